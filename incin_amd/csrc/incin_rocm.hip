@@ -925,7 +925,7 @@ int incin_rocm_lds_fill(int32_t dev, uint32_t pattern, void* sink, void* stream)
 size_t incin_rocm_sizeof_sdpa_bwd_desc(void) { return sizeof(incin_rocm_sdpa_bwd_desc_t); }
 
 // Validates a backward request; *empty is set when there is nothing to compute, *kind says which kernels take it:
-// 0 the generic ones, 1 the 16-bit matrix-core ones, 2 the IEEE-f32 matrix-core ones.
+// 0 the generic ones, 1 the 16-bit matrix-core ones, 2 the IEEE-f32 matrix-core ones, 3 the 16-bit ones above head dimension 128.
 static int check_bwd(const incin_rocm_sdpa_bwd_desc_t* bd, bool* empty, int* kind)
 {
     static const char* OP = "scaled_dot_product_attention backward";
@@ -948,7 +948,9 @@ static int check_bwd(const incin_rocm_sdpa_bwd_desc_t* bd, bool* empty, int* kin
     const bool f32 = d->dtype == INCIN_ROCM_F32;
     const int vec = f32 ? 4 : 8;
     // (head dimensions up to 128 in whole 16-byte vectors, D and Dv not necessarily equal: zero-padded into the 64 / 128 instances)
-    bool ok = d->D > 0 && d->D <= 128 && d->Dv <= 128 && d->D % vec == 0 && d->Dv % vec == 0 && std::isfinite(d->scale) && (f32 || d->scale > 0.0f);
+    // (16-bit storage without a dense mask: up to 256, in an instance for that)
+    const bool wide = d->D > 128 || d->Dv > 128;
+    bool ok = d->D > 0 && !(wide && (f32 || d->add_mask)) && d->D % vec == 0 && d->Dv % vec == 0 && std::isfinite(d->scale) && (f32 || wide || d->scale > 0.0f);
     ok = ok && fast_layout_ok(d, vec) && aligned16(bd->d_o) && aligned16(bd->d_q) && aligned16(bd->d_k) && aligned16(bd->d_v);
     for (int a = 0; a < 3; ++a)
         ok = ok && bd->d_o_stride[a] % vec == 0 && bd->d_q_stride[a] % vec == 0 && bd->d_k_stride[a] % vec == 0 && bd->d_v_stride[a] % vec == 0;
@@ -958,11 +960,11 @@ static int check_bwd(const incin_rocm_sdpa_bwd_desc_t* bd, bool* empty, int* kin
     if (d->add_mask)      // a tile's mask values are addressed with 32-bit byte offsets from the tile's first row
         ok = ok && d->mask_stride[2] >= 0 && d->mask_stride[3] >= 0 &&
              (64 * d->mask_stride[2] + (d->Skv > 0 ? d->Skv - 1 : 0) * d->mask_stride[3] + 1) * (f32 ? 4 : 2) < (int64_t)0x7fffffff;
-    const int fast = f32 ? 2 : 1;
+    const int fast = f32 ? 2 : wide ? 3 : 1;
     if (d->impl == INCIN_ROCM_IMPL_AUTO) *kind = ok ? fast : 0;
     else if (d->impl == INCIN_ROCM_IMPL_GENERIC) *kind = 0;
     else if (d->impl == INCIN_ROCM_IMPL_MFMA) {
-        if (!ok)
+        if (!ok || wide)      // (what MFMA names stops at 128; the kernels above that are AUTO's only)
             return fail(INCIN_ROCM_EUNSUPPORTED, "%s: the MFMA kernels need D and Dv <= 128 in whole 16-byte vectors, a finite scale (f16 / bf16: "
                         "positive), 64 rows of a dense mask within 2 GiB, and rows 16-byte aligned with strides that are multiples of 16 bytes below 2^%d elements",
                         OP, f32 ? 22 : 24);
@@ -998,9 +1000,25 @@ static size_t bwd_flags_bytes(const incin_rocm_sdpa_desc_t* d, int kind)
 // x 8192 0.72 (2 parts; 4: 0.85); 32 on 4 x 4096 0.80 (2); D = 64 8 on 1 x 8192 0.40; not worth it for short walks (8 heads x
 // 2048 keys without groups, 32 tiles per block: 1.19 in 2 parts) - a part keeps at least 64 tiles.  The kernel takes up to 8
 // parts, the rule stops at 4.
+// Head dimensions above 128 (kind 3): one launch holds the blocks of all three gradients (sdpa_bwd_wide.hip), a dK or dV block
+// walks every head of its group, and the launch ends with its longest item at the earliest: a walk is dealt to more workgroups
+// when it alone would take more than twice what a compute unit's share of the whole launch is.  Measured (bf16, D = 256, causal,
+// backward call, in 1 / 2 / 4 / 8 parts): 8 query heads on 1 KV head x 2048 positions 847 / 424 / 229 / 137 us, x 4096 1678 / 854 /
+// 483 / 405, 64 on 8 x 700 299 / 172 / 142 / 162; where a walk is not the longest thing in the launch the planes (written, read
+// and summed in f32) only cost: 2 x 16 on 8 x 1024 126 / 142 / 167 / 239, 8 x 16 x 512 159 / 292.
+static int bwd_wide_parts(const incin_rocm_sdpa_desc_t* d)
+{
+    const int64_t G = d->Hq / d->Hkv, nqb = (d->Sq + 127) / 128, nkb = (d->Skv + 127) / 128;
+    const int64_t walk = G * ((d->Sq + 31) / 32);            // tiles of the longest dK item, four products each; dV: three, dQ: four
+    int64_t all = d->B * d->Hkv * (nkb * walk * 7 + nqb * G * ((d->Skv + 31) / 32) * 4);
+    if (d->causal) all /= 2;
+    int parts = 1;
+    while (parts < 8 && walk * 4 > 2 * parts * (all / compute_units_of(d->device)) && walk >= 32 * parts) parts *= 2;
+    return parts;
+}
 static int bwd_parts(const incin_rocm_sdpa_desc_t* d, int kind, int which)
 {
-    if (kind == 0 || (kind == 1 && which == 0)) return 1;
+    if (kind == 0 || (kind != 2 && which == 0)) return 1;
     const char* forced = getenv("INCIN_ROCM_BWD_PARTS");      // (1, 2, 4 or 8 for every kernel that takes parts: a test knob)
     const int64_t blocks = which == 0 ? ((d->Sq + 127) / 128) * d->Hq * d->B : ((d->Skv + 127) / 128) * d->Hkv * d->B;
     const int64_t slots = (int64_t)(kind == 1 || d->D > 64 || d->Dv > 64 ? 1 : 2) * compute_units_of(d->device);
@@ -1008,10 +1026,11 @@ static int bwd_parts(const incin_rocm_sdpa_desc_t* d, int kind, int which)
     int parts = 1;
     const int f = forced ? atoi(forced) : 0;
     if (f == 1 || f == 2 || f == 4 || f == 8) {
-        parts = std::min(f, kind == 1 ? 8 : 4);
+        parts = std::min(f, kind != 2 ? 8 : 4);
         while (parts > 1 && walk < 4 * parts) parts >>= 1;
         return parts;
     }
+    if (kind == 3) return bwd_wide_parts(d);
     while (parts < 4 && 2 * parts * blocks <= slots) parts *= 2;
     // (f32: four tiles per part are enough to pay for the planes; 16-bit storage, whose tiles take an eighth of the time: 64)
     while (parts > 1 && walk < (kind == 1 ? 64 : 4) * parts) parts >>= 1;
@@ -1034,7 +1053,7 @@ static size_t bwd_planes_bytes(const incin_rocm_sdpa_desc_t* d, int kind, int pa
     const size_t k = round256((size_t)(d->B * d->Hkv * d->Skv * d->D) * sizeof(float));
     const size_t v = round256((size_t)(d->B * d->Hkv * d->Skv * d->Dv) * sizeof(float));
     // (f32: part 0 writes the gradient itself; 16-bit storage: every part of a divided walk writes a plane)
-    const int planes_kv = kind == 1 ? (parts_kv > 1 ? parts_kv : 0) : parts_kv - 1;
+    const int planes_kv = kind != 2 ? (parts_kv > 1 ? parts_kv : 0) : parts_kv - 1;
     return (size_t)(parts_q - 1) * q + (size_t)planes_kv * (k + v);
 }
 
@@ -1104,7 +1123,7 @@ int incin_rocm_sdpa_bwd(const incin_rocm_sdpa_bwd_desc_t* bd, void* stream)
         bp.part_dq = (float*)at;
         at += (size_t)(parts_q - 1) * round256((size_t)(d->B * d->Hq * d->Sq * d->D) * sizeof(float));
         bp.part_dk = (float*)at;
-        at += (size_t)(kind == 1 ? parts_kv : parts_kv - 1) * round256((size_t)(d->B * d->Hkv * d->Skv * d->D) * sizeof(float));
+        at += (size_t)(kind != 2 ? parts_kv : parts_kv - 1) * round256((size_t)(d->B * d->Hkv * d->Skv * d->D) * sizeof(float));
         bp.part_dv = (float*)at;
     }
     if (flag_bytes) {
@@ -1116,6 +1135,7 @@ int incin_rocm_sdpa_bwd(const incin_rocm_sdpa_bwd_desc_t* bd, void* stream)
     }
     hipError_t e = kind == 2   ? incin_rocm::launch_sdpa_bwd_f32(bp, (hipStream_t)stream)
                    : kind == 1 ? incin_rocm::launch_sdpa_bwd_mfma(bp, bd->fwd.dtype, (hipStream_t)stream)
+                   : kind == 3 ? incin_rocm::launch_sdpa_bwd_wide(bp, bd->fwd.dtype, (hipStream_t)stream)
                                : incin_rocm::launch_sdpa_bwd_generic(bp, bd->fwd.dtype, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "attention backward launch");
     return 0;

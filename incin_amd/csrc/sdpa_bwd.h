@@ -30,6 +30,10 @@ struct SdpaBwdParams {
 };
 
 hipError_t launch_sdpa_bwd_mfma(const SdpaBwdParams& bp, int dtype, hipStream_t stream);
+hipError_t launch_sdpa_bwd_wide(const SdpaBwdParams& bp, int dtype, hipStream_t stream);
+// (of sdpa_bwd_mfma.hip: the row dots, and the sum of the planes of a call with parts_kv > 1 into dK and dV)
+hipError_t launch_sdpa_bwd_delta(const SdpaBwdParams& bp, int dtype, hipStream_t stream);
+hipError_t launch_sdpa_bwd_sum_planes(const SdpaBwdParams& bp, int dtype, hipStream_t stream);
 hipError_t launch_sdpa_bwd_f32(const SdpaBwdParams& bp, hipStream_t stream);
 hipError_t launch_sdpa_bwd_generic(const SdpaBwdParams& bp, int dtype, hipStream_t stream);
 

@@ -1,6 +1,7 @@
 // Generic attention backward: fp32 FMA arithmetic, any of f32/f16/bf16 storage, D and Dv up to DMAX, dense additive
-// mask + causal + per-batch key lengths.  The kernel every backward request can fall back on (the reference's own
-// dtype, f32, comes through here); the MFMA kernels of sdpa_bwd_mfma.hip cover f16/bf16 at D = 128.
+// mask + causal + per-batch key lengths.  The kernel every backward request can fall back on;
+// the matrix-core kernels (sdpa_bwd_mfma.hip, sdpa_bwd_wide.hip, sdpa_bwd_f32.hip) leave it rows that are not whole
+// 16-byte vectors, f32 above head dimension 128 and dense masks there.
 //
 // The gradients are those of the reference's taped composition (crates/incin-backends/src/cpu/ops/shape_ops.rs:1245-1269
 // walked by cpu/tape.rs:149-176; matmul rule cpu/ops/matmul.rs:264-281, log-softmax chain cpu/ops/elementwise.rs:1062-1077):

@@ -925,6 +925,29 @@ __global__ __launch_bounds__(256) void sdpa_bwd_sum_planes_kernel(SumPlanesJob<T
     *(vec4*)(j.dst + b * j.sb + h * j.sh + (int64_t)s * j.ss + c) = w;
 }
 
+template <typename T>
+static void sum_planes(const SdpaBwdParams& bp, hipStream_t stream)
+{
+    const SdpaParams& p = bp.f;
+    const SumPlanesJob<T> jk = {(T*)bp.d_k, bp.part_dk, bp.dk_sb, bp.dk_sh, bp.dk_ss, p.B, p.Hkv, p.Skv, p.D};
+    const SumPlanesJob<T> jv = {(T*)bp.d_v, bp.part_dv, bp.dv_sb, bp.dv_sh, bp.dv_ss, p.B, p.Hkv, p.Skv, p.Dv};
+    const int64_t n4 = (int64_t)p.B * p.Hkv * p.Skv * (max(p.D, p.Dv) >> 2);
+    hipLaunchKernelGGL((sdpa_bwd_sum_planes_kernel<T>), dim3((unsigned)((n4 + 255) / 256), 2), dim3(256), 0, stream, jk, jv, bp.parts_kv);
+}
+hipError_t launch_sdpa_bwd_sum_planes(const SdpaBwdParams& bp, int dtype, hipStream_t stream)
+{
+    if (dtype == 1) sum_planes<f16_t>(bp, stream);
+    else sum_planes<bf16_t>(bp, stream);
+    return hipGetLastError();
+}
+hipError_t launch_sdpa_bwd_delta(const SdpaBwdParams& bp, int dtype, hipStream_t stream)
+{
+    const int64_t rows = (int64_t)bp.f.B * bp.f.Hq * bp.f.Sq;
+    if (dtype == 1) hipLaunchKernelGGL((sdpa_bwd_delta_kernel<f16_t>), dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, stream, bp);
+    else hipLaunchKernelGGL((sdpa_bwd_delta_kernel<bf16_t>), dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, stream, bp);
+    return hipGetLastError();
+}
+
 // The dQ kernel goes to a side stream where one is to be had (side_stream.h) - it and the dK/dV kernel read the same inputs
 // and the row dots, and write different outputs - when the call is short of work: at most two rounds of dQ workgroups (two
 // per compute unit at a time), or D = 64.  Measured, whole call, forked against one stream (bf16, causal): 8 heads x 1024
@@ -951,12 +974,7 @@ static hipError_t launch_bwd_t(const SdpaBwdParams& bp, hipStream_t stream)
         const dim3 grid((unsigned)((int64_t)nkb * p.Hkv * p.B), parts);
         if (DENSE && p.mask_chunks) hipLaunchKernelGGL((sdpa_bwd_dkv_kernel<T, D, DENSE ? 2 : 0>), grid, dim3(512), 0, stream, bp);
         else hipLaunchKernelGGL((sdpa_bwd_dkv_kernel<T, D, DENSE ? 1 : 0>), grid, dim3(512), 0, stream, bp);
-        if (parts > 1) {
-            const SumPlanesJob<T> jk = {(T*)bp.d_k, bp.part_dk, bp.dk_sb, bp.dk_sh, bp.dk_ss, p.B, p.Hkv, p.Skv, p.D};
-            const SumPlanesJob<T> jv = {(T*)bp.d_v, bp.part_dv, bp.dv_sb, bp.dv_sh, bp.dv_ss, p.B, p.Hkv, p.Skv, p.Dv};
-            const int64_t n4 = (int64_t)p.B * p.Hkv * p.Skv * (max(p.D, p.Dv) >> 2);
-            hipLaunchKernelGGL((sdpa_bwd_sum_planes_kernel<T>), dim3((unsigned)((n4 + 255) / 256), 2), dim3(256), 0, stream, jk, jv, (int)parts);
-        }
+        if (parts > 1) sum_planes<T>(bp, stream);
     }
     if (rows > 0) {
         hipStream_t sq = forked ? side.stream() : stream;

@@ -253,13 +253,14 @@ int incin_rocm_sdpa_fwd_static(const incin_rocm_sdpa_desc_t* desc, void* stream)
  * Covered: f32 / f16 / bf16, D and Dv up to 256, dense additive mask, causal, kv_lens, q_lens (padding query rows: their
  * O, lse and d_o rows are never read, their d_q rows are written as zero and they add nothing to d_k and d_v).
  * fwd.impl picks the kernels: AUTO = matrix-core kernels where they apply - D and Dv up to 128 in whole 16-byte vectors (zero-padded
- * into instances for 64 and 128); f16 / bf16 with a positive scale, f32 (IEEE single-precision matrix instructions) with any finite
+ * into instances for 64 and 128; f16 / bf16 without a dense mask: up to 256); f16 / bf16 with a positive scale (above 128: any finite
+ * scale), f32 (IEEE single-precision matrix instructions) with any finite
  * scale; both with 16-byte aligned rows, and a dense mask of non-negative strides of which 64 rows fit 32-bit byte offsets
- * - and generic f32-arithmetic kernels otherwise; GENERIC and MFMA pin one or the other.  A query row with no visible key (NaN in the forward) gets a zero gradient and
+ * - and generic f32-arithmetic kernels otherwise; GENERIC and MFMA (up to 128) pin one or the other.  A query row with no visible key (NaN in the forward) gets a zero gradient and
  * contributes nothing to d_k and d_v, where the reference's tape would spread NaN over the whole head.
  * The workspace holds two floats per query row (2 x [B, Hq, Sq]) and, for a dense mask on the matrix-core kernels, a byte
  * per 32 rows x 32 keys of the mask behind them, and for a call on the matrix-core kernels that does not fill the device
- * (f32; 16-bit storage with few KV heads) up to four f32 copies of the gradients' shapes, which workgroups that share a block
+ * (f32; 16-bit storage with few KV heads) up to four (16-bit above head dimension 128: eight) f32 copies of the gradients' shapes, which workgroups that share a block
  * of rows or keys sum into (ask incin_rocm_sdpa_bwd_workspace for the size: it depends on the device's compute-unit count);
  * d_q, d_k, d_v are fully overwritten.
  * Streams: everything the call launches is ordered behind the work already on `stream` and ahead of whatever `stream` gets

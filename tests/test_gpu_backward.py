@@ -629,3 +629,50 @@ def test_backward_of_a_padded_batch(gpu, case):
         compare("dk[%d]" % b, dk[b:b + 1, :, :n], rk.reshape(1, Hkv, n, D), tol)
         compare("dv[%d]" % b, dv[b:b + 1, :, :n], rv.reshape(1, Hkv, n, D), tol)
         assert not dq[b, :, n:].any() and not dk[b, :, n:].any() and not dv[b, :, n:].any()
+
+
+@pytest.mark.parametrize("parts", ["1", "4"])
+@pytest.mark.parametrize("dtype", [capi.BF16, capi.F16], ids=lambda x: dtypes.NAMES[x])
+@pytest.mark.parametrize("shape", [
+    # B, Hq, Hkv, Sq, Skv, D, Dv, causal, kv_lens, q_lens, scale
+    (1, 1, 1, 1, 1, 256, 256, True, None, None, None),                      # one query, one key
+    (1, 2, 1, 33, 31, 136, 144, False, None, None, None),                   # a row past and a row short of a tile; the narrowest heads
+    (2, 4, 2, 127, 129, 256, 256, True, None, None, None),                  # a row short of and a row past a block
+    (1, 2, 2, 161, 97, 192, 128, True, None, None, None),                   # more queries than keys: rows that see none; D != Dv
+    (3, 4, 1, 300, 420, 160, 256, True, [420, 131, 0], None, None),         # key counts, one sequence without keys
+    (2, 2, 2, 300, 300, 256, 192, True, [300, 70], [300, 70], None),        # a padded batch
+    (1, 8, 2, 260, 520, 256, 256, False, None, None, -0.05),                # a negative scale
+    (1, 2, 1, 1057, 1057, 256, 256, True, None, None, None),                # many tiles: every stage of the ring, four parts by themselves
+], ids=["one", "narrow", "block_edges", "rect", "ragged", "padded", "negative_scale", "long"])
+def test_matrix_core_backward_above_128(gpu, monkeypatch, parts, dtype, shape):
+    """Head dimensions above 128 on the matrix cores, with the walks of the dK and dV blocks whole and dealt to four workgroups.  P
+    and dS enter their products as two 16-bit values, so what is left is the rounding of the results (half a step of the storage
+    type, 2^-9 and 2^-12, of values up to the largest) and of the forward's O and normalisers: 4 times that half step of the largest magnitude."""
+    B, Hq, Hkv, Sq, Skv, D, Dv, causal, lens, qlens, scale = shape
+    G = Hq // Hkv
+    monkeypatch.setenv("INCIN_ROCM_BWD_PARTS", parts)
+    say("matrix-core backward above 128, %s in %s parts: %s" % (dtypes.NAMES[dtype], parts, shape))
+    q, k, v, go = make_d(131 + Sq, B, Hq, Hkv, Sq, Skv, D, Dv, dtype)
+    lens_a = None if lens is None else np.asarray(lens, np.int32)
+    qlens_a = None if qlens is None else np.asarray(qlens, np.int32)
+    out, dq, dk, dv = host.sdpa_backward(q, k, v, go, dtype, impl=capi.IMPL_AUTO, causal=causal, kv_lens=lens_a, q_lens=qlens_a, scale=scale,
+                                         poison_padding=qlens is not None)
+    tol = 2.0 ** -7 if dtype == capi.BF16 else 2.0 ** -10
+    for b in range(B):
+        nq = Sq if qlens is None else int(qlens[b])
+        nk = Skv if lens is None else int(lens[b])
+        if nk > 0:
+            tri = np.triu(np.full((Sq, Skv), -np.inf, np.float32), 1 + Skv - Sq)[:nq, :nk].reshape(1, 1, 1, nq, nk) if causal else None
+            rows = np.isfinite(tri).any(axis=-1).reshape(nq) if causal else np.ones(nq, bool)      # (rows that see a key: the others have zero gradients here)
+            sel = lambda x: x[b:b + 1, :, :nq][:, :, rows]
+            tri = None if tri is None else tri[:, :, :, rows]
+            n = int(rows.sum())
+            rq, rk, rv = BW.sdpa_backward(sel(q).reshape(1, Hkv, G, n, D), k[b:b + 1, :, None, :nk], v[b:b + 1, :, None, :nk],
+                                          sel(go).reshape(1, Hkv, G, n, Dv), mask=tri, scale=scale)
+            compare("dq[%d]" % b, sel(dq), rq.reshape(1, Hq, n, D), tol=tol)
+            compare("dk[%d]" % b, dk[b:b + 1, :, :nk], rk.reshape(1, Hkv, nk, D), tol=tol)
+            compare("dv[%d]" % b, dv[b:b + 1, :, :nk], rv.reshape(1, Hkv, nk, Dv), tol=tol)
+            assert not dq[b, :, :nq][:, ~rows].any()
+        else:
+            assert not dq[b].any()
+        assert not dq[b, :, nq:].any() and not dk[b, :, nk:].any() and not dv[b, :, nk:].any()
