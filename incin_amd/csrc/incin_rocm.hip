@@ -984,22 +984,40 @@ static size_t bwd_flags_bytes(const incin_rocm_sdpa_desc_t* d, int kind)
     return (size_t)(nbh * ((d->Sq + 31) / 32) * ((d->Skv + 31) / 32) + 255) / 256 * 256;
 }
 
-// Matrix-core kernels: into how many workgroups the key tiles of a block of 128 rows (dQ kernel, which = 0) or the query
-// tiles of a block of 128 keys (dK/dV kernel, which = 1) are dealt.  A launch of half a round of workgroups or less leaves
-// most of the device idle - under a causal mask every SIMD has one wavefront and all wait for the one with the longest
-// walk - so its tiles go to 2 workgroups (up to half a round) or 4 (up to a quarter), each with at least four tiles of 64 to
-// walk; the sums meet in planes of the workspace and a pass adds them (sdpa_bwd.h).
-// f32 (kind 2), both kernels.  Measured, whole call, against one workgroup per block (causal, with the dQ kernel on its side
-// stream either way): 8 heads x 1024 keys 0.36 (D = 64, 4 parts) / 0.56 (128); 32 heads x 1024 0.86 (D = 64, 2 parts: config
-// 2's shape) and 0.99 at D = 128 (a full round: not split); 16 query heads on 4 KV heads x 2048 0.38 / 0.41; from a full round
-// on 1.0 - 1.13: not split.
-// 16-bit storage (kind 1), the dK/dV kernel only - a workgroup of it fills a compute unit, a round is one per compute unit,
-// and with grouped queries a key block walks every head of its group: few KV heads on a device (a model's KV heads
-// divided over devices) leave most compute units without a block.  Measured, whole call, bf16 causal D = 128: 8 query heads on
-// 1 KV head x 8192 keys 1.66 -> 0.73 ms (4 parts; 2: 0.54 of the time, 8: 0.46), x 4096 0.84 -> 0.25 (8 parts: 0.28); 16 on 2
-// x 8192 0.72 (2 parts; 4: 0.85); 32 on 4 x 4096 0.80 (2); D = 64 8 on 1 x 8192 0.40; not worth it for short walks (8 heads x
-// 2048 keys without groups, 32 tiles per block: 1.19 in 2 parts) - a part keeps at least 64 tiles.  The kernel takes up to 8
-// parts, the rule stops at 4.
+// 16-bit storage (kind 1), the dK/dV kernel only: with grouped queries a key block walks every head of its group, and few KV
+// heads on a device (a model's KV heads divided over devices) leave most compute units without a block.
+// The paired kernel (bwd16_narrow says which) fills a compute unit with a workgroup: 2 parts up to half a round of blocks, 4 up to a
+// quarter, 16 tiles per part at least.  Measured, whole call, bf16 causal D = 128: 8 query heads on 1 KV head x 8192 keys 1.66 ->
+// 0.73 ms (4 parts; 2: 0.54 of the time, 8: 0.46), 16 on 2 x 8192 0.72 (2 parts; 4: 0.85), 32 on 8 x 1024 120 -> 79 us (4 parts).
+// One query head per KV head: half as many - the dQ launch is as small then and takes the compute units that are left (1 head x 16384:
+// 404 us undivided, 483 in 2 parts; without a mask 444 / 743) - of 64 tiles.
+// Up to a full round of key blocks with very long walks (8 query heads on 1 KV head x 32768 keys: 256 blocks of up to 4096
+// tiles): under a causal mask the longest walk is twice the average and the round ends with it - four parts make four rounds
+// of shorter items (10.2 -> 7.3 ms there; 16 heads on 2 x 16384, 2048 tiles: 0.84; at 512 tiles 1.05).
+// ... and two parts already from 256 tiles on when the dQ kernel is too large to run beside this one (bwd16_forks).  One sequence of
+// 4096 tokens, D = 128: 64 query heads on 8 KV heads 1.28 -> 1.01 ms, 128 on 8 2.62 -> 1.91, 48 on 8 0.97 -> 0.79, 2 x 32 on 4 1.29 ->
+// 1.02; with the dQ kernel beside it (2 x 8 on 2 x 8192) two parts cost 19 %.
+// The other kernel runs three workgroups per compute unit: walks are dealt until there are two per compute unit, 16 tiles per
+// part at least, and with grouped queries until there are three if a part keeps 64.  Bf16 causal D = 64, in 1 / 2 / 4 / 8 parts, us:
+// 32 on 8 x 1024 89 / 62 / 55 / 55, 16 on 2 x 4096 576 / 314 / 192 / 178, 8 on 1 x 8192 1129 / 600 / 353 / 301, 64 on 8 x 4096 682 / 547 /
+// 466 / 489, 8 x 8192 278 / 283 / 276 / 305.
+static int bwd16_parts(const incin_rocm_sdpa_desc_t* d, int64_t blocks, int64_t walk)
+{
+    const int64_t cus = compute_units_of(d->device), G = d->Hq / d->Hkv;
+    int parts = 1;
+    if (incin_rocm::bwd16_narrow(d->D, d->Dv, d->add_mask != nullptr, G, blocks, walk, cus)) {
+        while (parts < 8 && ((parts * blocks < 2 * cus && walk >= 32 * parts) || (G > 1 && parts * blocks < 3 * cus && walk >= 128 * parts))) parts *= 2;
+        return parts;
+    }
+    const bool uneven = d->causal || d->add_mask;
+    while (parts < 4 && (G > 1 ? 2 : 4) * parts * blocks <= cus) parts *= 2;
+    while (parts > 1 && walk < (G > 1 ? 16 : 64) * parts) parts >>= 1;
+    if (parts == 1 && G > 1 && blocks <= cus && uneven) {
+        if (walk >= 2048) parts = 4;
+        else if (walk >= 256 && ((d->Sq + 127) / 128) * d->Hq * d->B > 4 * cus) parts = 2;
+    }
+    return parts;
+}
 // Head dimensions above 128 (kind 3): one launch holds the blocks of all three gradients (sdpa_bwd_wide.hip), a dK or dV block
 // walks every head of its group, and the launch ends with its longest item at the earliest: a walk is dealt to more workgroups
 // when it alone would take more than twice what a compute unit's share of the whole launch is.  Measured (bf16, D = 256, causal,
@@ -1016,12 +1034,21 @@ static int bwd_wide_parts(const incin_rocm_sdpa_desc_t* d)
     while (parts < 8 && walk * 4 > 2 * parts * (all / compute_units_of(d->device)) && walk >= 32 * parts) parts *= 2;
     return parts;
 }
+// Matrix-core kernels: into how many workgroups the key tiles of a block of 128 rows (dQ kernel, which = 0) or the query
+// tiles of a block of 128 keys (dK/dV kernel, which = 1) are dealt.  A launch of half a round of workgroups or less leaves
+// most of the device idle - under a causal mask every SIMD has one wavefront and all wait for the one with the longest
+// walk - so its tiles go to 2 workgroups (up to half a round) or 4 (up to a quarter), each with at least four tiles of 64 to
+// walk; the sums meet in planes of the workspace and a pass adds them (sdpa_bwd.h).
+// f32 (kind 2), both kernels.  Measured, whole call, against one workgroup per block (causal, with the dQ kernel on its side
+// stream either way): 8 heads x 1024 keys 0.36 (D = 64, 4 parts) / 0.56 (128); 32 heads x 1024 0.86 (D = 64, 2 parts: config
+// 2's shape) and 0.99 at D = 128 (a full round: not split); 16 query heads on 4 KV heads x 2048 0.38 / 0.41; from a full round
+// on 1.0 - 1.13: not split.
 static int bwd_parts(const incin_rocm_sdpa_desc_t* d, int kind, int which)
 {
     if (kind == 0 || (kind != 2 && which == 0)) return 1;
     const char* forced = getenv("INCIN_ROCM_BWD_PARTS");      // (1, 2, 4 or 8 for every kernel that takes parts: a test knob)
     const int64_t blocks = which == 0 ? ((d->Sq + 127) / 128) * d->Hq * d->B : ((d->Skv + 127) / 128) * d->Hkv * d->B;
-    const int64_t slots = (int64_t)(kind == 1 || d->D > 64 || d->Dv > 64 ? 1 : 2) * compute_units_of(d->device);
+    const int64_t slots = (int64_t)(d->D > 64 || d->Dv > 64 ? 1 : 2) * compute_units_of(d->device);
     const int64_t walk = (which == 0 ? d->Skv : d->Sq * (d->Hq / d->Hkv)) / 64;
     int parts = 1;
     const int f = forced ? atoi(forced) : 0;
@@ -1031,19 +1058,9 @@ static int bwd_parts(const incin_rocm_sdpa_desc_t* d, int kind, int which)
         return parts;
     }
     if (kind == 3) return bwd_wide_parts(d);
+    if (kind == 1) return bwd16_parts(d, blocks, walk);
     while (parts < 4 && 2 * parts * blocks <= slots) parts *= 2;
-    // (f32: four tiles per part are enough to pay for the planes; 16-bit storage, whose tiles take an eighth of the time: 64)
-    while (parts > 1 && walk < (kind == 1 ? 64 : 4) * parts) parts >>= 1;
-    // 16-bit storage, up to a full round of key blocks with very long walks (8 query heads on 1 KV head x 32768 keys: 256 blocks
-    // of up to 4096 tiles): under a causal mask the longest walk is twice the average and the round ends with it - four parts
-    // make four rounds of shorter items (10.2 -> 7.3 ms there; 16 heads on 2 x 16384, 2048 tiles: 0.84; at 512 tiles 1.05)
-    if (kind == 1 && parts == 1 && blocks <= slots && walk >= 2048 && (d->causal || d->add_mask)) parts = 4;
-    // ... and two parts already from 256 tiles on when the dQ kernel is not running beside this one to fill the compute units the
-    // short walks leave idle (the launcher's rule: D = 64, or at most four dQ blocks per compute unit).  One sequence of 4096
-    // tokens, D = 128: 64 query heads on 8 KV heads 1.28 -> 1.01 ms, 128 on 8 2.62 -> 1.91, 48 on 8 0.97 -> 0.79, 2 x 32 on 4 1.29 ->
-    // 1.02; with the dQ kernel beside it (2 x 8 on 2 x 8192) two parts cost 19 %.
-    const bool dq_beside = (d->D <= 64 && d->Dv <= 64) || ((d->Sq + 127) / 128) * d->Hq * d->B <= 4 * (int64_t)compute_units_of(d->device);
-    if (kind == 1 && parts == 1 && blocks <= slots && walk >= 256 && !dq_beside && (d->causal || d->add_mask)) parts = 2;
+    while (parts > 1 && walk < 4 * parts) parts >>= 1;      // (four tiles per part are enough to pay for the planes)
     return parts;
 }
 static size_t round256(size_t n) { return (n + 255) / 256 * 256; }

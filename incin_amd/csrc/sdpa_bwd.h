@@ -14,6 +14,7 @@ struct SdpaBwdParams {
     void* d_v;
     float* neg_l2;                 // workspace, [B, Hq, Sq]: -L_i log2(e) (the normalisers, negated, in log2 units)
     float* neg_delta;              // workspace, [B, Hq, Sq]: -D_i = -(dO_i . O_i)
+    int32_t dots_in_dq;            // 16-bit matrix-core kernels up to 128: the dQ kernel computes the two rows above (it runs first), else a kernel of its own
     int64_t do_sb, do_sh, do_ss;
     int64_t dq_sb, dq_sh, dq_ss;
     int64_t dk_sb, dk_sh, dk_ss;
@@ -28,6 +29,36 @@ struct SdpaBwdParams {
     float* part_dk;                // workspace, f32: [parts_kv - 1][B, Hkv, Skv, D]; 16-bit storage: [parts_kv][...]
     float* part_dv;                // workspace, likewise [..][B, Hkv, Skv, Dv]
 };
+
+// 16-bit storage up to head dimension 128, the rules that the planner of the workspace and the launcher share.
+//   blocks: 128-key blocks of all (batch, KV head) pairs; walk: 64-row query tiles of a block's walk over its group's heads.
+//
+// Which dK/dV kernel.  Head dimensions up to 64 without a mask tensor: the kernel with one wavefront per 32 keys (the other
+// pairs them) wherever there is more than one workgroup per compute unit to cover its latencies or the walks can be dealt to
+// more: 8 x 32 heads x 4096, causal, whole call 2.32 -> 1.80 ms, 32 x 12 x 512 144 -> 96 us.  A launch of one query head per KV head
+// that gives it less than a workgroup per compute unit, for walks of some length, keeps the paired kernel, whose eight
+// wavefronts per 128 keys are twice as many (8 heads x 2048 62 us against 70, 4 x 4096 94 against 106; at 16 tiles 48 against 44).
+inline bool bwd16_narrow(int64_t D, int64_t Dv, bool mask, int64_t G, int64_t blocks, int64_t walk, int64_t cus)
+{
+    return D <= 64 && Dv <= 64 && !mask && (G > 1 || blocks >= cus || walk < 32);
+}
+// Whether the dQ kernel runs on a stream of its own beside the dK/dV kernel.  The fork and the join cost 5 - 7 us, and the call a
+// kernel for the row dots, which the dQ kernel computes where it runs first (8 x 16 heads x 256, D = 64: 40 us forked, 21 in
+// order; 4 x 16 x 512, D = 128: 69 and 47).  It pays where the dK/dV kernel leaves compute units idle for long enough:
+//   paired kernel (one workgroup fills a compute unit): at most half the compute units (8 x 2048, D = 128: 78 forked, 111 in
+//   order; 16 x 1024 57 / 67; from 12 tiles of walk on: 12 x 768 48 / 55, 8 x 512 44 / 42); under a causal mask, whose blocks end
+//   at different times, up to two rounds of workgroups with walks of 32 tiles (64 when they are dealt) if the dQ launch is at
+//   most two rounds too (8 x 8192 457 / 488, 2 x 32 / 8 x 2048 268 / 309, 16 / 4 x 2048 in 4 parts 145 / 126, 64 / 8 x 4096 975 / 891;
+//   without a mask 8 x 8192 942 / 823);
+//   the other: walks of 32 tiles under a causal mask or with grouped queries (8 x 8192, causal 278 / 305, 64 / 8 x 4096 466 / 518,
+//   4 x 32 / 8 x 4096 894 / 986; 32 x 12 x 512 118 / 103; without either 2 x 16 x 2048 135 / 121).
+inline bool bwd16_forks(bool narrow, bool causal, int64_t G, int64_t blocks, int64_t parts, int64_t walk, int64_t dq_blocks, int64_t cus)
+{
+    const int64_t w = walk / parts;
+    if (narrow) return w >= 32 && (causal || G > 1);
+    if (2 * parts * blocks <= cus && w >= 12) return true;
+    return causal && parts * blocks <= 2 * cus && dq_blocks <= 4 * cus && w >= (parts > 1 ? 64 : 32);
+}
 
 hipError_t launch_sdpa_bwd_mfma(const SdpaBwdParams& bp, int dtype, hipStream_t stream);
 hipError_t launch_sdpa_bwd_wide(const SdpaBwdParams& bp, int dtype, hipStream_t stream);

@@ -25,13 +25,13 @@
 namespace incin_rocm {
 
 // ---- D_i = dO_i . O_i ---------------------------------------------------------------------------------------------
-// Sixteen lanes per row (16 bytes of O and of dO each), four rows per wavefront.
-template <typename T>
+// LPR lanes per row (16 bytes of O and of dO each): sixteen, or eight when a row is no longer than that.
+template <typename T, int LPR>
 __global__ __launch_bounds__(256) void sdpa_bwd_delta_kernel(SdpaBwdParams p)
 {
     typedef typename Mma<T>::vec8 vec8;
-    const int lane = threadIdx.x & 63, sub = lane & 15;
-    const int64_t row = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 4 + (lane >> 4);     // (b * Hq + hq) * Sq + i
+    const int lane = threadIdx.x & 63, sub = lane & (LPR - 1);
+    const int64_t row = (int64_t)blockIdx.x * (256 / LPR) + threadIdx.x / LPR;     // (b * Hq + hq) * Sq + i
     const int64_t rows = (int64_t)p.f.B * p.f.Hq * p.f.Sq;
     float acc = 0.0f;
     if (row < rows) {
@@ -40,14 +40,14 @@ __global__ __launch_bounds__(256) void sdpa_bwd_delta_kernel(SdpaBwdParams p)
         const int hq = (int)(bh % p.f.Hq), b = (int)(bh / p.f.Hq);
         const T* o = (const T*)p.f.o + b * p.f.o_sb + hq * p.f.o_sh + (int64_t)i * p.f.o_ss;
         const T* g = (const T*)p.d_o + b * p.do_sb + hq * p.do_sh + (int64_t)i * p.do_ss;
-        for (int d = sub * 8; d < p.f.Dv; d += 128) {
+        for (int d = sub * 8; d < p.f.Dv; d += 8 * LPR) {
             const vec8 x = *(const vec8*)(o + d), y = *(const vec8*)(g + d);
 #pragma unroll
             for (int e = 0; e < 8; ++e) acc = fmaf((float)x[e], (float)y[e], acc);
         }
     }
 #pragma unroll
-    for (int off = 8; off >= 1; off >>= 1) acc += __shfl_xor(acc, off, 64);
+    for (int off = LPR / 2; off >= 1; off >>= 1) acc += __shfl_xor(acc, off, 64);
     if (row < rows && sub == 0) {
         // A row without a visible key (L_i = -inf, O and so D_i NaN) gets -inf and 0: its P is then 0 everywhere.
         const float l = p.f.lse[row];
@@ -224,6 +224,8 @@ void sdpa_bwd_dq_kernel(SdpaBwdParams bp)
     // wavefront's 4 KiB of the V buffers (fetch_q_rows / stage_q_rows), which nothing is copied into before the barrier below.
     vec8 qreg[NSTEP], greg[NSTEP];
     const int qi = min(my_i, Sq - 1);
+    const int64_t stat = ((int64_t)b * p.Hq + hq) * Sq + qi;
+    float l2, dlt;      // L_i log2(e) and D_i of the lane's query
     const unsigned lds0 = lds_address(smem);
     if (t_first < n_tiles) tl.issue(0, kp, p.k_ss, Skv, t_first * PF_BN, lds0 + (t_first & 1) * L::TILE_BYTES, wave);
     {
@@ -239,14 +241,44 @@ void sdpa_bwd_dq_kernel(SdpaBwdParams bp)
         for (int s = 0; s < NSTEP; ++s)
 #pragma unroll
             for (int e = 0; e < 8; ++e) qreg[s][e] = (T)((float)qreg[s][e] * c2);
+        if (bp.dots_in_dq) {
+            // dO . O of the wavefront's rows as the two tensors' rows are fetched: 16 bytes of each per lane, then the sum over a row's
+            // eight lanes (in the order of sdpa_bwd_delta_kernel, to the bit), then through LDS to the lanes that own the rows
+            const T* op = (const T*)p.o + (int64_t)b * p.o_sb + (int64_t)hq * p.o_sh;
+            uint4v oraw[NSTEP / 4][4];
+            fetch_q_rows(oraw, op, q0 + wave * 32, Sq, p.o_ss, p.Dv, lane);
+#pragma unroll
+            for (int ps = 0; ps < 4; ++ps) {
+                float dot = 0.0f;
+#pragma unroll
+                for (int h = 0; h < NSTEP / 4; ++h) {
+                    const vec8 x = __builtin_bit_cast(vec8, oraw[h][ps]), y = __builtin_bit_cast(vec8, graw[h][ps]);
+                    float part = 0.0f;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) part = fmaf((float)x[e], (float)y[e], part);
+                    dot = h == 0 ? part : dot + part;
+                }
+#pragma unroll
+                for (int off = 4; off >= 1; off >>= 1) dot += __shfl_xor(dot, off, 64);
+                if ((lane & 7) == 0) ((float*)stage)[ps * 8 + (lane >> 3)] = dot;
+            }
+            const float l = p.lse[stat];
+            l2 = l == -INFINITY ? INFINITY : l * 1.4426950408889634f;
+            dlt = l == -INFINITY ? 0.0f : ((const float*)stage)[ql];
+            if (g == 0 && my_i < Sq) {
+                bp.neg_l2[stat] = -l2;
+                bp.neg_delta[stat] = -dlt;
+            }
+        }
+    }
+    if (!bp.dots_in_dq) {
+        l2 = -bp.neg_l2[stat];
+        dlt = -bp.neg_delta[stat];
     }
     __syncthreads();      // every wavefront has its rows out of the V buffers
     if (t_first < n_tiles) tl.issue(1, vp, p.v_ss, Skv, t_first * PF_BN, lds0 + (2 + (t_first & 1)) * L::TILE_BYTES, wave);
-    const int64_t stat = ((int64_t)b * p.Hq + hq) * Sq + qi;
     [[maybe_unused]] const T* mrow = nullptr;      // DENSE: this lane's row of the mask
     if (DENSE) mrow = (const T*)p.mask + (int64_t)b * p.m_sb + (int64_t)hq * p.m_sh + (int64_t)qi * p.m_si;
-    const float l2 = -bp.neg_l2[stat];
-    const float dlt = -bp.neg_delta[stat];
 
     floatx16 dq_acc[NDB];
 #pragma unroll
@@ -428,7 +460,9 @@ constexpr int BWD_RING = 4;        // matrix operands in flight from LDS (reads 
 // computes S, dP of tile t, then dV, dK of tile t - 1 with the exponentials and products that make P, dS of tile t
 // issued between those matrix instructions (the workgroup's barriers keep the two wavefronts of a SIMD in the same
 // phase, so what overlaps a wavefront's matrix instructions has to come from its own stream), and writes P, dS of tile
-// t after a barrier.  Tiles t - 1 and t stay resident while tile t + 1 is copied: three stages.  The S and dP
+// t after a barrier.  (The order is asked of the compiler by name - values pinned in place, scheduling barriers, the first tile's step
+// a copy of its own: left to itself it gathers the exponentials on one side of the matrix instructions.  With that and the second
+// half's first operands asked for at the end of the first: 8 x 16 heads x 4096 2.00 -> 1.955 ms per call, 4 x 32 / 8 x 2048 617 -> 593 us.)  Tiles t - 1 and t stay resident while tile t + 1 is copied: three stages.  The S and dP
 // accumulators do not start from zero but from -L_i log2(e) and -D_i (staged per tile next to the Q and dO rows), so
 // P = exp2(S) and dS = P * dP need no subtraction.
 // DENSE: a dense additive mask, with one flag per block of 32 rows x 32 keys (mask_classify_kernel ran before).  Tiles before
@@ -616,7 +650,7 @@ void sdpa_bwd_dkv_kernel(SdpaBwdParams bp)
     // One step of the pipeline: S, dP of tile t (16 matrix instructions), then dV, dK of tile t - 1 (16 more, operands from
     // that tile's stage and from the exchange buffer) with P and dS of tile t computed on the vector ALU between them, then
     // - after a barrier, when everyone has read tile t - 1's P and dS - this wavefront's P and dS of tile t into the buffer.
-    // WITH_A = false is the step after the last tile: only the second half.
+    // WITH_A = false is the step after the last tile: only the second half; WITH_B = false the first tile's.
     // DENSE: the mask's column of this lane's key, for the query head in hand; and the flags of this wavefront's 32 keys -
     // per block of 32 query rows: 1 says the mask is zero there, 2 that it hides the keys from all of the rows (neither needs
     // the mask's values)
@@ -673,8 +707,9 @@ void sdpa_bwd_dkv_kernel(SdpaBwdParams bp)
         for (int r = 0; r < 16; ++r)
             mnext[r] = (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(rs, m_lane, (8 * (r / 4) + (r % 4)) * m_row2, 0);
     };
-    auto step = [&](int stage, int pstage, int i0, bool has_prev, [[maybe_unused]] int f_own, auto WITH_A_) __attribute__((always_inline)) {
-        constexpr bool WITH_A = decltype(WITH_A_)::value;
+    auto step = [&](int stage, int pstage, int i0, [[maybe_unused]] int f_own, auto WITH_A_, auto WITH_B_) __attribute__((always_inline)) {
+        constexpr bool WITH_A = decltype(WITH_A_)::value, WITH_B = decltype(WITH_B_)::value;
+        constexpr bool AHEAD = WITH_A && WITH_B && MASK != 1;      // (the instance with the mask's values in registers would spill)
         const char* qt = smem + stage * STAGE;
         const char* gt = qt + L::TILE_BYTES;
         const char* nl = gt + L::TILE_BYTES + role * 128;
@@ -682,13 +717,26 @@ void sdpa_bwd_dkv_kernel(SdpaBwdParams bp)
         const char* pg = pq + L::TILE_BYTES;
         vec8 ring[R];
         floatx16 sa, da;
-        vec8 pp[2], ds[2];
+        uint4v pp[2], ds[2];
         [[maybe_unused]] bool own_hidden = false, own_zero = false;
         if (WITH_A && DENSE) {
             own_hidden = f_own == 2;
             own_zero = f_own == 1;
         }
         [[maybe_unused]] const bool own_values = WITH_A && DENSE && !own_zero && !own_hidden;
+        // Matrix instruction m of the second half: group m / (2 NCB) = (own query block, rows 0-15), (own, 16-31),
+        // (partner's, 0-15), (partner's, 16-31); column block (m / 2) % NCB of this wavefront's; dV from dO^T and P (even m),
+        // dK from Q^T and dS (odd).
+        auto fetch_b = [&](int m) __attribute__((always_inline)) {
+            const int grp = m / (2 * NCB);
+            ring[m % R] = tl.tr_op((m % 2 ? pq : pg) + (grp < 2 ? own_rows : other_rows), (m / 2) % NCB, grp % 2);
+        };
+        vec8 bp_[2], bs_[2];        // P and dS of a group, two groups in flight
+        auto fetch_group = [&](int grp) __attribute__((always_inline)) {
+            const char* x = (grp < 2 ? (const char*)xmine : xother) + (grp % 2) * 1024;
+            bp_[grp % 2] = *(const vec8*)x;
+            bs_[grp % 2] = *(const vec8*)(x + 2048);
+        };
         if (WITH_A) {
             // The accumulators start from -L_i log2(e) and -D_i.  What the mask hides starts from -inf instead and ends as
             // P = 0, dS = 0 * (finite): only the causal edge needs that here, rows past Sq arrive as zeros throughout (dO = 0,
@@ -706,6 +754,7 @@ void sdpa_bwd_dkv_kernel(SdpaBwdParams bp)
             };
 #pragma unroll
             for (int i = 0; i < R; ++i) fetch_a(i);
+            __builtin_amdgcn_sched_barrier(0);
             if (DENSE && own_hidden) {      // (as at the causal edge: S starts from -inf; the products run all the same - branches
                                             //  around them cost every tile more than these tiles save)
                 asm volatile("" ::: "memory");
@@ -724,6 +773,10 @@ void sdpa_bwd_dkv_kernel(SdpaBwdParams bp)
                 if (i % 2 == 0) sa = Mma<T>::run(ring[i % R], kreg[i / 2], sa);
                 else da = Mma<T>::run(ring[i % R], vreg[i / 2], da);
                 if (i + R < NA) fetch_a(i + R);
+                else if (AHEAD) fetch_b(i + R - NA);      // (the second half's first operands)
+                if (AHEAD && i == NA - R - 2) fetch_group(0);
+                if (AHEAD && i == NA - R) fetch_group(1);
+                __builtin_amdgcn_sched_barrier(0);      // (the scheduler would put every read right in front of its matrix instruction)
             }
             if (own_values) {       // (the mask's values are no longer needed past this point: the second half has no room for them)
 #pragma unroll
@@ -731,30 +784,20 @@ void sdpa_bwd_dkv_kernel(SdpaBwdParams bp)
             }
         }
         // P and dS of register r of the own query block, rounded for the next products
-        auto soft = [&](int r) __attribute__((always_inline)) {
-            if (!WITH_A) return;
-            const float pr = __builtin_amdgcn_exp2f(sa[r]);
-            pp[r / 8][r % 8] = (T)pr;
-            ds[r / 8][r % 8] = (T)(pr * da[r]);
+        auto soft = [&](int r) __attribute__((always_inline)) {      // (two registers at a time: r is even)
+            if (!WITH_A || r % 2) return;
+            const float p0 = __builtin_amdgcn_exp2f(sa[r]), p1 = __builtin_amdgcn_exp2f(sa[r + 1]);
+            pp[r / 8][(r % 8) / 2] = pinned(pack2<T>(p0, p1));
+            ds[r / 8][(r % 8) / 2] = pinned(pack2<T>(p0 * da[r], p1 * da[r + 1]));
         };
-        if (has_prev) {
-            // Matrix instruction m of the second half: group m / (2 NCB) = (own query block, rows 0-15), (own, 16-31),
-            // (partner's, 0-15), (partner's, 16-31); column block (m / 2) % NCB of this wavefront's; dV from dO^T and P (even m),
-            // dK from Q^T and dS (odd).
-            auto fetch_b = [&](int m) __attribute__((always_inline)) {
-                const int grp = m / (2 * NCB);
-                ring[m % R] = tl.tr_op((m % 2 ? pq : pg) + (grp < 2 ? own_rows : other_rows), (m / 2) % NCB, grp % 2);
-            };
-            vec8 bp_[2], bs_[2];        // P and dS of a group, two groups in flight
-            auto fetch_group = [&](int grp) __attribute__((always_inline)) {
-                const char* x = (grp < 2 ? (const char*)xmine : xother) + (grp % 2) * 1024;
-                bp_[grp % 2] = *(const vec8*)x;
-                bs_[grp % 2] = *(const vec8*)(x + 2048);
-            };
-            fetch_group(0);
-            fetch_group(1);
+        if constexpr (WITH_B) {
+            if constexpr (!AHEAD) {
+                fetch_group(0);
+                fetch_group(1);
 #pragma unroll
-            for (int m = 0; m < R; ++m) fetch_b(m);
+                for (int m = 0; m < R; ++m) fetch_b(m);
+                __builtin_amdgcn_sched_barrier(0);
+            }
 #pragma unroll
             for (int m = 0; m < NB2; ++m) {
                 const int d = (m / 2) % NCB, grp = m / (2 * NCB);
@@ -764,6 +807,7 @@ void sdpa_bwd_dkv_kernel(SdpaBwdParams bp)
                 if (m % (2 * NCB) == 2 * NCB - 1 && grp + 2 < 4) fetch_group(grp + 2);
 #pragma unroll
                 for (int r = m * (16 / NB2); r < (m + 1) * (16 / NB2); ++r) soft(r);
+                __builtin_amdgcn_sched_barrier(0);
             }
         } else {
 #pragma unroll
@@ -771,10 +815,10 @@ void sdpa_bwd_dkv_kernel(SdpaBwdParams bp)
         }
         if (WITH_A) {
             __syncthreads();            // everyone has read the previous tile's P and dS
-            *(vec8*)(xmine) = pp[0];
-            *(vec8*)(xmine + 1024) = pp[1];
-            *(vec8*)(xmine + 2048) = ds[0];
-            *(vec8*)(xmine + 3072) = ds[1];
+            *(uint4v*)(xmine) = pp[0];
+            *(uint4v*)(xmine + 1024) = pp[1];
+            *(uint4v*)(xmine + 2048) = ds[0];
+            *(uint4v*)(xmine + 3072) = ds[1];
         }
     };
 
@@ -792,7 +836,7 @@ void sdpa_bwd_dkv_kernel(SdpaBwdParams bp)
         }
         if (f_cur == 0) { if (STAGED) tile_copy(n_lo); else tile_values(n_lo); }
     }
-    for (int t = n_lo; t < n_tiles; ++t) {
+    auto walk_tile = [&](int t, auto WITH_B_) __attribute__((always_inline)) {
         // Tile t has landed for everyone, tile t - 1's P and dS are in the exchange buffer, and everyone is done with tile
         // t - 2: its stage is free for tile t + 1.
         __builtin_amdgcn_s_waitcnt(0x0F70);             // vmcnt(0)
@@ -831,15 +875,19 @@ void sdpa_bwd_dkv_kernel(SdpaBwdParams bp)
         }
         // Every wavefront computes every tile: one whose keys no row of the tile sees (the first tile or two under a
         // causal mask) works on -inf, and would wait at the barriers for the others anyway.
-        step(stage, pstage, i0, t > n_lo, f_cur, std::true_type{});
+        step(stage, pstage, i0, f_cur, std::true_type{}, WITH_B_);
         pstage = stage;
         stage = nstage;
         i0 = i0 + PF_BN >= n_qt * PF_BN ? t_begin * PF_BN : i0 + PF_BN;      // (then: next head of the group)
         f_cur = f_next;
-    }
+    };
     if (n_lo < n_tiles) {
+        // (the first tile's step, which has no second half, is code of its own: with a branch inside the loop the compiler moves
+        //  the exponentials, which both of its sides have, in front of it and away from the matrix instructions)
+        walk_tile(n_lo, std::false_type{});
+        for (int t = n_lo + 1; t < n_tiles; ++t) walk_tile(t, std::true_type{});
         __syncthreads();
-        step(stage, pstage, i0, true, 0, std::false_type{});
+        step(stage, pstage, i0, 0, std::false_type{}, std::true_type{});
     }
 
     if (parts > 1) {
@@ -885,6 +933,206 @@ void sdpa_bwd_dkv_kernel(SdpaBwdParams bp)
                 if (col < p.Dv) *(vec4*)(vrow + d * 32 + r4 * 8 + g * 4) = wv;
             }
     }
+#endif
+}
+
+// ---- dK, dV for head dimensions up to 64, without a mask tensor ---------------------------------------------------------------
+// Here a wavefront has room for the whole of its 32 keys - K' and V rows 32 registers, dK and dV 64, a block's S and dP 32 - at
+// three wavefronts per SIMD, so none of the 128-wide kernel's pairing is needed: no exchange buffer, one barrier per tile, 33 KiB of
+// LDS per workgroup of four wavefronts, and three workgroups on a compute unit to cover each other's start, waits and vector
+// work (at 64 a block of 32 x 32 has 16 matrix instructions for its 16 exponentials per lane, half of what it has at 128).  The
+// kernel is the dQ kernel with the roles swapped: keys owned, Q / dO tiles streamed.
+constexpr int BN_WAVES = 3;        // wavefronts per SIMD
+template <typename T>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BN_WAVES, BN_WAVES))) void sdpa_bwd_dkv_narrow_kernel(SdpaBwdParams bp)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    constexpr int D = 64;
+    typedef typename Mma<T>::vec8 vec8;
+    typedef PfLayout<D> L;
+    typedef float float4v __attribute__((ext_vector_type(4)));
+    constexpr int NSTEP = D / 16, NDB = D / 32;
+    constexpr int R = 2;      // matrix operands in flight from LDS: three would spill at three wavefronts per SIMD
+    constexpr int STAGE = 2 * L::TILE_BYTES + 512;      // Q rows, dO rows, 64 x -L_i log2(e), 64 x -D_i
+    const SdpaParams& p = bp.f;
+    __shared__ __attribute__((aligned(1024))) char smem[2 * STAGE];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ql = lane & 31, g = lane >> 5;
+    const int Sq = p.Sq, Skv = p.Skv;
+    const int nkb = (Skv + BWD_KEYS - 1) / BWD_KEYS;
+    int kblk, bhkv;      // (a pair's key blocks on one XCD, the one with the most visible queries first: see sdpa_bwd_dkv_kernel)
+    if (((p.B * p.Hkv) & 7) == 0) {
+        const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+        kblk = slot % nkb;
+        bhkv = (slot / nkb) * 8 + xcd;
+    } else {
+        kblk = blockIdx.x % nkb;
+        bhkv = blockIdx.x / nkb;
+    }
+    const int hkv = bhkv % p.Hkv, b = bhkv / p.Hkv;
+    const int j0 = kblk * BWD_KEYS, wave_j0 = j0 + wave * 32, my_j = wave_j0 + ql;
+
+    const T* kp = (const T*)p.k + (int64_t)b * p.k_sb + (int64_t)hkv * p.k_sh;
+    const T* vp = (const T*)p.v + (int64_t)b * p.v_sb + (int64_t)hkv * p.v_sh;
+    T* dkp = (T*)bp.d_k + (int64_t)b * bp.dk_sb + (int64_t)hkv * bp.dk_sh;
+    T* dvp = (T*)bp.d_v + (int64_t)b * bp.dv_sb + (int64_t)hkv * bp.dv_sh;
+
+    const int kv_len = p.kv_lens ? clampi(p.kv_lens[b], 0, Skv) : Skv;
+    const int coff = Skv - Sq;
+    const int rows_b = p.q_lens ? clampi(p.q_lens[b], 0, Sq) : Sq;
+    // tiles from the first row that sees the workgroup's first key; a wavefront computes them from the first row that sees its
+    // own first key on (not at all when its keys are padding), and needs no mask from the first row that sees all of them on
+    const int t_begin = p.causal ? clampi(j0 - coff, 0, Sq) / PF_BN : 0;
+    const int i_wave = wave_j0 >= kv_len ? 0x40000000 : p.causal ? max(wave_j0 - coff, 0) : 0;
+    const int i_all_wave = p.causal ? max(wave_j0 + 31 - coff, 0) : 0;
+    const int lo_i = p.causal ? my_j - coff : -0x40000000;
+    const int n_qt = (rows_b + PF_BN - 1) / PF_BN;
+    const int tiles_per_head = j0 < kv_len ? max(n_qt - t_begin, 0) : 0;
+    const int n_all = tiles_per_head * p.G;
+    const int part = blockIdx.y, parts = gridDim.y;      // (a stretch of the walk: see sdpa_bwd_dkv_kernel)
+    const int n_lo = parts > 1 ? (int)((int64_t)n_all * part / parts) : 0;
+    const int n_hi = parts > 1 ? (int)((int64_t)n_all * (part + 1) / parts) : n_all;
+
+    BwdTiles<T, D, 4, NDB> tl;
+    tl.init(wave, lane, p.q_ss, bp.do_ss, p.D, p.Dv, 0);
+    const unsigned lds0 = lds_address(smem);
+    auto issue = [&](int n, int stage) __attribute__((always_inline)) {
+        const int h = n / tiles_per_head, r0 = (t_begin + n - h * tiles_per_head) * PF_BN;
+        const int hq = hkv * p.G + h;
+        const T* qb = (const T*)p.q + (int64_t)b * p.q_sb + (int64_t)hq * p.q_sh;
+        const T* gb = (const T*)bp.d_o + (int64_t)b * bp.do_sb + (int64_t)hq * bp.do_sh;
+        tl.issue(0, qb, p.q_ss, rows_b, r0, lds0 + stage * STAGE, wave);
+        tl.issue(1, gb, bp.do_ss, rows_b, r0, lds0 + stage * STAGE + L::TILE_BYTES, wave);
+        if (wave < 2)           // 64 floats of one of the two per-row arrays; rows past the last one arrive as zeros
+            dma_copy4(dma_descriptor((wave == 0 ? bp.neg_l2 : bp.neg_delta) + ((int64_t)b * p.Hq + hq) * Sq + r0, (rows_b - r0) * 4),
+                      lds0 + stage * STAGE + 2 * L::TILE_BYTES + wave * 256, lane * 4);
+    };
+    if (n_lo < n_hi) issue(n_lo, n_lo & 1);
+
+    // this lane's key: K row (scaled into log2 units) and V row as B operands, through 4 KiB per wavefront of the other stage
+    vec8 kreg[NSTEP], vreg[NSTEP];
+    {
+        char* stage = smem + ((n_lo + 1) & 1) * STAGE + wave * 4096;
+        static_assert(STAGE >= 4 * 4096, "a 4 KiB staging area per wavefront");
+        uint4v kraw[1][4], vraw[1][4];
+        fetch_q_rows(kraw, kp, wave_j0, Skv, p.k_ss, p.D, lane);
+        fetch_q_rows(vraw, vp, wave_j0, Skv, p.v_ss, p.Dv, lane);
+        stage_q_rows(kreg, kraw, stage, lane);
+        stage_q_rows(vreg, vraw, stage, lane);
+        const float c2 = p.scale * 1.4426950408889634f;
+#pragma unroll
+        for (int s = 0; s < NSTEP; ++s)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) kreg[s][e] = (T)((float)kreg[s][e] * c2);
+    }
+
+    floatx16 dk_acc[NDB], dv_acc[NDB];
+#pragma unroll
+    for (int d = 0; d < NDB; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) { dk_acc[d][r] = 0.0f; dv_acc[d][r] = 0.0f; }
+
+    int i0 = (t_begin + (n_lo < n_hi ? n_lo % tiles_per_head : 0)) * PF_BN;
+    for (int n = n_lo; n < n_hi; ++n) {
+        // tile n has landed for everyone and everyone is done with tile n - 1: its stage is free for tile n + 1
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (n + 1 < n_hi) issue(n + 1, (n + 1) & 1);
+        const char* qt = smem + (n & 1) * STAGE;
+        const char* gt = qt + L::TILE_BYTES;
+        const char* nl = gt + L::TILE_BYTES;
+#pragma unroll
+        for (int blk = 0; blk < 2; ++blk) {
+            const int ib = i0 + 32 * blk;
+            if (ib + 31 < i_wave) continue;      // no row of the block sees a key of the wavefront
+            // S and dP start from -L_i log2(e) and -D_i (what the mask hides from -inf: P = 0, dS = 0)
+            floatx16 s_acc, dp_acc;
+#pragma unroll
+            for (int r4 = 0; r4 < 4; ++r4) {
+                const float4v a = *(const float4v*)(nl + (32 * blk + 8 * r4 + 4 * g) * 4);
+                const float4v d = *(const float4v*)(nl + 256 + (32 * blk + 8 * r4 + 4 * g) * 4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) { s_acc[4 * r4 + e] = a[e]; dp_acc[4 * r4 + e] = d[e]; }
+            }
+            if (ib < i_all_wave) {      // some row of the block does not see every key of the wavefront
+                asm volatile("" ::: "memory");      // (a real branch)
+                const int rel = lo_i - ib - 4 * g;      // register r is row ib + 8 (r / 4) + 4 g + r % 4
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    if (8 * (r / 4) + (r % 4) < rel) s_acc[r] = -INFINITY;
+            }
+            // Operand i of the block: Q rows (even) and dO rows (odd) of k-step i / 2, then dO^T and Q^T of (16 rows h, column block d) in
+            // turn; R of them in flight ahead of their matrix instructions
+            vec8 ring[R];
+            auto fetch = [&](int i) __attribute__((always_inline)) {
+                const int m = i - 2 * NSTEP;
+                ring[i % R] = i < 2 * NSTEP ? tl.rows_op(i % 2 ? gt : qt, blk, i / 2) : tl.tr_op(m % 2 ? qt : gt, (m / 2) % NDB, 2 * blk + m / (2 * NDB));
+            };
+#pragma unroll
+            for (int i = 0; i < R; ++i) fetch(i);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 2 * NSTEP; ++i) {
+                if (i % 2 == 0) s_acc = Mma<T>::run(ring[i % R], kreg[i / 2], s_acc);
+                else dp_acc = Mma<T>::run(ring[i % R], vreg[i / 2], dp_acc);
+                fetch(i + R);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            // P and dS of 16 rows, then their products with P and dS of the other 16 between them
+            uint4v pp[2], ds[2];
+            auto soft = [&](int r) __attribute__((always_inline)) {
+                const float p0 = __builtin_amdgcn_exp2f(s_acc[r]), p1 = __builtin_amdgcn_exp2f(s_acc[r + 1]);
+                pp[r / 8][(r % 8) / 2] = pinned(pack2<T>(p0, p1));
+                ds[r / 8][(r % 8) / 2] = pinned(pack2<T>(p0 * dp_acc[r], p1 * dp_acc[r + 1]));
+            };
+#pragma unroll
+            for (int r = 0; r < 8; r += 2) soft(r);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int m = 0; m < 4 * NDB; ++m) {
+                const int d = (m / 2) % NDB, h = m / (2 * NDB);
+                if (m % 2 == 0) dv_acc[d] = Mma<T>::run(ring[(2 * NSTEP + m) % R], __builtin_bit_cast(vec8, pp[h]), dv_acc[d]);
+                else dk_acc[d] = Mma<T>::run(ring[(2 * NSTEP + m) % R], __builtin_bit_cast(vec8, ds[h]), dk_acc[d]);
+                if (m + R < 4 * NDB) fetch(2 * NSTEP + m + R);
+                if (m < 4) soft(8 + 2 * m);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        i0 = i0 + PF_BN >= n_qt * PF_BN ? t_begin * PF_BN : i0 + PF_BN;      // (then: next head of the group)
+    }
+
+    if (my_j >= kv_len) {      // (a key past the count met no mask above: its sums are not gradients)
+#pragma unroll
+        for (int d = 0; d < NDB; ++d)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) { dk_acc[d][r] = 0.0f; dv_acc[d][r] = 0.0f; }
+    }
+    if (parts > 1) {
+        if (my_j < Skv) {
+            const int64_t r = (((int64_t)part * p.B + b) * p.Hkv + hkv) * Skv + my_j;
+#pragma unroll
+            for (int d = 0; d < NDB; ++d)
+#pragma unroll
+                for (int r4 = 0; r4 < 4; ++r4) {
+                    float4v wk, wv;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        wk[e] = dk_acc[d][r4 * 4 + e] * p.scale;
+                        wv[e] = dv_acc[d][r4 * 4 + e];
+                    }
+                    const int col = d * 32 + r4 * 8 + g * 4;
+                    if (col < p.D) *(float4v*)(bp.part_dk + r * p.D + col) = wk;
+                    if (col < p.Dv) *(float4v*)(bp.part_dv + r * p.Dv + col) = wv;
+                }
+        }
+        return;
+    }
+    // (staged through the stage the last tile did not use: everyone is past that tile's barrier, i.e. done with the tile before it)
+    char* stage = smem + ((n_hi > n_lo ? n_hi : n_lo + 1) & 1) * STAGE + wave * 4096;
+    store_o_rows(dk_acc, p.scale, stage, dkp, wave_j0, Skv, bp.dk_ss, p.D, lane);
+    store_o_rows(dv_acc, 1.0f, stage, dvp, wave_j0, Skv, bp.dv_ss, p.Dv, lane);
 #endif
 }
 
@@ -940,21 +1188,23 @@ hipError_t launch_sdpa_bwd_sum_planes(const SdpaBwdParams& bp, int dtype, hipStr
     else sum_planes<bf16_t>(bp, stream);
     return hipGetLastError();
 }
-hipError_t launch_sdpa_bwd_delta(const SdpaBwdParams& bp, int dtype, hipStream_t stream)
+template <typename T>
+static void row_dots(const SdpaBwdParams& bp, hipStream_t stream)
 {
     const int64_t rows = (int64_t)bp.f.B * bp.f.Hq * bp.f.Sq;
-    if (dtype == 1) hipLaunchKernelGGL((sdpa_bwd_delta_kernel<f16_t>), dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, stream, bp);
-    else hipLaunchKernelGGL((sdpa_bwd_delta_kernel<bf16_t>), dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, stream, bp);
+    if (bp.f.Dv <= 64) hipLaunchKernelGGL((sdpa_bwd_delta_kernel<T, 8>), dim3((unsigned)((rows + 31) / 32)), dim3(256), 0, stream, bp);
+    else hipLaunchKernelGGL((sdpa_bwd_delta_kernel<T, 16>), dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, stream, bp);
+}
+hipError_t launch_sdpa_bwd_delta(const SdpaBwdParams& bp, int dtype, hipStream_t stream)
+{
+    if (dtype == 1) row_dots<f16_t>(bp, stream);
+    else row_dots<bf16_t>(bp, stream);
     return hipGetLastError();
 }
 
-// The dQ kernel goes to a side stream where one is to be had (side_stream.h) - it and the dK/dV kernel read the same inputs
-// and the row dots, and write different outputs - when the call is short of work: at most two rounds of dQ workgroups (two
-// per compute unit at a time), or D = 64.  Measured, whole call, forked against one stream (bf16, causal): 8 heads x 1024
-// 0.80 (D = 128) / 0.91 (64), 8 heads x 8192 0.875 / 0.98, 32 heads x 2048 0.98 / 0.89, 128 heads x 4096 1.00 - 1.03 / 0.96,
-// 32 heads x 8192 1.01 / 0.94: at D = 128 two launches that each fill the device only disturb each other's longest-first
-// order, at D = 64 the dQ kernel's workgroups still fill the dK/dV kernel's tail.  (The fork and join cost about 5 us: 32
-// heads x 1024, 256 workgroups in a call of 52 - 74 us, is 8 - 9 % slower forked.)
+// The dQ kernel first, computing the row dots that the dK/dV kernel needs too; or, where that pays (bwd16_forks), a kernel for the
+// row dots and the dQ kernel on a side stream (side_stream.h): it and the dK/dV kernel read the same inputs and write different
+// outputs.
 template <typename T, int D, bool DENSE = false>
 static hipError_t launch_bwd_t(const SdpaBwdParams& bp, hipStream_t stream)
 {
@@ -962,30 +1212,38 @@ static hipError_t launch_bwd_t(const SdpaBwdParams& bp, hipStream_t stream)
     const int64_t rows = (int64_t)p.B * p.Hq * p.Sq;
     const int nkb = (p.Skv + BWD_KEYS - 1) / BWD_KEYS;
     const bool with_dkv = (int64_t)nkb * p.Hkv * p.B > 0;
-    const int64_t dq_total = (int64_t)((p.Sq + PF_BM - 1) / PF_BM) * p.Hq * p.B;
-    SideStreamLease side(stream, rows > 0 && with_dkv && (D == 64 || dq_total <= 4 * (int64_t)device_cus()));
+    const int64_t cus = device_cus(), blocks = (int64_t)nkb * p.Hkv * p.B, walk = (int64_t)p.Sq * p.G / PF_BN, dq_blocks = (int64_t)((p.Sq + PF_BM - 1) / PF_BM) * p.Hq * p.B;
+    const bool narrow = bwd16_narrow(p.D, p.Dv, DENSE, p.G, blocks, walk, cus);
+    SideStreamLease side(stream, rows > 0 && with_dkv && bwd16_forks(narrow, p.causal || DENSE, p.G, blocks, max(bp.parts_kv, 1), walk, dq_blocks, cus));
+    SdpaBwdParams bq = bp;      // the dQ kernel: two workgroups per CU, an eighth of the CUs per XCD
+    const int nqb = (p.Sq + PF_BM - 1) / PF_BM;
+    const int64_t total = dq_blocks;
+    auto launch_dq = [&](hipStream_t s) {
+        bq.f.interleave = work_interleave(p.causal != 0 || p.mask != nullptr, 2 * device_cus() / 8, p.G, nqb, (total & 7) == 0 ? total >> 3 : total);
+        bq.f.deal_groups = (total & 7) == 0 ? work_deal(bq.f.interleave, p.G, nqb, total >> 3, p.causal != 0 || p.mask != nullptr) : 0;
+        if (DENSE && p.mask_chunks) hipLaunchKernelGGL((sdpa_bwd_dq_kernel<T, D, DENSE ? 2 : 0>), dim3((unsigned)total), dim3(256), 0, s, bq);
+        else hipLaunchKernelGGL((sdpa_bwd_dq_kernel<T, D, DENSE ? 1 : 0>), dim3((unsigned)total), dim3(256), 0, s, bq);
+    };
     bool forked = false;
     if (rows > 0) {
-        hipLaunchKernelGGL((sdpa_bwd_delta_kernel<T>), dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, stream, bp);
-        forked = with_dkv && side.active() && side.fork() == hipSuccess;
+        if (side.active()) {
+            row_dots<T>(bp, stream);
+            forked = side.fork() == hipSuccess;
+            if (!forked) launch_dq(stream);
+        } else {
+            bq.dots_in_dq = 1;
+            launch_dq(stream);
+        }
     }
     if (with_dkv) {
         const unsigned parts = bp.parts_kv > 1 ? (unsigned)bp.parts_kv : 1u;
         const dim3 grid((unsigned)((int64_t)nkb * p.Hkv * p.B), parts);
-        if (DENSE && p.mask_chunks) hipLaunchKernelGGL((sdpa_bwd_dkv_kernel<T, D, DENSE ? 2 : 0>), grid, dim3(512), 0, stream, bp);
+        if (narrow) hipLaunchKernelGGL((sdpa_bwd_dkv_narrow_kernel<T>), grid, dim3(256), 0, stream, bp);
+        else if (DENSE && p.mask_chunks) hipLaunchKernelGGL((sdpa_bwd_dkv_kernel<T, D, DENSE ? 2 : 0>), grid, dim3(512), 0, stream, bp);
         else hipLaunchKernelGGL((sdpa_bwd_dkv_kernel<T, D, DENSE ? 1 : 0>), grid, dim3(512), 0, stream, bp);
         if (parts > 1) sum_planes<T>(bp, stream);
     }
-    if (rows > 0) {
-        hipStream_t sq = forked ? side.stream() : stream;
-        const int nqb = (p.Sq + PF_BM - 1) / PF_BM;
-        const int64_t total = (int64_t)nqb * p.Hq * p.B;
-        SdpaBwdParams bq = bp;      // two workgroups per CU, an eighth of the CUs per XCD
-        bq.f.interleave = work_interleave(p.causal != 0 || p.mask != nullptr, 2 * device_cus() / 8, p.G, nqb, (total & 7) == 0 ? total >> 3 : total);
-        bq.f.deal_groups = (total & 7) == 0 ? work_deal(bq.f.interleave, p.G, nqb, total >> 3, p.causal != 0 || p.mask != nullptr) : 0;
-        if (DENSE && p.mask_chunks) hipLaunchKernelGGL((sdpa_bwd_dq_kernel<T, D, DENSE ? 2 : 0>), dim3((unsigned)total), dim3(256), 0, sq, bq);
-        else hipLaunchKernelGGL((sdpa_bwd_dq_kernel<T, D, DENSE ? 1 : 0>), dim3((unsigned)total), dim3(256), 0, sq, bq);
-    }
+    if (forked) launch_dq(side.stream());
     const hipError_t launched = hipGetLastError();
     if (forked) {
         const hipError_t e = side.join();      // (also after a failed launch: whatever did reach the side stream is ordered before the caller's next work)

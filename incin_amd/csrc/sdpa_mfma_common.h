@@ -309,6 +309,21 @@ __device__ __forceinline__ void store_o_rows_f32(const floatx16 (&o_acc)[NDB], f
     }
 }
 
+// A place in the order of the program for a value the matrix instructions around it do not need: what makes `x` comes before,
+// what uses it behind.  The compiler orders pure arithmetic by its uses and would gather a tile's exponentials behind the last
+// matrix instruction that they are written between; with this (no instruction) and __builtin_amdgcn_sched_barrier(0) they stay.
+__device__ __forceinline__ unsigned pinned(unsigned x)
+{
+    asm volatile("" : "+v"(x));
+    return x;
+}
+template <typename T> __device__ __forceinline__ unsigned pack2(float a, float b)
+{
+    typedef T vec2 __attribute__((ext_vector_type(2)));
+    const vec2 v = {(T)a, (T)b};
+    return __builtin_bit_cast(unsigned, v);
+}
+
 __device__ __forceinline__ float xor32_max(float x)
 {
     // lanes l and l^32 exchange; both end with the maximum

@@ -676,3 +676,53 @@ def test_matrix_core_backward_above_128(gpu, monkeypatch, parts, dtype, shape):
         else:
             assert not dq[b].any()
         assert not dq[b, :, nq:].any() and not dk[b, :, nk:].any() and not dv[b, :, nk:].any()
+
+
+@pytest.mark.parametrize("parts", ["1", "4"])
+@pytest.mark.parametrize("dtype", [capi.BF16, capi.F16], ids=lambda x: dtypes.NAMES[x])
+@pytest.mark.parametrize("shape", [
+    # B, Hq, Hkv, Sq, Skv, D, Dv, causal, kv_lens, q_lens
+    (2, 130, 130, 1, 33, 64, 64, True, None, None),                         # enough blocks without groups: one query, a key past a 32-key share
+    (1, 260, 260, 65, 31, 64, 64, False, None, None),                       # a row past a tile, a key short of a share
+    (2, 6, 3, 200, 333, 64, 48, True, [333, 70], None),                     # grouped queries, D != Dv, a count inside the first block
+    (1, 8, 1, 1030, 640, 40, 64, False, None, None),                        # many tiles of eight heads
+    (1, 4, 2, 700, 260, 64, 64, True, None, None),                          # rows that see no key
+    (3, 4, 2, 300, 300, 64, 64, True, [300, 131, 0], [300, 131, 1]),        # a padded batch, a sequence without keys
+], ids=["one_row", "rect", "ragged", "gqa8", "no_keys_seen", "padded"])
+def test_matrix_core_backward_narrow_heads(gpu, monkeypatch, parts, dtype, shape):
+    """The dK/dV kernel for head dimensions up to 64 (one wavefront per 32 keys) against the f64 oracle, walks whole and dealt to
+    four workgroups; and the same call with the row dots computed inside the dQ kernel (one stream) bit-identical to the
+    call that has a kernel for them and the dQ kernel beside (where the rule takes a second stream)."""
+    B, Hq, Hkv, Sq, Skv, D, Dv, causal, lens, qlens = shape
+    G = Hq // Hkv
+    monkeypatch.setenv("INCIN_ROCM_BWD_PARTS", parts)
+    say("matrix-core backward, narrow heads, %s in %s parts: %s" % (dtypes.NAMES[dtype], parts, shape))
+    q, k, v, go = make_d(141 + Sq, B, Hq, Hkv, Sq, Skv, D, Dv, dtype)
+    lens_a = None if lens is None else np.asarray(lens, np.int32)
+    qlens_a = None if qlens is None else np.asarray(qlens, np.int32)
+    res = []
+    for streams in (None, "1"):
+        if streams:
+            monkeypatch.setenv("INCIN_ROCM_BWD_STREAMS", streams)
+        res.append(host.sdpa_backward(q, k, v, go, dtype, impl=capi.IMPL_MFMA, causal=causal, kv_lens=lens_a, q_lens=qlens_a,
+                                      poison_padding=qlens is not None))
+    for a, b in zip(res[0][1:], res[1][1:]):
+        assert np.array_equal(a, b)
+    out, dq, dk, dv = res[0]
+    for b in range(B):
+        nq = Sq if qlens is None else int(qlens[b])
+        nk = Skv if lens is None else int(lens[b])
+        if nk > 0:
+            tri = np.triu(np.full((Sq, Skv), -np.inf, np.float32), 1 + Skv - Sq)[:nq, :nk] if causal else np.zeros((nq, nk), np.float32)
+            rows = np.isfinite(tri).any(axis=-1)                            # (rows that see a key: the others have zero gradients here)
+            sel = lambda x: x[b:b + 1, :, :nq][:, :, rows]
+            n = int(rows.sum())
+            rq, rk, rv = BW.sdpa_backward(sel(q).reshape(1, Hkv, G, n, D), k[b:b + 1, :, None, :nk], v[b:b + 1, :, None, :nk],
+                                          sel(go).reshape(1, Hkv, G, n, Dv), mask=tri[rows].reshape(1, 1, 1, n, nk))
+            compare("dq[%d]" % b, sel(dq), rq.reshape(1, Hq, n, D))
+            compare("dk[%d]" % b, dk[b:b + 1, :, :nk], rk.reshape(1, Hkv, nk, D))
+            compare("dv[%d]" % b, dv[b:b + 1, :, :nk], rv.reshape(1, Hkv, nk, Dv))
+            assert not dq[b, :, :nq][:, ~rows].any()
+        else:
+            assert not dq[b].any()
+        assert not dq[b, :, nq:].any() and not dk[b, :, nk:].any() and not dv[b, :, nk:].any()
