@@ -1348,3 +1348,48 @@ def test_copy_strided_gathers_any_view(gpu):
     bad = (C.c_int64 * 9)(*[1] * 9)
     assert lib.incin_rocm_copy_strided(0, None, None, 9, bad, bad, 4, None) == capi.ESHAPE
     assert lib.incin_rocm_copy_strided(0, None, None, 1, bad, bad, 3, None) == capi.EDTYPE
+
+
+@pytest.mark.parametrize("dtype", [capi.BF16, capi.F16], ids=lambda x: dtypes.NAMES[x])
+@pytest.mark.parametrize("shape", [
+    # B, Hq, Hkv, Sq, Skv, D, Dv, causal, kv_lens, q_lens
+    (3, 3, 3, 1, 1, 64, 64, False, None, None),               # a pair per wavefront, the last workgroup a quarter full
+    (2, 5, 5, 32, 17, 128, 128, True, None, None),            # ... rows that see no key (the diagonal is anchored at the last)
+    (3, 5, 5, 33, 64, 64, 64, True, None, None),              # two wavefronts a pair, an odd number of pairs
+    (1, 3, 3, 64, 33, 40, 64, False, None, None),
+    (2, 8, 2, 70, 65, 64, 64, False, [65, 31], None),         # grouped heads, three blocks of keys
+    (1, 4, 4, 129, 128, 128, 96, True, None, None),           # as many keys as D = 128 takes here
+    (1, 2, 2, 200, 97, 80, 80, False, None, None),
+    (3, 4, 4, 197, 197, 64, 64, False, [197, 160, 1], None),  # seven blocks, counts that end on a block and on its first key
+    (2, 4, 2, 224, 225, 64, 48, True, [225, 0], None),        # eight blocks, a sequence without keys
+    (2, 4, 2, 256, 256, 64, 64, True, [256, 100], [256, 100]),   # as many keys as D = 64 takes here; padding rows
+    (1, 2, 1, 2100, 77, 64, 64, False, None, None),           # many rows over few keys: several items per wavefront
+    (8, 40, 40, 90, 120, 64, 64, False, None, None),          # a workgroup per pair walking all its rows
+], ids=lambda s: "x".join(str(x) for x in s[:7]))
+def test_prefill_with_all_keys_in_lds(gpu, dtype, shape):
+    """The prefill kernel for up to 256 keys (128 at head dimensions above 64): outputs and row normalisers against the oracle."""
+    B, Hq, Hkv, Sq, Skv, D, Dv, causal, lens, qlens = shape
+    q, k, v = inputs(1500 + Sq + Skv, B, Hq, Hkv, Sq, Skv, D, Dv, dtype)
+    lens_a = None if lens is None else np.asarray(lens, np.int32)
+    qlens_a = None if qlens is None else np.asarray(qlens, np.int32)
+    say("all keys in LDS: %s %r" % (dtypes.NAMES[dtype], shape))
+    got, lse, info = host.sdpa(q, k, v, dtype, causal=causal, kv_lens=lens_a, q_lens=qlens_a, impl=capi.IMPL_MFMA, return_info=True, return_lse=True)
+    assert info["impl"] == capi.IMPL_MFMA and info["workspace_bytes"] == 0
+    ref = oracle_full(q, k, v, G=Hq // Hkv, causal=causal, kv_lens=lens_a)
+    kk = np.repeat(k, Hq // Hkv, axis=1).astype(np.float64)
+    x = np.matmul(q.astype(np.float64), np.swapaxes(kk, -1, -2)) * float(np.float32(1.0 / np.sqrt(D)))
+    if causal:
+        x = x + np.triu(np.full((Sq, Skv), -np.inf), 1 + Skv - Sq)
+    if lens is not None:
+        x = np.where(np.arange(Skv) < lens_a[:, None, None, None], x, -np.inf)
+    with np.errstate(divide="ignore", invalid="ignore"):
+        m = x.max(-1)
+        ref_lse = np.where(m == -np.inf, -np.inf, m + np.log(np.exp(x - np.where(m == -np.inf, 0.0, m)[..., None]).sum(-1)))
+    for b in range(B):
+        n = Sq if qlens is None else qlens[b]
+        check(got[b, :, :n], ref[b, :, :n], TOL[dtype], "output[%d]" % b)
+        a, r = lse[b, :, :n], ref_lse[b, :, :n]
+        assert np.array_equal(np.isneginf(a), np.isneginf(r))
+        seen = ~np.isneginf(r)
+        # (the scale is folded into Q, which is rounded again: half a step of the storage type on every term of a score)
+        assert not seen.any() or np.abs(a[seen] - r[seen]).max() <= (2e-2 if dtype == capi.BF16 else 3e-3)
