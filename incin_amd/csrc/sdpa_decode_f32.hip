@@ -46,19 +46,21 @@ __device__ __forceinline__ float quad_sum(float x)
     return xor32_sum(x);
 }
 
+// DC: the columns that are multiplied, D or fewer: the head dimensions are at most DC, and the products with the zeros beyond are
+// left out (the LDS rows keep the layout of D).
 //
 // LIMS: the launch is one half of a request with a mask tensor (one query head per KV head, or whole 128-row blocks per head):
 // mask_row_limits_kernel wrote, per mask row, n if the row is n zeros and then -inf, else -1.  A workgroup whose 128-row
 // block of rows all have a limit takes the limits - the tensor says nothing more - and the others leave at once: the f32
 // prefill kernel's dense-mask launch that follows computes those, and leaves the blocks computed here alone.
-template <int D, int NSLOT, int NRB, bool LIMS = false>
+template <int D, int NSLOT, int NRB, bool LIMS = false, int DC = D>
 __global__ __launch_bounds__(256) void sdpa_decode_f32_kernel(SdpaParams p)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
     typedef F32Layout<D> L;
-    constexpr int NJ = D / 16;                         // groups of four k-steps of the S^T product
-    constexpr int NDB = D / 16;                        // 16-wide blocks of the head dimension
-    constexpr int NDBW = NDB / 4;                      // of which a wavefront stores this many at the end
+    constexpr int NJ = DC / 16;                        // groups of four k-steps of the S^T product
+    constexpr int NDB = DC / 16;                       // 16-wide blocks of the head dimension
+    constexpr int NDBW = (NDB + 3) / 4;                // of which a wavefront stores at most this many at the end
     constexpr int SLOT = D > 128 ? 2 * DM_SLOT_BYTES : DM_SLOT_BYTES;      // a slot holds 8 KiB, at D = 256 the 16 KiB of 16 keys
     constexpr int BLOCK = SLOT / L::ROWB;              // keys per block: 16 (D = 128, 256), 32 (D = 64)
     constexpr int KB = BLOCK / 16;                     // 16-key sub-blocks of a block
@@ -389,6 +391,7 @@ __global__ __launch_bounds__(256) void sdpa_decode_f32_kernel(SdpaParams p)
 #pragma unroll
         for (int d2 = 0; d2 < NDBW; ++d2) {
             const int db = wave * NDBW + d2;
+            if (NDB % 4 != 0 && db >= NDB) continue;
             floatx4 o = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (int w = 0; w < 4; ++w)
@@ -418,14 +421,14 @@ __global__ __launch_bounds__(256) void sdpa_decode_f32_kernel(SdpaParams p)
 
 hipError_t launch_sdpa_combine(const SdpaParams& p, int dtype, hipStream_t stream);
 
-template <int D, int NSLOT, int NRB, bool LIMS = false>
+template <int D, int NSLOT, int NRB, bool LIMS = false, int DC = D>
 static hipError_t launch_decode_f32_t(const SdpaParams& p, hipStream_t stream)
 {
     // the rings, or what the wavefronts' results need when they meet at the end, whichever is more
     constexpr size_t slot_bytes = D > 128 ? 2 * DM_SLOT_BYTES : DM_SLOT_BYTES;
-    constexpr size_t ring_bytes = (size_t)4 * NSLOT * slot_bytes, merge_bytes = (size_t)NRB * (4 * 16 * 2 + 4 * (D / 16) * 4 * 64) * sizeof(float);
+    constexpr size_t ring_bytes = (size_t)4 * NSLOT * slot_bytes, merge_bytes = (size_t)NRB * (4 * 16 * 2 + 4 * (DC / 16) * 4 * 64) * sizeof(float);
     constexpr size_t lds = ring_bytes > merge_bytes ? ring_bytes : merge_bytes;
-    auto kern = sdpa_decode_f32_kernel<D, NSLOT, NRB, LIMS>;
+    auto kern = sdpa_decode_f32_kernel<D, NSLOT, NRB, LIMS, DC>;
     // the dynamic-LDS limit of this instance is raised once per device, not per launch
     static std::atomic<uint64_t> prepared{0};
     int dev = 0;
@@ -455,7 +458,12 @@ static hipError_t launch_decode_f32_d(const SdpaParams& p, bool two_slots, hipSt
     // 32 rows: always the two-slot rings, two workgroups per compute unit - one wavefront per SIMD leaves nothing to cover a
     // wavefront's start-up, softmax and waits (measured against five slots on prefill and decode shapes alike: level to 1.3
     // times ahead, config 2 of the benchmark 65 -> 51 us)
-    if (decode_f32_chunk_rows(p.G * p.Sq) == 32) return launch_decode_f32_t<D, 2, 2>(p, stream);
+    if (decode_f32_chunk_rows(p.G * p.Sq) == 32) {
+        // (and up to head dimension 96 only three quarters of the products, whose time is what bounds these shapes: 4 x 8 x 1643 at
+        // 80 377 -> 297 us, 12 x 501 causal 24.4 -> 20.6)
+        if (D == 128 && p.D <= 96 && p.Dv <= 96) return launch_decode_f32_t<128, 2, 2, false, 96>(p, stream);
+        return launch_decode_f32_t<D, 2, 2>(p, stream);
+    }
     return two_slots ? launch_decode_f32_t<D, 2, 1>(p, stream) : launch_decode_f32_t<D, DM_NSLOT, 1>(p, stream);
 }
 
@@ -476,6 +484,7 @@ hipError_t launch_sdpa_decode_f32(const SdpaParams& p, bool two_slots, hipStream
 // Dv <= 128, and p.mask_lims written.
 hipError_t launch_sdpa_decode_f32_limits(const SdpaParams& p, hipStream_t stream)
 {
+    if (p.Dp == 128 && p.D <= 96 && p.Dv <= 96) return launch_decode_f32_t<128, 2, 2, true, 96>(p, stream);
     return p.Dp == 128 ? launch_decode_f32_t<128, 2, 2, true>(p, stream) : launch_decode_f32_t<64, 2, 2, true>(p, stream);
 }
 

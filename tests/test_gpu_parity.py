@@ -1393,3 +1393,24 @@ def test_prefill_with_all_keys_in_lds(gpu, dtype, shape):
         seen = ~np.isneginf(r)
         # (the scale is folded into Q, which is rounded again: half a step of the storage type on every term of a score)
         assert not seen.any() or np.abs(a[seen] - r[seen]).max() <= (2e-2 if dtype == capi.BF16 else 3e-3)
+
+
+@pytest.mark.parametrize("D,Dv", [(68, 96), (80, 80), (96, 72), (96, 96), (100, 96), (96, 100)])
+def test_f32_kernels_up_to_96_columns(gpu, D, Dv):
+    """Head dimensions of 65 - 96 on the f32 prefill kernel and the split-KV kernel's 32-row form multiply 96 columns of the 128-column layout: both sides of
+    the edge, D and Dv apart, whole and split, the causal flag, row limits from a mask tensor, rows that end inside a block."""
+    dt = capi.F32
+    for B, Hq, Hkv, Sq, Skv, splits in ((2, 3, 3, 67, 67, 1), (1, 4, 2, 33, 900, 3)):
+        q, k, v = inputs(7000 + D + Dv + Sq, B, Hq, Hkv, Sq, Skv, D, Dv, dt)
+        for causal in (False, True):
+            ref = oracle_full(q, k, v, Hq // Hkv, causal=causal)
+            got, info = host.sdpa(q, k, v, dt, causal=causal, impl=capi.IMPL_SPLITKV_MFMA, num_splits=splits, return_info=True)
+            assert info["impl"] == capi.IMPL_SPLITKV_MFMA and (info["splits"] > 1) == (splits > 1)
+            check(got, ref, TOL[dt], "causal %s, %d splits" % (causal, info["splits"]))
+    q, k, v = inputs(7100 + D + Dv, 1, 2, 2, 150, 150, D, Dv, dt)
+    check(host.sdpa(q, k, v, dt, mask=O.causal_additive_mask(150, 150)), oracle_full(q, k, v, 1, causal=True), TOL[dt], "causal mask tensor")
+    q, k, v = inputs(7200 + D + Dv, 1, 2, 1, 150, 333, D, Dv, dt)
+    m = np.where(rng(9).random((1, 1, 150, 333)) < 0.3, -np.inf, rng(8).standard_normal((1, 1, 150, 333))).astype(np.float32)
+    check(host.sdpa(q, k, v, dt, mask=m, impl=capi.IMPL_MFMA), oracle_full(q, k, v, 2, mask=m), TOL[dt], "the prefill kernel, a mask of values")
+    for splits in (1, 2):
+        check(host.sdpa(q, k, v, dt, causal=True, impl=capi.IMPL_MFMA, num_splits=splits), oracle_full(q, k, v, 2, causal=True), TOL[dt], "the prefill kernel, %d splits" % splits)
