@@ -1034,21 +1034,54 @@ static int bwd_wide_parts(const incin_rocm_sdpa_desc_t* d)
     while (parts < 8 && walk * 4 > 2 * parts * (all / compute_units_of(d->device)) && walk >= 32 * parts) parts *= 2;
     return parts;
 }
-// Matrix-core kernels: into how many workgroups the key tiles of a block of 128 rows (dQ kernel, which = 0) or the query
-// tiles of a block of 128 keys (dK/dV kernel, which = 1) are dealt.  A launch of half a round of workgroups or less leaves
-// most of the device idle - under a causal mask every SIMD has one wavefront and all wait for the one with the longest
-// walk - so its tiles go to 2 workgroups (up to half a round) or 4 (up to a quarter), each with at least four tiles of 64 to
-// walk; the sums meet in planes of the workspace and a pass adds them (sdpa_bwd.h).
-// f32 (kind 2), both kernels.  Measured, whole call, against one workgroup per block (causal, with the dQ kernel on its side
-// stream either way): 8 heads x 1024 keys 0.36 (D = 64, 4 parts) / 0.56 (128); 32 heads x 1024 0.86 (D = 64, 2 parts: config
-// 2's shape) and 0.99 at D = 128 (a full round: not split); 16 query heads on 4 KV heads x 2048 0.38 / 0.41; from a full round
-// on 1.0 - 1.13: not split.
+// f32 (kind 2): one launch holds the blocks of dQ and of dK / dV, four wavefronts a workgroup (sdpa_bwd_f32.hip).
+//
+// How many of the four share the walk of one block of 32 rows or keys (the others take more blocks beside it): the more share, the
+// more and the shorter the items, and the more each tile that is copied into LDS costs.  Head dimensions above 64: two (one leaves
+// 1.02 - 1.7 times the time, everywhere).  Up to 64: four - whose tiles fill a compute unit with one workgroup - where that gives
+// at most one workgroup per compute unit, two up to eight rounds of two workgroups per compute unit.  Measured, backward
+// call, causal, 1 / 2 / 4 sharing: 4 heads x 300 51 / 31 / 24 us, 8 x 512 (not causal) 76 / 44 / 29, 56 x 65 21.2 / 18.8 / 21.8,
+// 32 x 1024 234 / 143 / 204, 64 x 2048 969 / 987 / 1368.
+static int bwd_f32_share(const incin_rocm_sdpa_desc_t* d)
+{
+    if (d->D > 64 || d->Dv > 64) return 2;
+    const int64_t cus = compute_units_of(d->device);
+    auto blocks = [&](int64_t own) { return ((d->Skv + own - 1) / own * d->Hkv + (d->Sq + own - 1) / own * d->Hq) * d->B; };
+    return blocks(32) <= cus ? 4 : blocks(64) < 16 * cus ? 2 : 1;
+}
+// Into how many workgroups a block's walk is dealt on top of that (which = 0: dQ, 1: dK / dV): the launch ends with its longest
+// item at the earliest, so where that alone would take more than twice a workgroup slot's share of the whole launch (one and a half
+// times where a workgroup has its compute unit to itself) the walks are divided, eight tiles of 64 per part at least (an item
+// costs about 10 us beside its tiles, and the planes are written, read and added).  And once where the items are equal (no mask)
+// and either leave the last of two rounds more than a quarter empty or are one round, which the dK / dV items alone then end (from
+// 16 tiles per part on).  Measured, backward call, in 1 / 2 / 4 parts (both kinds of item): 8 heads x 1259 x 64 causal 117 / 83 /
+// 86 us, 16 on 4 x 2048 x 64 causal 637 / 365 / 300, 8 x 1024 x 128 causal 158 / 108 / 130, 12 x 1024 x 80 causal 155 / 130 / 137 (dK / dV
+// alone in 2: 154), 24 x 544 x 80 causal 74 / 96, 24 x 1024 x 64 causal 115 / 136 / 162, 32 x 1024 x 64 causal 143 / 173 / 209, 8 x 1464 x 80
+// 296 / 259 / 269, 4 x 2048 x 128 303 / 283 / 305.
+static int bwd_f32_parts(const incin_rocm_sdpa_desc_t* d, int which)
+{
+    const int share = bwd_f32_share(d);
+    const int64_t own = 128 / share, tile = share == 4 ? 128 : 64, G = d->Hq / d->Hkv;
+    const int64_t slots = (int64_t)(d->D > 64 || d->Dv > 64 || share == 4 ? 1 : 2) * compute_units_of(d->device);
+    const int64_t n_kv = (d->Skv + own - 1) / own * d->Hkv * d->B, n_q = (d->Sq + own - 1) / own * d->Hq * d->B;
+    const int64_t walk_kv = (d->Sq + tile - 1) / tile * G, walk_q = (d->Skv + tile - 1) / tile;      // four products a tile; three
+    const bool uneven = d->causal || d->add_mask;
+    const int64_t all = (n_kv * walk_kv * 8 + n_q * walk_q * 6) / (uneven ? 2 : 1);
+    const int64_t longest = std::max(walk_q * 6, walk_kv * 8), tiles = (which == 0 ? d->Skv : d->Sq * G) / 64;
+    const int64_t over = slots > compute_units_of(d->device) ? 4 : 3;      // halves of a slot's share
+    int parts = 1;
+    while (parts < 4 && 2 * longest * slots > over * all * parts && tiles >= 16 * parts) parts *= 2;
+    const int64_t rounds = (n_kv + n_q + slots - 1) / slots;
+    if (parts == 1 && !uneven && tiles >= 16 && (rounds == 1 ? tiles >= 32 : rounds == 2 && 4 * (n_kv + n_q) <= 3 * rounds * slots)) parts = 2;
+    return parts;
+}
+// Matrix-core kernels: into how many workgroups the key tiles of a dQ block (which = 0) or the query tiles of a dK/dV block (which =
+// 1) are dealt; the sums meet in planes of the workspace and a pass adds them (sdpa_bwd.h).
 static int bwd_parts(const incin_rocm_sdpa_desc_t* d, int kind, int which)
 {
     if (kind == 0 || (kind != 2 && which == 0)) return 1;
     const char* forced = getenv("INCIN_ROCM_BWD_PARTS");      // (1, 2, 4 or 8 for every kernel that takes parts: a test knob)
     const int64_t blocks = which == 0 ? ((d->Sq + 127) / 128) * d->Hq * d->B : ((d->Skv + 127) / 128) * d->Hkv * d->B;
-    const int64_t slots = (int64_t)(d->D > 64 || d->Dv > 64 ? 1 : 2) * compute_units_of(d->device);
     const int64_t walk = (which == 0 ? d->Skv : d->Sq * (d->Hq / d->Hkv)) / 64;
     int parts = 1;
     const int f = forced ? atoi(forced) : 0;
@@ -1059,9 +1092,7 @@ static int bwd_parts(const incin_rocm_sdpa_desc_t* d, int kind, int which)
     }
     if (kind == 3) return bwd_wide_parts(d);
     if (kind == 1) return bwd16_parts(d, blocks, walk);
-    while (parts < 4 && 2 * parts * blocks <= slots) parts *= 2;
-    while (parts > 1 && walk < 4 * parts) parts >>= 1;      // (four tiles per part are enough to pay for the planes)
-    return parts;
+    return bwd_f32_parts(d, which);
 }
 static size_t round256(size_t n) { return (n + 255) / 256 * 256; }
 static size_t bwd_planes_bytes(const incin_rocm_sdpa_desc_t* d, int kind, int parts_q, int parts_kv)
@@ -1134,6 +1165,7 @@ int incin_rocm_sdpa_bwd(const incin_rocm_sdpa_bwd_desc_t* bd, void* stream)
     bp.f.mask_lims = nullptr;
     bp.parts_q = parts_q;
     bp.parts_kv = parts_kv;
+    bp.share = kind == 2 ? bwd_f32_share(&bd->fwd) : 0;
     if (plane_bytes) {
         const incin_rocm_sdpa_desc_t* d = &bd->fwd;
         char* at = (char*)bd->workspace + bwd_rows_bytes(d) + flag_bytes;

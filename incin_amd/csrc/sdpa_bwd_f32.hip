@@ -6,43 +6,45 @@
 //   P_ij = exp(x_ij - L_i)      dP_ij = dO_i . V_j      D_i = dO_i . O_i      dS_ij = P_ij (dP_ij - D_i)
 //   dV_j = sum_i P_ij dO_i      dK_j = s sum_i dS_ij Q_i      dQ_i = s sum_j dS_ij K_j
 //
-// Three kernels, no atomics (results are the same on every run), P and dP recomputed in both big ones - the plan of
-// sdpa_bwd_mfma.hip with the operand layouts of sdpa_prefill_f32.hip:
-//   bwd_f32_delta_kernel   per query row, into the workspace: -L_i log2(e) and -D_i, the values both big kernels start
+// No atomics (results are the same on every run), P and dP recomputed for both kinds of gradient - the plan of sdpa_bwd_mfma.hip
+// with the operand layouts of sdpa_prefill_f32.hip:
+//   bwd_f32_delta_kernel   per query row, into the workspace: -L_i log2(e) and -D_i, the values both kinds of block start
 //                          their S and dP accumulators from
-//   bwd_f32_dq_kernel      the forward's shape of work: a wavefront owns 32 query rows (Q' and dO rows resident as B
+//   bwd_f32_kernel         one launch of both: dK / dV blocks first, dQ blocks behind them
+//     dQ block             the forward's shape of work: a wavefront owns 32 query rows (Q' and dO rows resident as B
 //                          operands), K / V tiles stream through LDS; S^T = K Q'^T and dP^T = V dO^T land in the
 //                          lane-owns-a-query layout, which is the B-operand layout of dQ^T += K^T dS^T (K^T read from
 //                          the K tile as 32 consecutive floats of one row per half-wavefront)
-//   bwd_f32_dkv_kernel     the roles swapped: a wavefront owns 32 keys (K' and V rows resident as B operands), Q / dO
+//     dK / dV block        the roles swapped: a wavefront owns 32 keys (K' and V rows resident as B operands), Q / dO
 //                          tiles of the group's query heads stream through LDS; S = Q K'^T and dP = dO V^T land in a
 //                          lane-owns-a-key layout, the B-operand layout of dV^T += dO^T P and dK^T += Q^T dS
 // A matrix instruction occupies its pipe for 64 cycles and takes one register per operand, so nothing else is near a
-// limit and the loops are plain.  At D = 128 the resident rows and the accumulators of a wavefront exceed 256
-// registers: those instances run one wavefront per SIMD.
+// limit and the loops are plain; what decides is how evenly the items fill the device (BwdF32Shape, and the rules of the C ABI
+// layer).  At D = 128 the resident rows and the accumulators of a wavefront exceed 256 registers: those instances run one
+// wavefront per SIMD.  The call, causal, against two kernels on two streams with four blocks of 32 side by side in a workgroup: 32
+// heads x 1024, D = 64 214 -> 143 us (106 TFLOP/s of 153 that a large matrix product reaches), 64 x 2048 1129 -> 970, 12 x 501 at 80
+// 159 -> 66, 24 x 79 44 -> 14.
 #include <type_traits>
 
 #include "sdpa_bwd.h"
 #include "sdpa_mfma_common.h"
-#include "side_stream.h"
 
 namespace incin_rocm {
 
 typedef float float4v __attribute__((ext_vector_type(4)));
 
-// The LDS tile layout of sdpa_prefill_f32.hip: 16 KiB tiles of unpadded rows, 16-byte chunks XOR-swizzled by f(row).
-template <int D> struct F32Tile {
-    static constexpr int ROWB = D * 4, CPR = D / 4, TILE_BYTES = 16384;
-    static constexpr int ROWS = TILE_BYTES / ROWB;           // 64 (D = 64), 32 (D = 128)
-    static constexpr int NB = ROWS / 32, LPW = TILE_BYTES / 1024 / 4;
+// The LDS tile layout of sdpa_prefill_f32.hip: NB blocks of 32 unpadded rows, 16-byte chunks XOR-swizzled by f(row).
+template <int D, int NB> struct F32Tile {
+    static constexpr int ROWB = D * 4, CPR = D / 4, ROWS = 32 * NB, TILE_BYTES = ROWS * ROWB;
+    static constexpr int LPW = TILE_BYTES / 1024 / 4;
     static __device__ __forceinline__ int f(int r) { return (r & 3) | ((r & 4) << 1) | ((r & 8) >> 1); }
 };
 
 // Per-lane addressing of a tile, for both ways a tile is read: by rows (lane (ql, g): 16 bytes of row ql, floats
 // 8 j + 4 g ..: an A operand whose M index is the row) and by columns (lane (ql, g), k-step r: float 32 db + ql of row
 // 8 (r / 4) + 4 g + r % 4: an A operand whose M index is the column), and of the global -> LDS copies.
-template <int D> struct F32Addr {
-    typedef F32Tile<D> L;
+template <int D, int NB> struct F32Addr {
+    typedef F32Tile<D, NB> L;
     int row_base;                  // by rows: address = row_base ^ (j << 5)
     int col_low[8], col_high[D / 32];
     int voff[2][L::LPW];
@@ -87,27 +89,63 @@ template <int D> struct F32Addr {
 };
 
 // ---- -L_i log2(e) and -D_i ------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void bwd_f32_delta_kernel(SdpaBwdParams p)
+// LPR lanes of 16 bytes to a row of O and of dO.
+template <int LPR> __global__ __launch_bounds__(256) void bwd_f32_delta_kernel(SdpaBwdParams p)
 {
-    const int lane = threadIdx.x & 63;
-    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);     // (b * Hq + hq) * Sq + i
+    const int c = (threadIdx.x % LPR) * 4;
+    const int64_t row = (int64_t)blockIdx.x * (256 / LPR) + threadIdx.x / LPR;     // (b * Hq + hq) * Sq + i
     const int64_t rows = (int64_t)p.f.B * p.f.Hq * p.f.Sq;
     if (row >= rows) return;
     const int i = (int)(row % p.f.Sq);
     const int64_t bh = row / p.f.Sq;
     const int hq = (int)(bh % p.f.Hq), b = (int)(bh / p.f.Hq);
-    const float* o = (const float*)p.f.o + b * p.f.o_sb + hq * p.f.o_sh + (int64_t)i * p.f.o_ss;
-    const float* g = (const float*)p.d_o + b * p.do_sb + hq * p.do_sh + (int64_t)i * p.do_ss;
+    const float* o = (const float*)p.f.o + b * p.f.o_sb + hq * p.f.o_sh + (int64_t)i * p.f.o_ss + c;
+    const float* g = (const float*)p.d_o + b * p.do_sb + hq * p.do_sh + (int64_t)i * p.do_ss + c;
     float acc = 0.0f;
-    for (int d = lane; d < p.f.Dv; d += 64) acc = fmaf(o[d], g[d], acc);
+    if (c < p.f.Dv) {
+        const float4v x = *(const float4v*)o, y = *(const float4v*)g;
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) acc += __shfl_xor(acc, off, 64);
-    if (lane == 0) {
+        for (int e = 0; e < 4; ++e) acc = fmaf(x[e], y[e], acc);
+    }
+#pragma unroll
+    for (int off = LPR / 2; off >= 1; off >>= 1) acc += __shfl_xor(acc, off, 64);
+    if (c == 0) {
         // a row without a visible key (L_i = -inf, O and so D_i NaN) gets -inf and 0: its P is then 0 everywhere
         const float l = p.f.lse[row];
         p.neg_delta[row] = l == -INFINITY ? 0.0f : -acc;
         p.neg_l2[row] = l == -INFINITY ? -INFINITY : -l * 1.4426950408889634f;
     }
+}
+
+// ---- the shape of a workgroup ---------------------------------------------------------------------------------------
+// Four wavefronts: RW of them share the walk over the other axis for each of the 4 / RW blocks of 32 rows (dQ) or keys (dK, dV)
+// of the workgroup - wavefront w has block w % KW and of every tile the blocks of 32 with index w / KW modulo RW - and what they
+// sum meets in LDS at the end, added in a fixed order.
+template <int D, int RW> struct BwdF32Shape {
+    static constexpr int KW = 4 / RW, OWN = 32 * KW;                 // wavefronts side by side, rows or keys of the workgroup
+    static constexpr int NB0 = D == 64 ? 2 : 1, NB = RW > NB0 ? RW : NB0, NBW = NB / RW;      // blocks of a tile, and of a wavefront
+    typedef F32Tile<D, NB> Tile;
+    static constexpr int STAGE = 2 * Tile::TILE_BYTES + 1024;        // Q tile, dO tile, the two per-row arrays of the tile
+    static constexpr int LDS = 2 * STAGE;
+};
+
+// The registers of NX accumulators of 16 of each of the RW wavefronts of a block, through LDS: element u (four registers of an
+// accumulator: u / 4 names it) of the sum is left with wavefront u % RW.
+template <int NX, int RW, int KW> __device__ __forceinline__ void meet(const floatx16 (&acc)[NX], int first, char* smem, int own, int rs, int lane, int total)
+{
+    float4v* red = (float4v*)smem + ((int64_t)(own * RW + rs) * total + first) * 64 + lane;
+#pragma unroll
+    for (int x = 0; x < NX; ++x)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4) red[(x * 4 + r4) * 64] = float4v{acc[x][r4 * 4], acc[x][r4 * 4 + 1], acc[x][r4 * 4 + 2], acc[x][r4 * 4 + 3]};
+}
+template <int RW, int KW> __device__ __forceinline__ float4v met(const char* smem, int own, int u, int lane, int total)
+{
+    const float4v* red = (const float4v*)smem + ((int64_t)own * RW * total + u) * 64 + lane;
+    float4v w = red[0];
+#pragma unroll
+    for (int r = 1; r < RW; ++r) w += red[r * total * 64];
+    return w;
 }
 
 // ---- dQ ----------------------------------------------------------------------------------------------------------------
@@ -116,27 +154,30 @@ __global__ __launch_bounds__(256) void bwd_f32_delta_kernel(SdpaBwdParams p)
 // of the mask, asked for one tile ahead (right after the next tile's copies are issued) so that they arrive with that
 // tile.  The mask's block flags (mask_classify_kernel ran before) give the first and the last tile in which any row of the
 // workgroup sees a key: the tiles outside are left out.
-template <int D, bool DENSE = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 128 ? 1 : 2, D == 128 ? 1 : 2)))
-void bwd_f32_dq_kernel(SdpaBwdParams bp)
+template <int D, int DC, int RW, bool DENSE>
+__device__ __forceinline__ void bwd_f32_dq_body(const SdpaBwdParams& bp, char* smem, int id)      // smem: K buffers 0, 1, V buffers 0, 1
 {
 #if defined(__HIP_DEVICE_COMPILE__)
-    typedef F32Tile<D> L;
-    constexpr int NJ = D / 8, NDB = D / 32, KT = L::ROWS, NB = L::NB;
+    typedef BwdF32Shape<D, RW> W;
+    typedef typename W::Tile L;
+    constexpr int NJ = DC / 8, NDB = DC / 32, KT = L::ROWS, NB = W::NB, NBW = W::NBW, OWN = W::OWN;
     const SdpaParams& p = bp.f;
-    __shared__ __attribute__((aligned(1024))) char smem[4 * L::TILE_BYTES];      // K buffers 0, 1, V buffers 0, 1
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int own = wave % W::KW, rs = wave / W::KW;
     const int ql = lane & 31, g = lane >> 5;
     const int Sq = p.Sq, Skv = p.Skv;
-    const int nqb = (Sq + PF_BM - 1) / PF_BM;
-    const int total = gridDim.x;
-    const WorkItem wi = (total & 7) == 0 ? work_item_of_share(blockIdx.x & 7, blockIdx.x >> 3, total >> 3, p.interleave, p.G, nqb, p.deal_groups)
-                                         : work_item(blockIdx.x, p.interleave, p.G, nqb);
+    const int nqb = (Sq + OWN - 1) / OWN;
+    const int parts = bp.parts_q, total = nqb * p.Hq * p.B;
+    // (the parts of a block one behind the other, the blocks in the order of the work list)
+    const bool eighths = (total & 7) == 0;
+    const int part = eighths ? (id >> 3) % parts : id % parts;
+    const WorkItem wi = eighths ? work_item_of_share(id & 7, (id >> 3) / parts, total >> 3, p.interleave, p.G, nqb, p.deal_groups)
+                                : work_item(id / parts, p.interleave, p.G, nqb);
     const int hkv = wi.bhkv % p.Hkv, b = wi.bhkv / p.Hkv;
     const int hq = hkv * p.G + wi.gq;
-    const int q0 = wi.qblk * PF_BM;
+    const int q0 = wi.qblk * OWN;
 
     const float* qp = (const float*)p.q + (int64_t)b * p.q_sb + (int64_t)hq * p.q_sh;
     const float* gp = (const float*)bp.d_o + (int64_t)b * bp.do_sb + (int64_t)hq * bp.do_sh;
@@ -151,17 +192,17 @@ void bwd_f32_dq_kernel(SdpaBwdParams bp)
     const int rows_b = p.q_lens ? clampi(p.q_lens[b], 0, Sq) : Sq;
     const int coff = Skv - Sq;
     int j_end = kv_len;
-    const int my_i = q0 + wave * 32 + ql;
+    const int my_i = q0 + own * 32 + ql;
     int lim_lane = kv_len, lim_wave_min = kv_len, lim_wave_max = kv_len;
     if (p.causal) {
-        const int last_row = min(q0 + PF_BM - 1, rows_b - 1);
+        const int last_row = min(q0 + OWN - 1, rows_b - 1);
         j_end = clampi(last_row + coff + 1, 0, kv_len);
         lim_lane = clampi(my_i + coff + 1, 0, kv_len);
-        lim_wave_min = clampi(q0 + wave * 32 + coff + 1, 0, kv_len);
-        lim_wave_max = clampi(min(q0 + wave * 32 + 31, rows_b - 1) + coff + 1, 0, kv_len);
+        lim_wave_min = clampi(q0 + own * 32 + coff + 1, 0, kv_len);
+        lim_wave_max = clampi(min(q0 + own * 32 + 31, rows_b - 1) + coff + 1, 0, kv_len);
     }
     if (q0 >= rows_b) j_end = 0;
-    if (q0 + wave * 32 >= rows_b) lim_wave_min = lim_wave_max = 0;
+    if (q0 + own * 32 >= rows_b) lim_wave_min = lim_wave_max = 0;
     int n_tiles = (j_end + KT - 1) / KT, t_first = 0;
     const int n_act = lim_wave_max > 0 ? (lim_wave_max + KT - 1) / KT : 0;
     if (DENSE && p.mask_flags) {
@@ -174,7 +215,7 @@ void bwd_f32_dq_kernel(SdpaBwdParams bp)
         for (int c = tid; c < min(NB * n_tiles, nkb32); c += 256) {
             bool seen = false;
 #pragma unroll
-            for (int w = 0; w < 4; ++w) seen = seen || fl[(int64_t)min((q0 >> 5) + w, nrb32 - 1) * nkb32 + c] != 2;
+            for (int w = 0; w < W::KW; ++w) seen = seen || fl[(int64_t)min((q0 >> 5) + w, nrb32 - 1) * nkb32 + c] != 2;
             if (seen) { lo = min(lo, c); hi = max(hi, c); }
         }
         if (hi >= 0) { atomicMin(&s_seen[0], lo); atomicMax(&s_seen[1], hi); }
@@ -183,16 +224,15 @@ void bwd_f32_dq_kernel(SdpaBwdParams bp)
         n_tiles = s_seen[1] < 0 ? 0 : min(n_tiles, __builtin_amdgcn_readfirstlane(s_seen[1]) / NB + 1);
     }
 
-    // this workgroup's share of the tiles (bp.parts_q workgroups per block of rows: blockIdx.y says which)
-    const int part = blockIdx.y;
-    if (gridDim.y > 1) {
-        const int span = max(n_tiles - t_first, 0), parts = gridDim.y;
+    // this workgroup's share of the tiles (bp.parts_q workgroups per block of rows)
+    if (parts > 1) {
+        const int span = max(n_tiles - t_first, 0);
         const int lo = t_first + (int)((int64_t)span * part / parts), hi = t_first + (int)((int64_t)span * (part + 1) / parts);
         t_first = lo;
         n_tiles = hi;
     }
 
-    F32Addr<D> ad;
+    F32Addr<D, NB> ad;
     ad.init(wave, lane, p.k_ss, p.v_ss, p.D, p.Dv);
     const unsigned lds0 = lds_address(smem);
     auto issue_kv = [&](int t) __attribute__((always_inline)) {
@@ -237,8 +277,8 @@ void bwd_f32_dq_kernel(SdpaBwdParams bp)
         for (int r = 0; r < 16; ++r) dq_acc[db][r] = 0.0f;
 
     // DENSE: this lane's row of the mask; the values of a tile's keys, register r of block kb being key
-    // t * KT + 32 * kb + 8 * (r / 4) + 4 * g + r % 4
-    [[maybe_unused]] float4v m_next[NB][4], m_cur[NB][4];
+    // t * KT + 32 * (rs + RW * kb) + 8 * (r / 4) + 4 * g + r % 4
+    [[maybe_unused]] float4v m_next[NBW][4], m_cur[NBW][4];
     [[maybe_unused]] const float* mrow = nullptr;
     [[maybe_unused]] bool m_vec = false;
     if (DENSE) {
@@ -247,10 +287,10 @@ void bwd_f32_dq_kernel(SdpaBwdParams bp)
     }
     [[maybe_unused]] auto load_mask = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
-        for (int kb = 0; kb < NB; ++kb)
+        for (int kb = 0; kb < NBW; ++kb)
 #pragma unroll
             for (int r4 = 0; r4 < 4; ++r4) {
-                const int j = t * KT + 32 * kb + 8 * r4 + 4 * g;
+                const int j = t * KT + 32 * (rs + RW * kb) + 8 * r4 + 4 * g;
                 if (m_vec && j + 3 < Skv) m_next[kb][r4] = *(const float4v*)(mrow + j);
                 else {
 #pragma unroll
@@ -267,7 +307,7 @@ void bwd_f32_dq_kernel(SdpaBwdParams bp)
         __syncthreads();
         if (DENSE) {      // (arrived: a wait the compiler places for them is placed here, before the next copies are issued)
 #pragma unroll
-            for (int kb = 0; kb < NB; ++kb)
+            for (int kb = 0; kb < NBW; ++kb)
 #pragma unroll
                 for (int r4 = 0; r4 < 4; ++r4) {
                     m_cur[kb][r4] = m_next[kb][r4];
@@ -282,8 +322,8 @@ void bwd_f32_dq_kernel(SdpaBwdParams bp)
         const char* kt = smem + (t & 1) * L::TILE_BYTES;
         const char* vt = smem + (2 + (t & 1)) * L::TILE_BYTES;
 #pragma unroll
-        for (int kb = 0; kb < NB; ++kb) {
-            const int j0 = t * KT + kb * 32;
+        for (int x = 0; x < NBW; ++x) {
+            const int kb = rs + RW * x, j0 = t * KT + kb * 32;
             if (j0 >= lim_wave_max) break;
             // S^T - L and dP^T - D: the accumulators start from the per-query values.  Operands of step j + 1 are read
             // from LDS before the matrix instructions of step j are issued (the fences keep the compiler from moving
@@ -322,7 +362,7 @@ void bwd_f32_dq_kernel(SdpaBwdParams bp)
             }
             if (DENSE) {
 #pragma unroll
-                for (int r = 0; r < 16; ++r) s[r] = __builtin_fmaf(m_cur[kb][r / 4][r % 4], 1.4426950408889634f, s[r]);
+                for (int r = 0; r < 16; ++r) s[r] = __builtin_fmaf(m_cur[x][r / 4][r % 4], 1.4426950408889634f, s[r]);
             }
             // dS^T = P^T (dP^T - D); a masked pair has P = 0 and a finite second factor
 #pragma unroll
@@ -342,63 +382,66 @@ void bwd_f32_dq_kernel(SdpaBwdParams bp)
             }
         }
     }
+    constexpr int NU = NDB * 4;
+    if (RW > 1) {
+        __syncthreads();
+        meet<NDB, RW, W::KW>(dq_acc, 0, smem, own, rs, lane, NU);
+        __syncthreads();
+    }
     if (my_i < Sq) {
         float* row = dqp + (int64_t)my_i * bp.dq_ss;
         if (part > 0)      // (a plane of the workspace: contiguous rows of D floats)
             row = bp.part_dq + ((((int64_t)(part - 1) * p.B + b) * p.Hq + hq) * Sq + my_i) * p.D;
 #pragma unroll
-        for (int db = 0; db < NDB; ++db)
+        for (int x = 0; x < NU / RW; ++x) {
+            const int u = RW > 1 ? rs + RW * x : x;
+            float4v w;
+            if constexpr (RW > 1) w = met<RW, W::KW>(smem, own, u, lane, NU);
+            else w = float4v{dq_acc[x / 4][x % 4 * 4], dq_acc[x / 4][x % 4 * 4 + 1], dq_acc[x / 4][x % 4 * 4 + 2], dq_acc[x / 4][x % 4 * 4 + 3]};
 #pragma unroll
-            for (int r4 = 0; r4 < 4; ++r4) {
-                float4v w;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) w[e] = my_i < rows_b ? dq_acc[db][r4 * 4 + e] * p.scale : 0.0f;
-                if (db * 32 + r4 * 8 + g * 4 < p.D) *(float4v*)(row + db * 32 + r4 * 8 + g * 4) = w;
-            }
+            for (int e = 0; e < 4; ++e) w[e] = my_i < rows_b ? w[e] * p.scale : 0.0f;
+            if (u * 8 + g * 4 < p.D) *(float4v*)(row + u * 8 + g * 4) = w;
+        }
     }
 #endif
 }
 
 // ---- dK, dV ------------------------------------------------------------------------------------------------------------
-constexpr int BWD32_KEYS = 128;      // keys per workgroup: 32 per wavefront
-
 // DENSE: a dense additive mask.  A lane owns a key and holds 16 query rows of a block: its values are 16 loads down a column
 // of the mask (one buffer descriptor per tile that starts at the tile's first row and ends with the head's last - rows past
 // Sq read zeros - one lane offset for the key's column and the lane's first row, a scalar offset per register; the host has
 // checked that a tile's rows fit 32-bit offsets), asked for one tile ahead like the dQ kernel's.  The block flags trim the
 // tiles to those between the first and the last block of rows, over the group's heads, that see any key of the workgroup.
-template <int D, bool DENSE = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 128 ? 1 : 2, D == 128 ? 1 : 2)))
-void bwd_f32_dkv_kernel(SdpaBwdParams bp)
+template <int D, int DC, int RW, bool DENSE>
+__device__ __forceinline__ void bwd_f32_dkv_body(const SdpaBwdParams& bp, char* smem, int id)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
-    typedef F32Tile<D> L;
-    constexpr int NJ = D / 8, NDB = D / 32, QT = L::ROWS, NB = L::NB;
-    constexpr int STAGE = 2 * L::TILE_BYTES + 1024;          // Q tile, dO tile, the two per-row arrays of the tile
+    typedef BwdF32Shape<D, RW> W;
+    typedef typename W::Tile L;
+    constexpr int NJ = DC / 8, NDB = DC / 32, QT = L::ROWS, NB = W::NB, NBW = W::NBW, OWN = W::OWN, STAGE = W::STAGE;
     const SdpaParams& p = bp.f;
-    __shared__ __attribute__((aligned(1024))) char smem[2 * STAGE];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int own = wave % W::KW, rs = wave / W::KW;
     const int ql = lane & 31, g = lane >> 5;
     const int Sq = p.Sq, Skv = p.Skv;
-    const int nkb = (Skv + BWD32_KEYS - 1) / BWD32_KEYS;
-    // all key blocks of a (batch, KV head) pair read the same Q and dO rows: a pair is given to one XCD
-    int kblk, bhkv;
+    const int nkb = (Skv + OWN - 1) / OWN;
+    // All key blocks of a (batch, KV head) pair read the same Q and dO rows: a pair is given to one XCD.  Under a mask the blocks
+    // of all the pairs of an XCD go first blocks first (a causal mask leaves those the most rows): what starts last is short.
+    int kblk, bhkv, part;
     {
-        const int pairs = p.B * p.Hkv;
-        if ((pairs & 7) == 0) {
-            const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-            kblk = slot % nkb;
-            bhkv = (slot / nkb) * 8 + xcd;
-        } else {
-            kblk = blockIdx.x % nkb;
-            bhkv = blockIdx.x / nkb;
-        }
+        const int pairs = p.B * p.Hkv, parts = bp.parts_kv, xcds = (pairs & 7) == 0 ? 8 : 1;
+        const int xcd = xcds == 8 ? id & 7 : 0, slot = xcds == 8 ? id >> 3 : id, per = pairs / xcds;
+        part = slot % parts;
+        const int r = slot / parts;
+        const bool uneven = p.causal || DENSE;
+        kblk = uneven ? r / per : r % nkb;
+        bhkv = (uneven ? r % per : r / nkb) * xcds + xcd;
     }
     const int hkv = bhkv % p.Hkv, b = bhkv / p.Hkv;
-    const int j0 = kblk * BWD32_KEYS;
-    const int my_j = j0 + wave * 32 + ql;              // this lane's key
+    const int j0 = kblk * OWN;
+    const int my_j = j0 + own * 32 + ql;              // this lane's key
 
     const float* kp = (const float*)p.k + (int64_t)b * p.k_sb + (int64_t)hkv * p.k_sh;
     const float* vp = (const float*)p.v + (int64_t)b * p.v_sb + (int64_t)hkv * p.v_sh;
@@ -411,7 +454,10 @@ void bwd_f32_dkv_kernel(SdpaBwdParams bp)
     // query rows that see any key of this workgroup: i >= j - coff for its first key (causal)
     const int i_begin_wg = p.causal ? clampi(j0 - coff, 0, Sq) : 0;
     // first query row that sees every key of this wavefront: tiles from there on need no mask
-    const int i_all_wave = p.causal ? max(j0 + wave * 32 + 31 - coff, 0) : 0;
+    const int i_all_wave = p.causal ? max(j0 + own * 32 + 31 - coff, 0) : 0;
+    // ... and first that sees any
+    const int i_first_wave = p.causal ? j0 + own * 32 - coff : -0x40000000;
+    const bool wave_past = j0 + own * 32 >= kv_len;
     int t_begin = i_begin_wg / QT;
     // query rows at and beyond rows_b are padding (q_lens): the tiles end there, and the rows between there and the end of
     // the last tile arrive as zeros like rows past Sq
@@ -419,7 +465,7 @@ void bwd_f32_dkv_kernel(SdpaBwdParams bp)
     int n_qt = (rows_b + QT - 1) / QT;
     if (DENSE && p.mask_flags) {
         __shared__ int s_seen[2];
-        const int nkb32 = (Skv + 31) >> 5, nrb32 = (Sq + 31) >> 5, c0 = kblk * 4;
+        const int nkb32 = (Skv + 31) >> 5, nrb32 = (Sq + 31) >> 5, c0 = kblk * W::KW;
         if (tid == 0) { s_seen[0] = 0x7fffffff; s_seen[1] = -1; }
         __syncthreads();
         int lo = 0x7fffffff, hi = -1;
@@ -429,7 +475,7 @@ void bwd_f32_dkv_kernel(SdpaBwdParams bp)
             const uint8_t* fl = mask_flags_of(p, b, hkv * p.G + x / r_n) + (int64_t)rb * nkb32;
             bool seen = false;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) seen = seen || fl[min(c0 + c, nkb32 - 1)] != 2;
+            for (int c = 0; c < W::KW; ++c) seen = seen || fl[min(c0 + c, nkb32 - 1)] != 2;
             if (seen) { lo = min(lo, rb); hi = max(hi, rb); }
         }
         if (hi >= 0) { atomicMin(&s_seen[0], lo); atomicMax(&s_seen[1], hi); }
@@ -442,11 +488,10 @@ void bwd_f32_dkv_kernel(SdpaBwdParams bp)
     }
     const int tiles_per_head = j0 < kv_len ? max(n_qt - t_begin, 0) : 0;
     const int n_all = tiles_per_head * p.G;             // the group's query heads one after another
-    // this workgroup's share of the walk (bp.parts_kv workgroups per key block: blockIdx.y says which)
-    const int part = blockIdx.y;
-    const int n_lo = (int)((int64_t)n_all * part / (int)gridDim.y), n_tiles = (int)((int64_t)n_all * (part + 1) / (int)gridDim.y);
+    // this workgroup's share of the walk (bp.parts_kv workgroups per key block)
+    const int n_lo = (int)((int64_t)n_all * part / bp.parts_kv), n_tiles = (int)((int64_t)n_all * (part + 1) / bp.parts_kv);
 
-    F32Addr<D> ad;
+    F32Addr<D, NB> ad;
     ad.init(wave, lane, p.q_ss, bp.do_ss, p.D, p.Dv);
 
     // this lane's key: K' = K * scale * log2(e) and V rows as B operands
@@ -488,26 +533,28 @@ void bwd_f32_dkv_kernel(SdpaBwdParams bp)
         const unsigned st = lds0 + stage * STAGE;
         ad.issue(0, (const float*)p.q + (int64_t)b * p.q_sb + (int64_t)hq * p.q_sh, p.q_ss, rows_b, r0, st, wave);
         ad.issue(1, (const float*)bp.d_o + (int64_t)b * bp.do_sb + (int64_t)hq * bp.do_sh, bp.do_ss, rows_b, r0, st + L::TILE_BYTES, wave);
-        if (wave < 2) {          // 64 floats (a tile has at most that many rows) of one of the two per-row arrays; rows past Sq arrive as zeros
-            const float* src = (wave == 0 ? bp.neg_l2 : bp.neg_delta) + ((int64_t)b * p.Hq + hq) * Sq + r0;
-            dma_copy4(dma_descriptor(src, (rows_b - r0) * 4), st + 2 * L::TILE_BYTES + wave * 256, lane * 4);
+        // 64 floats of one of the two per-row arrays, 512 bytes apart (a tile has 32, 64 or 128 rows); rows past Sq arrive as zeros
+        if (wave < (NB > 2 ? 4 : 2)) {
+            const int r1 = r0 + (wave >> 1) * 64;
+            const float* src = ((wave & 1) == 0 ? bp.neg_l2 : bp.neg_delta) + ((int64_t)b * p.Hq + hq) * Sq + r1;
+            dma_copy4(dma_descriptor(src, max(rows_b - r1, 0) * 4), st + 2 * L::TILE_BYTES + (wave & 1) * 512 + (wave >> 1) * 256, lane * 4);
         }
     };
 
-    // DENSE: the mask's values of a tile, register r of block qb being query row r0 + 32 * qb + 8 * (r / 4) + 4 * g + r % 4
-    [[maybe_unused]] float m_next[NB][16], m_cur[NB][16];
+    // DENSE: the mask's values of a tile, register r of block x being query row r0 + 32 * (rs + RW * x) + 8 * (r / 4) + 4 * g + r % 4
+    [[maybe_unused]] float m_next[NBW][16], m_cur[NBW][16];
     [[maybe_unused]] const int m_lane = (int)(((int64_t)min(my_j, Skv - 1) * p.m_sj + (int64_t)(4 * g) * p.m_si) * 4);
     [[maybe_unused]] const int m_row4 = (int)(p.m_si * 4);
     [[maybe_unused]] auto load_mask = [&](int n) __attribute__((always_inline)) {
-        const int h = n / tiles_per_head, r0 = (t_begin + n % tiles_per_head) * QT;
+        const int h = n / tiles_per_head, r0 = (t_begin + n % tiles_per_head) * QT + 32 * rs;
         const float* mc = (const float*)p.mask + (int64_t)b * p.m_sb + (int64_t)(hkv * p.G + h) * p.m_sh + (int64_t)r0 * p.m_si;
         const int64_t left = r0 < Sq ? ((int64_t)(Sq - 1 - r0) * p.m_si + (int64_t)(Skv - 1) * p.m_sj + 1) * 4 : 0;
-        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)mc, 0, (int)min(left, (int64_t)0x7fffffff), 0x00020000);
+        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)mc, 0, (int)min(left, (int64_t)0x7fffffff), 0x00020000);
 #pragma unroll
-        for (int qb = 0; qb < NB; ++qb)
+        for (int x = 0; x < NBW; ++x)
 #pragma unroll
             for (int r = 0; r < 16; ++r)
-                m_next[qb][r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, m_lane, (32 * qb + 8 * (r / 4) + (r % 4)) * m_row4, 0));
+                m_next[x][r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, m_lane, (32 * RW * x + 8 * (r / 4) + (r % 4)) * m_row4, 0));
     };
     if (n_lo < n_tiles) {
         issue(n_lo, n_lo & 1);
@@ -518,11 +565,11 @@ void bwd_f32_dkv_kernel(SdpaBwdParams bp)
         __syncthreads();
         if (DENSE) {      // (arrived: a wait the compiler places for them is placed here, before the next copies are issued)
 #pragma unroll
-            for (int qb = 0; qb < NB; ++qb)
+            for (int x = 0; x < NBW; ++x)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    m_cur[qb][r] = m_next[qb][r];
-                    asm volatile("" : "+v"(m_cur[qb][r]));
+                    m_cur[x][r] = m_next[x][r];
+                    asm volatile("" : "+v"(m_cur[x][r]));
                 }
         }
         if (n + 1 < n_tiles) {
@@ -534,16 +581,17 @@ void bwd_f32_dkv_kernel(SdpaBwdParams bp)
         const char* nl = gt + L::TILE_BYTES;
         const int i0 = (t_begin + n % tiles_per_head) * QT;
 #pragma unroll
-        for (int qb = 0; qb < NB; ++qb) {
-            const int ib = i0 + qb * 32;               // first query row of the block
+        for (int x = 0; x < NBW; ++x) {
+            const int qb = rs + RW * x, ib = i0 + qb * 32;      // first query row of the block
             if (ib >= rows_b) break;
+            if (ib + 31 < i_first_wave || wave_past) continue;  // no row of the block sees a key of this wavefront
             // S - L and dP - D in the lane-owns-a-key layout: register r is query row ib + 8 (r / 4) + 4 g + r % 4.
             // Operands of a step are read from LDS one step ahead, as in the dQ kernel.
             floatx16 s, dp;
 #pragma unroll
             for (int r4 = 0; r4 < 4; ++r4) {
                 const float4v a = *(const float4v*)(nl + (qb * 32 + 8 * r4 + 4 * g) * 4);
-                const float4v d = *(const float4v*)(nl + 256 + (qb * 32 + 8 * r4 + 4 * g) * 4);
+                const float4v d = *(const float4v*)(nl + 512 + (qb * 32 + 8 * r4 + 4 * g) * 4);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) { s[4 * r4 + e] = a[e]; dp[4 * r4 + e] = d[e]; }
             }
@@ -578,7 +626,7 @@ void bwd_f32_dkv_kernel(SdpaBwdParams bp)
             }
             if (DENSE) {
 #pragma unroll
-                for (int r = 0; r < 16; ++r) s[r] = __builtin_fmaf(m_cur[qb][r], 1.4426950408889634f, s[r]);
+                for (int r = 0; r < 16; ++r) s[r] = __builtin_fmaf(m_cur[x][r], 1.4426950408889634f, s[r]);
             }
             // rows past Sq arrive as zeros throughout (L' = 0, dO = 0: P = exp2(q.k) finite times dP = 0 for dS, and their
             // P meets dO = 0 in dV); rows without any visible key carry -inf already
@@ -609,6 +657,13 @@ void bwd_f32_dkv_kernel(SdpaBwdParams bp)
         }
     }
 
+    constexpr int NU = 2 * NDB * 4;      // dK's, then dV's
+    if (RW > 1) {
+        __syncthreads();
+        meet<NDB, RW, W::KW>(dk_acc, 0, smem, own, rs, lane, NU);
+        meet<NDB, RW, W::KW>(dv_acc, NU / 2, smem, own, rs, lane, NU);
+        __syncthreads();
+    }
     if (my_j < Skv) {
         float* krow = dkp + (int64_t)my_j * bp.dk_ss;
         float* vrow = dvp + (int64_t)my_j * bp.dv_ss;
@@ -619,33 +674,46 @@ void bwd_f32_dkv_kernel(SdpaBwdParams bp)
         }
         const bool live = my_j < kv_len;               // (a key past kv_len met no mask above: its sums are not gradients)
 #pragma unroll
-        for (int db = 0; db < NDB; ++db)
-#pragma unroll
-            for (int r4 = 0; r4 < 4; ++r4) {
-                float4v wk, wv;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    wk[e] = live ? dk_acc[db][r4 * 4 + e] * p.scale : 0.0f;
-                    wv[e] = live ? dv_acc[db][r4 * 4 + e] : 0.0f;
-                }
-                if (db * 32 + r4 * 8 + g * 4 < p.D) *(float4v*)(krow + db * 32 + r4 * 8 + g * 4) = wk;
-                if (db * 32 + r4 * 8 + g * 4 < p.Dv) *(float4v*)(vrow + db * 32 + r4 * 8 + g * 4) = wv;
+        for (int x = 0; x < NU / RW; ++x) {
+            const int u = RW > 1 ? rs + RW * x : x;
+            const bool is_k = u < NU / 2;
+            const int c = (is_k ? u : u - NU / 2) * 8 + g * 4;
+            float4v w;
+            if constexpr (RW > 1) w = met<RW, W::KW>(smem, own, u, lane, NU);
+            else {
+                const floatx16& a = x < NU / 2 ? dk_acc[x % (NU / 2) / 4] : dv_acc[x % (NU / 2) / 4];
+                w = float4v{a[x % 4 * 4], a[x % 4 * 4 + 1], a[x % 4 * 4 + 2], a[x % 4 * 4 + 3]};
             }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[e] = live ? (is_k ? w[e] * p.scale : w[e]) : 0.0f;
+            if (c < (is_k ? p.D : p.Dv)) *(float4v*)((is_k ? krow : vrow) + c) = w;
+        }
     }
 #endif
 }
 
+// One launch: the dK/dV blocks, whose items are the longer ones, then the dQ blocks.
+template <int D, int DC, int RW, bool DENSE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 && RW < 4 ? 2 : 1, D == 64 && RW < 4 ? 2 : 1)))
+void bwd_f32_kernel(SdpaBwdParams bp, int n_dkv)
+{
+    __shared__ __attribute__((aligned(1024))) char smem[BwdF32Shape<D, RW>::LDS];
+    const int id = blockIdx.x;
+    if (id < n_dkv) bwd_f32_dkv_body<D, DC, RW, DENSE>(bp, smem, id);
+    else bwd_f32_dq_body<D, DC, RW, DENSE>(bp, smem, id - n_dkv);
+}
+
 // dst rows [B, H, S, D] by strides += planes 0 .. nplanes - 1 of src ([nplanes][B, H, S, D] contiguous), in that order; blockIdx.y
-// picks one of two such jobs (dK and dV share a launch).  A thread takes four floats.
+// picks one of three such jobs.  A thread takes four floats.
 struct AddPlanesJob {
     float* dst;
     const float* src;
     int64_t sb, sh, ss;
-    int B, H, S, D;
+    int B, H, S, D, planes;
 };
-__global__ __launch_bounds__(256) void bwd_f32_add_planes_kernel(AddPlanesJob j0, AddPlanesJob j1, int nplanes)
+__global__ __launch_bounds__(256) void bwd_f32_add_planes_kernel(AddPlanesJob j0, AddPlanesJob j1, AddPlanesJob j2)
 {
-    const AddPlanesJob& j = blockIdx.y == 0 ? j0 : j1;
+    const AddPlanesJob& j = blockIdx.y == 0 ? j0 : blockIdx.y == 1 ? j1 : j2;
     const int d4 = j.D >> 2;
     const int64_t n = (int64_t)j.B * j.H * j.S * d4;
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -659,7 +727,7 @@ __global__ __launch_bounds__(256) void bwd_f32_add_planes_kernel(AddPlanesJob j0
     float* d = j.dst + b * j.sb + h * j.sh + (int64_t)s * j.ss + c;
     float4v acc = *(const float4v*)d;
     const int64_t plane = (int64_t)j.B * j.H * j.S * j.D;
-    for (int k = 0; k < nplanes; ++k) {
+    for (int k = 0; k < j.planes; ++k) {
         const float4v x = *(const float4v*)(j.src + k * plane + row * j.D + c);
 #pragma unroll
         for (int e = 0; e < 4; ++e) acc[e] += x[e];
@@ -667,66 +735,51 @@ __global__ __launch_bounds__(256) void bwd_f32_add_planes_kernel(AddPlanesJob j0
     *(float4v*)d = acc;
 }
 
-template <int D, bool DENSE = false>
-static hipError_t launch_bwd_f32_t(const SdpaBwdParams& bp, hipStream_t stream)
+template <int D, int DC, int RW, bool DENSE>
+static hipError_t launch_bwd_f32_t(const SdpaBwdParams& bp0, hipStream_t stream)
 {
-    const SdpaParams& p = bp.f;
+    typedef BwdF32Shape<D, RW> W;
+    SdpaBwdParams bp = bp0;
+    SdpaParams& p = bp.f;
+    bp.parts_q = bp.parts_q > 1 ? bp.parts_q : 1;
+    bp.parts_kv = bp.parts_kv > 1 ? bp.parts_kv : 1;
     const int64_t rows = (int64_t)p.B * p.Hq * p.Sq;
-    const int nqb = (p.Sq + PF_BM - 1) / PF_BM;
-    const int64_t total = (int64_t)nqb * p.Hq * p.B;
-    if (total > 0x7fffffffLL) return hipErrorInvalidValue;
-    const int nkb = (p.Skv + BWD32_KEYS - 1) / BWD32_KEYS;
-    const bool with_dkv = (int64_t)nkb * p.Hkv * p.B > 0;
-    // the dQ kernel on a side stream where one is to be had (side_stream.h) - it and the dK/dV kernel read the same inputs and
-    // the row dots, and write different outputs - when the call is short of work: at most two rounds of dQ workgroups (one
-    // per compute unit at a time at D = 128, two at 64).  Measured, whole call, forked against one stream (causal): 8 heads x
-    // 1024 0.60 (D = 128) / 0.76 (64), 32 heads x 1024 0.82 / 0.97, 32 heads x 2048 0.87 / 0.71, 8 heads x 8192 1.03 / 0.73; with
-    // more work than that 0.95 - 1.06 (128 heads x 2048 0.95 / 1.02, 64 heads x 4096 without a mask 1.02 / 1.06): not forked.
-    SideStreamLease side(stream, rows > 0 && with_dkv && total <= 2 * (int64_t)(D == 128 ? 1 : 2) * device_cus());
-    bool forked = false;
+    const int nqb = (p.Sq + W::OWN - 1) / W::OWN, nkb = (p.Skv + W::OWN - 1) / W::OWN;
+    const int64_t total = (int64_t)nqb * p.Hq * p.B, n_dkv = (int64_t)nkb * p.Hkv * p.B * bp.parts_kv, n_dq = total * bp.parts_q;
+    if (n_dkv + n_dq > 0x7fffffffLL) return hipErrorInvalidValue;
+    if (n_dkv + n_dq == 0) return hipSuccess;
     if (rows > 0) {
-        hipLaunchKernelGGL(bwd_f32_delta_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, bp);
-        forked = with_dkv && side.active() && side.fork() == hipSuccess;
+        if (p.Dv <= 64) hipLaunchKernelGGL(bwd_f32_delta_kernel<16>, dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, stream, bp);
+        else hipLaunchKernelGGL(bwd_f32_delta_kernel<32>, dim3((unsigned)((rows + 7) / 8)), dim3(256), 0, stream, bp);
     }
-    const unsigned parts_q = bp.parts_q > 1 ? (unsigned)bp.parts_q : 1u, parts_kv = bp.parts_kv > 1 ? (unsigned)bp.parts_kv : 1u;
-    if (with_dkv) {
-        const unsigned parts = parts_kv;
-        hipLaunchKernelGGL((bwd_f32_dkv_kernel<D, DENSE>), dim3((unsigned)((int64_t)nkb * p.Hkv * p.B), parts), dim3(256), 0, stream, bp);
-        if (parts > 1) {
-            const AddPlanesJob jk = {(float*)bp.d_k, bp.part_dk, bp.dk_sb, bp.dk_sh, bp.dk_ss, p.B, p.Hkv, p.Skv, p.D};
-            const AddPlanesJob jv = {(float*)bp.d_v, bp.part_dv, bp.dv_sb, bp.dv_sh, bp.dv_ss, p.B, p.Hkv, p.Skv, p.Dv};
-            const int64_t n4 = (int64_t)p.B * p.Hkv * p.Skv * (max(p.D, p.Dv) >> 2);
-            hipLaunchKernelGGL(bwd_f32_add_planes_kernel, dim3((unsigned)((n4 + 255) / 256), 2), dim3(256), 0, stream, jk, jv, (int)parts - 1);
-        }
+    p.interleave = work_interleave(p.causal != 0 || p.mask != nullptr, (D == 128 || RW == 4 ? 1 : 2) * device_cus() / 8, p.G, nqb, (total & 7) == 0 ? total >> 3 : total);
+    p.deal_groups = (total & 7) == 0 ? work_deal(p.interleave, p.G, nqb, total >> 3, p.causal != 0 || p.mask != nullptr) : 0;
+    hipLaunchKernelGGL((bwd_f32_kernel<D, DC, RW, DENSE>), dim3((unsigned)(n_dkv + n_dq)), dim3(256), 0, stream, bp, (int)n_dkv);
+    if (bp.parts_q > 1 || bp.parts_kv > 1) {
+        const AddPlanesJob jq = {(float*)bp.d_q, bp.part_dq, bp.dq_sb, bp.dq_sh, bp.dq_ss, p.B, p.Hq, p.Sq, p.D, bp.parts_q - 1};
+        const AddPlanesJob jk = {(float*)bp.d_k, bp.part_dk, bp.dk_sb, bp.dk_sh, bp.dk_ss, p.B, p.Hkv, p.Skv, p.D, bp.parts_kv - 1};
+        const AddPlanesJob jv = {(float*)bp.d_v, bp.part_dv, bp.dv_sb, bp.dv_sh, bp.dv_ss, p.B, p.Hkv, p.Skv, p.Dv, bp.parts_kv - 1};
+        const int64_t nq = bp.parts_q > 1 ? rows * (p.D >> 2) : 0, nk = bp.parts_kv > 1 ? (int64_t)p.B * p.Hkv * p.Skv * (max(p.D, p.Dv) >> 2) : 0;
+        const unsigned blocks = (unsigned)((max(nq, nk) + 255) / 256);
+        if (nq == 0) hipLaunchKernelGGL(bwd_f32_add_planes_kernel, dim3(blocks, 2), dim3(256), 0, stream, jk, jv, jv);
+        else hipLaunchKernelGGL(bwd_f32_add_planes_kernel, dim3(blocks, nk == 0 ? 1 : 3), dim3(256), 0, stream, jq, jk, jv);
     }
-    if (rows > 0) {
-        hipStream_t sq = forked ? side.stream() : stream;
-        const unsigned parts = parts_q;
-        SdpaBwdParams bq = bp;
-        bq.f.interleave = work_interleave(p.causal != 0 || p.mask != nullptr, (D == 128 ? 1 : 2) * device_cus() / 8, p.G, nqb, (total & 7) == 0 ? total >> 3 : total);
-        bq.f.deal_groups = (total & 7) == 0 ? work_deal(bq.f.interleave, p.G, nqb, total >> 3, p.causal != 0 || p.mask != nullptr) : 0;
-        hipLaunchKernelGGL((bwd_f32_dq_kernel<D, DENSE>), dim3((unsigned)total, parts), dim3(256), 0, sq, bq);
-        if (parts > 1) {
-            const AddPlanesJob jq = {(float*)bp.d_q, bp.part_dq, bp.dq_sb, bp.dq_sh, bp.dq_ss, p.B, p.Hq, p.Sq, p.D};
-            const int64_t n4 = (int64_t)p.B * p.Hq * p.Sq * (p.D >> 2);
-            hipLaunchKernelGGL(bwd_f32_add_planes_kernel, dim3((unsigned)((n4 + 255) / 256), 1), dim3(256), 0, sq, jq, jq, (int)parts - 1);
-        }
-    }
-    const hipError_t launched = hipGetLastError();
-    if (forked) {
-        const hipError_t e = side.join();      // (also after a failed launch: whatever did reach the side stream is ordered before the caller's next work)
-        if (e != hipSuccess) return e;
-    }
-    return launched;
+    return hipGetLastError();
 }
 
 // Host has validated: f32, D and Dv <= 128 in whole 16-byte vectors (bp.f.Dp = the instance: 64 or 128), finite scale, unit last-axis strides, 16-byte aligned rows,
 // row strides below 2^22 elements, lse and the workspace present; a dense mask (the DENSE instances) of any non-negative strides
 // of which 64 rows fit 32-bit byte offsets, its block flags computed.
+template <int D, int DC, int RW> static hipError_t launch_bwd_f32_d(const SdpaBwdParams& bp, hipStream_t stream)
+{
+    return bp.f.mask ? launch_bwd_f32_t<D, DC, RW, true>(bp, stream) : launch_bwd_f32_t<D, DC, RW, false>(bp, stream);
+}
 hipError_t launch_sdpa_bwd_f32(const SdpaBwdParams& bp, hipStream_t stream)
 {
-    if (bp.f.mask) return bp.f.Dp == 128 ? launch_bwd_f32_t<128, true>(bp, stream) : launch_bwd_f32_t<64, true>(bp, stream);
-    return bp.f.Dp == 128 ? launch_bwd_f32_t<128>(bp, stream) : launch_bwd_f32_t<64>(bp, stream);
+    if (bp.f.Dp == 64)
+        return bp.share == 4 ? launch_bwd_f32_d<64, 64, 4>(bp, stream) : bp.share == 2 ? launch_bwd_f32_d<64, 64, 2>(bp, stream) : launch_bwd_f32_d<64, 64, 1>(bp, stream);
+    // (up to head dimension 96 in the 128 layout: three quarters of the products)
+    return bp.f.D <= 96 && bp.f.Dv <= 96 ? launch_bwd_f32_d<128, 96, 2>(bp, stream) : launch_bwd_f32_d<128, 128, 2>(bp, stream);
 }
 
 }  // namespace incin_rocm

@@ -1,4 +1,4 @@
-// A second stream for launches of one call that do not depend on each other (the backward's dQ and dK/dV kernels: both
+// A second stream for launches of one call that do not depend on each other (the 16-bit backward's dQ and dK/dV kernels: both
 // read what the row-dots kernel wrote, neither reads what the other writes).  On shapes that do not fill the device the two
 // kernels share it instead of waiting for each other; the callers hold the rule for when that pays.
 //

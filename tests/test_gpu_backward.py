@@ -726,3 +726,61 @@ def test_matrix_core_backward_narrow_heads(gpu, monkeypatch, parts, dtype, shape
         else:
             assert not dq[b].any()
         assert not dq[b, :, nq:].any() and not dk[b, :, nk:].any() and not dv[b, :, nk:].any()
+
+
+@pytest.mark.parametrize("shape", [
+    # B, Hq, Hkv, Sq, Skv, D, Dv, causal, kv_lens, q_lens, mask
+    (1, 1, 1, 1, 1, 64, 64, False, None, None, False),                      # four wavefronts to a walk of one row
+    (2, 3, 3, 33, 129, 64, 32, True, [129, 97], None, False),               # ... a tile of 128 rows and one more
+    (1, 4, 2, 260, 131, 64, 64, True, None, None, False),                   # ... rows that see no key, grouped queries
+    (1, 2, 2, 161, 300, 40, 64, False, None, None, True),                   # ... a mask of values
+    (3, 4, 4, 193, 193, 64, 64, True, [193, 64, 0], [193, 64, 1], False),   # ... a padded batch, a sequence without keys
+    (4, 20, 20, 97, 95, 64, 64, True, None, None, True),                    # two: more blocks of 32 than compute units
+    (8, 36, 36, 450, 450, 64, 64, True, None, None, False),                 # one: many rounds of blocks
+    (1, 2, 1, 65, 63, 80, 80, True, None, None, False),                     # 96 of 128 columns: a row past and a key short of a tile
+    (2, 4, 2, 127, 200, 96, 68, False, [200, 33], None, True),
+    (1, 3, 3, 130, 97, 100, 96, True, None, None, False),                   # ... and past their edge
+    (3, 4, 4, 193, 193, 128, 128, True, [193, 64, 0], [193, 64, 1], False),
+    (2, 8, 8, 1464, 1464, 80, 80, False, None, None, False),                # dealt to two workgroups because a round would be left part empty
+], ids=lambda s: "x".join(str(x) for x in s[:7]))
+def test_matrix_core_backward_f32_walks_shared(gpu, shape):
+    """The f32 backward launch with 1, 2 and 4 wavefronts of a workgroup to a block's walk, as the sizes choose: 1e-5 of the largest
+    gradient magnitude against the f64 oracle (sampled batch entries of the large ones), exact zeros where padding is."""
+    B, Hq, Hkv, Sq, Skv, D, Dv, causal, lens, qlens, values = shape
+    G = Hq // Hkv
+    say("matrix-core backward f32, walks shared: %s" % (shape,))
+    q, k, v, go = make_d(171 + Sq, B, Hq, Hkv, Sq, Skv, D, Dv, capi.F32)
+    r = np.random.Generator(np.random.PCG64(172))
+    mask = None
+    if values:
+        mask = r.standard_normal((1, Hq, Sq, Skv), dtype=np.float32)
+        mask[r.random(mask.shape) < 0.25] = -np.inf
+        mask[..., 0] = 0.0
+    lens_a = None if lens is None else np.asarray(lens, np.int32)
+    qlens_a = None if qlens is None else np.asarray(qlens, np.int32)
+    out, dq, dk, dv = host.sdpa_backward(q, k, v, go, capi.F32, impl=capi.IMPL_MFMA, causal=causal, kv_lens=lens_a, q_lens=qlens_a, mask=mask,
+                                         poison_padding=qlens is not None)
+    for b in (range(B) if B * Hq < 200 else (0, B - 1)):
+        nq = Sq if qlens is None else int(qlens[b])
+        nk = Skv if lens is None else int(lens[b])
+        if nk > 0:
+            m = np.triu(np.full((Sq, Skv), -np.inf, np.float32), 1 + Skv - Sq)[:nq, :nk] if causal else np.zeros((nq, nk), np.float32)
+            rows = np.isfinite(m).any(axis=-1)                              # (rows that see a key: the others have zero gradients here)
+            n = int(rows.sum())
+            sel = lambda x: x[b:b + 1, :, :nq][:, :, rows]
+            m5 = m[rows].reshape(1, 1, 1, n, nk)
+            if values:
+                m5 = m5 + mask[:, :, :nq, :nk][:, :, rows].reshape(1, Hkv, G, n, nk)
+            rq, rk, rv = BW.sdpa_backward(sel(q).reshape(1, Hkv, G, n, D), k[b:b + 1, :, None, :nk], v[b:b + 1, :, None, :nk],
+                                          sel(go).reshape(1, Hkv, G, n, Dv), mask=m5)
+            # (one visible key leaves dS = 0, and what f32 leaves of it is the rounding of dP - D: measured on dP's scale instead)
+            for name, x, y in (("dq", sel(dq), rq.reshape(1, Hq, n, D)), ("dk", dk[b:b + 1, :, :nk], rk.reshape(1, Hkv, nk, D)),
+                               ("dv", dv[b:b + 1, :, :nk], rv.reshape(1, Hkv, nk, Dv))):
+                if nk == 1 and name != "dv":
+                    assert np.abs(x).max() <= 1e-5 * float(np.abs(v).max() * np.abs(go).max() * Dv)
+                else:
+                    compare("%s[%d]" % (name, b), x, y, tol=1e-5)
+            assert not dq[b, :, :nq][:, ~rows].any()
+        else:
+            assert not dq[b].any()
+        assert not dq[b, :, nq:].any() and not dk[b, :, nk:].any() and not dv[b, :, nk:].any()
