@@ -1001,11 +1001,19 @@ static size_t bwd_flags_bytes(const incin_rocm_sdpa_desc_t* d, int kind)
 // part at least, and with grouped queries until there are three if a part keeps 64.  Bf16 causal D = 64, in 1 / 2 / 4 / 8 parts, us:
 // 32 on 8 x 1024 89 / 62 / 55 / 55, 16 on 2 x 4096 576 / 314 / 192 / 178, 8 on 1 x 8192 1129 / 600 / 353 / 301, 64 on 8 x 4096 682 / 547 /
 // 466 / 489, 8 x 8192 278 / 283 / 276 / 305.
+// Its instance for head dimensions 65 - 96 runs two workgroups per compute unit: grouped queries only (without, the other kernel takes
+// the launches that would want parts), 8 tiles per part up to one workgroup per compute unit, 96 beyond.  Bf16 causal D = 96, likewise:
+// 16 on 4 x 500 68 / 51 / 41 / 41, 32 on 8 x 1000 109 / 86 / 68 / 69, 8 on 1 x 2048 366 / 200 / 115 / 87, 2 x 32 on 8 x 2000 239 / 207 / 240 /
+// 263, 4 x 32 on 8 x 1000 133 / 153 / 166 / 192, 64 on 8 x 4000 874 / 703 / 683 / 719.
 static int bwd16_parts(const incin_rocm_sdpa_desc_t* d, int64_t blocks, int64_t walk)
 {
     const int64_t cus = compute_units_of(d->device), G = d->Hq / d->Hkv;
     int parts = 1;
     if (incin_rocm::bwd16_narrow(d->D, d->Dv, d->add_mask != nullptr, G, blocks, walk, cus)) {
+        if (d->D > 64 || d->Dv > 64) {
+            while (parts < 8 && G > 1 && ((parts * blocks < cus && walk >= 8 * parts) || (parts * blocks < 3 * cus && walk >= 96 * parts))) parts *= 2;
+            return parts;
+        }
         while (parts < 8 && ((parts * blocks < 2 * cus && walk >= 32 * parts) || (G > 1 && parts * blocks < 3 * cus && walk >= 128 * parts))) parts *= 2;
         return parts;
     }

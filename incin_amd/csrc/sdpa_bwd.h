@@ -34,14 +34,16 @@ struct SdpaBwdParams {
 // 16-bit storage up to head dimension 128, the rules that the planner of the workspace and the launcher share.
 //   blocks: 128-key blocks of all (batch, KV head) pairs; walk: 64-row query tiles of a block's walk over its group's heads.
 //
-// Which dK/dV kernel.  Head dimensions up to 64 without a mask tensor: the kernel with one wavefront per 32 keys (the other
+// Which dK/dV kernel.  Head dimensions up to 96 without a mask tensor: the kernel with one wavefront per 32 keys (the other
 // pairs them) wherever there is more than one workgroup per compute unit to cover its latencies or the walks can be dealt to
 // more: 8 x 32 heads x 4096, causal, whole call 2.32 -> 1.80 ms, 32 x 12 x 512 144 -> 96 us.  A launch of one query head per KV head
 // that gives it less than a workgroup per compute unit, for walks of some length, keeps the paired kernel, whose eight
 // wavefronts per 128 keys are twice as many (8 heads x 2048 62 us against 70, 4 x 4096 94 against 106; at 16 tiles 48 against 44).
+// From 65 to 96 likewise, from walks of 12 tiles on (paired / narrow: 60 x 12 x 400 at 80 289 / 216 us, 87 x 16 x 98 98 / 83, 8 x 16 x 2553 at 96 causal
+// 719 / 605, 8 x 32 x 220 47 / 36, 2 x 32 on 8 x 2000 228 / 207; 2 heads x 5224 139 / 162, 16 x 1000 50 / 56).
 inline bool bwd16_narrow(int64_t D, int64_t Dv, bool mask, int64_t G, int64_t blocks, int64_t walk, int64_t cus)
 {
-    return D <= 64 && Dv <= 64 && !mask && (G > 1 || blocks >= cus || walk < 32);
+    return D <= 96 && Dv <= 96 && !mask && (G > 1 || blocks >= cus || walk < (D <= 64 && Dv <= 64 ? 32 : 12));
 }
 // Whether the dQ kernel runs on a stream of its own beside the dK/dV kernel.  The fork and the join cost 5 - 7 us, and the call a
 // kernel for the row dots, which the dQ kernel computes where it runs first (8 x 16 heads x 256, D = 64: 40 us forked, 21 in

@@ -134,9 +134,10 @@ struct BwdTiles {
 // on the scores, copies the same half of the next tile into the place they left: the copy has most of a tile's time to
 // land and no load sits inside the tile.  (The buffers of two workgroups and their tiles fill a compute unit's LDS to the
 // byte: the two words of the tile-range search live in the buffers before the first copy.)
+// DC: the columns that are multiplied, D or fewer (96 of 128 where the head dimensions end there: the zeros beyond are left out).
 // Wavefronts per SIMD: two; three for D = 64 without a mask tensor, which fits 168 registers without a spill (48 KiB of LDS
 // per workgroup: three workgroups per compute unit) - the masked instances would spill 11 - 42 registers there.
-template <typename T, int D, int MASK = 0>
+template <typename T, int D, int MASK = 0, int DC = D>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((D == 64 && MASK == 0) ? 3 : 2, (D == 64 && MASK == 0) ? 3 : 2)))
 void sdpa_bwd_dq_kernel(SdpaBwdParams bp)
 {
@@ -144,7 +145,7 @@ void sdpa_bwd_dq_kernel(SdpaBwdParams bp)
 #if defined(__HIP_DEVICE_COMPILE__)
     typedef typename Mma<T>::vec8 vec8;
     typedef PfLayout<D> L;
-    constexpr int NSTEP = D / 16, NDB = D / 32;
+    constexpr int NSTEP = DC / 16, NDB = DC / 32, NQH = (NSTEP + 3) / 4;
     const SdpaParams& p = bp.f;
     __shared__ __attribute__((aligned(1024))) char smem[4 * L::TILE_BYTES + (STAGED ? 4 * 4096 : 0)];      // K buffers 0, 1, V buffers 0, 1 (, mask values)
 
@@ -231,7 +232,7 @@ void sdpa_bwd_dq_kernel(SdpaBwdParams bp)
     {
         static_assert(2 * L::TILE_BYTES >= 4 * 4096, "the V buffers hold a 4 KiB staging area per wavefront");
         char* stage = smem + 2 * L::TILE_BYTES + wave * 4096;
-        uint4v qraw[NSTEP / 4][4], graw[NSTEP / 4][4];
+        uint4v qraw[NQH][4], graw[NQH][4];
         fetch_q_rows(qraw, qp, q0 + wave * 32, Sq, p.q_ss, p.D, lane);
         fetch_q_rows(graw, gp, q0 + wave * 32, Sq, bp.do_ss, p.Dv, lane);
         stage_q_rows(qreg, qraw, stage, lane);
@@ -245,13 +246,13 @@ void sdpa_bwd_dq_kernel(SdpaBwdParams bp)
             // dO . O of the wavefront's rows as the two tensors' rows are fetched: 16 bytes of each per lane, then the sum over a row's
             // eight lanes (in the order of sdpa_bwd_delta_kernel, to the bit), then through LDS to the lanes that own the rows
             const T* op = (const T*)p.o + (int64_t)b * p.o_sb + (int64_t)hq * p.o_sh;
-            uint4v oraw[NSTEP / 4][4];
+            uint4v oraw[NQH][4];
             fetch_q_rows(oraw, op, q0 + wave * 32, Sq, p.o_ss, p.Dv, lane);
 #pragma unroll
             for (int ps = 0; ps < 4; ++ps) {
                 float dot = 0.0f;
 #pragma unroll
-                for (int h = 0; h < NSTEP / 4; ++h) {
+                for (int h = 0; h < NQH; ++h) {
                     const vec8 x = __builtin_bit_cast(vec8, oraw[h][ps]), y = __builtin_bit_cast(vec8, graw[h][ps]);
                     float part = 0.0f;
 #pragma unroll
@@ -936,23 +937,24 @@ void sdpa_bwd_dkv_kernel(SdpaBwdParams bp)
 #endif
 }
 
-// ---- dK, dV for head dimensions up to 64, without a mask tensor ---------------------------------------------------------------
+// ---- dK, dV for head dimensions up to 96, without a mask tensor ---------------------------------------------------------------
 // Here a wavefront has room for the whole of its 32 keys - K' and V rows 32 registers, dK and dV 64, a block's S and dP 32 - at
 // three wavefronts per SIMD, so none of the 128-wide kernel's pairing is needed: no exchange buffer, one barrier per tile, 33 KiB of
 // LDS per workgroup of four wavefronts, and three workgroups on a compute unit to cover each other's start, waits and vector
 // work (at 64 a block of 32 x 32 has 16 matrix instructions for its 16 exponentials per lane, half of what it has at 128).  The
 // kernel is the dQ kernel with the roles swapped: keys owned, Q / dO tiles streamed.
-constexpr int BN_WAVES = 3;        // wavefronts per SIMD
-template <typename T>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BN_WAVES, BN_WAVES))) void sdpa_bwd_dkv_narrow_kernel(SdpaBwdParams bp)
+// D = 128 with DC = 96: head dimensions of 65 - 96 in the 128-column LDS layout, 96 columns of it multiplied - dK and dV 96 registers, K' and V
+// 48, two wavefronts per SIMD, two workgroups of 65 KiB on a compute unit.  (At 128 columns the registers would not do.)  With the dQ kernel cut
+// to 96 columns too, the call at 60 x 12 heads x 400, D = 80, f16 315 -> 216 us, 16 x 8 x 900 181 -> 133, 8 x 16 x 2553, D = 96, causal 787 -> 605.
+template <typename T, int D, int DC>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 3 : 2, D == 64 ? 3 : 2))) void sdpa_bwd_dkv_narrow_kernel(SdpaBwdParams bp)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
-    constexpr int D = 64;
     typedef typename Mma<T>::vec8 vec8;
     typedef PfLayout<D> L;
     typedef float float4v __attribute__((ext_vector_type(4)));
-    constexpr int NSTEP = D / 16, NDB = D / 32;
-    constexpr int R = 2;      // matrix operands in flight from LDS: three would spill at three wavefronts per SIMD
+    constexpr int NSTEP = DC / 16, NDB = DC / 32, NQH = (NSTEP + 3) / 4;
+    constexpr int R = D == 64 ? 2 : 4;      // matrix operands in flight from LDS (at 64 three would spill at three wavefronts per SIMD)
     constexpr int STAGE = 2 * L::TILE_BYTES + 512;      // Q rows, dO rows, 64 x -L_i log2(e), 64 x -D_i
     const SdpaParams& p = bp.f;
     __shared__ __attribute__((aligned(1024))) char smem[2 * STAGE];
@@ -1016,7 +1018,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BN_WAVES, B
     {
         char* stage = smem + ((n_lo + 1) & 1) * STAGE + wave * 4096;
         static_assert(STAGE >= 4 * 4096, "a 4 KiB staging area per wavefront");
-        uint4v kraw[1][4], vraw[1][4];
+        uint4v kraw[NQH][4], vraw[NQH][4];
         fetch_q_rows(kraw, kp, wave_j0, Skv, p.k_ss, p.D, lane);
         fetch_q_rows(vraw, vp, wave_j0, Skv, p.v_ss, p.Dv, lane);
         stage_q_rows(kreg, kraw, stage, lane);
@@ -1221,7 +1223,8 @@ static hipError_t launch_bwd_t(const SdpaBwdParams& bp, hipStream_t stream)
     auto launch_dq = [&](hipStream_t s) {
         bq.f.interleave = work_interleave(p.causal != 0 || p.mask != nullptr, 2 * device_cus() / 8, p.G, nqb, (total & 7) == 0 ? total >> 3 : total);
         bq.f.deal_groups = (total & 7) == 0 ? work_deal(bq.f.interleave, p.G, nqb, total >> 3, p.causal != 0 || p.mask != nullptr) : 0;
-        if (DENSE && p.mask_chunks) hipLaunchKernelGGL((sdpa_bwd_dq_kernel<T, D, DENSE ? 2 : 0>), dim3((unsigned)total), dim3(256), 0, s, bq);
+        if (D == 128 && !DENSE && p.D <= 96 && p.Dv <= 96) hipLaunchKernelGGL((sdpa_bwd_dq_kernel<T, D, 0, D == 128 ? 96 : D>), dim3((unsigned)total), dim3(256), 0, s, bq);
+        else if (DENSE && p.mask_chunks) hipLaunchKernelGGL((sdpa_bwd_dq_kernel<T, D, DENSE ? 2 : 0>), dim3((unsigned)total), dim3(256), 0, s, bq);
         else hipLaunchKernelGGL((sdpa_bwd_dq_kernel<T, D, DENSE ? 1 : 0>), dim3((unsigned)total), dim3(256), 0, s, bq);
     };
     bool forked = false;
@@ -1238,7 +1241,8 @@ static hipError_t launch_bwd_t(const SdpaBwdParams& bp, hipStream_t stream)
     if (with_dkv) {
         const unsigned parts = bp.parts_kv > 1 ? (unsigned)bp.parts_kv : 1u;
         const dim3 grid((unsigned)((int64_t)nkb * p.Hkv * p.B), parts);
-        if (narrow) hipLaunchKernelGGL((sdpa_bwd_dkv_narrow_kernel<T>), grid, dim3(256), 0, stream, bp);
+        if (narrow && D == 64) hipLaunchKernelGGL((sdpa_bwd_dkv_narrow_kernel<T, 64, 64>), grid, dim3(256), 0, stream, bp);
+        else if (narrow) hipLaunchKernelGGL((sdpa_bwd_dkv_narrow_kernel<T, 128, 96>), grid, dim3(256), 0, stream, bp);
         else if (DENSE && p.mask_chunks) hipLaunchKernelGGL((sdpa_bwd_dkv_kernel<T, D, DENSE ? 2 : 0>), grid, dim3(512), 0, stream, bp);
         else hipLaunchKernelGGL((sdpa_bwd_dkv_kernel<T, D, DENSE ? 1 : 0>), grid, dim3(512), 0, stream, bp);
         if (parts > 1) sum_planes<T>(bp, stream);

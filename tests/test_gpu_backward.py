@@ -688,9 +688,16 @@ def test_matrix_core_backward_above_128(gpu, monkeypatch, parts, dtype, shape):
     (1, 8, 1, 1030, 640, 40, 64, False, None, None),                        # many tiles of eight heads
     (1, 4, 2, 700, 260, 64, 64, True, None, None),                          # rows that see no key
     (3, 4, 2, 300, 300, 64, 64, True, [300, 131, 0], [300, 131, 1]),        # a padded batch, a sequence without keys
-], ids=["one_row", "rect", "ragged", "gqa8", "no_keys_seen", "padded"])
+    (2, 130, 130, 1, 33, 96, 96, True, None, None),                         # the same edges in the instance for 65 - 96
+    (1, 260, 260, 65, 31, 80, 72, False, None, None),
+    (2, 6, 3, 200, 333, 72, 96, True, [333, 70], None),
+    (1, 8, 1, 1030, 640, 96, 40, False, None, None),
+    (1, 4, 2, 700, 260, 40, 96, True, None, None),
+    (3, 4, 2, 300, 300, 96, 80, True, [300, 131, 0], [300, 131, 1]),
+    (1, 4, 2, 200, 200, 96, 104, True, None, None),                         # past its edge: the paired kernel
+], ids=["one_row", "rect", "ragged", "gqa8", "no_keys_seen", "padded", "one_row_96", "rect_96", "ragged_96", "gqa8_96", "no_keys_seen_96", "padded_96", "edge_104"])
 def test_matrix_core_backward_narrow_heads(gpu, monkeypatch, parts, dtype, shape):
-    """The dK/dV kernel for head dimensions up to 64 (one wavefront per 32 keys) against the f64 oracle, walks whole and dealt to
+    """The dK/dV kernel for head dimensions up to 64, or 96 (one wavefront per 32 keys) against the f64 oracle, walks whole and dealt to
     four workgroups; and the same call with the row dots computed inside the dQ kernel (one stream) bit-identical to the
     call that has a kernel for them and the dQ kernel beside (where the rule takes a second stream)."""
     B, Hq, Hkv, Sq, Skv, D, Dv, causal, lens, qlens = shape
