@@ -1102,6 +1102,26 @@ static int bwd_parts(const incin_rocm_sdpa_desc_t* d, int kind, int which)
     if (kind == 1) return bwd16_parts(d, blocks, walk);
     return bwd_f32_parts(d, which);
 }
+// The parts that any accepted workspace has room for: by 128-row blocks and rounds of workgroups alone.  Callers hold workspaces of
+// that size, so bwd_parts - measured on kernels that deal their work otherwise - may neither ask for more (a call whose
+// workspace does not hold its planes takes these parts) nor make a smaller one acceptable.
+static int bwd_parts_held(const incin_rocm_sdpa_desc_t* d, int kind, int which)
+{
+    if (kind == 0 || kind == 3 || (kind == 1 && which == 0)) return 1;
+    if (getenv("INCIN_ROCM_BWD_PARTS")) return bwd_parts(d, kind, which);
+    const int64_t cus = compute_units_of(d->device), q_blocks = ((d->Sq + 127) / 128) * d->Hq * d->B;
+    const int64_t blocks = which == 0 ? q_blocks : ((d->Skv + 127) / 128) * d->Hkv * d->B;
+    const int64_t slots = (kind == 1 || d->D > 64 || d->Dv > 64 ? 1 : 2) * cus;
+    const int64_t walk = (which == 0 ? d->Skv : d->Sq * (d->Hq / d->Hkv)) / 64;
+    int parts = 1;
+    while (parts < 4 && 2 * parts * blocks <= slots) parts *= 2;
+    while (parts > 1 && walk < (kind == 1 ? 64 : 4) * parts) parts >>= 1;
+    if (kind == 1 && parts == 1 && blocks <= slots && (d->causal || d->add_mask)) {
+        if (walk >= 2048) parts = 4;
+        else if (walk >= 256 && (d->D > 64 || d->Dv > 64) && q_blocks > 4 * cus) parts = 2;
+    }
+    return parts;
+}
 static size_t round256(size_t n) { return (n + 255) / 256 * 256; }
 static size_t bwd_planes_bytes(const incin_rocm_sdpa_desc_t* d, int kind, int parts_q, int parts_kv)
 {
@@ -1113,6 +1133,13 @@ static size_t bwd_planes_bytes(const incin_rocm_sdpa_desc_t* d, int kind, int pa
     return (size_t)(parts_q - 1) * q + (size_t)planes_kv * (k + v);
 }
 
+// A call's workspace: two f32 per query row, the mask's block flags, the planes of a split call.
+static size_t bwd_bytes(const incin_rocm_sdpa_desc_t* d, int kind, int parts_q, int parts_kv)
+{
+    const size_t more = bwd_flags_bytes(d, kind) + bwd_planes_bytes(d, kind, parts_q, parts_kv);
+    return more ? bwd_rows_bytes(d) + more : 2 * (size_t)(d->B * d->Hq * d->Sq) * sizeof(float);
+}
+
 int incin_rocm_sdpa_bwd_workspace(const incin_rocm_sdpa_bwd_desc_t* bd, size_t* bytes)
 {
     if (!bytes) return fail(INCIN_ROCM_EINVAL, "scaled_dot_product_attention backward: null output");
@@ -1121,9 +1148,8 @@ int incin_rocm_sdpa_bwd_workspace(const incin_rocm_sdpa_bwd_desc_t* bd, size_t* 
     int kind = 0;
     if (int rc = check_bwd(bd, &empty, &kind)) return rc;
     if (!empty) {
-        const size_t flags = bwd_flags_bytes(&bd->fwd, kind);
-        const size_t planes = bwd_planes_bytes(&bd->fwd, kind, bwd_parts(&bd->fwd, kind, 0), bwd_parts(&bd->fwd, kind, 1));
-        *bytes = flags || planes ? bwd_rows_bytes(&bd->fwd) + flags + planes : 2 * (size_t)(bd->fwd.B * bd->fwd.Hq * bd->fwd.Sq) * sizeof(float);
+        *bytes = std::max(bwd_bytes(&bd->fwd, kind, bwd_parts(&bd->fwd, kind, 0), bwd_parts(&bd->fwd, kind, 1)),
+                          bwd_bytes(&bd->fwd, kind, bwd_parts_held(&bd->fwd, kind, 0), bwd_parts_held(&bd->fwd, kind, 1)));
     }
     return 0;
 }
@@ -1147,13 +1173,17 @@ int incin_rocm_sdpa_bwd(const incin_rocm_sdpa_bwd_desc_t* bd, void* stream)
         return 0;
     }
     const size_t flag_bytes = bwd_flags_bytes(&bd->fwd, kind);
-    const int parts_q = bwd_parts(&bd->fwd, kind, 0), parts_kv = bwd_parts(&bd->fwd, kind, 1);
-    const size_t plane_bytes = bwd_planes_bytes(&bd->fwd, kind, parts_q, parts_kv);
-    const size_t need = flag_bytes || plane_bytes ? bwd_rows_bytes(&bd->fwd) + flag_bytes + plane_bytes
-                                   : 2 * (size_t)(bd->fwd.B * bd->fwd.Hq * bd->fwd.Sq) * sizeof(float);      // two f32 per query row (+ the mask's block flags, + the planes of a split call)
+    const int held_q = bwd_parts_held(&bd->fwd, kind, 0), held_kv = bwd_parts_held(&bd->fwd, kind, 1);
+    const size_t need = bwd_bytes(&bd->fwd, kind, held_q, held_kv);
     if (!bd->workspace || bd->workspace_bytes < need || !aligned16(bd->workspace))
         return fail(INCIN_ROCM_EWORKSPACE, "scaled_dot_product_attention backward: %zu workspace bytes needed (16-byte aligned), %zu given",
                     need, bd->workspace ? bd->workspace_bytes : (size_t)0);
+    int parts_q = bwd_parts(&bd->fwd, kind, 0), parts_kv = bwd_parts(&bd->fwd, kind, 1);
+    if (bd->workspace_bytes < bwd_bytes(&bd->fwd, kind, parts_q, parts_kv)) {
+        parts_q = held_q;
+        parts_kv = held_kv;
+    }
+    const size_t plane_bytes = bwd_planes_bytes(&bd->fwd, kind, parts_q, parts_kv);
     if (int rc = use_device(bd->fwd.device)) return rc;
     Plan plan;
     plan.impl = INCIN_ROCM_IMPL_GENERIC;

@@ -791,3 +791,47 @@ def test_matrix_core_backward_f32_walks_shared(gpu, shape):
         else:
             assert not dq[b].any()
         assert not dq[b, :, nq:].any() and not dk[b, :, nk:].any() and not dv[b, :, nk:].any()
+
+
+@pytest.mark.parametrize("case", [
+    # dtype, B, Hq, Hkv, S, D
+    (capi.BF16, 1, 8, 1, 1024, 256),
+    (capi.BF16, 1, 8, 2, 512, 64),
+    (capi.F16, 1, 4, 1, 512, 96),
+    (capi.F32, 1, 2, 2, 192, 64),
+], ids=["wide", "narrow64", "narrow96", "f32"])
+def test_backward_with_the_smallest_workspace(gpu, case):
+    """A call whose workspace holds the per-row floats but not the planes of the walks that it would divide by itself: the same gradients
+    (planes change the order of f32 sums and nothing else: one rounding step of the storage type of the largest magnitude); a byte less is refused."""
+    dtype, B, Hq, Hkv, S, D = case
+    say("backward, smallest workspace: %s" % (case,))
+    q, k, v, go = make(173 + D, B, Hq, Hkv, S, S, D, dtype)
+    tq, tk, tv, tg = (host.DeviceTensor.from_f32(x, dtype) for x in (q, k, v, go))
+    to, tdq, tdk, tdv = (host.DeviceTensor(t.shape, dtype) for t in (tq, tq, tk, tv))
+    lse = capi.DeviceBuffer(B * Hq * S * 4)
+    bd = capi.SdpaBwdDesc()
+    bd.fwd = host.make_desc(tq, tk, tv, to, causal=True, lse=lse)
+    fneed = capi.sdpa_workspace(bd.fwd)[0]
+    fws = capi.DeviceBuffer(max(fneed, 256))
+    bd.fwd.workspace, bd.fwd.workspace_bytes = fws.ptr, fneed
+    for name, t in (("d_o", tg), ("d_q", tdq), ("d_k", tdk), ("d_v", tdv)):
+        setattr(bd, name, t.ptr)
+        for i, s in enumerate(host._strides3(t.shape)):
+            getattr(bd, name + "_stride")[i] = s
+    capi.sdpa_fwd(bd.fwd)
+    least, full = 2 * B * Hq * S * 4, capi.sdpa_bwd_workspace(bd)
+    assert full >= least
+    ws = capi.DeviceBuffer(full)
+    got = []
+    for given in (full, least):
+        bd.workspace, bd.workspace_bytes = ws.ptr, given
+        capi.sdpa_bwd(bd)
+        capi.sync()
+        got.append([t.to_f32() for t in (tdq, tdk, tdv)])
+    step = {capi.BF16: 2.0 ** -8, capi.F16: 2.0 ** -11, capi.F32: 1e-5}[dtype]
+    for name, a, b in zip(("dq", "dk", "dv"), *got):
+        compare(name, b, a, tol=step)
+    bd.workspace_bytes = least - 1
+    with pytest.raises(capi.RocmError) as e:
+        capi.sdpa_bwd(bd)
+    assert e.value.code == capi.EWORKSPACE
