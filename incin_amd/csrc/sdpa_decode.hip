@@ -79,9 +79,8 @@ __global__ __launch_bounds__(256) void sdpa_decode_split_kernel(SdpaParams p)
     const int dl = (lane % LPR) * VEC;
     const int R = p.G * p.Sq;
     const int nchunks = (R + RMAX - 1) / RMAX;
-    const int split = blockIdx.x;
     const int hkv = blockIdx.y / nchunks, r0 = (blockIdx.y % nchunks) * RMAX;
-    const int b = blockIdx.z;
+    const int b = blockIdx.z, split = work_split(p, b * p.Hkv + hkv);
     const int Skv = p.Skv, Sq = p.Sq;
 
     int kv_len = Skv;

@@ -75,10 +75,10 @@ __global__ __launch_bounds__(256) void sdpa_decode_f32_kernel(SdpaParams p)
     const int Sq = p.Sq, Skv = p.Skv;
     const int R = p.G * Sq;
     const int nchunks = (R + CHUNK - 1) / CHUNK;
-    const int split = blockIdx.x;
     int hkv, chunk_id;
     int b;
     decode_work_item(nchunks, (p.causal || LIMS) && p.G == 1, NSLOT == 2, &b, &hkv, &chunk_id);
+    const int split = work_split(p, b * p.Hkv + hkv);
     const int r0 = chunk_id * CHUNK;
 
     int kv_len = Skv;

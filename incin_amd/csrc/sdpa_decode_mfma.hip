@@ -59,10 +59,10 @@ __global__ __launch_bounds__(256) void sdpa_decode_mfma_kernel(SdpaParams p)
     const int R = p.G * Sq;
     constexpr int CHUNK = 32 * NRB;                    // rows per workgroup
     const int nchunks = (R + CHUNK - 1) / CHUNK;
-    const int split = blockIdx.x;
     int hkv, chunk_id;
     int b;
     decode_work_item(nchunks, p.causal && p.G == 1, NSLOT == 2, &b, &hkv, &chunk_id);
+    const int split = work_split(p, b * p.Hkv + hkv);
     const int r0 = chunk_id * CHUNK;
 
     int kv_len = Skv;

@@ -1414,3 +1414,35 @@ def test_f32_kernels_up_to_96_columns(gpu, D, Dv):
     check(host.sdpa(q, k, v, dt, mask=m, impl=capi.IMPL_MFMA), oracle_full(q, k, v, 2, mask=m), TOL[dt], "the prefill kernel, a mask of values")
     for splits in (1, 2):
         check(host.sdpa(q, k, v, dt, causal=True, impl=capi.IMPL_MFMA, num_splits=splits), oracle_full(q, k, v, 2, causal=True), TOL[dt], "the prefill kernel, %d splits" % splits)
+
+
+@pytest.mark.parametrize("dtype", [capi.BF16, capi.F32], ids=lambda x: dtypes.NAMES[x])
+@pytest.mark.parametrize("case", [
+    # impl, B, Hq, Hkv, Sq, Skv, D, splits: the splits are dealt to the grid shifted from (batch, KV head) to the next, by up to the power of two in their number
+    (capi.IMPL_SPLITKV_MFMA, 4, 6, 3, 1, 2048, 128, 8),
+    (capi.IMPL_SPLITKV_MFMA, 9, 4, 1, 2, 1536, 64, 6),
+    (capi.IMPL_SPLITKV_MFMA, 5, 2, 2, 1, 4096, 128, 16),
+    (capi.IMPL_SPLITKV, 4, 6, 3, 1, 2048, 128, 4),
+    (capi.IMPL_SPLITKV, 7, 2, 2, 1, 2048, 64, 2),
+], ids=["mfma8", "mfma6", "mfma16", "vector4", "vector2"])
+def test_decode_splits_shifted_between_groups(gpu, dtype, case):
+    """Key counts from none to all of the cache: every split of every group is written once - the ones without keys as empty - and the
+    rows of a sequence without keys are NaN."""
+    impl, B, Hq, Hkv, Sq, Skv, D, splits = case
+    say("decode, splits shifted between groups: %s %s" % (dtypes.NAMES[dtype], case))
+    r = np.random.Generator(np.random.PCG64(211 + Skv))
+    mk = lambda *s: dtypes.round_to(r.standard_normal(s, dtype=np.float32), dtype)
+    q, k, v = mk(B, Hq, Sq, D), mk(B, Hkv, Skv, D), mk(B, Hkv, Skv, D)
+    lens = np.linspace(0, Skv, B).astype(np.int32)
+    lens[1] = 1
+    got = host.sdpa(q, k, v, dtype, kv_lens=lens, impl=impl, num_splits=splits)
+    assert np.isnan(got[0]).all()
+    for b in range(1, B):
+        n, G = int(lens[b]), Hq // Hkv
+        kk, vv = (np.repeat(x[b, :, :n].astype(np.float64), G, axis=0) for x in (k, v))
+        s = np.einsum("hid,hjd->hij", q[b].astype(np.float64), kk) / np.sqrt(D)
+        e = np.exp(s - s.max(-1, keepdims=True))
+        ref = np.einsum("hij,hjd->hid", e / e.sum(-1, keepdims=True), vv)
+        # f32: sums of at most 4096 terms; bf16: P and the result rounded to 2^-9 of values up to the largest, with the sums' spread
+        tol = 1e-5 if dtype == capi.F32 else 2.0 ** -7
+        assert np.abs(got[b] - ref).max() <= tol * max(1.0, np.abs(ref).max()), b
