@@ -21,11 +21,15 @@
 // (Without the pairs - a wavefront alone on its SIMD with 461 registers, half of them accumulation registers - nothing covers a
 // wavefront's LDS latencies and vector work: 144 us for the backward of 2 x 16 / 8 heads x 1024, causal, against 133.)
 //
-// P and dS enter the third product as two 16-bit values each - the rounded value and what the rounding left, 16 significant bits
-// in bf16 and 22 in f16 - through two matrix instructions that share one LDS operand: the f32 arithmetic such a call got
-// before (sdpa_bwd_generic.hip) keeps its precision (bf16 gradients 1.7 - 1.9e-3 off the float64 result in the 2-norm, which is
-// the rounding of the gradients themselves; with P and dS rounded once: 3e-3), for 176 matrix instructions per block over the
-// three items instead of 128.
+// P and dS enter the third product as two 16-bit values each - the rounded value and what the rounding left - through two matrix
+// instructions that share one LDS operand, so that such a call keeps the precision of f32 arithmetic (sdpa_bwd_generic.hip), for
+// 176 matrix instructions per block over the three items instead of 128.  bf16 leaves 16 significant bits of them whatever their size:
+// gradients 1.7 - 1.9e-3 off the float64 result in the 2-norm, as with f32 arithmetic, which is the rounding of the gradients
+// themselves (with P and dS rounded once: 3e-3).  f16 ends at 65504 above and at steps of 2^-24 below, so there they are split times
+// a power of two of the owned row's own, which follows the largest value the row has met (k_acc below): 22 bits of the largest, 2^-36 of it
+// for the others, no overflow.  Off the float64 result in the 2-norm, dQ, unscaled / so / f32 arithmetic: 8192 positions, dO of 1e-2
+// 5.7e-4 / 2.1e-4 / 2.1e-4, of 1e-3 5.4e-3 / 9.4e-4 / 9.4e-4 (subnormal gradients); and a dS beyond 65504 was a NaN in its row.  It costs
+// f16 2 - 4 % of the call (2 x 16 on 8 x 1024, causal 136 -> 138 us, 8 on 1 x 4096 520 -> 536).
 //
 // Tiles of 32 rows (16 KiB each of both tensors), three stages: t - 1 and t in use, t + 1 arriving by global -> LDS copies.  A
 // step is the first products of tile t, a barrier, and the third product of tile t - 1 with the exponentials and splits of
@@ -49,7 +53,9 @@ constexpr int BW_ROWS = 128;                                    // rows of a gra
 constexpr int BW_KT = 32;                                       // rows per streamed tile
 constexpr int BW_TILE = BW_KT * BW_D * 2;                       // 16 KiB
 constexpr int BW_STAGE = 2 * BW_TILE + 512;                     // both tensors' tiles; 32 x -L_i log2(e), 32 x -D_i (64 floats arrive)
-constexpr int BW_XCHG = 4 * 8192;                               // exchange areas of the four pairs
+constexpr int BW_PAIR = 8192 + 512;                             // a pair's exchange area: 8 KiB of values, two exponents per owned row
+constexpr int BW_XCHG = 4 * BW_PAIR;
+constexpr int BW_TOP = 15, BW_AIM = 11, BW_LOOSE = 60;          // f16: powers of two that bound and place the split values (see bwd_wide_item)
 constexpr int BW_RING = 4;                                      // LDS operands in flight ahead of their matrix instructions
 
 enum { BW_DQ = 0, BW_DK = 1, BW_DV = 2 };
@@ -64,6 +70,7 @@ __device__ __forceinline__ void bwd_wide_item(const SdpaBwdParams& bp, char* sme
     constexpr int R = BW_RING, LPW = BW_TILE / 1024 / 8;
     constexpr int NA = WITH_DP ? BW_D / 16 : BW_D / 32;      // matrix instructions (k-steps) of a wavefront's share of the first products
     constexpr int NDB = BW_D / 64;                           // 32-wide column blocks of its half of the gradient
+    constexpr bool SCALED = std::is_same<T, f16_t>::value;
     const SdpaParams& p = bp.f;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -196,8 +203,9 @@ __device__ __forceinline__ void bwd_wide_item(const SdpaBwdParams& bp, char* sme
     }
     // Exchange areas of the pair: what a role sends of its first products (8 floats per lane), and its half of dS (dV: P) as two
     // operands of 16 bytes per lane.
-    char* const x1 = smem + 3 * BW_STAGE + pr * 8192 + lane * 16;
+    char* const x1 = smem + 3 * BW_STAGE + pr * BW_PAIR + lane * 16;
     char* const x2 = x1 + 4096;
+    [[maybe_unused]] int* const x3 = (int*)(smem + 3 * BW_STAGE + pr * BW_PAIR + 8192) + lane;      // f16: what power of two a role's half is times
 
     floatx16 acc[NDB];
 #pragma unroll
@@ -206,15 +214,22 @@ __device__ __forceinline__ void bwd_wide_item(const SdpaBwdParams& bp, char* sme
         for (int r = 0; r < 16; ++r) acc[db][r] = 0.0f;
 
     vec8 w_hi, w_lo;      // this role's half of dS (dV: P) of the previous tile: the rounded value and the rest
+    // f16: the lane's owned row, and with it its column of the third product, has a power of two of its own.  k_acc: the accumulators
+    // are the sums times 2^k_acc, and the next tile is split times that; k_w: w_hi and w_lo are times 2^k_w <= 2^k_acc.  It starts
+    // so high that what it leaves unsplit is nothing, and comes down to where a tile's largest value is 2^BW_AIM whenever one
+    // passes 2^BW_TOP: the largest has its 22 bits, all others of the row 2^-36 of it, and nothing overflows.
+    [[maybe_unused]] int k_acc = BW_LOOSE, k_w = BW_LOOSE;
     // One tile: the first products of tile t, whose eight registers that the partner needs go to the exchange area; a barrier;
     // the third product of tile t - 1 with P and dS of tile t made between its matrix instructions.
     auto step = [&](const char* st, const char* pst, int r0, auto WITH_A_, auto WITH_B_) __attribute__((always_inline)) {
         constexpr bool WITH_A = decltype(WITH_A_)::value, WITH_B = decltype(WITH_B_)::value;
         floatx16 f;
         vec8 o_hi, o_lo;
+        [[maybe_unused]] int k_o = 0;
         if constexpr (WITH_B) {      // the partner's half of tile t - 1's dS
             o_hi = *(const vec8*)(x2 + (1 - role) * 2048);
             o_lo = *(const vec8*)(x2 + (1 - role) * 2048 + 1024);
+            if constexpr (SCALED) k_o = x3[(1 - role) * 64];
         }
         float4v nl[2], nd[2];
         if constexpr (WITH_A) {
@@ -256,12 +271,36 @@ __device__ __forceinline__ void bwd_wide_item(const SdpaBwdParams& bp, char* sme
             *(float4v*)(x1 + role * 2048 + 1024) = float4v{f[12], f[13], f[14], f[15]};
             __syncthreads();
         }
+        if constexpr (WITH_B && SCALED) {
+            const int k = min(k_w, k_o);
+            if (__builtin_amdgcn_ballot_w64(k_w != k_acc || k_o != k_acc)) {      // (rare: a row's largest value so far grew eightfold or more)
+                auto shift = [](vec8& v, int d) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) v[e] = (T)__builtin_ldexpf((float)v[e], d);
+                };
+                shift(w_hi, k - k_w);
+                shift(w_lo, k - k_w);
+                shift(o_hi, k - k_o);
+                shift(o_lo, k - k_o);
+#pragma unroll
+                for (int db = 0; db < NDB; ++db)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[db][r] = __builtin_ldexpf(acc[db][r], k - k_acc);
+                k_acc = k;
+            }
+        }
         float4v other[2];
         if constexpr (WITH_A) {
             other[0] = *(const float4v*)(x1 + (1 - role) * 2048);
             other[1] = *(const float4v*)(x1 + (1 - role) * 2048 + 1024);
         }
         vec8 n_hi, n_lo;
+        auto split = [&](int r, float x) __attribute__((always_inline)) {
+            const T hi = (T)x;
+            n_hi[r] = hi;
+            n_lo[r] = (T)(x - (float)hi);
+        };
+        [[maybe_unused]] const float two_k = __builtin_bit_cast(float, (127 + k_acc) << 23);
         auto soft = [&](int r) __attribute__((always_inline)) {
             if constexpr (WITH_A) {
                 const float a = f[r], o = other[r / 4][r % 4];
@@ -271,9 +310,11 @@ __device__ __forceinline__ void bwd_wide_item(const SdpaBwdParams& bp, char* sme
                     x = __builtin_amdgcn_exp2f(__builtin_fmaf(s, c2, nl[r / 4][r % 4])) * (d + nd[r / 4][r % 4]);
                 } else
                     x = __builtin_amdgcn_exp2f(__builtin_fmaf(a + o, c2, nl[r / 4][r % 4]));
-                const T hi = (T)x;
-                n_hi[r] = hi;
-                n_lo[r] = (T)(x - (float)hi);
+                if constexpr (SCALED) {
+                    f[r] = x;
+                    split(r, x * two_k);
+                } else
+                    split(r, x);
             }
         };
         if constexpr (WITH_B) {
@@ -299,6 +340,21 @@ __device__ __forceinline__ void bwd_wide_item(const SdpaBwdParams& bp, char* sme
         } else {
 #pragma unroll
             for (int r = 0; r < 8; ++r) soft(r);
+        }
+        if constexpr (WITH_A && SCALED) {
+            k_w = k_acc;
+            float top = 0.0f;
+#pragma unroll
+            for (int r = 0; r < 8; ++r) top = fmaxf(top, fabsf(f[r]));
+            constexpr float LIMIT = 1 << BW_TOP;
+            if (__builtin_amdgcn_ballot_w64(top * two_k > LIMIT)) {
+                top = xor32_max(top);      // (the other half of the row's values)
+                if (top * two_k > LIMIT) k_w = BW_AIM + 127 - (__builtin_bit_cast(int, top) >> 23);
+                const float two_w = __builtin_bit_cast(float, (127 + k_w) << 23);
+#pragma unroll
+                for (int r = 0; r < 8; ++r) split(r, f[r] * two_w);
+            }
+            x3[role * 64] = k_w;
         }
         if constexpr (WITH_A) {      // (the partner has read tile t - 1's before this step's barrier)
             w_hi = n_hi;
@@ -341,7 +397,7 @@ __device__ __forceinline__ void bwd_wide_item(const SdpaBwdParams& bp, char* sme
     }
 
     // ---- out: this role's half of the columns -----------------------------------------------------------------------------------
-    const float out_scale = ROLE == BW_DV ? 1.0f : p.scale;
+    const float unit = ROLE == BW_DV ? 1.0f : p.scale, out_scale = SCALED ? __builtin_ldexpf(unit, -k_acc) : unit;
     const int width = ROLE == BW_DV ? p.Dv : p.D, c0 = role * (BW_D / 2);
     if (mine >= (ROLE == BW_DQ ? rows_b : kv_len)) {      // padding rows and keys past the count: zeros
 #pragma unroll

@@ -835,3 +835,87 @@ def test_backward_with_the_smallest_workspace(gpu, case):
     with pytest.raises(capi.RocmError) as e:
         capi.sdpa_bwd(bd)
     assert e.value.code == capi.EWORKSPACE
+
+
+class Gradients:
+    """One forward with row normalisers, and backward calls on what it left, by whichever kernels a call names."""
+
+    def __init__(self, q, k, v, go, dtype, **kw):
+        self.dtype = dtype
+        self.t = {n: host.DeviceTensor.from_f32(x, dtype) for n, x in (("q", q), ("k", k), ("v", v), ("d_o", go))}
+        self.t["o"] = host.DeviceTensor(go.shape, dtype)
+        for n in ("q", "k", "v"):
+            self.t["d_" + n] = host.DeviceTensor(self.t[n].shape, dtype)
+        self.lens = {n: capi.DeviceBuffer.from_numpy(np.asarray(kw.pop(n), np.int32)) for n in ("kv_lens", "q_lens") if kw.get(n) is not None}
+        self.lse = capi.DeviceBuffer(int(np.prod(go.shape[:3])) * 4)
+        self.bd = bd = capi.SdpaBwdDesc()
+        bd.fwd = host.make_desc(self.t["q"], self.t["k"], self.t["v"], self.t["o"], lse=self.lse, **{**kw, **self.lens})
+        self.fws = capi.DeviceBuffer(max(capi.sdpa_workspace(bd.fwd)[0], 256))
+        bd.fwd.workspace, bd.fwd.workspace_bytes = self.fws.ptr, self.fws.nbytes
+        for n in ("d_o", "d_q", "d_k", "d_v"):
+            setattr(bd, n, self.t[n].ptr)
+            for a, s in enumerate(host._strides3(self.t[n].shape)):
+                getattr(bd, n + "_stride")[a] = s
+        capi.sdpa_fwd(bd.fwd)
+        capi.sync()
+
+    def workspace(self, impl):
+        self.bd.fwd.impl = impl
+        return capi.sdpa_bwd_workspace(self.bd)
+
+    def run(self, impl):
+        ws = capi.DeviceBuffer(self.workspace(impl))
+        self.bd.workspace, self.bd.workspace_bytes = ws.ptr, ws.nbytes
+        capi.sdpa_bwd(self.bd)
+        capi.sync()
+        ws.free()
+        return [self.t[n].to_f32() for n in ("d_q", "d_k", "d_v")]
+
+
+def step_of(x, dtype):
+    """The distance between neighbouring values of the storage type at magnitude x."""
+    bits, least = (11, -24) if dtype == capi.F16 else (8, -133)
+    return 2.0 ** np.maximum(np.floor(np.log2(np.maximum(np.abs(x), 2.0 ** -140))) + 1 - bits, least)
+
+
+def assert_same_but_for_the_last_rounding(name, got, ref, dtype):
+    """Both rounded from sums whose terms are exact to 16 bits (bf16) or 22 (f16) at least, where the storage type has 8 and 11: a result
+    is the neighbouring value where the two sums lie on either side of a rounding border, about one in 2^8 of them; with terms
+    rounded to the storage type once, one in three or four.  (A result far below its row's others is looked at in their steps.)"""
+    rms = np.sqrt((ref.astype(np.float64) ** 2).mean(-1, keepdims=True))
+    assert np.isfinite(got).all() and np.isfinite(ref).all(), name
+    steps = np.abs(got.astype(np.float64) - ref) / step_of(np.maximum(np.abs(ref), rms), dtype)
+    say("   %s: %.2e of the results differ, by %.2f steps at most" % (name, (got != ref).mean(), steps.max()))
+    assert steps.max() <= 1.0, name
+    assert (got != ref).mean() <= 2.0 ** -5, name
+
+
+@pytest.mark.parametrize("parts", ["1", "4"])
+@pytest.mark.parametrize("dtype", [capi.BF16, capi.F16], ids=lambda x: dtypes.NAMES[x])
+@pytest.mark.parametrize("magnitudes", ["one", "small", "rising", "falling", "opposed_pair"])
+def test_backward_above_128_has_the_precision_of_f32_arithmetic(gpu, monkeypatch, parts, dtype, magnitudes):
+    """Head dimensions above 128 on the matrix cores against the generic kernels' f32 arithmetic on the same forward: gradients of any
+    magnitude that the storage type holds.  small: an unscaled mean loss; rising, falling: the rows of dO and V over a
+    factor of 2^16, so that in either walk what a row has to hold grows again and again, or only shrinks; opposed_pair: two keys with equal
+    scores and opposed values under a scaled loss, whose dS pass what f16 holds while the gradients do not come near it."""
+    monkeypatch.setenv("INCIN_ROCM_BWD_PARTS", parts)
+    say("backward above 128 against f32 arithmetic: %s, %s, %s parts" % (magnitudes, dtypes.NAMES[dtype], parts))
+    if magnitudes == "opposed_pair":
+        B, Hq, Hkv, Sq, Skv, D, Dv, causal = 1, 2, 1, 50, 2, 256, 256, False
+    else:
+        B, Hq, Hkv, Sq, Skv, D, Dv, causal = 2, 4, 2, 333, 420, 256, 192, True
+    q, k, v, go = make_d(241, B, Hq, Hkv, Sq, Skv, D, Dv, dtype)
+    if magnitudes == "small":
+        go *= 2.0 ** -10
+    elif magnitudes in ("rising", "falling"):
+        up = lambda n: (2.0 ** np.linspace(-8, 8, n)[:: 1 if magnitudes == "rising" else -1]).astype(np.float32)[:, None]
+        go, v = go * up(Sq) / 16, v * up(Skv) / 16
+    elif magnitudes == "opposed_pair":
+        q, go = q / 64, np.full_like(go, 512.0)
+        v[:, :, 0], v[:, :, 1] = 1.0, -1.0
+    q, go, v = (dtypes.round_to(x, dtype) for x in (q, go, v))
+    g = Gradients(q, k, v, go, dtype, causal=causal)
+    if parts == "4" and magnitudes != "opposed_pair":      # (planes of f32 sums: the generic kernels have none)
+        assert g.workspace(capi.IMPL_AUTO) > g.workspace(capi.IMPL_GENERIC)
+    for name, a, b in zip(("dq", "dk", "dv"), g.run(capi.IMPL_AUTO), g.run(capi.IMPL_GENERIC)):
+        assert_same_but_for_the_last_rounding(name, a, b, dtype)
