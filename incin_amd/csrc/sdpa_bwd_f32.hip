@@ -754,7 +754,12 @@ static hipError_t launch_bwd_f32_t(const SdpaBwdParams& bp0, hipStream_t stream)
     }
     p.interleave = work_interleave(p.causal != 0 || p.mask != nullptr, (D == 128 || RW == 4 ? 1 : 2) * device_cus() / 8, p.G, nqb, (total & 7) == 0 ? total >> 3 : total);
     p.deal_groups = (total & 7) == 0 ? work_deal(p.interleave, p.G, nqb, total >> 3, p.causal != 0 || p.mask != nullptr) : 0;
-    hipLaunchKernelGGL((bwd_f32_kernel<D, DC, RW, DENSE>), dim3((unsigned)(n_dkv + n_dq)), dim3(256), 0, stream, bp, (int)n_dkv);
+    auto launch = [&](int64_t blocks, int64_t n) { hipLaunchKernelGGL((bwd_f32_kernel<D, DC, RW, DENSE>), dim3((unsigned)blocks), dim3(256), 0, stream, bp, (int)n); };
+    if (n_dkv + n_dq <= max_blocks(256)) launch(n_dkv + n_dq, n_dkv);
+    else {
+        if (n_dkv > 0) launch(n_dkv, n_dkv);
+        if (n_dq > 0) launch(n_dq, 0);
+    }
     if (bp.parts_q > 1 || bp.parts_kv > 1) {
         const AddPlanesJob jq = {(float*)bp.d_q, bp.part_dq, bp.dq_sb, bp.dq_sh, bp.dq_ss, p.B, p.Hq, p.Sq, p.D, bp.parts_q - 1};
         const AddPlanesJob jk = {(float*)bp.d_k, bp.part_dk, bp.dk_sb, bp.dk_sh, bp.dk_ss, p.B, p.Hkv, p.Skv, p.D, bp.parts_kv - 1};

@@ -433,7 +433,7 @@ __device__ __forceinline__ void bwd_wide_item(const SdpaBwdParams& bp, char* sme
 // blocks of every head - dK and dV blocks of all (batch, KV head) pairs, then dQ blocks of all heads, the pairs innermost, so that
 // with a multiple of 8 pairs one XCD has all items of a pair.
 template <typename T>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void sdpa_bwd_wide_kernel(SdpaBwdParams bp)
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void sdpa_bwd_wide_kernel(SdpaBwdParams bp, int first)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
     __shared__ __attribute__((aligned(1024))) char smem[3 * BW_STAGE + BW_XCHG];
@@ -441,7 +441,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int nqb = (p.Sq + BW_ROWS - 1) / BW_ROWS, nkb = (p.Skv + BW_ROWS - 1) / BW_ROWS;
     const int pairs = p.B * p.Hkv, parts = bp.parts_kv;
     const int kv_items = 2 * parts * pairs, q_items = p.G * pairs, both = min(nqb, nkb);
-    int id = blockIdx.x, rank;
+    int id = first + (int)blockIdx.x, rank;
     bool kv;
     if (id < both * (kv_items + q_items)) {
         rank = id / (kv_items + q_items);
@@ -472,9 +472,12 @@ hipError_t launch_sdpa_bwd_wide(const SdpaBwdParams& bp, int dtype, hipStream_t 
     if (total > 0x7fffffffLL) return hipErrorInvalidValue;
     hipError_t e = launch_sdpa_bwd_delta(bp, dtype, stream);
     if (e != hipSuccess) return e;
-    if (dtype == 1) hipLaunchKernelGGL((sdpa_bwd_wide_kernel<f16_t>), dim3((unsigned)total), dim3(512), 0, stream, bp);
-    else hipLaunchKernelGGL((sdpa_bwd_wide_kernel<bf16_t>), dim3((unsigned)total), dim3(512), 0, stream, bp);
-    e = hipGetLastError();
+    for (int64_t first = 0; first < total && e == hipSuccess; first += max_blocks(512)) {
+        const dim3 grid((unsigned)min(total - first, max_blocks(512)));
+        if (dtype == 1) hipLaunchKernelGGL((sdpa_bwd_wide_kernel<f16_t>), grid, dim3(512), 0, stream, bp, (int)first);
+        else hipLaunchKernelGGL((sdpa_bwd_wide_kernel<bf16_t>), grid, dim3(512), 0, stream, bp, (int)first);
+        e = hipGetLastError();
+    }
     if (e == hipSuccess && bp.parts_kv > 1) e = launch_sdpa_bwd_sum_planes(bp, dtype, stream);
     return e;
 }

@@ -919,3 +919,48 @@ def test_backward_above_128_has_the_precision_of_f32_arithmetic(gpu, monkeypatch
         assert g.workspace(capi.IMPL_AUTO) > g.workspace(capi.IMPL_GENERIC)
     for name, a, b in zip(("dq", "dk", "dv"), g.run(capi.IMPL_AUTO), g.run(capi.IMPL_GENERIC)):
         assert_same_but_for_the_last_rounding(name, a, b, dtype)
+
+
+@pytest.mark.parametrize("case", [
+    # dtype, B, heads, D: one query over one key; more blocks of all gradients together than one launch takes, though not of any one
+    (capi.BF16, 60000, 48, 256),
+    (capi.F32, 60000, 150, 68),
+], ids=["wide", "f32"])
+def test_backward_of_more_heads_than_one_launch_takes(gpu, case):
+    """Heads of one query and one key, the inputs the same in every batch entry (strides of 0): P = 1, so dV is dO (P to 1e-5: in bf16
+    the same or the neighbouring value) and dQ, dK are what rounding leaves of dP - D = 0."""
+    dtype, B, H, D = case
+    say("backward of %d x %d heads, %s, D = %d" % (B, H, dtypes.NAMES[dtype], D))
+    r = np.random.Generator(np.random.PCG64(251))
+    q, k, v, go = (dtypes.round_to(r.standard_normal((1, H, 1, D), dtype=np.float32), dtype) for _ in range(4))
+    scale = host.resolve_scale(None, D)
+    lse = np.broadcast_to((q.astype(np.float64) * k).sum(-1).reshape(1, H) * scale, (B, H)).astype(np.float32)
+    ins = [host.DeviceTensor.from_f32(x, dtype) for x in (q, k, v, v, go)]      # (O is V)
+    size = dtypes.ITEMSIZE[dtype]
+    grads = [capi.DeviceBuffer(B * H * D * size) for _ in range(3)]
+    for g in grads:
+        capi.check(capi.load().incin_rocm_memset(0, g.ptr, 0x7f, g.nbytes))
+    tl = capi.DeviceBuffer.from_numpy(np.ascontiguousarray(lse))
+    bd = capi.SdpaBwdDesc()
+    bd.fwd = host.make_desc(*ins[:4], lse=tl)
+    bd.fwd.B = B
+    for name in ("q_stride", "k_stride", "v_stride", "o_stride"):
+        getattr(bd.fwd, name)[0] = 0
+    bd.d_o = ins[4].ptr
+    bd.d_q, bd.d_k, bd.d_v = (g.ptr for g in grads)
+    for name in ("d_o", "d_q", "d_k", "d_v"):
+        for a, s in enumerate((0 if name == "d_o" else H * D, D, D)):
+            getattr(bd, name + "_stride")[a] = s
+    ws = capi.DeviceBuffer(capi.sdpa_bwd_workspace(bd))
+    bd.workspace, bd.workspace_bytes = ws.ptr, ws.nbytes
+    capi.sdpa_bwd(bd)
+    capi.sync()
+    most = float(np.abs(v).max() * np.abs(go).max() * D)
+    for b in list(range(0, B, 997)) + [B - 1]:
+        for g, name in zip(grads, ("dq", "dk", "dv")):
+            raw = np.empty((H, D), dtypes.storage_numpy_dtype(dtype))
+            capi.check(capi.load().incin_rocm_memcpy_d2h(0, raw.ctypes.data, g.ptr + b * raw.nbytes, raw.nbytes))
+            x, ref = dtypes.decode(raw, dtype), go[0, :, 0] if name == "dv" else 0.0
+            assert np.isfinite(x).all() and (np.abs(x - ref) <= (np.abs(ref) * (2.0 ** -7 if dtype == capi.BF16 else 1e-5) if name == "dv" else 1e-5 * most)).all(), (b, name)
+    for x in grads:
+        x.free()
