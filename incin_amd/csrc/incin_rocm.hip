@@ -450,6 +450,7 @@ void fill_params(const incin_rocm_sdpa_desc_t* d, const Plan& plan, SdpaParams* 
     p->deal_groups = 0;
     p->num_splits = plan.splits;
     p->split_len = plan.split_len;
+    p->split_turn = incin_rocm::split_turn_of(d->kv_lens != nullptr, p->B, plan.splits);
     if (plan.impl == INCIN_ROCM_IMPL_MFMA) p->mask_flags = d->add_mask ? (const uint8_t*)d->workspace : nullptr;
     if (plan.impl == INCIN_ROCM_IMPL_MFMA && d->add_mask && plan.lims_offset) p->mask_lims = (const int32_t*)((const char*)d->workspace + plan.lims_offset);
     if (!(plan.impl == INCIN_ROCM_IMPL_MFMA && d->add_mask)) p->ws_acc = (float*)d->workspace;
@@ -811,6 +812,7 @@ static int launch_fwd(const incin_rocm_sdpa_desc_t* desc, const Plan& plan, void
                 if (plan.lims_splitkv) {
                     SdpaParams pl = p;
                     pl.num_splits = 1;
+                    pl.split_turn = 0;
                     pl.split_len = (int)((desc->Skv + 255) / 256 * 256);
                     e = incin_rocm::launch_sdpa_decode_f32_limits(pl, s);
                     if (e != hipSuccess) break;

@@ -30,6 +30,7 @@ struct SdpaParams {
     // split-KV only
     int32_t num_splits;
     int32_t split_len;         // keys per split (multiple of the kernel's key tile)
+    int32_t split_turn;        // largest shift of work_split (a power of two minus one; 0: none)
     float* ws_acc;             // [B, Hq, Sq, num_splits, Dp] f32 partial numerators (Dp == Dv for the vector-ALU kernel)
     float* ws_ml;              // [B, Hq, Sq, num_splits, 2]  running max (natural-log domain) and denominator
     // matrix-core prefill kernels with a dense mask: one byte per block of 32 query rows x 32 keys (0 mixed, 1 all zero,
@@ -75,18 +76,25 @@ __device__ __forceinline__ const int32_t* mask_lims_of(const SdpaParams& p, int 
 }
 
 // Which split of the keys a workgroup of a split-KV launch takes (grid: x splits, y and z groups; group is the (batch, KV head)
-// pair).  Workgroups reach the 8 XCDs round-robin in dispatch order, so an even number of splits by itself gives an XCD the
+// pair): x, shifted from group to group by up to split_turn where the launcher asks for that.
+// Workgroups reach the 8 XCDs round-robin in dispatch order, so an even number of splits by itself gives an XCD the
 // same few splits of every group; with key counts the last splits of short sequences are empty, and the XCDs that hold them run
-// out of work.  There the splits are dealt to x shifted from group to group, by 0 .. d - 1 with d = 2, 4 or 8 the power of two in the
+// out of work.  There split_turn is d - 1 with d = 2, 4 or 8 the power of two in the
 // number of splits; g + g / 2 + g / 4 takes every such value whatever g is modulo 2, 4 or 8.  Counts spread from an eighth of the
 // capacity to all of it, us before and after: 33 sequences x 8 KV heads x 4096 x 64 (8 splits) 39.7 -> 29.6, 24 31.2 -> 25.4, 16 x 2 x 32768 x
 // 128 (8) 68.3 -> 59.4, 8 x 8 x 8192 x 128 (8) 39.1 -> 34.8, f32 8 x 8 x 4096 39.7 -> 36.3, 64 x 1 x 60000 (4) 196 -> 182; 4 sequences level, 2 or 3
-// have little to balance (17.0 / 17.5) and are left alone.
+// have little to balance (17.0 / 17.5) and are left alone.  (The host decides: worked out by every workgroup, the rule cost the
+// launches that it leaves alone 0.2 - 0.5 us - 8 x 1 x 60000 44.7 without it, 45.3 so, 44.7 now; 8 x 12 x 2048 x 256 50.7 / 51.0 / 50.8.)
+inline int split_turn_of(bool key_counts, int B, int num_splits)
+{
+    const int d = num_splits & -num_splits;
+    return key_counts && B >= 4 && num_splits > 1 ? (d < 8 ? d : 8) - 1 : 0;
+}
 __device__ __forceinline__ int work_split(const SdpaParams& p, int group)
 {
-    const int x = blockIdx.x, d = p.num_splits & -p.num_splits;
-    if (!p.kv_lens || d == 1 || p.B < 4) return x;
-    const int y = x + ((group + (group >> 1) + (group >> 2)) & (min(d, 8) - 1));
+    const int x = blockIdx.x;
+    if (p.split_turn == 0) return x;
+    const int y = x + ((group + (group >> 1) + (group >> 2)) & p.split_turn);
     return y >= p.num_splits ? y - p.num_splits : y;
 }
 
