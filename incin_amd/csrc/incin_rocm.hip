@@ -18,6 +18,7 @@
 #include "kv_append.h"
 #include "sdpa_bwd.h"
 #include "sdpa_params.h"
+#include "side_stream.h"
 
 namespace incin_rocm {
 hipError_t launch_sdpa_generic(const SdpaParams& p, int dtype, hipStream_t stream);
@@ -1229,6 +1230,8 @@ int incin_rocm_sdpa_bwd(const incin_rocm_sdpa_bwd_desc_t* bd, void* stream)
     if (e != hipSuccess) return hip_fail(e, "attention backward launch");
     return 0;
 }
+
+uint64_t incin_rocm_side_stream_forks(void) { return incin_rocm::side_stream_forks().load(std::memory_order_relaxed); }
 
 size_t incin_rocm_sizeof_kv_append_desc(void) { return sizeof(incin_rocm_kv_append_desc_t); }
 

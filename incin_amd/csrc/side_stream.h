@@ -19,6 +19,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
@@ -41,6 +42,13 @@ inline std::vector<SideStreamSet>& side_stream_pool()
 {
     static std::vector<SideStreamSet>* pool = new std::vector<SideStreamSet>();      // (never freed: streams outlive static destructors)
     return *pool;
+}
+
+// Forks since the process began: what tells a test that a call did use a second stream.
+inline std::atomic<uint64_t>& side_stream_forks()
+{
+    static std::atomic<uint64_t> n{0};
+    return n;
 }
 
 class SideStreamLease {
@@ -96,7 +104,9 @@ public:
     hipError_t fork()
     {
         hipError_t e = hipEventRecord(set_.fork, main_);
-        return e != hipSuccess ? e : hipStreamWaitEvent(set_.stream, set_.fork, 0);
+        if (e == hipSuccess) e = hipStreamWaitEvent(set_.stream, set_.fork, 0);
+        if (e == hipSuccess) side_stream_forks().fetch_add(1, std::memory_order_relaxed);
+        return e;
     }
     // the main stream waits for everything enqueued on the side stream so far
     hipError_t join()

@@ -285,6 +285,8 @@ size_t incin_rocm_sizeof_sdpa_bwd_desc(void);
 int incin_rocm_sdpa_bwd_workspace(const incin_rocm_sdpa_bwd_desc_t* desc, size_t* bytes);
 int incin_rocm_sdpa_bwd(const incin_rocm_sdpa_bwd_desc_t* desc, void* stream);
 
+/* How many backward calls of this process have put a kernel on a second stream so far (any device, any thread). */
+uint64_t incin_rocm_side_stream_forks(void);
 /* ---- diagnostics ------------------------------------------------------------------
  * No counterpart in the reference.  One launch of a loop of bf16 matrix instructions (v_mfma_f32_32x32x16_bf16, one
  * workgroup of two wavefronts per SIMD on every compute unit, `iterations` x 4 instructions per wavefront) whose operands

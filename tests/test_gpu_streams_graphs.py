@@ -264,12 +264,13 @@ class BackwardPair:
 
 @pytest.mark.parametrize("dtype, D", [(capi.BF16, 128), (capi.BF16, 64), (capi.F32, 128), (capi.F32, 64)],
                          ids=["bf16_d128", "bf16_d64", "f32_d128", "f32_d64"])
-def test_backward_with_its_dq_kernel_on_a_side_stream(gpu, dtype, D, monkeypatch):
+def test_backward_with_its_dq_kernel_on_a_side_stream(gpu, dtype, D, monkeypatch, **sizes):
     """A backward call short of work puts its dQ kernel on a stream of the library's own beside the dK/dV kernel and joins
     the caller's stream afterwards.  Against the same calls held to one stream (INCIN_ROCM_BWD_STREAMS=1): bit-identical
     gradients of two dependent calls, back to back on a stream of the caller's, and from three host threads at once, each on
-    a stream of its own with problems of its own (the library's streams come out of a shared pool)."""
-    pairs = [BackwardPair(500 + i, dtype, D) for i in range(3)]
+    a stream of its own with problems of its own (the library's streams come out of a shared pool).  (The rule takes the calls
+    of these sizes, and every f32 call, to one stream; the test below this one has calls that fork, and counts that they do.)"""
+    pairs = [BackwardPair(500 + i, dtype, D, **sizes) for i in range(3)]
     monkeypatch.setenv("INCIN_ROCM_BWD_STREAMS", "1")
     expect = []
     for p in pairs:
@@ -310,3 +311,63 @@ def test_backward_with_its_dq_kernel_on_a_side_stream(gpu, dtype, D, monkeypatch
     for i, (p, exp) in enumerate(zip(pairs, expect)):
         for name, got, e in zip(("dq1", "dk1", "dv1", "dq2", "dk2", "dv2"), p.read(), exp):
             assert np.array_equal(got, e), "thread %d, %s" % (i, name)
+
+
+@pytest.mark.parametrize("dtype, D, sizes", [
+    (capi.BF16, 128, dict(B=2, Hq=4, Hkv=2, S=1024)),       # the paired dK/dV kernel: 64 workgroups of it, walks of 16 tiles
+    (capi.F16, 128, dict(B=1, Hq=4, Hkv=4, S=2048)),        # ... without groups, walks undivided
+    (capi.BF16, 64, dict(B=1, Hq=16, Hkv=2, S=2048)),       # the one for narrow heads: eight parts of 32 tiles
+    (capi.F16, 96, dict(B=1, Hq=16, Hkv=2, S=2048)),
+], ids=["paired_dealt", "paired", "narrow64", "narrow96"])
+def test_backward_that_forks(gpu, dtype, D, sizes, monkeypatch):
+    """The test above at sizes whose calls fork, on any device of 256 compute units: one fork per call."""
+    forks = capi.load().incin_rocm_side_stream_forks
+    before = forks()
+    test_backward_with_its_dq_kernel_on_a_side_stream(gpu, dtype, D, monkeypatch, **sizes)
+    # two calls a run: once per pair on one stream (none forks), 5 repetitions of one pair, 15 of three in threads of their own
+    assert forks() - before == 2 * (5 + 3 * 15)
+
+
+@pytest.mark.parametrize("dtype, D, sizes", [
+    (capi.BF16, 256, dict(B=2, Hq=4, Hkv=2, S=300)),
+    (capi.F16, 256, dict(B=1, Hq=8, Hkv=1, S=600)),         # walks dealt to workgroups, planes
+], ids=["bf16_d256", "f16_d256_dealt_walks"])
+def test_backward_above_128_from_threads(gpu, dtype, D, sizes, monkeypatch):
+    """Head dimensions above 128 (one stream): two dependent calls, and three threads of them at once."""
+    test_backward_with_its_dq_kernel_on_a_side_stream(gpu, dtype, D, monkeypatch, **sizes)
+
+
+@pytest.mark.parametrize("dtype, D, sizes", [
+    (capi.BF16, 64, dict(B=2, Hq=4, Hkv=2, S=200)),         # the dK/dV kernel for narrow heads; a forward with all keys in LDS
+    (capi.BF16, 64, dict(B=1, Hq=16, Hkv=2, S=2048)),       # ... that forks outside a capture, walks dealt to workgroups
+    (capi.F16, 80, dict(B=2, Hq=4, Hkv=2, S=333)),
+    (capi.BF16, 256, dict(B=2, Hq=4, Hkv=2, S=300)),        # above 128
+    (capi.F16, 256, dict(B=1, Hq=8, Hkv=1, S=600)),         # ... walks dealt to workgroups
+    (capi.F32, 64, dict(B=1, Hq=8, Hkv=8, S=1259)),
+], ids=["narrow64", "narrow64_dealt_walks", "narrow96", "bf16_d256", "f16_d256_dealt_walks", "f32_d64_dealt_walks"])
+def test_dependent_backward_calls_in_a_graph(gpu, dtype, D, sizes):
+    """A forward and two dependent backward calls recorded into one launch graph: every replay gives the bytes of the eager calls,
+    with the program's own eager work between replays, and nothing of the capture runs on a second stream."""
+    pair = BackwardPair(600, dtype, D, **sizes)
+    pair.run()
+    capi.sync()
+    expect = pair.read()
+    say("graph capture: forward and two backward calls, dtype %d, D %d" % (dtype, D))
+    stream = capi.Stream()
+    before = capi.load().incin_rocm_side_stream_forks()
+    with capi.Graph.record(stream) as graph:
+        capi.sdpa_fwd(pair.descs[0].fwd, stream.ptr)
+        pair.run(stream.ptr)
+    assert capi.load().incin_rocm_side_stream_forks() == before
+    for replay in range(3):
+        pair.clear()
+        graph.launch()
+        stream.sync()
+        for name, got, e in zip(("dq1", "dk1", "dv1", "dq2", "dk2", "dv2"), pair.read(), expect):
+            assert np.array_equal(got, e), "%s, replay %d" % (name, replay)
+        pair.run()              # eager work of the program's own between replays
+        capi.sync()
+        for got, e in zip(pair.read(), expect):
+            assert np.array_equal(got, e)
+    graph.destroy()
+    stream.destroy()
