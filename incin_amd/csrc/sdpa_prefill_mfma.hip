@@ -1015,7 +1015,7 @@ static hipError_t launch_prefill_t(const SdpaParams& p0, hipStream_t stream)
 // elements (tile offsets fit the 32-bit buffer offset).
 hipError_t launch_sdpa_prefill_mfma(const SdpaParams& p, int dtype, hipStream_t stream)
 {
-    // (all keys of a head fit into LDS: never behind this file's kernel there; INCIN_ROCM_PREFILL_BLOCK_ROWS names a form of this one)
+    // (all keys of a head fit into LDS, and that kernel is ahead of this file's there; INCIN_ROCM_PREFILL_BLOCK_ROWS names a form of this one)
     if (prefill_short_fits(p) && !getenv("INCIN_ROCM_PREFILL_BLOCK_ROWS")) return launch_sdpa_prefill_short(p, dtype, stream);
     if (p.mask) {
         if (dtype == 1) return p.Dp == 128 ? launch_prefill_t<f16_t, 128, 1>(p, stream) : launch_prefill_t<f16_t, 64, 1>(p, stream);

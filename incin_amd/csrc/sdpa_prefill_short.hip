@@ -13,10 +13,10 @@
 // products; the next rows' Q fetched meanwhile.  Heads of up to 32 or 64 rows and keys come four or two to a workgroup, a
 // wavefront or two each, so that no wavefront idles.
 //
-// Measured against that kernel (f16 / bf16; us): 64 x 12 heads x 197 x 64 30.4 -> 24 (3.2 TB/s), 256 x 12 x 197 109 -> 84,
-// 256 x 16 x 64 38 -> 26 (5.2 TB/s), 256 x 12 x 17 28 -> 10, 119 x 16 x 43 x 128 29 -> 19, 64 x 32 / 8 x 128 x 128 causal 48 -> 34,
-// 32 x 12 x 224 causal 17.4 -> 13.3, 8 x 32 x 4096 rows over 77 keys 106 -> 63; level where a head's rows are one item per
-// wavefront already (64 x 16 x 128 x 128: 26.6, at the rate of a copy).
+// Measured against that kernel (f16 / bf16; us a call, calls back to back): 64 x 12 heads x 197 x 64 28.8 -> 25.1 (3.1 TB/s), 256 x 12 x 197 111 -> 90,
+// 256 x 16 x 64 39.4 -> 26.3 (5.1 TB/s), 256 x 12 x 17 28.0 -> 8.7, 119 x 16 x 43 x 128 29.6 -> 18.9, 64 x 32 / 8 x 128 x 128 causal 45.9 -> 35.7,
+// 32 x 12 x 224 causal 17.4 -> 14.5, 8 x 32 x 4096 rows over 77 keys 105 -> 73; behind it by up to a fifth in the launches that
+// tiles_are_ahead names, which stay with it.
 #include <algorithm>
 #include <type_traits>
 
@@ -266,17 +266,50 @@ static hipError_t launch_short_t(const SdpaParams& p, int64_t pairs, int64_t ite
     return launch_short<T, 64, 8, 4>(p, nb, pairs, chunks, stream);
 }
 
-bool prefill_short_fits(const SdpaParams& p) { return !p.mask && p.num_splits <= 1 && p.Skv >= 1 && p.Skv <= (p.Dp == 64 ? 256 : 128) && p.Dp <= 128; }
+// Workgroups per pair: as many as give every compute unit two, at most one item per wavefront; more only read K and V more often
+// (in us, by chunks: 8 x 12 heads x 197 keys 7.8 with 2, 10.5 with 1; 8 x 16 x 4096 rows over 77 keys at D = 128 66 / 62 / 57 / 66 / 108 with
+// 32 / 8 / 4 / 2 / 1; 64 x 12 x 197 27.8 with 2, 25 with 1).
+static int64_t short_chunks(int64_t pairs, int64_t items) { return std::min((items + 3) / 4, std::max<int64_t>(1, (2 * (int64_t)device_cus() + pairs - 1) / pairs)); }
+
+// Which of the launches whose keys fit come here: all but those that the kernel that walks tiles of 64 keys is ahead on.  That one's
+// workgroups are lighter - more of them on a compute unit - and where its last tile is nearly full and no wavefront here has a
+// second item whose Q rows arrive under the first, nothing is left to gain (us, tiles / here, bf16, no mask):
+//   D <= 64, 185 - 192 or 225 - 256 keys, one item per wavefront: 8 x 16 x 192 6.2 / 6.5, 20 x 16 x 192 11.9 / 12.7, 16 x 16 x 256 9.4 / 9.9, 8 x
+//     32 / 8 x 192 8.2 / 8.8; or a last round of workgroups at most a quarter full: 36 x 16 x 256 22.1 / 23.5, 66 x 16 x 256 36.1 / 37.0 (but
+//     32 x 16 x 256 19.3 / 17.4, 42 x 16 x 192 20.4 / 19.2, 20 x 16 x 161 13.3 / 13.0; with a causal mask 16 x 16 x 256 9.8 / 9.3);
+//   D <= 64, more than 160 keys, at most 128 rows, more than a round: 64 x 16 x 64 rows over 256 keys 17.6 / 21.4, over 200 18.0 / 19.4 (over 160
+//     16.6 / 16.1);
+//   D > 64, 97 - 128 keys, at most 128 rows, more than a round: 64 x 16 x 128 25.0 / 26.2, 48 x 16 20.7 / 21.6, causal 20.7 / 21.3; level from seven
+//     workgroups per compute unit on (128 x 16 46.9 / 46.3), and D <= 96, whose products are the fewer there, from one to ten: 64 x 16 x
+//     128 x 96 22.3 / 24.0, 18 x 16 8.7 / 9.2 (160 x 16 50.9 / 51.0; 64 x 16 x 100 x 80 19.3 / 19.2); 49 - 64 keys under 97 - 128 rows 19.2 / 20.4.
+static bool tiles_are_ahead(const SdpaParams& p)
+{
+    const int64_t cus = device_cus(), pairs = (int64_t)p.B * p.Hkv, items = ((int64_t)(p.Sq + 31) / 32) * p.G;
+    if (3 * p.G * ((p.Sq + 127) / 128) > 4 * ((items + 3) / 4)) return false;      // (its blocks of 128 rows of one head would be half empty)
+    if (p.Dp == 64) {
+        if (p.causal || p.Skv <= 160) return false;
+        if (items <= 4 && pairs > 2 * cus) return true;
+        if (!(p.Skv > 224 || (p.Skv > 184 && p.Skv <= 192))) return false;
+        const int64_t chunks = short_chunks(pairs, items), round = 2 * cus, blocks = pairs * chunks, last = blocks % round;
+        return 4 * chunks >= items || (blocks > round && blocks < 3 * round && last > 0 && 4 * last <= round);
+    }
+    if (items > 4) return false;
+    const bool wide = p.D > 96 || p.Dv > 96;
+    if (pairs <= (wide || p.causal ? 2 : 1) * cus || pairs >= (wide ? 7 : 10) * cus) return false;
+    if (p.Skv > (p.causal ? 112 : wide ? 96 : 100)) return p.Sq > 32;
+    return !p.causal && p.Skv > 48 && p.Skv <= 64 && p.Sq > 96 && pairs > 2 * cus;
+}
+bool prefill_short_fits(const SdpaParams& p)
+{
+    return !p.mask && p.num_splits <= 1 && p.Skv >= 1 && p.Skv <= (p.Dp == 64 ? 256 : 128) && p.Dp <= 128 && !tiles_are_ahead(p);
+}
 
 // Host has validated what sdpa_prefill_mfma.hip asks for; the keys fit (prefill_short_fits).
 hipError_t launch_sdpa_prefill_short(const SdpaParams& p, int dtype, hipStream_t stream)
 {
     const int64_t pairs = (int64_t)p.B * p.Hkv;
     const int64_t items = ((int64_t)(p.Sq + 31) / 32) * p.G;      // 32-row items of a pair
-    // Workgroups per pair: as many as give every compute unit two, at most one item per wavefront; more only read K and V more often
-    // (in us, by chunks: 8 x 12 heads x 197 keys 7.8 with 2, 10.5 with 1; 8 x 16 x 4096 rows over 77 keys at D = 128 66 / 62 / 57 / 66 / 108 with
-    // 32 / 8 / 4 / 2 / 1; 64 x 12 x 197 27.8 with 2, 25 with 1).
-    const int64_t chunks = std::min((items + 3) / 4, std::max<int64_t>(1, (2 * (int64_t)device_cus() + pairs - 1) / pairs));
+    const int64_t chunks = short_chunks(pairs, items);
     if (pairs * chunks > 0x7fffffffLL) return hipErrorInvalidValue;
     return dtype == 1 ? launch_short_t<f16_t>(p, pairs, items, (int)chunks, stream) : launch_short_t<bf16_t>(p, pairs, items, (int)chunks, stream);
 }

@@ -1395,6 +1395,36 @@ def test_prefill_with_all_keys_in_lds(gpu, dtype, shape):
         assert not seen.any() or np.abs(a[seen] - r[seen]).max() <= (2e-2 if dtype == capi.BF16 else 3e-3)
 
 
+@pytest.mark.parametrize("dtype", [capi.BF16, capi.F16], ids=lambda x: dtypes.NAMES[x])
+@pytest.mark.parametrize("case", [
+    # B, Hq, Hkv, Sq, Skv, D, causal, whether the kernel that walks tiles takes it (256 compute units)
+    (2, 2, 2, 256, 256, 64, False, True),             # nearly full tiles, one item of 32 rows per wavefront
+    (2, 4, 2, 192, 192, 64, False, True),
+    (2, 2, 2, 256, 256, 64, True, False),
+    (2, 2, 2, 200, 200, 64, False, False),
+    (2, 4, 1, 32, 256, 64, False, False),             # blocks of 128 rows would be a quarter full
+    (33, 16, 16, 40, 200, 64, False, True),           # few rows, more than a round of workgroups
+    (33, 16, 16, 40, 160, 64, False, False),
+    (33, 16, 16, 100, 128, 128, True, True),
+    (33, 16, 16, 100, 96, 128, False, False),
+    (17, 16, 16, 60, 128, 80, False, True),
+    (17, 16, 16, 100, 100, 80, False, False),
+], ids=lambda c: "x".join(str(x) for x in c[:6]) + ("causal" if c[6] else ""))
+def test_which_prefill_kernel_takes_short_keys(gpu, monkeypatch, dtype, case):
+    """Launches whose keys fit into LDS at once but which the kernel that walks tiles is ahead on are that kernel's: the bytes of a call that names
+    one of its forms, and others where the exponents are taken from another maximum."""
+    B, Hq, Hkv, Sq, Skv, D, causal, tiles = case
+    say("prefill over short keys: %s %r" % (dtypes.NAMES[dtype], case))
+    q, k, v = inputs(1700 + Sq + Skv, B, Hq, Hkv, Sq, Skv, D, D, dtype)
+    got = host.sdpa(q, k, v, dtype, causal=causal, impl=capi.IMPL_MFMA)
+    monkeypatch.setenv("INCIN_ROCM_PREFILL_BLOCK_ROWS", "128")
+    named = host.sdpa(q, k, v, dtype, causal=causal, impl=capi.IMPL_MFMA)
+    if capi.device_info(0).compute_units == 256:
+        assert np.array_equal(got, named) == tiles
+    ref = oracle_full(q[-1:], k[-1:], v[-1:], G=Hq // Hkv, causal=causal)
+    check(got[-1:], ref, TOL[dtype], "output")
+
+
 @pytest.mark.parametrize("D,Dv", [(68, 96), (80, 80), (96, 72), (96, 96), (100, 96), (96, 100)])
 def test_f32_kernels_up_to_96_columns(gpu, D, Dv):
     """Head dimensions of 65 - 96 on the f32 prefill kernel and the split-KV kernel's 32-row form multiply 96 columns of the 128-column layout: both sides of
