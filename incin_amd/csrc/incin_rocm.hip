@@ -1048,24 +1048,41 @@ static int bwd_wide_parts(const incin_rocm_sdpa_desc_t* d)
 // f32 (kind 2): one launch holds the blocks of dQ and of dK / dV, four wavefronts a workgroup (sdpa_bwd_f32.hip).
 //
 // How many of the four share the walk of one block of 32 rows or keys (the others take more blocks beside it): the more share, the
-// more and the shorter the items, and the more each tile that is copied into LDS costs.  Head dimensions above 64: two (one leaves
-// 1.02 - 1.7 times the time, everywhere).  Up to 64: four - whose tiles fill a compute unit with one workgroup - where that gives
-// at most one workgroup per compute unit, two up to eight rounds of two workgroups per compute unit.  Measured, backward
-// call, causal, 1 / 2 / 4 sharing: 4 heads x 300 51 / 31 / 24 us, 8 x 512 (not causal) 76 / 44 / 29, 56 x 65 21.2 / 18.8 / 21.8,
-// 32 x 1024 234 / 143 / 204, 64 x 2048 969 / 987 / 1368.
+// more and the shorter the items, and the more each tile that is copied into LDS costs.  Measured, backward call:
+// Head dimensions up to 64: four - whose tiles fill a compute unit with one workgroup - where that gives at most one workgroup per
+// compute unit; one from eight rounds of two workgroups per compute unit on; two between.  1 / 2 / 4 sharing, causal: 4 heads x 300 51 / 31 /
+// 24 us, 8 x 512 (not causal) 76 / 44 / 29, 56 x 65 21.2 / 18.8 / 21.8, 32 x 1024 234 / 143 / 204, 64 x 2048 969 / 987 / 1368.  And one where that issues
+// fewer products - blocks of 128 walked in 32s, against blocks of 64 in 64s - and there are items enough: 1000 heads x 65 112 / 156,
+// 300 x 96 49 / 58, 400 x 200 197 / 220, causal 300 x 65 48 / 50, 400 x 200 159 / 164, but 200 x 200 99 / 92.
+// Above 64: two, or one where that issues no more products, from two workgroups per compute unit on - under a mask, whose longer items
+// then end the launch, from four if there are grouped queries or as many products; grouped queries without one, whose dK / dV walks are
+// dealt below, from one and a quarter.  D = 128, 1 / 2 sharing: 1000 heads x 65 266 / 404, 1000 x 96 297 / 416, 250 x 200 270 / 338, 2048 x 128 775 / 896,
+// 128 x 1024 2104 / 2266, 32 x 1024 527 / 552, 16 on 4 x 2048 1045 / 1069, but 16 x 1024 305 / 280, 500 x 190 478 / 430, 1024 x 60 200 / 156; causal 1000 x 65
+// 261 / 325, 128 x 2048 4418 / 4647, 512 x 512 1490 / 1530, 8 x 16384 16206 / 16556, but 48 x 1024 504 / 499, 128 x 256 151 / 128, 8 x 1024 169 / 112.
 static int bwd_f32_share(const incin_rocm_sdpa_desc_t* d)
 {
-    if (d->D > 64 || d->Dv > 64) return 2;
     const int64_t cus = compute_units_of(d->device);
-    auto blocks = [&](int64_t own) { return ((d->Skv + own - 1) / own * d->Hkv + (d->Sq + own - 1) / own * d->Hq) * d->B; };
-    return blocks(32) <= cus ? 4 : blocks(64) < 16 * cus ? 2 : 1;
+    const bool wide = d->D > 64 || d->Dv > 64, uneven = d->causal || d->add_mask, grouped = d->Hq > d->Hkv;
+    auto ceil_div = [](int64_t n, int64_t m) { return (n + m - 1) / m; };
+    auto blocks = [&](int64_t own) { return (ceil_div(d->Skv, own) * d->Hkv + ceil_div(d->Sq, own) * d->Hq) * d->B; };
+    if (!wide && blocks(32) <= cus) return 4;
+    if (!wide && blocks(64) >= 16 * cus) return 1;
+    // (products per head: three of a dQ block, four of a dK / dV block)
+    auto work = [&](int64_t own, int64_t tile) { return 3 * ceil_div(d->Sq, own) * ceil_div(d->Skv, tile) + 4 * ceil_div(d->Skv, own) * ceil_div(d->Sq, tile); };
+    const int64_t one = work(128, 32), two = work(64, 64);
+    if (one > two || (!wide && (one == two || grouped))) return 2;
+    const bool one_block = d->Sq <= 128 && d->Skv <= 128;
+    const int64_t quarters = wide ? (uneven ? (one == two || grouped ? 16 : 8) : grouped ? 5 : 8) : uneven && !one_block ? 24 : 6;
+    return 4 * blocks(128) >= quarters * cus ? 1 : 2;
 }
 // Into how many workgroups a block's walk is dealt on top of that (which = 0: dQ, 1: dK / dV): the launch ends with its longest
 // item at the earliest, so where that alone would take more than twice a workgroup slot's share of the whole launch (one and a half
 // times where a workgroup has its compute unit to itself) the walks are divided, eight tiles of 64 per part at least (an item
 // costs about 10 us beside its tiles, and the planes are written, read and added).  And once where the items are equal (no mask)
 // and either leave the last of two rounds more than a quarter empty or are one round, which the dK / dV items alone then end (from
-// 16 tiles per part on).  Measured, backward call, in 1 / 2 / 4 parts (both kinds of item): 8 heads x 1259 x 64 causal 117 / 83 /
+// 16 tiles per part on).  Grouped queries without a mask at head dimensions above 64: a dK / dV item that takes a tenth more than the
+// share is divided (D = 128, dK / dV in 1 / 2 / 4 parts: 32 on 8 x 1024 1148 / 618 / 539, 16 on 4 x 2048 2249 / 1181 / 1045, 32 on 8 x 2048 2303 / 2039 / 2050).
+// Measured, backward call, in 1 / 2 / 4 parts (both kinds of item): 8 heads x 1259 x 64 causal 117 / 83 /
 // 86 us, 16 on 4 x 2048 x 64 causal 637 / 365 / 300, 8 x 1024 x 128 causal 158 / 108 / 130, 12 x 1024 x 80 causal 155 / 130 / 137 (dK / dV
 // alone in 2: 154), 24 x 544 x 80 causal 74 / 96, 24 x 1024 x 64 causal 115 / 136 / 162, 32 x 1024 x 64 causal 143 / 173 / 209, 8 x 1464 x 80
 // 296 / 259 / 269, 4 x 2048 x 128 303 / 283 / 305.
@@ -1080,8 +1097,9 @@ static int bwd_f32_parts(const incin_rocm_sdpa_desc_t* d, int which)
     const int64_t all = (n_kv * walk_kv * 8 + n_q * walk_q * 6) / (uneven ? 2 : 1);
     const int64_t longest = std::max(walk_q * 6, walk_kv * 8), tiles = (which == 0 ? d->Skv : d->Sq * G) / 64;
     const int64_t over = slots > compute_units_of(d->device) ? 4 : 3;      // halves of a slot's share
+    const bool tight = which == 1 && G > 1 && !uneven && (d->D > 64 || d->Dv > 64);
     int parts = 1;
-    while (parts < 4 && 2 * longest * slots > over * all * parts && tiles >= 16 * parts) parts *= 2;
+    while (parts < 4 && (tight ? 10 * longest * slots > 11 * all * parts : 2 * longest * slots > over * all * parts) && tiles >= 16 * parts) parts *= 2;
     const int64_t rounds = (n_kv + n_q + slots - 1) / slots;
     if (parts == 1 && !uneven && tiles >= 16 && (rounds == 1 ? tiles >= 32 : rounds == 2 && 4 * (n_kv + n_q) <= 3 * rounds * slots)) parts = 2;
     return parts;

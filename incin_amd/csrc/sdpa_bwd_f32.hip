@@ -784,7 +784,8 @@ hipError_t launch_sdpa_bwd_f32(const SdpaBwdParams& bp, hipStream_t stream)
     if (bp.f.Dp == 64)
         return bp.share == 4 ? launch_bwd_f32_d<64, 64, 4>(bp, stream) : bp.share == 2 ? launch_bwd_f32_d<64, 64, 2>(bp, stream) : launch_bwd_f32_d<64, 64, 1>(bp, stream);
     // (up to head dimension 96 in the 128 layout: three quarters of the products)
-    return bp.f.D <= 96 && bp.f.Dv <= 96 ? launch_bwd_f32_d<128, 96, 2>(bp, stream) : launch_bwd_f32_d<128, 128, 2>(bp, stream);
+    if (bp.f.D <= 96 && bp.f.Dv <= 96) return bp.share == 1 ? launch_bwd_f32_d<128, 96, 1>(bp, stream) : launch_bwd_f32_d<128, 96, 2>(bp, stream);
+    return bp.share == 1 ? launch_bwd_f32_d<128, 128, 1>(bp, stream) : launch_bwd_f32_d<128, 128, 2>(bp, stream);
 }
 
 }  // namespace incin_rocm

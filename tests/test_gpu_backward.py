@@ -1033,3 +1033,33 @@ def test_training_step_on_views(gpu, monkeypatch, parts, case):
             assert np.array_equal(got, ref, equal_nan=True), (n, turn)
         for x in bufs.values():
             x.free()
+
+
+@pytest.mark.parametrize("case", [
+    # B, Hq, Hkv, Sq, Skv, D, Dv, causal, key counts, mask
+    (4, 66, 66, 65, 65, 128, 128, True, None, False),           # a row past a tile
+    (4, 66, 66, 65, 70, 80, 72, False, None, True),
+    (4, 66, 66, 96, 96, 128, 128, True, None, True),            # whole tiles, a mask of values
+    (3, 90, 90, 200, 97, 128, 100, False, [97, 33, 0], False),  # two blocks of rows, the second not full; a sequence without keys
+    (3, 32, 8, 384, 384, 128, 128, False, None, False),         # grouped queries: dK / dV walks dealt to two workgroups
+    (4, 70, 70, 65, 65, 40, 64, False, None, False),
+    (4, 70, 70, 96, 70, 64, 48, True, None, True),
+], ids=lambda c: "x".join(str(x) for x in c[:7]))
+def test_matrix_core_backward_f32_of_many_short_heads(gpu, case):
+    """Launches in which a wavefront walks its block of 32 alone because that issues fewer products (on 256 compute units): many heads of 65 - 96
+    positions, and blocks of 128 that fill the device, against the generic kernels on the same forward."""
+    B, Hq, Hkv, Sq, Skv, D, Dv, causal, lens, masked = case
+    say("f32 backward of many short heads: %s" % (case,))
+    q, k, v, go = make_d(331 + Sq, B, Hq, Hkv, Sq, Skv, D, Dv, capi.F32)
+    kw = {}
+    if masked:
+        r = np.random.Generator(np.random.PCG64(337))
+        m = r.standard_normal((1, 1, Sq, Skv), dtype=np.float32)
+        m[..., 1:][r.random((1, 1, Sq, Skv - 1)) < 0.3] = -np.inf
+        m[..., :32, 32:64] = -np.inf
+        tm = capi.DeviceBuffer.from_numpy(m)
+        kw = dict(mask=tm, mask_strides=host.mask_strides_for(m.shape, B, Hq, Sq, Skv))
+    g = Gradients(q, k, v, go, capi.F32, causal=causal, kv_lens=lens, **kw)
+    got, ref = g.run(capi.IMPL_MFMA), g.run(capi.IMPL_GENERIC)
+    for name, a, b in zip(("dq", "dk", "dv"), got, ref):
+        compare(name, a, b, tol=1e-5)
