@@ -1003,9 +1003,11 @@ static size_t bwd_flags_bytes(const incin_rocm_sdpa_desc_t* d, int kind)
 // The other kernel runs three workgroups per compute unit: walks are dealt until there are two per compute unit, 16 tiles per
 // part at least, and with grouped queries until there are three if a part keeps 64.  Bf16 causal D = 64, in 1 / 2 / 4 / 8 parts, us:
 // 32 on 8 x 1024 89 / 62 / 55 / 55, 16 on 2 x 4096 576 / 314 / 192 / 178, 8 on 1 x 8192 1129 / 600 / 353 / 301, 64 on 8 x 4096 682 / 547 /
-// 466 / 489, 8 x 8192 278 / 283 / 276 / 305.
+// 466 / 489, 8 x 8192 278 / 283 / 276 / 305.  Not without grouped queries: there a launch of this kernel has a workgroup per compute unit, and undivided it
+// takes the dQ kernel beside it under a causal mask (24 x 2048 81 / 95 / 104, 6 x 8192 273 / 318 / 293); without one from 96 tiles on (6 x 8192 392 / 376 / 385,
+// 12 x 4096 204 / 203, 28 x 2048 116 / 137).
 // Its instance for head dimensions 65 - 96 runs two workgroups per compute unit: grouped queries only (without, the other kernel takes
-// the launches that would want parts), 8 tiles per part up to one workgroup per compute unit, 96 beyond.  Bf16 causal D = 96, likewise:
+// the launches that would want parts), 4 tiles per part up to one workgroup per compute unit, 48 beyond, up to three.  Bf16 causal D = 96, likewise:
 // 16 on 4 x 500 68 / 51 / 41 / 41, 32 on 8 x 1000 109 / 86 / 68 / 69, 8 on 1 x 2048 366 / 200 / 115 / 87, 2 x 32 on 8 x 2000 239 / 207 / 240 /
 // 263, 4 x 32 on 8 x 1000 133 / 153 / 166 / 192, 64 on 8 x 4000 874 / 703 / 683 / 719.
 static int bwd16_parts(const incin_rocm_sdpa_desc_t* d, int64_t blocks, int64_t walk)
@@ -1017,6 +1019,7 @@ static int bwd16_parts(const incin_rocm_sdpa_desc_t* d, int64_t blocks, int64_t 
             while (parts < 8 && G > 1 && ((parts * blocks < cus && walk >= 8 * parts) || (parts * blocks < 3 * cus && walk >= 96 * parts))) parts *= 2;
             return parts;
         }
+        if (G == 1 && (d->causal || walk < 96)) return 1;
         while (parts < 8 && ((parts * blocks < 2 * cus && walk >= 32 * parts) || (G > 1 && parts * blocks < 3 * cus && walk >= 128 * parts))) parts *= 2;
         return parts;
     }

@@ -51,7 +51,8 @@ inline bool bwd16_narrow(int64_t D, int64_t Dv, bool mask, int64_t G, int64_t bl
 //   paired kernel (one workgroup fills a compute unit): at most half the compute units (8 x 2048, D = 128: 78 forked, 111 in
 //   order; 16 x 1024 57 / 67; from 12 tiles of walk on: 12 x 768 48 / 55, 8 x 512 44 / 42); under a causal mask, whose blocks end
 //   at different times, up to two rounds of workgroups with walks of 32 tiles (64 when they are dealt) if the dQ launch is at
-//   most two rounds too (8 x 8192 457 / 488, 2 x 32 / 8 x 2048 268 / 309, 16 / 4 x 2048 in 4 parts 145 / 126, 64 / 8 x 4096 975 / 891;
+//   most two rounds too - of 16 tiles up to one and a half rounds, undivided: the second one leaves half of the compute units idle (40 x 1024 84 / 89,
+//   48 x 1024 88 / 92, 56 x 1024 113 / 105) - (8 x 8192 457 / 488, 2 x 32 / 8 x 2048 268 / 309, 16 / 4 x 2048 in 4 parts 145 / 126, 64 / 8 x 4096 975 / 891;
 //   without a mask 8 x 8192 942 / 823);
 //   the other: walks of 32 tiles under a causal mask or with grouped queries (8 x 8192, causal 278 / 305, 64 / 8 x 4096 466 / 518,
 //   4 x 32 / 8 x 4096 894 / 986; 32 x 12 x 512 118 / 103; without either 2 x 16 x 2048 135 / 121).
@@ -60,6 +61,7 @@ inline bool bwd16_forks(bool narrow, bool causal, int64_t G, int64_t blocks, int
     const int64_t w = walk / parts;
     if (narrow) return w >= 32 && (causal || G > 1);
     if (2 * parts * blocks <= cus && w >= 12) return true;
+    if (causal && parts == 1 && blocks > cus && 2 * blocks <= 3 * cus && dq_blocks <= 2 * cus && w >= 16) return true;
     return causal && parts * blocks <= 2 * cus && dq_blocks <= 4 * cus && w >= (parts > 1 ? 64 : 32);
 }
 

@@ -318,7 +318,9 @@ def test_backward_with_its_dq_kernel_on_a_side_stream(gpu, dtype, D, monkeypatch
     (capi.F16, 128, dict(B=1, Hq=4, Hkv=4, S=2048)),        # ... without groups, walks undivided
     (capi.BF16, 64, dict(B=1, Hq=16, Hkv=2, S=2048)),       # the one for narrow heads: eight parts of 32 tiles
     (capi.F16, 96, dict(B=1, Hq=16, Hkv=2, S=2048)),
-], ids=["paired_dealt", "paired", "narrow64", "narrow96"])
+    (capi.BF16, 128, dict(B=1, Hq=40, Hkv=40, S=1024)),     # the paired kernel in a round and a quarter
+    (capi.BF16, 64, dict(B=1, Hq=24, Hkv=24, S=2048)),      # the one for narrow heads without groups, undivided
+], ids=["paired_dealt", "paired", "narrow64", "narrow96", "paired_second_round", "narrow64_undivided"])
 def test_backward_that_forks(gpu, dtype, D, sizes, monkeypatch):
     """The test above at sizes whose calls fork, on any device of 256 compute units: one fork per call."""
     forks = capi.load().incin_rocm_side_stream_forks
