@@ -57,12 +57,10 @@ TRAFFIC_KIB = {   # leg/shape/variant: (FETCH_SIZE, WRITE_SIZE)
     "prefill_chunk/bf16_sq512_kv32768/auto": (67708 + 17448.5, 33677.2 + 4096), "prefill_chunk/bf16_sq512_kv32768/unsplit": (67735.5, 4096),
     "prefill_chunk/f32_sq128_kv32768/auto": (132204 + 16680, 33316.9 + 2048), "prefill_chunk/f32_sq128_kv32768/unsplit": (132192, 2048),
     "f32/f32_c1": (187.2, 32), "f32/f32_c2": (12378.4, 8192), "f32/f32_large": (1523050, 262144),
-    "backward/bf16_d128": (133150 + 367216 + 264788, 4096 + 131072 + 262324),          # (row dots + dQ + dK/dV kernels)
-    "backward/bf16_d64": (135199 + 309173 + 266324, 8192 + 131072 + 262152),
-    # (config 2's shape in f32: blocks dealt to two workgroups - the kernels write a plane each beside the gradients, and the two
-    #  passes that add the planes follow)
-    "backward/f32_d64": (8735 + 16613 + 16883 + 8219 + 16411, 512 + 16384 + 32778.2 + 8192 + 16384),
-    "backward/f32_d128": (270367 + 875814 + 924203, 8192 + 262144 + 524288),
+    "backward/bf16_d128": (432606 + 264544, 135168 + 262439),          # (dQ kernel with the row dots, dK/dV kernel)
+    "backward/bf16_d64": (133152 + 313584 + 269509, 8192 + 131072 + 270332),          # (row dots, dQ and dK/dV kernels)
+    "backward/f32_d64": (8350 + 26826, 256 + 24576),          # (row dots, one launch of all gradients)
+    "backward/f32_d128": (266271 + 3539515, 4096 + 786432),
 }
 TRAFFIC_PROFILE = "profiles/fetch_write_size_bench_legs.txt"
 
@@ -429,8 +427,8 @@ def decode_step_graph(w, B, H, Skv, D, steps):
 
 def backward_leg(steps, warmup, dtype=capi.BF16, B=8, H=16, S=4096, D=128, what="BASELINE config 3's shape"):
     """Forward (keeping the row normalisers) and then the timed backward: dQ, dK, dV for a synthetic upstream gradient.
-    The figure counts 2.5 x the forward's FLOPs (five matrix products against the forward's two; the recomputation of S
-    and dP in both big kernels is not counted)."""
+    The figure counts 2.5 x the forward's FLOPs (five matrix products against the forward's two; S and dP, which
+    are computed for dQ and again for dK and dV, count once)."""
     name = {capi.BF16: "bf16", capi.F16: "f16", capi.F32: "f32"}[dtype]
     q, k, v = make_inputs(SEED0 + 5, B, H, H, S, S, D, dtype)
     g = rng(SEED0 + 6).standard_normal((B, H, S, D), dtype=np.float32)
@@ -471,7 +469,8 @@ def backward_leg(steps, warmup, dtype=capi.BF16, B=8, H=16, S=4096, D=128, what=
     peak = PEAK_F32_TFLOPS if dtype == capi.F32 else PEAK_BF16_TFLOPS
     return {"workload": "backward of %s: %s causal B=%d H=%d S=%d D=%d, dQ dK dV from Q K V O dO and the "
                         "forward's row normalisers" % (what, name, B, H, S, D),
-            "step": "one incin_rocm_sdpa_bwd call (3 kernels: row dots, dQ, dK/dV)", "dtype": name,
+            "step": "one incin_rocm_sdpa_bwd call (%s)" % ("row dots, then dQ and dK/dV blocks in one launch" if dtype == capi.F32 else
+                                                           "dQ and dK/dV kernels; row dots in the dQ kernel, or in one of their own where those two run side by side"), "dtype": name,
             "metric": "attn bwd TFLOP/s (2.5 x forward FLOPs)", "value": flops / (wall * 1e-3) / 1e12, "unit": "TFLOP/s",
             "ms_per_step": wall, "steps": steps, "frac_of_%s_mfma_peak" % ("fp32" if dtype == capi.F32 else "bf16"): flops / (wall * 1e-3) / 1e12 / peak,
             "traffic": traffic_of("backward/%s_d%d" % (name, D))[0], "traffic_source": TRAFFIC_PROFILE,

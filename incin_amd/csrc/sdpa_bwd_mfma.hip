@@ -954,7 +954,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 3
     typedef PfLayout<D> L;
     typedef float float4v __attribute__((ext_vector_type(4)));
     constexpr int NSTEP = DC / 16, NDB = DC / 32, NQH = (NSTEP + 3) / 4;
-    constexpr int R = D == 64 ? 2 : 4;      // matrix operands in flight from LDS (at 64 three would spill at three wavefronts per SIMD)
+    constexpr int R = D == 64 ? 2 : 4;      // matrix operands in flight from LDS (three would spill inside the loop at three wavefronts per SIMD; with two one register is put away across it)
     constexpr int STAGE = 2 * L::TILE_BYTES + 512;      // Q rows, dO rows, 64 x -L_i log2(e), 64 x -D_i
     const SdpaParams& p = bp.f;
     __shared__ __attribute__((aligned(1024))) char smem[2 * STAGE];

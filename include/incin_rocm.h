@@ -246,7 +246,7 @@ int incin_rocm_sdpa_fwd_static(const incin_rocm_sdpa_desc_t* desc, void* stream)
  * The reference has no backward kernel for attention: its gradient is what walking the tape of the composed ops
  * gives (crates/incin-backends/src/cpu/ops/shape_ops.rs:1245-1269 records matmul, mul_scalar, add, log_softmax,
  * exp, matmul; crates/incin-backends/src/cpu/tape.rs:149-176 walks it).  This computes the same dq, dk, dv in
- * three launches from q, k, v, the forward's output o and row normalisers lse, and the upstream gradient d_o.
+ * two or three launches (one more where a mask is classified, one where walks are divided) from q, k, v, the forward's output o and row normalisers lse, and the upstream gradient d_o.
  *
  * `fwd` is the forward's descriptor as it was launched with `lse` set (o and lse are inputs here); causal,
  * kv_lens and the grouped-query layout carry over; d_k and d_v are summed over the query heads of a group.
@@ -260,9 +260,9 @@ int incin_rocm_sdpa_fwd_static(const incin_rocm_sdpa_desc_t* desc, void* stream)
  * contributes nothing to d_k and d_v, where the reference's tape would spread NaN over the whole head.
  * The workspace holds two floats per query row (2 x [B, Hq, Sq]) and, for a dense mask on the matrix-core kernels, a byte
  * per 32 rows x 32 keys of the mask behind them, and for a call on the matrix-core kernels that does not fill the device
- * (f32; 16-bit storage with few KV heads) up to four (16-bit above head dimension 128: eight) f32 copies of the gradients' shapes, which workgroups that share a block
- * of rows or keys sum into (ask incin_rocm_sdpa_bwd_workspace for the size: it depends on the device's compute-unit count);
- * d_q, d_k, d_v are fully overwritten.
+ * evenly - too few blocks of rows or keys for it, or a few long ones - f32 copies of the gradients' shapes, up to four (16-bit storage without a mask at head
+ * dimensions up to 96 and above 128: eight), which workgroups that share a block of rows or keys sum into (ask incin_rocm_sdpa_bwd_workspace for the size: it depends on the device's compute-unit count);
+ * d_q, d_k, d_v are fully overwritten, in no particular order: they overlap neither each other nor anything the call reads.
  * Streams: everything the call launches is ordered behind the work already on `stream` and ahead of whatever `stream` gets
  * next.  A call of the matrix-core kernels that is short of work may run its dQ kernel on a stream of the library's own
  * beside the dK/dV kernel (forked from and joined to `stream` with events; the library's streams have the default priority,
