@@ -452,6 +452,16 @@ void fill_params(const incin_rocm_sdpa_desc_t* d, const Plan& plan, SdpaParams* 
     p->num_splits = plan.splits;
     p->split_len = plan.split_len;
     p->split_turn = incin_rocm::split_turn_of(d->kv_lens != nullptr, p->B, plan.splits);
+    if (plan.impl == INCIN_ROCM_IMPL_SPLITKV || plan.impl == INCIN_ROCM_IMPL_SPLITKV_MFMA) {
+        // workgroups of the launch against what the device holds at a time (four per compute unit of the vector-ALU kernel)
+        const int64_t R = (d->Hq / d->Hkv) * d->Sq, cus = compute_units_of(d->device);
+        const bool vector = plan.impl == INCIN_ROCM_IMPL_SPLITKV;
+        const int64_t chunk = vector ? (R <= 1 ? 1 : R <= 2 ? 2 : R <= 4 ? 4 : 8) : incin_rocm::decode_mfma_chunk_rows((int)std::min<int64_t>(R, 1 << 20), d->dtype, p->Dp);
+        const int64_t wgs = d->B * d->Hkv * ((R + chunk - 1) / chunk) * plan.splits;
+        const int64_t slots = cus * (vector ? 4 : incin_rocm::decode_mfma_workgroups_per_cu((int)chunk, plan.split_len, d->dtype, p->Dp));
+        p->split_even = incin_rocm::split_even_of(d->kv_lens != nullptr, p->B, plan.splits, wgs <= slots, (int64_t)plan.split_len * p->Dp * (int64_t)dtype_size(d->dtype), p->Dp);
+        if (p->split_even) p->split_turn = 0;
+    }
     if (plan.impl == INCIN_ROCM_IMPL_MFMA) p->mask_flags = d->add_mask ? (const uint8_t*)d->workspace : nullptr;
     if (plan.impl == INCIN_ROCM_IMPL_MFMA && d->add_mask && plan.lims_offset) p->mask_lims = (const int32_t*)((const char*)d->workspace + plan.lims_offset);
     if (!(plan.impl == INCIN_ROCM_IMPL_MFMA && d->add_mask)) p->ws_acc = (float*)d->workspace;

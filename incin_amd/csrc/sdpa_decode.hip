@@ -85,9 +85,8 @@ __global__ __launch_bounds__(256) void sdpa_decode_split_kernel(SdpaParams p)
 
     int kv_len = Skv;
     if (p.kv_lens) kv_len = clampi(p.kv_lens[b], 0, Skv);
-    const int k_begin = split * p.split_len;
-    int k_end = k_begin + p.split_len;
-    if (k_end > kv_len) k_end = kv_len;
+    const KeyRange keys = split_keys(p, split, kv_len, KT);
+    const int k_begin = keys.begin, k_end = keys.end;
 
     const float sc = p.scale * Softexp<T>::kPre;
     float qf[RMAX][VEC];
@@ -97,7 +96,7 @@ __global__ __launch_bounds__(256) void sdpa_decode_split_kernel(SdpaParams p)
     for (int r = 0; r < RMAX; ++r) {
         const int row = r0 + r;
         const bool valid = row < R;
-        const int g = valid ? row / Sq : 0, i = valid ? row % Sq : 0;
+        const int g = !valid ? 0 : Sq > 1 ? row / Sq : row, i = valid ? row - g * Sq : 0;      // (a division is some forty instructions)
         const T* qp = (const T*)p.q + (int64_t)b * p.q_sb + (int64_t)(hkv * p.G + g) * p.q_sh + (int64_t)i * p.q_ss + dl;
         vec_t qv = *(const vec_t*)qp;
 #pragma unroll
@@ -215,7 +214,7 @@ __global__ __launch_bounds__(256) void sdpa_decode_split_kernel(SdpaParams p)
             L = fmaf(w, s_ml[(s2 * RMAX + r) * 2 + 1], L);
             A = fmaf(w, s_acc[(s2 * RMAX + r) * D + d], A);
         }
-        const int g = row / Sq, i = row % Sq;
+        const int g = Sq > 1 ? row / Sq : row, i = row - g * Sq;
         const int hq = hkv * p.G + g;
         if (p.num_splits == 1) {
             T* op = (T*)p.o + (int64_t)b * p.o_sb + (int64_t)hq * p.o_sh + (int64_t)i * p.o_ss;

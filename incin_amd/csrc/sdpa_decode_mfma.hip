@@ -67,7 +67,8 @@ __global__ __launch_bounds__(256) void sdpa_decode_mfma_kernel(SdpaParams p)
 
     int kv_len = Skv;
     if (p.kv_lens) kv_len = clampi(p.kv_lens[b], 0, Skv);
-    const int k_begin = split * p.split_len;
+    const KeyRange keys = split_keys(p, split, kv_len, BLOCK);
+    const int k_begin = keys.begin;
 
     // this lane's rows, one per block of 32 (lanes l and l + 32 share them), and the keys each may see inside this split
     bool valid[NRB];
@@ -77,10 +78,10 @@ __global__ __launch_bounds__(256) void sdpa_decode_mfma_kernel(SdpaParams p)
     for (int rb = 0; rb < NRB; ++rb) {
         const int row = r0 + 32 * rb + ql;
         valid[rb] = row < R;
-        const int gq = valid[rb] ? row / Sq : 0;
-        qi[rb] = valid[rb] ? row % Sq : 0;
+        const int gq = !valid[rb] ? 0 : Sq > 1 ? row / Sq : row;      // (a division is some forty instructions)
+        qi[rb] = valid[rb] ? row - gq * Sq : 0;
         hq[rb] = hkv * p.G + gq;
-        int l = min(k_begin + p.split_len, kv_len);
+        int l = keys.end;
         if (p.causal) l = min(l, causal_limit(qi[rb], Sq, Skv));
         lim[rb] = valid[rb] ? l : 0;
         lim_hi = max(lim_hi, lim[rb]);

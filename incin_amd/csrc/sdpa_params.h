@@ -31,6 +31,7 @@ struct SdpaParams {
     int32_t num_splits;
     int32_t split_len;         // keys per split (multiple of the kernel's key tile)
     int32_t split_turn;        // largest shift of work_split (a power of two minus one; 0: none)
+    int32_t split_even;        // splits are equal shares of a batch entry's keys, not of the capacity (split_keys)
     float* ws_acc;             // [B, Hq, Sq, num_splits, Dp] f32 partial numerators (Dp == Dv for the vector-ALU kernel)
     float* ws_ml;              // [B, Hq, Sq, num_splits, 2]  running max (natural-log domain) and denominator
     // matrix-core prefill kernels with a dense mask: one byte per block of 32 query rows x 32 keys (0 mixed, 1 all zero,
@@ -89,6 +90,32 @@ inline int split_turn_of(bool key_counts, int B, int num_splits)
 {
     const int d = num_splits & -num_splits;
     return key_counts && B >= 4 && num_splits > 1 ? (d < 8 ? d : 8) - 1 : 0;
+}
+// Which keys of a batch entry with kv_len of them a split holds: split_len of the capacity's, or - split_even_of says where - an equal share of
+// those there are, in whole blocks of `unit` keys.
+struct KeyRange { int begin, end; };
+__device__ __forceinline__ KeyRange split_keys(const SdpaParams& p, int split, int kv_len, int unit)
+{
+    KeyRange r;
+    if (p.split_even) {
+        const int blocks = (kv_len + unit - 1) / unit, each = blocks / p.num_splits, more = blocks - each * p.num_splits;
+        r.begin = (each * split + min(split, more)) * unit;      // (the first `more` splits take one block more)
+        r.end = min(r.begin + (each + (split < more ? 1 : 0)) * unit, kv_len);
+    } else {
+        r.begin = split * p.split_len;
+        r.end = min(r.begin + p.split_len, kv_len);
+    }
+    return r;
+}
+// Equal shares where one round of workgroups is the whole launch (`one_round`), so that its longest is what the launch takes, and the
+// splits are short (`split_bytes` of K: 256 KiB at most), so that a workgroup is bound by its own latencies and not by the memory system - there
+// splits of one length are the better ones: those of short sequences that are empty leave their bandwidth to the others, and all
+// end together.  From 8 sequences on the shift above balances as well.  Bf16, us, splits of the capacity / equal shares: 32 on 8 heads x 4 sequences of 3000 - 16000
+// keys 34.0 / 29.8, 2 of 4096 - 32768 at D = 64 20.8 / 17.3, 3 x 4 x 832 - 2386 11.8 / 10.4, 6 x 8 x 1650 - 2037 19.8 / 18.6, f32 1 x 2 x 2058 18.4 / 14.7, one of 407 at D = 256 17.5 /
+// 15.4; but 8 x 8 x 1024 - 8192 31.8 / 32.2, 16 x 8 x 512 - 4096 31.8 / 32.9, 4 x 8 x 7000 - 60000 (7500 a split) 95 / 101, 2 x 2 x 10000 - 29999 at D = 256 27.2 / 27.5.
+inline int split_even_of(bool key_counts, int B, int num_splits, bool one_round, int64_t split_bytes, int Dp)
+{
+    return key_counts && num_splits > 1 && one_round && split_bytes <= (256 << 10) && B < (Dp > 128 ? 2 : 8);
 }
 __device__ __forceinline__ int work_split(const SdpaParams& p, int group)
 {

@@ -1476,3 +1476,20 @@ def test_decode_splits_shifted_between_groups(gpu, dtype, case):
         # f32: sums of at most 4096 terms; bf16: P and the result rounded to 2^-9 of values up to the largest, with the sums' spread
         tol = 1e-5 if dtype == capi.F32 else 2.0 ** -7
         assert np.abs(got[b] - ref).max() <= tol * max(1.0, np.abs(ref).max()), b
+
+
+@pytest.mark.parametrize("dtype,D,G,Sq,impl", [
+    (capi.BF16, 128, 4, 1, capi.IMPL_SPLITKV_MFMA), (capi.F16, 64, 8, 1, capi.IMPL_SPLITKV_MFMA), (capi.BF16, 256, 2, 1, capi.IMPL_SPLITKV_MFMA),
+    (capi.BF16, 64, 16, 3, capi.IMPL_SPLITKV_MFMA), (capi.F32, 128, 4, 1, capi.IMPL_SPLITKV_MFMA), (capi.F32, 64, 8, 5, capi.IMPL_SPLITKV_MFMA),
+    (capi.F32, 256, 1, 1, capi.IMPL_SPLITKV_MFMA), (capi.BF16, 128, 1, 1, capi.IMPL_SPLITKV), (capi.F16, 64, 2, 2, capi.IMPL_SPLITKV), (capi.F32, 128, 1, 1, capi.IMPL_SPLITKV),
+], ids=lambda x: str(x))
+def test_key_counts_in_equal_shares(dtype, D, G, Sq, impl):
+    """Split-KV launches of one round give each split an equal share of the keys a sequence has, in whole blocks: counts of no
+    key, fewer blocks than splits, a block more or less than whole shares, all keys."""
+    Hkv, Skv, splits = 2, 1030, 4
+    # one call per count - a single sequence, which takes the rule at every head dimension - and one with several at once
+    for lens in ([0], [1], [31], [32], [33], [64], [127], [128], [129], [255], [257], [513], [1023], [1029], [1030], [5, 1030, 0, 700, 96, 97, 511]):
+        q, k, v = inputs(SEED0 + 77 + lens[0], len(lens), Hkv * G, Hkv, Sq, Skv, D, D, dtype)
+        got, info = host.sdpa(q, k, v, dtype, causal=Sq > 1, kv_lens=np.asarray(lens, np.int32), num_splits=splits, impl=impl, return_info=True)
+        assert info["impl"] == impl and info["splits"] > 1
+        check(got, oracle_full(q, k, v, G=G, causal=Sq > 1, kv_lens=lens), TOL[dtype], "equal shares of %r" % (lens,))
