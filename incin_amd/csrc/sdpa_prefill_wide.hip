@@ -36,10 +36,16 @@ constexpr int PW_KT = 32;      // keys per tile
 // MASK: 0 no mask tensor; 1 (DENSE) a dense additive mask by flags and values; 2 (LIMS) the launch for the 128-row blocks all
 // of whose rows the mask gives n zeros and then -inf (sdpa_prefill_mfma.hip has the scheme: a masked request is the LIMS
 // launch, whose other workgroups leave at once, and then the DENSE launch, whose workgroups leave if LIMS took their block).
-template <typename T, int MASK, bool SPLIT = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void sdpa_prefill_wide_kernel(SdpaParams p)
+//
+// KG: wavefronts per 32 query rows.  With 2 (no mask tensor, no splits) a workgroup is eight wavefronts, each group of four with tile
+// buffers of its own: the first walks the even tiles of the block, the second the odd ones, and the two partial results of a row
+// meet in LDS at the end, either group finishing half of the columns.  For launches of at most a workgroup per compute unit,
+// whose wavefronts would otherwise be alone on their SIMDs and walk all keys one tile after the other.
+template <typename T, int MASK, bool SPLIT = false, int KG = 1>
+__global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(2, 2))) void sdpa_prefill_wide_kernel(SdpaParams p)
 {
     constexpr bool DENSE = MASK == 1, LIMS = MASK == 2;
+    static_assert(KG == 1 || (KG == 2 && MASK == 0 && !SPLIT), "two groups of wavefronts: the plain launch only");
 #if defined(__HIP_DEVICE_COMPILE__)
     typedef typename Mma<T>::vec8 vec8;
     constexpr int D = 256;
@@ -47,10 +53,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     constexpr int NSTEP = D / 16, NDB = D / 32;
     constexpr int TILE = PW_KT * L::ROWB;              // 16 KiB
     constexpr int LPW = TILE / 1024 / 4;               // wavefront-wide 1 KiB copies per tensor per tile: 4
-    __shared__ __attribute__((aligned(1024))) char smem[4 * TILE];      // K buffers 0, 1, V buffers 0, 1
+    __shared__ __attribute__((aligned(1024))) char smem_all[KG * 4 * TILE];
 
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave_id = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = KG == 2 ? wave_id & 3 : wave_id, grp = KG == 2 ? wave_id >> 2 : 0;      // which 32 rows, which tiles (t % KG)
+    char* const smem = smem_all + grp * 4 * TILE;      // the group's: K buffers 0, 1, V buffers 0, 1
+    auto parity = [](int t) __attribute__((always_inline)) { return KG == 2 ? (t >> 1) & 1 : t & 1; };      // which buffers tile t goes into
     const int ql = lane & 31, g = lane >> 5;
     const int Sq = p.Sq, Skv = p.Skv;
 
@@ -171,10 +180,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int c = 0; c < LPW; ++c) dma_copy16(r, dst + c * 1024, voff[c]);
     };
     auto issue_kv = [&](int t) __attribute__((always_inline)) {
-        issue(kp, k_tile_bytes, p.k_ss, p.D, t, t & 1, k_voff);
-        issue(vp, v_tile_bytes, p.v_ss, p.Dv, t, 2 + (t & 1), v_voff);
+        issue(kp, k_tile_bytes, p.k_ss, p.D, t, parity(t), k_voff);
+        issue(vp, v_tile_bytes, p.v_ss, p.Dv, t, 2 + parity(t), v_voff);
     };
-    if (n_tiles > t_first) issue_kv(t_first);
+    if (n_tiles > t_first + grp) issue_kv(t_first + grp);
     int flag_next = 1;      // the flag of the next tile, read one tile ahead
     if (DENSE && n_tiles > t_first) flag_next = mflags[t_first];
 
@@ -186,7 +195,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     {
         uint4v qraw[NSTEP / 4][4];
         fetch_q_rows(qraw, qp, q0 + wave * 32, Sq, p.q_ss, p.D, lane);
-        stage_q_rows(qreg, qraw, smem + ((t_first + 1) & 1) * TILE + wave * 4096, lane);
+        stage_q_rows(qreg, qraw, smem + (parity(t_first) ^ 1) * TILE + wave * 4096, lane);
         // scale * log2(e) folded into Q once (rounded back to the storage type, as sdpa_prefill_mfma.hip does): the product
         // then yields the scores in the log2 units the softmax works in, whatever the sign of the scale
         const float c2 = p.scale * 1.4426950408889634f;
@@ -219,19 +228,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int r = 0; r < 16; ++r) o_acc[db][r] = 0.0f;
 
-    for (int t = t_first; t < n_tiles; ++t) {
-        // K(t), V(t) have arrived for everyone, everyone is done with tile t - 1: its buffers take tile t + 1
+    for (int t0 = t_first; t0 < n_tiles; t0 += KG) {
+        const int t = t0 + grp;
+        // K(t), V(t) have arrived for everyone, everyone is done with tile t - KG: its buffers take tile t + KG
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        if (t + 1 < n_tiles) issue_kv(t + 1);
+        if (t + KG < n_tiles) issue_kv(t + KG);
         int flag = 1;
         if (DENSE) {      // (arrived with the tile: the wait above covers it)
             flag = __builtin_amdgcn_readfirstlane(flag_next);
             if (t + 1 < n_tiles) flag_next = mflags[t + 1];
         }
-        if (t >= n_act || t < w_first) continue;      // nothing of this tile is visible to the wavefront's rows
-        const char* kb = smem + (t & 1) * TILE;
-        const char* vb = smem + (2 + (t & 1)) * TILE;
+        if (t >= n_act || t < w_first) continue;      // nothing of this tile is visible to the wavefront's rows (or there is no such tile)
+        const char* kb = smem + parity(t) * TILE;
+        const char* vb = smem + (2 + parity(t)) * TILE;
         const int j0 = t * PW_KT;
         // ---- S^T = K Q^T ----
         floatx16 sacc;
@@ -325,6 +335,53 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
 
     // ---- normalise and store --------------------------------------------------------------------------------------
+    if constexpr (KG == 2) {
+        // The two groups' results of a row meet: each wavefront hands the columns that its partner (the same rows, the other
+        // tiles) finishes to it, unscaled, with its reference and sum, and adds the partner's to its own.  16 KiB per wavefront: all
+        // of the tile buffers; a wavefront reads the area that its partner wrote and nobody else looks at it.
+        constexpr int HALF = NDB / 2;
+        __shared__ float s_ml[8][2][64];
+        typedef float f4 __attribute__((ext_vector_type(4)));
+        const float l_mine = xor32_sum(l_run);
+        const int other = wave_id ^ 4;
+        __syncthreads();      // (everyone is done with the tiles; no copy is in flight)
+        s_ml[wave_id][0][lane] = m_run;
+        s_ml[wave_id][1][lane] = l_mine;
+        f4* const give = (f4*)(smem_all + wave_id * 4 * 4096) + lane;
+        floatx16 o_half[HALF];
+#pragma unroll
+        for (int d = 0; d < HALF; ++d)
+#pragma unroll
+            for (int r4 = 0; r4 < 4; ++r4) {
+                f4 w;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float lo = o_acc[d][4 * r4 + e], hi = o_acc[HALF + d][4 * r4 + e];
+                    w[e] = grp ? lo : hi;
+                    o_half[d][4 * r4 + e] = grp ? hi : lo;
+                }
+                give[(d * 4 + r4) * 64] = w;
+            }
+        __syncthreads();
+        const float m_o = s_ml[other][0][lane], l_o = s_ml[other][1][lane], m_all = fmaxf(m_run, m_o), m_use = m_all == -INFINITY ? 0.0f : m_all;
+        const float f_mine = __builtin_amdgcn_exp2f(m_run - m_use), f_o = __builtin_amdgcn_exp2f(m_o - m_use);      // (no key in a group's tiles: 0)
+        const f4* const take = (const f4*)(smem_all + other * 4 * 4096) + lane;
+#pragma unroll
+        for (int d = 0; d < HALF; ++d)
+#pragma unroll
+            for (int r4 = 0; r4 < 4; ++r4) {
+                const f4 w = take[(d * 4 + r4) * 64];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o_half[d][4 * r4 + e] = o_half[d][4 * r4 + e] * f_mine + w[e] * f_o;
+            }
+        const float l_all = l_mine * f_mine + l_o * f_o;
+        const float inv = (l_all == 0.0f) ? __builtin_nanf("") : 1.0f / l_all;      // no visible key: NaN, as the reference
+        if (my_i < rows_b && p.lse && grp == 0 && g == 0)
+            p.lse[((int64_t)b * p.Hq + hq) * Sq + my_i] = l_all == 0.0f ? -INFINITY : (m_all + __builtin_log2f(l_all)) * 0.6931471805599453f;
+        const int c0 = grp * HALF * 32;
+        store_o_rows(o_half, inv, smem_all + other * 4 * 4096, op + c0, q0 + wave * 32, rows_b, p.o_ss, p.Dv - c0, lane);
+        return;
+    }
     const float l_tot = xor32_sum(l_run);
     if constexpr (SPLIT) {
         // partial result of this split: unnormalised O, and (reference, sum) in the log2 units the combine kernel takes for 16-bit
@@ -354,6 +411,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // tile, i.e. done with the tile before it, and nothing has been copied since
     store_o_rows(o_acc, inv, smem + (n_tiles & 1) * TILE + wave * 4096, op, q0 + wave * 32, rows_b, p.o_ss, p.Dv, lane);
 #endif
+}
+
+// Where the form with two groups of wavefronts per block is ahead (bf16, D = 256, us with one / two; launches of Hq x S, workgroups in
+// brackets).  At most one workgroup per compute unit - with one group its wavefronts are alone on their SIMDs: causal 2 x 16 x 1024 (256)
+// 50.4 / 36.9, 16 x 2048 (256) 92 / 65, 3 x 12 x 640 (180) 35.1 / 28.5, nothing masked 16 x 2048 92 / 70.  Up to two, where blocks differ in
+// length by a causal flag and heads have eight of them or more: with one group the two longest meet on a compute unit and end the
+// launch.  16 x 4096 (512) 191 / 148, 8 x 8192 (512) 370 / 271, 2 x 16 x 1536 (384) 74 / 53, 4 x 16 x 1024 (512) 55.4 / 53.4; but 6 x 16 x 512 (384)
+// 31.8 / 34.3, 16 x 8 x 300 (384) 22 / 30, nothing masked 2 x 16 x 2048 (512) 124 / 137, 4 x 16 x 2048 (1024) 139 / 164.
+static bool two_groups(const SdpaParams& p, int64_t total, int nqb)
+{
+    const int64_t cus = device_cus();
+    return total <= cus || (total <= 2 * cus && p.causal && nqb >= 8 && p.Skv - p.Sq <= p.Sq / 4);
 }
 
 // Host has validated: dtype f16 / bf16, 128 < max(D, Dv) <= 256 in whole 16-byte vectors, finite scale; with a dense mask its
@@ -387,6 +456,9 @@ hipError_t launch_sdpa_prefill_wide(const SdpaParams& p0, int dtype, hipStream_t
     if (p.mask) {
         if (dtype == 1) hipLaunchKernelGGL((sdpa_prefill_wide_kernel<f16_t, 1>), dim3((unsigned)total), dim3(256), 0, stream, p);
         else hipLaunchKernelGGL((sdpa_prefill_wide_kernel<bf16_t, 1>), dim3((unsigned)total), dim3(256), 0, stream, p);
+    } else if (two_groups(p, total, nqb)) {
+        if (dtype == 1) hipLaunchKernelGGL((sdpa_prefill_wide_kernel<f16_t, 0, false, 2>), dim3((unsigned)total), dim3(512), 0, stream, p);
+        else hipLaunchKernelGGL((sdpa_prefill_wide_kernel<bf16_t, 0, false, 2>), dim3((unsigned)total), dim3(512), 0, stream, p);
     } else if (dtype == 1) hipLaunchKernelGGL((sdpa_prefill_wide_kernel<f16_t, 0>), dim3((unsigned)total), dim3(256), 0, stream, p);
     else hipLaunchKernelGGL((sdpa_prefill_wide_kernel<bf16_t, 0>), dim3((unsigned)total), dim3(256), 0, stream, p);
     return hipGetLastError();

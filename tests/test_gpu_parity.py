@@ -830,6 +830,41 @@ def test_head_dimensions_above_128(gpu, dtype, dims):
 
 
 @pytest.mark.parametrize("dtype", [capi.BF16, capi.F16], ids=lambda x: dtypes.NAMES[x])
+@pytest.mark.parametrize("dims", [(256, 256), (160, 248), (256, 72)], ids=lambda x: "D%d_Dv%d" % x)
+def test_two_groups_of_wavefronts_above_128(gpu, dtype, dims):
+    """A launch of at most a workgroup per compute unit above head dimension 128 deals the key tiles of a block to two groups of
+    wavefronts: a single tile (the second group has none), even and odd numbers of them, partial last tiles, rows whose keys
+    lie in one group's tiles only, sequences without keys, padded query rows, Dv in the first group's columns only."""
+    D, Dv = dims
+    tol = TOL[dtype]
+    for Sq, Skv, causal in ((5, 7, False), (33, 32, False), (64, 33, True), (129, 65, False), (100, 96, True), (200, 161, True), (257, 300, True)):
+        q, k, v = inputs(5100 + Sq, 3, 4, 2, Sq, Skv, D, Dv, dtype)
+        for kv_lens, q_lens in ((None, None), ([Skv, 0, 1], None), ([min(Skv, 33), Skv, min(Skv, 64)], [Sq, 1, max(Sq - 2, 1)])):
+            lens = None if kv_lens is None else np.array(kv_lens, np.int32)
+            got, lse = host.sdpa(q, k, v, dtype, causal=causal, kv_lens=lens, q_lens=None if q_lens is None else np.array(q_lens, np.int32),
+                                 impl=capi.IMPL_MFMA, return_lse=True)
+            _, lse_g = host.sdpa(q, k, v, dtype, causal=causal, kv_lens=lens, impl=capi.IMPL_GENERIC, return_lse=True)
+            ref = oracle_full(q, k, v, G=2, causal=causal, kv_lens=lens)
+            for b in range(3):
+                n = Sq if q_lens is None else q_lens[b]
+                check(got[b:b + 1, :, :n], ref[b:b + 1, :, :n], tol, "two groups, Sq=%d Skv=%d b=%d causal=%d" % (Sq, Skv, b, causal))
+                fin = np.isfinite(lse_g[b, :, :n])
+                assert np.array_equal(fin, np.isfinite(lse[b, :, :n])) and (not fin.any() or np.abs(lse[b, :, :n][fin] - lse_g[b, :, :n][fin]).max() < 2e-2)
+
+
+def test_two_groups_of_wavefronts_up_to_two_workgroups_per_compute_unit(gpu):
+    """... and so does a causal launch of more, up to two, whose heads have eight blocks or more: sampled rows of every block."""
+    cus = capi.device_info(0).compute_units
+    H, S = cus // 9 + 1, 1100      # 9 blocks a head
+    q, k, v = inputs(5200, 1, H, H, S, S, 256, 256, capi.BF16)
+    got, info = host.sdpa(q, k, v, capi.BF16, causal=True, return_info=True)
+    assert info["impl"] == capi.IMPL_MFMA and info["splits"] == 1
+    rows = np.array([[h, i] for h in (0, H // 2, H - 1) for i in (0, 31, 32, 127, 128, 500, 639, 900, 1023, 1024, 1099)])
+    ref = O.sdpa_rows(q.reshape(1, H, 1, S, 256), k[:, :, None], v[:, :, None], rows, causal=True)
+    assert np.abs(got.reshape(H, S, 256)[rows[:, 0], rows[:, 1]] - ref).max() <= TOL[capi.BF16]
+
+
+@pytest.mark.parametrize("dtype", [capi.BF16, capi.F16], ids=lambda x: dtypes.NAMES[x])
 @pytest.mark.parametrize("dims", [(256, 256), (192, 128)], ids=lambda x: "D%d_Dv%d" % x)
 def test_head_dimensions_above_128_with_a_dense_mask(gpu, dtype, dims):
     """The prefill kernel for 256 with a dense additive mask: a sliding window given as a [1, 1, Sq, Skv] tensor (tiles before
