@@ -33,12 +33,15 @@
 //
 // Tiles of 32 rows (16 KiB each of both tensors), three stages: t - 1 and t in use, t + 1 arriving by global -> LDS copies.  A
 // step is the first products of tile t, a barrier, and the third product of tile t - 1 with the exponentials and splits of
-// tile t between its matrix instructions.
+// tile t between its matrix instructions.  The copies of tile t + 1 are started behind the first LDS reads of tile t, and the first
+// operands of the third product are read before the barrier, with the last first products: neither then waits behind a barrier
+// (2 x 16 on 8 x 1024 causal 128.5 -> 126 us, nothing masked 234 -> 229, 8 x 2048 123.5 -> 119.5, 4 x 3000 at D = 160 161 -> 158).
 //
 // Measured, backward call, bf16: 2 x 16 heads on 8 x 1024 positions, D = 256, causal 13.86 -> 0.14 ms (302 TFLOP/s of
 // useful work; the generic kernels 3.1), 8 on 1 x 4096 0.48 ms, 4 x 16 on 4 x 1024 0.25 ms.  The matrix pipes are busy 45 % of the
-// time a workgroup is on a compute unit; the rest is the two barriers of a step, behind which all eight wavefronts wait for
-// their first LDS operands together, and the vector work of the splits.
+// time a workgroup is on a compute unit; beside them the LDS is the bound - in the first products every matrix instruction takes
+// 1 KiB of it, 128 bytes a clock over the four SIMDs.  With parts left out (2 x 16 on 8 x 1024, nothing masked, 229 us): no copies
+// 210, no exponentials and splits 209, neither 191.
 #include <type_traits>
 
 // (three bodies in one kernel spill scalar registers, copy descriptors among them: their copies take the five wait states)
@@ -221,17 +224,27 @@ __device__ __forceinline__ void bwd_wide_item(const SdpaBwdParams& bp, char* sme
     [[maybe_unused]] int k_acc = BW_LOOSE, k_w = BW_LOOSE;
     // One tile: the first products of tile t, whose eight registers that the partner needs go to the exchange area; a barrier;
     // the third product of tile t - 1 with P and dS of tile t made between its matrix instructions.
-    auto step = [&](const char* st, const char* pst, int r0, auto WITH_A_, auto WITH_B_) __attribute__((always_inline)) {
+    auto step = [&](const char* st, const char* pst, int r0, auto copies, auto WITH_A_, auto WITH_B_) __attribute__((always_inline)) {
         constexpr bool WITH_A = decltype(WITH_A_)::value, WITH_B = decltype(WITH_B_)::value;
         floatx16 f;
         vec8 o_hi, o_lo;
         [[maybe_unused]] int k_o = 0;
-        if constexpr (WITH_B) {      // the partner's half of tile t - 1's dS
-            o_hi = *(const vec8*)(x2 + (1 - role) * 2048);
-            o_lo = *(const vec8*)(x2 + (1 - role) * 2048 + 1024);
-            if constexpr (SCALED) k_o = x3[(1 - role) * 64];
-        }
+        auto read_partner = [&]() __attribute__((always_inline)) {      // the partner's half of tile t - 1's dS
+            if constexpr (WITH_B) {
+                o_hi = *(const vec8*)(x2 + (1 - role) * 2048);
+                o_lo = *(const vec8*)(x2 + (1 - role) * 2048 + 1024);
+                if constexpr (SCALED) k_o = x3[(1 - role) * 64];
+            }
+        };
         float4v nl[2], nd[2];
+        vec8 bring[R];
+        auto fetch_b = [&](int m) __attribute__((always_inline)) {      // m: column block m % NDB, rows 16 (role ^ (m / NDB)) .. + 15: the own half first
+            const char* tt = pst + (role ^ (m / NDB)) * 16 * L::ROWB;
+            short8v av;
+            av.lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((short4v __attribute__((address_space(3)))*)(tt + (tr_base[0] ^ ((m % NDB) << 6))));
+            av.hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((short4v __attribute__((address_space(3)))*)(tt + (tr_base[1] ^ ((m % NDB) << 6))));
+            bring[m % R] = __builtin_bit_cast(vec8, av);
+        };
         if constexpr (WITH_A) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) f[r] = 0.0f;
@@ -239,11 +252,15 @@ __device__ __forceinline__ void bwd_wide_item(const SdpaBwdParams& bp, char* sme
             auto fetch = [&](int i) __attribute__((always_inline)) { ring[i % R] = *(const vec8*)(st + (row_base ^ (i << 5))); };
 #pragma unroll
             for (int i = 0; i < R; ++i) fetch(i);
+            read_partner();
+            __builtin_amdgcn_sched_barrier(0);
+            copies();      // (behind the first reads: their latency covers what starting copies takes)
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int i = 0; i < NA; ++i) {
                 f = Mma<T>::run(ring[i % R], own[i], f);
                 if (i + R < NA) fetch(i + R);
+                else if (WITH_B) fetch_b(i + R - NA);      // (the third product's first operands are there when the barrier opens)
                 __builtin_amdgcn_sched_barrier(0);      // (the scheduler would put every read right in front of its matrix instruction)
             }
             // -L_i log2(e) and -D_i of the 16 rows this role makes P and dS of: register r is streamed row r0 + 16 role + 8 (r / 4) + 4 g + r % 4
@@ -270,6 +287,10 @@ __device__ __forceinline__ void bwd_wide_item(const SdpaBwdParams& bp, char* sme
             *(float4v*)(x1 + role * 2048) = float4v{f[8], f[9], f[10], f[11]};
             *(float4v*)(x1 + role * 2048 + 1024) = float4v{f[12], f[13], f[14], f[15]};
             __syncthreads();
+        } else {
+            read_partner();
+#pragma unroll
+            for (int m = 0; m < R; ++m) fetch_b(m);
         }
         if constexpr (WITH_B && SCALED) {
             const int k = min(k_w, k_o);
@@ -318,22 +339,12 @@ __device__ __forceinline__ void bwd_wide_item(const SdpaBwdParams& bp, char* sme
             }
         };
         if constexpr (WITH_B) {
-            vec8 ring[R];
-            auto fetch = [&](int m) __attribute__((always_inline)) {      // m: column block m % NDB, rows 16 (role ^ (m / NDB)) .. + 15: the own half first
-                const char* tt = pst + (role ^ (m / NDB)) * 16 * L::ROWB;
-                short8v av;
-                av.lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((short4v __attribute__((address_space(3)))*)(tt + (tr_base[0] ^ ((m % NDB) << 6))));
-                av.hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((short4v __attribute__((address_space(3)))*)(tt + (tr_base[1] ^ ((m % NDB) << 6))));
-                ring[m % R] = __builtin_bit_cast(vec8, av);
-            };
-#pragma unroll
-            for (int m = 0; m < R; ++m) fetch(m);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int m = 0; m < 2 * NDB; ++m) {
-                acc[m % NDB] = Mma<T>::run(ring[m % R], m < NDB ? w_hi : o_hi, acc[m % NDB]);
-                acc[m % NDB] = Mma<T>::run(ring[m % R], m < NDB ? w_lo : o_lo, acc[m % NDB]);
-                if (m + R < 2 * NDB) fetch(m + R);
+                acc[m % NDB] = Mma<T>::run(bring[m % R], m < NDB ? w_hi : o_hi, acc[m % NDB]);
+                acc[m % NDB] = Mma<T>::run(bring[m % R], m < NDB ? w_lo : o_lo, acc[m % NDB]);
+                if (m + R < 2 * NDB) fetch_b(m + R);
                 soft(m);
                 __builtin_amdgcn_sched_barrier(0);      // (likewise: the vector work would gather behind the matrix instructions)
             }
@@ -374,7 +385,6 @@ __device__ __forceinline__ void bwd_wide_item(const SdpaBwdParams& bp, char* sme
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         const int nstage = stage == 2 ? 0 : stage + 1;
-        if (n + 1 < n_hi) issue(nstage);
         return nstage;
     };
     auto advance = [&](int nstage) __attribute__((always_inline)) {
@@ -385,15 +395,15 @@ __device__ __forceinline__ void bwd_wide_item(const SdpaBwdParams& bp, char* sme
     };
     if (n_lo < n_hi) {
         const int first = next_tile();
-        step(smem, smem, r0, std::true_type{}, std::false_type{});
+        step(smem, smem, r0, [&]() __attribute__((always_inline)) { if (n + 1 < n_hi) issue(first); }, std::true_type{}, std::false_type{});
         advance(first);
         while (n < n_hi) {
             const int nstage = next_tile();
-            step(smem + stage * BW_STAGE, smem + pstage * BW_STAGE, r0, std::true_type{}, std::true_type{});
+            step(smem + stage * BW_STAGE, smem + pstage * BW_STAGE, r0, [&]() __attribute__((always_inline)) { if (n + 1 < n_hi) issue(nstage); }, std::true_type{}, std::true_type{});
             advance(nstage);
         }
         __syncthreads();      // (the last tile's dS)
-        step(smem, smem + pstage * BW_STAGE, 0, std::false_type{}, std::true_type{});
+        step(smem, smem + pstage * BW_STAGE, 0, []() {}, std::false_type{}, std::true_type{});
     }
 
     // ---- out: this role's half of the columns -----------------------------------------------------------------------------------
