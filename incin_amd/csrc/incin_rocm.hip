@@ -15,6 +15,7 @@
 
 #include "../../include/incin_rocm.h"
 #include "copy.h"
+#include "decode_deal.h"
 #include "kv_append.h"
 #include "sdpa_bwd.h"
 #include "sdpa_params.h"
@@ -31,6 +32,7 @@ hipError_t launch_mask_row_limits(const void* mask, int dtype, const int64_t sha
 hipError_t launch_sdpa_decode_f32_limits(const SdpaParams& p, hipStream_t stream);
 hipError_t launch_sdpa_decode(const SdpaParams& p, int dtype, hipStream_t stream);
 hipError_t launch_sdpa_decode_mfma(const SdpaParams& p, int dtype, hipStream_t stream);
+hipError_t launch_sdpa_decode_deal(const SdpaParams& p, int dtype, hipStream_t stream);
 hipError_t launch_read_rate(const void* src, void* sink, size_t bytes, int nontemporal, hipStream_t stream);
 hipError_t launch_lds_fill(void* sink, uint32_t pattern, hipStream_t stream);
 int decode_mfma_chunk_rows(int R, int dtype, int d_pad);
@@ -114,7 +116,8 @@ struct Plan {
     int impl;
     int splits;
     int split_len;
-    size_t ws_bytes;
+    int deal;        // workgroups of a launch that deals all sequences' keys (decode_deal.h); 0: by splits
+    size_t ws_bytes, deal_bytes;      // workspace of the launch by splits (it must have that), of the other (it is taken where there is that)
     size_t lims_offset;      // dense mask on the prefill kernels: where the mask's row limits start in the workspace (0: none)
     bool lims_splitkv;       // f32 with a dense mask: the blocks whose rows all have a limit go through the f32 split-KV kernel first
     bool empty;      // nothing to compute
@@ -160,6 +163,27 @@ bool mask_rows_stageable(const incin_rocm_sdpa_desc_t* d)
     return (32 * d->mask_stride[2] + d->Skv) < (1LL << 29);
 }
 
+// 16-bit decode with key counts: into how many workgroups the keys of all sequences are dealt (sdpa_decode_deal.hip), 0 for a launch
+// by splits of the capacity.  The host does not know the counts, so what speaks for it is what does not depend on them: a cache
+// large enough (300 MB) for the pass over the partial results and the division of the shares - 4 us and 1 - not to show, five sequences or
+// more, shares that hold few pieces (at most two rounds of (sequence, KV head) pairs, each of some thousand keys).  Bf16, four
+// query heads on each of 8 KV heads, counts spread evenly, us by splits / dealt: 32 x 1031 - 8192 106 / 98, 12 x 2048 - 16384 97 / 78.5,
+// 12 x 1000 - 8192 49.7 / 43.6, 24 x 512 - 4096 49.3 / 43.1, 48 x 1031 - 8192 156 / 144, 64 x 2000 - 16384 405 / 367, 20 of 4096 at D = 256 82 /
+// 70, 20 of 8192 on 12 KV heads 109 / 94, 20 of 8192 at D = 64 45 / 39; equal counts 32 x 4608 94.8 / 93.5, 8 x 12000 64.0 / 64.7, 64 x 16000 622 / 631.
+// Outside: 4 x 16384 30.6 / 33.2, 4 x 32768 58.6 / 61.5, 8 x 8192 33.2 / 33.0, 7 x 20000 on 1 KV head 18.1 / 21.2, 64 x 2048 54.9 / 57.7, 32 x 32 x 8192 351 / 356.
+// Two workgroups per compute unit where their LDS allows (rows x head dimension up to 512: 32 x 8192 ragged level, 24 x 4096 44.9 one, 43.1 two).
+// INCIN_ROCM_DECODE_DEAL forces a count of workgroups (0: by splits), for tests.
+int decode_deal_workgroups(const incin_rocm_sdpa_desc_t* d, int64_t R, int64_t d_pad)
+{
+    if (d->dtype == INCIN_ROCM_F32 || d->num_splits != 0 || d->add_mask || d->B > incin_rocm::DEAL_MAX_BATCH ||
+        R * d_pad > incin_rocm::DEAL_MAX_VALUES || d->B * d->Hkv * (d->Skv / 128 + 2) > (1LL << 30)) return 0;
+    const char* forced = getenv("INCIN_ROCM_DECODE_DEAL");
+    if (forced) return std::min(std::max(atoi(forced), 0), 4096);
+    const int64_t cus = compute_units_of(d->device), groups = d->B * d->Hkv, key_bytes = d->Skv * d_pad * 2;
+    if (d->impl != INCIN_ROCM_IMPL_AUTO || !d->kv_lens || d->B < 5 || groups > 2 * cus || 2 * groups * key_bytes < 300000000 || key_bytes < (groups > cus ? 1 << 20 : 3 << 18)) return 0;
+    return (int)(cus * (d_pad <= 128 && 2 * R * d_pad <= incin_rocm::DEAL_MAX_VALUES ? 2 : 1));
+}
+
 int make_plan(const incin_rocm_sdpa_desc_t* d, Plan* plan)
 {
     if (!d) return fail(INCIN_ROCM_EINVAL, "scaled_dot_product_attention: null descriptor");
@@ -174,6 +198,8 @@ int make_plan(const incin_rocm_sdpa_desc_t* d, Plan* plan)
     plan->splits = 1;
     plan->split_len = (int)d->Skv;
     plan->ws_bytes = 0;
+    plan->deal = 0;
+    plan->deal_bytes = 0;
     plan->lims_offset = 0;
     plan->lims_splitkv = false;
     plan->empty = (d->B == 0 || d->Hq == 0 || d->Sq == 0 || d->Dv == 0);
@@ -378,6 +404,8 @@ int make_plan(const incin_rocm_sdpa_desc_t* d, Plan* plan)
         plan->splits = (int)splits;
         plan->split_len = (int)split_len;
         plan->ws_bytes = splits > 1 ? (size_t)(d->B * d->Hq * d->Sq * splits) * (size_t)(d_pad + 2) * sizeof(float) : 0;
+        plan->deal = decode_deal_workgroups(d, R, d_pad);
+        if (plan->deal) plan->deal_bytes = incin_rocm::deal_workspace_bytes(plan->deal, (int)R, (int)d_pad);
     }
     if (impl == INCIN_ROCM_IMPL_MFMA && !d->add_mask && !d->q_lens && !(wide && d->dtype == INCIN_ROCM_F32)) {
         // The prefill kernels (16-bit and f32) run one workgroup per (batch, query head, 128 rows) and a compute unit holds two:
@@ -461,6 +489,7 @@ void fill_params(const incin_rocm_sdpa_desc_t* d, const Plan& plan, SdpaParams* 
         const int64_t slots = cus * (vector ? 4 : incin_rocm::decode_mfma_workgroups_per_cu((int)chunk, plan.split_len, d->dtype, p->Dp));
         p->split_even = incin_rocm::split_even_of(d->kv_lens != nullptr, p->B, plan.splits, wgs <= slots, (int64_t)plan.split_len * p->Dp * (int64_t)dtype_size(d->dtype), p->Dp);
         if (p->split_even) p->split_turn = 0;
+        p->deal = plan.deal;
     }
     if (plan.impl == INCIN_ROCM_IMPL_MFMA) p->mask_flags = d->add_mask ? (const uint8_t*)d->workspace : nullptr;
     if (plan.impl == INCIN_ROCM_IMPL_MFMA && d->add_mask && plan.lims_offset) p->mask_lims = (const int32_t*)((const char*)d->workspace + plan.lims_offset);
@@ -469,6 +498,7 @@ void fill_params(const incin_rocm_sdpa_desc_t* d, const Plan& plan, SdpaParams* 
         const size_t rows = (size_t)(d->B * d->Hq * d->Sq * plan.splits);
         p->ws_ml = (float*)d->workspace + rows * (size_t)p->Dp;      // partial rows are as wide as the kernel instance
     }
+    if (p->deal) p->ws_ml = (float*)d->workspace + (size_t)p->deal * 2 * (size_t)(p->G * p->Sq) * (size_t)p->Dp;
 }
 
 }  // namespace
@@ -792,16 +822,19 @@ int incin_rocm_sdpa_workspace(const incin_rocm_sdpa_desc_t* desc, size_t* bytes,
 {
     Plan plan;
     if (int rc = make_plan(desc, &plan)) return rc;
-    if (bytes) *bytes = plan.ws_bytes;
+    if (bytes) *bytes = std::max(plan.ws_bytes, plan.deal_bytes);
     if (splits) *splits = plan.splits;
     if (impl_out) *impl_out = plan.impl;
     return 0;
 }
 
 // Launches a validated request; the scratch memory is what desc->workspace names.
-static int launch_fwd(const incin_rocm_sdpa_desc_t* desc, const Plan& plan, void* stream)
+static int launch_fwd(const incin_rocm_sdpa_desc_t* desc, const Plan& planned, void* stream)
 {
-    if (plan.ws_bytes > 0) {
+    Plan plan = planned;
+    // (a workspace that is enough for the launch by splits, or none where that needs none, is not refused)
+    if (plan.deal && !(desc->workspace && desc->workspace_bytes >= plan.deal_bytes && aligned16(desc->workspace))) plan.deal = 0;
+    if (plan.ws_bytes > 0 && !plan.deal) {
         if (!desc->workspace || desc->workspace_bytes < plan.ws_bytes)
             return fail(INCIN_ROCM_EWORKSPACE,
                         "scaled_dot_product_attention: %s needs %zu workspace bytes, %zu given",
@@ -834,7 +867,7 @@ static int launch_fwd(const incin_rocm_sdpa_desc_t* desc, const Plan& plan, void
                                                 : incin_rocm::launch_sdpa_prefill_mfma(p, desc->dtype, s);
             break;
         case INCIN_ROCM_IMPL_SPLITKV: e = incin_rocm::launch_sdpa_decode(p, desc->dtype, s); break;
-        case INCIN_ROCM_IMPL_SPLITKV_MFMA: e = incin_rocm::launch_sdpa_decode_mfma(p, desc->dtype, s); break;
+        case INCIN_ROCM_IMPL_SPLITKV_MFMA: e = p.deal ? incin_rocm::launch_sdpa_decode_deal(p, desc->dtype, s) : incin_rocm::launch_sdpa_decode_mfma(p, desc->dtype, s); break;
         default: e = incin_rocm::launch_sdpa_generic(p, desc->dtype, s); break;
     }
     if (e != hipSuccess) return hip_fail(e, "attention kernel launch");
@@ -891,6 +924,8 @@ int incin_rocm_sdpa_fwd_static(const incin_rocm_sdpa_desc_t* desc, void* stream)
                     "sdpa_fwd_static: this request needs %zu bytes of scratch memory, the static buffer holds %zu "
                     "(fewer splits, or incin_rocm_sdpa_fwd with a workspace of the caller's)",
                     plan.ws_bytes, (size_t)INCIN_ROCM_STATIC_SCRATCH_BYTES);
+    // (a call that needs no scratch memory leaves the shared buffer alone: such calls may overlap)
+    if (plan.ws_bytes == 0) plan.deal = 0;
     incin_rocm_sdpa_desc_t d = *desc;
     d.workspace = nullptr;
     d.workspace_bytes = 0;

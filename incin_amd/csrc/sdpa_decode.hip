@@ -17,7 +17,7 @@
 // final output itself.
 #include <atomic>
 
-#include "sdpa_params.h"
+#include "decode_deal.h"
 
 namespace incin_rocm {
 
@@ -235,7 +235,10 @@ __global__ __launch_bounds__(256) void sdpa_decode_split_kernel(SdpaParams p)
 // thread holds 4 consecutive output elements; the D / 4 threads of a group walk the splits group, group + NG, ..., so
 // that NG splits are read side by side (a launch with hundreds of splits and few rows would otherwise walk them one
 // after the other), and the groups' sums meet in LDS.  blockDim.x = NG * D / 4, a multiple of 64.
-template <typename T, int D>
+//
+// DEAL: the partial results of a row are those of the shares that its sequence's units went to (decode_deal.h); rows of
+// sequences that one share holds are finished already.
+template <typename T, int D, bool DEAL = false>
 __global__ __launch_bounds__(256) void sdpa_combine_kernel(SdpaParams p)
 {
     constexpr int TPR = D / 4;
@@ -250,10 +253,25 @@ __global__ __launch_bounds__(256) void sdpa_combine_kernel(SdpaParams p)
     const int i = (int)(row % p.Sq);
     const int64_t bh = row / p.Sq;
     const int hq = (int)(bh % p.Hq), b = (int)(bh / p.Hq);
-    const float* ml = p.ws_ml + row * p.num_splits * 2;
-    const float* ac = p.ws_acc + row * p.num_splits * D;
+    int n = p.num_splits, w0 = 0, rows_per_place = 1, place_row = 0;
+    if constexpr (DEAL) {
+        const DealColumn column = deal_column<deal_unit<T, D>()>(p);
+        const DealShares shares(column.total * p.Hkv, p.deal);
+        int first, units;
+        deal_place(column, b, &first, &units);
+        first += hq / p.G * column.total;
+        w0 = shares.owner(first);
+        n = shares.owner(first + units - 1) - w0 + 1;
+        if (n == 1) return;      // (uniform)
+        rows_per_place = p.G * p.Sq;
+        place_row = (hq % p.G) * p.Sq + i;
+    }
+    // partial result s of the row: (maximum, sum) and numerators
+    const float* ml = DEAL ? p.ws_ml : p.ws_ml + row * p.num_splits * 2;
+    const float* ac = DEAL ? p.ws_acc : p.ws_acc + row * p.num_splits * D;
+    auto at = [&](int s) __attribute__((always_inline)) { return DEAL ? deal_slot(w0 + s, s < n - 1, rows_per_place, place_row) : (int64_t)s; };
     float m = -INFINITY;
-    for (int s = tid; s < p.num_splits; s += blockDim.x) m = fmaxf(m, ml[s * 2]);
+    for (int s = tid; s < n; s += blockDim.x) m = fmaxf(m, ml[at(s) * 2]);
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
     if ((tid & 63) == 0) s_max[tid >> 6] = m;
@@ -264,10 +282,11 @@ __global__ __launch_bounds__(256) void sdpa_combine_kernel(SdpaParams p)
     const int grp = tid / TPR, c = tid % TPR;
     f4 A = {0.0f, 0.0f, 0.0f, 0.0f};
     float L = 0.0f;
-    for (int s = grp; s < p.num_splits; s += ng) {
-        const float w = Softexp<T>::ex(ml[s * 2] - M_use);
-        L = fmaf(w, ml[s * 2 + 1], L);
-        const f4 a = *(const f4*)(ac + (int64_t)s * D + 4 * c);
+    for (int s = grp; s < n; s += ng) {
+        const int64_t slot = at(s);
+        const float w = Softexp<T>::ex(ml[slot * 2] - M_use);
+        L = fmaf(w, ml[slot * 2 + 1], L);
+        const f4 a = *(const f4*)(ac + slot * D + 4 * c);
 #pragma unroll
         for (int e = 0; e < 4; ++e) A[e] = fmaf(w, a[e], A[e]);
     }
@@ -297,6 +316,12 @@ static hipError_t launch_combine_t(const SdpaParams& p, hipStream_t stream)
 {
     constexpr int TPR = D / 4;
     int ng = 64 / TPR;                                  // at least one wavefront
+    if constexpr (sizeof(T) == 2) {
+        if (p.deal) {
+            hipLaunchKernelGGL((sdpa_combine_kernel<T, D, true>), dim3((unsigned)((int64_t)p.B * p.Hq * p.Sq)), dim3(256), 0, stream, p);
+            return hipGetLastError();
+        }
+    }
     while (ng < 256 / TPR && ng < p.num_splits) ng *= 2;
     hipLaunchKernelGGL((sdpa_combine_kernel<T, D>), dim3((unsigned)((int64_t)p.B * p.Hq * p.Sq)), dim3(ng * TPR), 0, stream, p);
     return hipGetLastError();

@@ -672,6 +672,75 @@ def test_decode_splitkv_matrix_cores_d64(gpu, dtype, shape, slots, monkeypatch):
         check(got, host.sdpa(q, k, v, dtype, causal=causal, kv_lens=lens, impl=capi.IMPL_SPLITKV), 8e-3, "matrix-core vs vector-ALU split-KV, D = 64")
 
 
+@pytest.mark.parametrize("dtype", [capi.BF16, capi.F16], ids=lambda x: dtypes.NAMES[x])
+@pytest.mark.parametrize("case", [
+    # Hq, Hkv, Sq, D, Dv, causal, Skv, key counts
+    (8, 2, 1, 128, 128, False, 1000, [1000, 0, 1, 127, 128, 129, 255, 700]),      # edges of a unit of 128 keys, an empty sequence
+    (8, 1, 1, 128, 128, False, 1300, [0, 0, 1300]),                               # eight rows; the first two sequences empty
+    (6, 3, 4, 64, 64, True, 1100, [1100, 255, 256, 257, 3, 900]),                 # causal among four positions, units of 256 keys
+    (4, 2, 1, 200, 256, False, 600, [600, 5, 128, 300, 600]),                     # the 256 instance, zero-padded
+    (16, 1, 1, 56, 64, False, 777, [777, 776, 1]),                                # sixteen rows
+    (2, 2, 3, 80, 96, True, 400, None),                                           # no counts: the capacity
+    (4, 4, 1, 128, 128, False, 130, [(37 * b) % 131 for b in range(200)]),        # more sequences than lanes
+])
+def test_keys_dealt_in_equal_shares(gpu, dtype, case, monkeypatch):
+    """Decode whose workgroups take equal shares of all sequences' keys (chosen for large ragged batches; forced here with counts of
+    workgroups that cut sequences, hold several of them, and outnumber the units): against the oracle, row normalisers against
+    the launch by splits, twice the same bytes, and with less workspace than it asks for the launch by splits itself."""
+    Hq, Hkv, Sq, D, Dv, causal, Skv, counts = case
+    B = 3 if counts is None else len(counts)
+    lens = None if counts is None else np.array(counts, np.int32)
+    q, k, v = inputs(5300 + Skv, B, Hq, Hkv, Sq, Skv, D, Dv, dtype)
+    ref = oracle_full(q, k, v, G=Hq // Hkv, causal=causal, kv_lens=lens)
+    monkeypatch.setenv("INCIN_ROCM_DECODE_DEAL", "0")
+    _, lse_s, info_s = host.sdpa(q, k, v, dtype, causal=causal, kv_lens=lens, impl=capi.IMPL_SPLITKV_MFMA, return_lse=True, return_info=True)
+    for workgroups in (1, 3, 7, 61, 600):
+        monkeypatch.setenv("INCIN_ROCM_DECODE_DEAL", str(workgroups))
+        say("dealt: %s %r workgroups=%d" % (dtypes.NAMES[dtype], case[:7], workgroups))
+        got, lse, info = host.sdpa(q, k, v, dtype, causal=causal, kv_lens=lens, impl=capi.IMPL_SPLITKV_MFMA, return_lse=True, return_info=True)
+        Dp = 64 if max(D, Dv) <= 64 else 128 if max(D, Dv) <= 128 else 256
+        assert info["workspace_bytes"] == max(info_s["workspace_bytes"], workgroups * 2 * (Hq // Hkv) * Sq * (Dp + 2) * 4)
+        check(got, ref, TOL[dtype], "dealt to %d workgroups" % workgroups)
+        fin = np.isfinite(lse_s)
+        # (either sum is of probabilities rounded to the storage type, 2^-9 or 2^-12 of each at most, against references of its own)
+        assert np.array_equal(fin, np.isfinite(lse)) and np.abs(lse[fin] - lse_s[fin]).max() <= 2.0 ** (-8 if dtype == capi.BF16 else -11)
+        again = host.sdpa(q, k, v, dtype, causal=causal, kv_lens=lens, impl=capi.IMPL_SPLITKV_MFMA)
+        assert np.array_equal(got, again, equal_nan=True)
+
+
+def test_keys_dealt_where_a_large_batch_is_ragged(gpu):
+    """The library's own choice for a large ragged batch: key counts change between two launches of one descriptor, and a descriptor
+    with no more workspace than the launch by splits needs is served as it was."""
+    B, Hq, Hkv, Skv, D = 12, 32, 8, 8192, 128
+    r = rng(5400)
+    mk = lambda *s: dtypes.round_to(r.standard_normal(s, dtype=np.float32), capi.BF16)
+    qf, kf, vf = mk(B, Hq, 1, D), mk(B, Hkv, Skv, D), mk(B, Hkv, Skv, D)
+    tq, tk, tv = (host.DeviceTensor.from_f32(x, capi.BF16) for x in (qf, kf, vf))
+    outs = []
+    lens = np.array([1000 + 600 * b for b in range(B)], np.int32)
+    for dealt in (True, False):
+        to, tl = host.DeviceTensor((B, Hq, 1, D), capi.BF16), capi.DeviceBuffer.from_numpy(lens)
+        desc = host.make_desc(tq, tk, tv, to, kv_lens=tl)
+        need, splits, impl = capi.sdpa_workspace(desc)
+        old = B * Hq * splits * (D + 2) * 4 if splits > 1 else 0
+        assert impl == capi.IMPL_SPLITKV_MFMA and need >= 2 * 256 * 4 * (D + 2) * 4
+        give = need if dealt else old
+        ws = capi.DeviceBuffer(give) if give else None
+        if ws is not None:
+            desc.workspace, desc.workspace_bytes = ws.ptr, give
+        for n in (lens, lens[::-1].copy()):
+            capi.check(capi.load().incin_rocm_memcpy_h2d(0, tl.ptr, n.ctypes.data, n.nbytes))
+            capi.sdpa_fwd(desc)
+            capi.sync()
+            outs.append(to.to_f32())
+    for a, b in ((0, 2), (1, 3)):
+        check(outs[a], outs[b], 8e-3, "dealt against splits")
+    for o, n in ((outs[0], lens), (outs[1], lens[::-1])):
+        rows = [0, 5, B - 1]
+        ref = oracle_full(qf[rows], kf[rows], vf[rows], G=Hq // Hkv, kv_lens=n[rows])
+        check(o[rows], ref, TOL[capi.BF16], "dealt, large batch")
+
+
 @pytest.mark.parametrize("D", [128, 64])
 @pytest.mark.parametrize("slots", ["2", "5"], ids=["two_slot_rings", "five_slot_rings"])
 @pytest.mark.parametrize("shape", [
