@@ -37,7 +37,7 @@ constexpr int PW_KT = 32;      // keys per tile
 // of whose rows the mask gives n zeros and then -inf (sdpa_prefill_mfma.hip has the scheme: a masked request is the LIMS
 // launch, whose other workgroups leave at once, and then the DENSE launch, whose workgroups leave if LIMS took their block).
 //
-// KG: wavefronts per 32 query rows.  With 2 (no mask tensor, no splits) a workgroup is eight wavefronts, each group of four with tile
+// KG: wavefronts per 32 query rows.  With 2 (no mask values, no splits) a workgroup is eight wavefronts, each group of four with tile
 // buffers of its own: the first walks the even tiles of the block, the second the odd ones, and the two partial results of a row
 // meet in LDS at the end, either group finishing half of the columns.  For launches of at most a workgroup per compute unit,
 // whose wavefronts would otherwise be alone on their SIMDs and walk all keys one tile after the other.
@@ -45,7 +45,7 @@ template <typename T, int MASK, bool SPLIT = false, int KG = 1>
 __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(2, 2))) void sdpa_prefill_wide_kernel(SdpaParams p)
 {
     constexpr bool DENSE = MASK == 1, LIMS = MASK == 2;
-    static_assert(KG == 1 || (KG == 2 && MASK == 0 && !SPLIT), "two groups of wavefronts: the plain launch only");
+    static_assert(KG == 1 || (KG == 2 && !DENSE && !SPLIT), "two groups of wavefronts: blocks that need no mask values, keys not split");
 #if defined(__HIP_DEVICE_COMPILE__)
     typedef typename Mma<T>::vec8 vec8;
     constexpr int D = 256;
@@ -422,7 +422,7 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(2, 2))
 static bool two_groups(const SdpaParams& p, int64_t total, int nqb)
 {
     const int64_t cus = device_cus();
-    return total <= cus || (total <= 2 * cus && p.causal && nqb >= 8 && p.Skv - p.Sq <= p.Sq / 4);
+    return total <= cus || (total <= 2 * cus && (p.causal || p.mask) && nqb >= 8 && p.Skv - p.Sq <= p.Sq / 4);
 }
 
 // Host has validated: dtype f16 / bf16, 128 < max(D, Dv) <= 256 in whole 16-byte vectors, finite scale; with a dense mask its
@@ -441,7 +441,10 @@ hipError_t launch_sdpa_prefill_wide(const SdpaParams& p0, int dtype, hipStream_t
     p.interleave = work_interleave(p.causal != 0 || p.mask != nullptr, 2 * device_cus() / 8, p.G, nqb, (total & 7) == 0 ? total >> 3 : total);
     p.deal_groups = (total & 7) == 0 ? work_deal(p.interleave, p.G, nqb, total >> 3, p.causal != 0 || p.mask != nullptr) : 0;
     if (p.mask && p.mask_lims) {       // the blocks whose rows all have a limit; then, below, the others
-        if (dtype == 1) hipLaunchKernelGGL((sdpa_prefill_wide_kernel<f16_t, 2>), dim3((unsigned)total), dim3(256), 0, stream, p);
+        if (two_groups(p, total, nqb)) {      // (as the launch of the flag that such a mask stands for)
+            if (dtype == 1) hipLaunchKernelGGL((sdpa_prefill_wide_kernel<f16_t, 2, false, 2>), dim3((unsigned)total), dim3(512), 0, stream, p);
+            else hipLaunchKernelGGL((sdpa_prefill_wide_kernel<bf16_t, 2, false, 2>), dim3((unsigned)total), dim3(512), 0, stream, p);
+        } else if (dtype == 1) hipLaunchKernelGGL((sdpa_prefill_wide_kernel<f16_t, 2>), dim3((unsigned)total), dim3(256), 0, stream, p);
         else hipLaunchKernelGGL((sdpa_prefill_wide_kernel<bf16_t, 2>), dim3((unsigned)total), dim3(256), 0, stream, p);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
