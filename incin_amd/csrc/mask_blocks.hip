@@ -8,7 +8,7 @@
 // One workgroup per strip of 32 rows x 256 keys (8 blocks): a thread takes 8 consecutive keys of 4 rows - one 16-byte
 // load each for 16-bit masks with unit key stride and aligned rows, element-wise loads otherwise - and the votes of a
 // block meet in LDS; rows beyond Sq and keys beyond Skv do not vote.
-#include "sdpa_params.h"
+#include "sdpa_mfma_common.h"
 
 namespace incin_rocm {
 
@@ -116,6 +116,67 @@ __global__ __launch_bounds__(256) void mask_row_limits_kernel(const T* mask, int
     if (lane == 0) lims[r] = ninf == Skv - first ? first : -1;
 }
 
+// Both in one pass over the mask: a workgroup of sixteen wavefronts takes 32 whole rows, two per wavefront, and has the limits of
+// the rows and the flags of their blocks at the end.  Row by row as above (first position that is not zero, number of -inf values),
+// the votes of a stretch of 4096 keys in LDS.
+template <typename T, bool VEC>
+__global__ __launch_bounds__(1024) void mask_scan_kernel(const T* mask, int64_t m_sb, int64_t m_sh, int64_t m_si, int64_t m_sj,
+                                                        int Hm, int Sq, int Skv, int nkb, uint8_t* flags, int32_t* lims, int rows_m)
+{
+    constexpr int STRETCH = 4096;
+    __shared__ int votes[STRETCH / 32][2];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int rb = blockIdx.x, bh = blockIdx.y;
+    const T* base = mask + (int64_t)(bh / Hm) * m_sb + (int64_t)(bh % Hm) * m_sh;
+    int first[2] = {Skv, Skv}, ninf[2] = {0, 0};
+    for (int s0 = 0; s0 < Skv; s0 += STRETCH) {
+        const int s1 = min(s0 + STRETCH, Skv);
+        if (threadIdx.x < 2 * STRETCH / 32) votes[threadIdx.x >> 1][threadIdx.x & 1] = 0;
+        __syncthreads();
+#pragma unroll 2
+        for (int j0 = s0 + lane * 8; j0 < s1; j0 += 512) {
+            int not_zero = 0, not_hidden = 0;
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                const int i = rb * 32 + wave + 16 * r;
+                if (i >= Sq) continue;
+                const T* row = base + (int64_t)i * m_si;
+                auto see = [&](float f, int j) __attribute__((always_inline)) {
+                    if (!(f == 0.0f)) first[r] = min(first[r], j);
+                    ninf[r] += f == -INFINITY;
+                    not_zero |= !(f == 0.0f);
+                    not_hidden |= !(f == -INFINITY);
+                };
+                if (VEC && j0 + 7 < Skv) {
+                    typedef T vec8 __attribute__((ext_vector_type(8)));
+                    const vec8 x = *(const vec8*)(row + j0);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) see(to_f32(x[e]), j0 + e);
+                } else {
+                    for (int e = 0; e < 8 && j0 + e < Skv; ++e) see(to_f32(row[(int64_t)(j0 + e) * m_sj]), j0 + e);
+                }
+            }
+            if (not_zero) atomicOr(&votes[(j0 - s0) >> 5][0], 1);
+            if (not_hidden) atomicOr(&votes[(j0 - s0) >> 5][1], 1);
+        }
+        __syncthreads();
+        const int kb = s0 / 32 + (int)threadIdx.x;
+        if (threadIdx.x < STRETCH / 32 && kb < nkb)
+            flags[((int64_t)bh * gridDim.x + rb) * nkb + kb] = !votes[threadIdx.x][0] ? 1 : (!votes[threadIdx.x][1] ? 2 : 0);
+        __syncthreads();
+    }
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) {
+            first[r] = min(first[r], __shfl_xor(first[r], off, 64));
+            ninf[r] += __shfl_xor(ninf[r], off, 64);
+        }
+        const int i = rb * 32 + wave + 16 * r;
+        if (lane == 0 && i < rows_m) lims[(int64_t)bh * rows_m + i] = ninf[r] == Skv - first[r] ? first[r] : -1;      // (rows that are repeated: one of them)
+    }
+}
+
 // Host has validated the extents; nbh = mask batch entries x mask heads (1 where the mask is broadcast).
 hipError_t launch_mask_classify(const SdpaParams& p, int dtype, hipStream_t stream)
 {
@@ -129,6 +190,21 @@ hipError_t launch_mask_classify(const SdpaParams& p, int dtype, hipStream_t stre
     // 8 consecutive elements in one vector load: unit key stride, every row start a multiple of the vector
     const bool vec = p.m_sj == 1 && ((uintptr_t)p.mask % (8 * esz)) == 0 && p.m_sb % 8 == 0 && p.m_sh % 8 == 0 && p.m_si % 8 == 0;
     const int rows_m = p.m_si ? p.Sq : 1;
+    // Limits and flags in one pass where its workgroups - one per 32 rows of the mask - are as many as compute units, or rows are so
+    // short that a launch is all there is to save; else two kernels, whose second reads nothing where all rows have limits.  Whole
+    // call, us, two / one: f32, a bias per head, 8 heads x 1024 x 1024 134 / 130, x 4096 887 / 824, 4 x 2048 x 16384 2200 / 2116, bf16 likewise 42.1 /
+    // 38.4, 231 / 231, 452 / 416; 129 x 129 30.7 / 27.7, 25.4 / 22.5; one causal mask of 256 x 256 19.6 / 18.2, 18.5 / 16.2, of 1024 x 1024 60.0 / 61.0,
+    // 24.5 / 24.9, 4096 x 4096 314 / 316, 74.4 / 79.3, 128 rows x 8192 291 / 304, 128 / 141.
+    if (p.mask_lims && (p.Skv <= 512 || (int64_t)nrb * Bm * Hm >= device_cus())) {
+#define SCAN(T, V) hipLaunchKernelGGL((mask_scan_kernel<T, V>), dim3(nrb, Bm * Hm), dim3(1024), 0, stream, (const T*)p.mask, p.m_sb, p.m_sh, p.m_si, p.m_sj, Hm, p.Sq, p.Skv, nkb, flags, (int32_t*)p.mask_lims, rows_m)
+        switch (dtype) {
+            case 0: if (vec) SCAN(float, true); else SCAN(float, false); break;
+            case 1: if (vec) SCAN(f16_t, true); else SCAN(f16_t, false); break;
+            default: if (vec) SCAN(bf16_t, true); else SCAN(bf16_t, false); break;
+        }
+#undef SCAN
+        return hipGetLastError();
+    }
     if (p.mask_lims) {       // the limits first: the flags of blocks whose rows all have one are not needed
         const int64_t n_rows = (int64_t)Bm * Hm * rows_m;
         const dim3 lgrid((unsigned)((n_rows + 3) / 4));

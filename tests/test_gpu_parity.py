@@ -438,6 +438,33 @@ def test_auto_splits_the_keys_of_a_wide_prefill_launch_that_fills_the_device(gpu
         assert np.abs(got.reshape(Hq, Sq, 256)[rows[:, 0], rows[:, 1]] - ref).max() <= TOL[capi.BF16]
 
 
+@pytest.mark.parametrize("dtype", [capi.F32, capi.BF16], ids=lambda x: dtypes.NAMES[x])
+@pytest.mark.parametrize("Skv", [4200, 4097, 4096, 8200])
+def test_mask_limits_and_flags_in_one_pass(gpu, dtype, Skv):
+    """A mask of 32-row strips enough for every compute unit is read once, 4096 keys at a time: rows with limits on both sides of a
+    stretch's end, rows whose zeros end and begin again behind it, values in the last keys only, an odd number of rows - against the
+    kernels that read the mask's values as they are."""
+    H, Sq, D = 52, 141, 64      # 5 strips a head, the last of 13 rows
+    q, k, v = inputs(5500 + Skv, 1, H, H, Sq, Skv, D, D, dtype)
+    r = rng(5501)
+    mask = np.zeros((1, H, Sq, Skv), np.float32)
+    for h in range(H):
+        m = mask[0, h]
+        if h % 4 == 0:      # limits around the end of a stretch
+            for i in range(Sq):
+                m[i, min(4090 + (i * 7 + h) % 16, Skv):] = -np.inf
+        elif h % 4 == 1:      # a hole
+            m[: 64, 4000:4090] = -np.inf
+            m[64:, 100:300] = -np.inf
+        elif h % 4 == 2:      # values in the last keys
+            m[:, Skv - 3:] = dtypes.round_to(r.standard_normal((Sq, 3), dtype=np.float32), dtype)
+        else:
+            m[:, 5 + 3 * h:] = -np.inf
+    got = host.sdpa(q, k, v, dtype, mask=mask)
+    ref = host.sdpa(q, k, v, dtype, mask=mask, impl=capi.IMPL_GENERIC)
+    check(got, ref, TOL[dtype], "mask in one pass, %d keys" % Skv)
+
+
 @pytest.mark.parametrize("dtype", [capi.BF16, capi.F16], ids=lambda x: dtypes.NAMES[x])
 @pytest.mark.parametrize("rows", ["128", "256"])
 @pytest.mark.parametrize("D", [128, 64])
