@@ -39,9 +39,9 @@ struct Error {
 };
 
 // One device allocation, released when the last storage that views it goes away.  Released, not freed: the buffer goes back
-// to a pool per device, stamped with an event on the stream the releasing thread works on, and is handed out again to
-// that same stream at once (its work is ordered behind what still uses the buffer) or to another stream once the event
-// has passed - the stream-ordered lifetime the reference's CUDA buffers have (cuda/storage.rs:171-177, 225-233).  So an
+// to a pool per device and is handed out again to the stream the releasing thread works on at once (its work is ordered behind
+// what still uses the buffer) or to another stream once an event on that one, recorded behind the release - at the latest when
+// the thread has left sixteen buffers or 64 MiB so -, has passed - the stream-ordered lifetime the reference's CUDA buffers have (cuda/storage.rs:171-177, 225-233).  So an
 // operator can drop temporaries and workspaces that its kernels are still using without waiting for the device.
 class RocmBuffer {
   public:

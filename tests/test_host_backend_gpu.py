@@ -499,6 +499,63 @@ def test_operators_do_not_allocate_once_the_pool_is_warm(gpu):
     assert RB.pool_stats()[2] == 0
 
 
+def test_blocks_left_in_stream_order_come_back(gpu):
+    """Released blocks that no event stands behind: the stream they were released on has them again at once; a thread that never
+    had that stream does not, while the thread that left them is there and on it - and does once that thread is gone, from the
+    pool; more releases than a thread may leave so, and then results are still those of eager calls on untouched buffers."""
+    import threading
+    from incin_amd import capi
+    q, k, v = (rnd(90 + i, (2, 4, 160, 64), RB.F32) for i in range(3))
+    ref = O.sdpa(q, k, v)
+    streams = [capi.Stream() for _ in range(2)]
+    RB.trim_pool()
+    done, go_on = threading.Event(), threading.Event()
+    results, stats = [], {}
+
+    def first():
+        RB.set_stream(streams[0].ptr)
+        S = [RB.RocmStorage.from_numpy(a) for a in (q, k, v)]
+        for _ in range(3):
+            kept = [RB.scaled_dot_product_attention(*S) for _ in range(24)]      # (24 outputs at once: beyond what may go without an event)
+            results.append(kept[-1].to_numpy())
+            del kept
+        one = RB.scaled_dot_product_attention(*S)
+        before = RB.pool_stats()
+        del one
+        for _ in range(5):
+            RB.scaled_dot_product_attention(*S)
+        stats["repeat"] = (before, RB.pool_stats())
+        del S
+        done.set()
+        go_on.wait(60)
+
+    t = threading.Thread(target=first)
+    t.start()
+    assert done.wait(60)
+    RB.set_stream(streams[1].ptr)
+    try:
+        S = [RB.RocmStorage.from_numpy(a) for a in (q, k, v)]
+        results.append(RB.scaled_dot_product_attention(*S).to_numpy())
+        go_on.set()
+        t.join()
+        before = RB.pool_stats()
+        kept = [RB.scaled_dot_product_attention(*S) for _ in range(24)]      # the gone thread's blocks among them
+        after = RB.pool_stats()
+        results.append(kept[0].to_numpy())
+        results.append(kept[-1].to_numpy())
+        del kept, S
+    finally:
+        RB.set_stream(None)
+    for r in results:
+        close(r, ref, TOL[RB.F32], "operator on pooled blocks")
+    assert stats["repeat"][1][0] == stats["repeat"][0][0], "a repeated operator finds its blocks on its own stream: %r" % (stats["repeat"],)
+    assert after[0] - before[0] < 8 and after[1] - before[1] >= 16, "blocks of a thread that is gone: %r -> %r" % (before, after)
+    RB.trim_pool()
+    assert RB.pool_stats()[2] == 0
+    for s in streams:
+        s.destroy()
+
+
 def test_recorded_operator_with_a_transposed_k(gpu):
     """The operator with k handed over as a transposed view (gathered into a temporary first), recorded into a launch graph on
     a stream of the caller's and replayed: no step of it waits for the device or allocates while recording; every replay -
