@@ -1,7 +1,9 @@
 """The attention op through the C++ host mirror of the reference's backend interface, written the way
 the reference's own tests use the op (crates/incin/tests/medium_priority_ops_tests.rs:57-67:
 storages in, optional mask and scale, storage out) and checked against the CPU oracle."""
+import os
 import sys
+import time
 
 import numpy as np
 import pytest
@@ -538,6 +540,10 @@ def test_blocks_left_in_stream_order_come_back(gpu):
         results.append(RB.scaled_dot_product_attention(*S).to_numpy())
         go_on.set()
         t.join()
+        for _ in range(2000):      # (join returns before the thread has left the process, and what it kept goes with it only then)
+            if not os.path.exists("/proc/self/task/%d" % t.native_id):
+                break
+            time.sleep(0.005)
         before = RB.pool_stats()
         kept = [RB.scaled_dot_product_attention(*S) for _ in range(24)]      # the gone thread's blocks among them
         after = RB.pool_stats()
