@@ -236,6 +236,12 @@ __global__ __launch_bounds__(256) void sdpa_decode_split_kernel(SdpaParams p)
 // that NG splits are read side by side (a launch with hundreds of splits and few rows would otherwise walk them one
 // after the other), and the groups' sums meet in LDS.  blockDim.x = NG * D / 4, a multiple of 64.
 //
+// Behind a small split-KV launch this is a chain of latencies, so a group asks for its first AHEAD splits - maxima, sums and
+// numerators - before the common maximum is known, and the row's place comes from the grid without a division.
+// With the split kernels' meeting of wavefronts 16 bytes at a time, us a call before / after: bf16, 32 on 8 heads, one sequence of 2085 keys 10.7 /
+// 10.2, four of 300 - 1000 10.5 / 10.3, 16 on 2 heads x 5 positions x 4 x 3000 18.6 / 17.3, 4 x 1000 - 3000 at D = 256 19.0 / 18.1; f32 2 x 8 on
+// 4 x 1000 - 2000 at D = 64 10.6 / 10.3.
+//
 // DEAL: the partial results of a row are those of the shares that its sequence's units went to (decode_deal.h); rows of
 // sequences that one share holds are finished already.
 template <typename T, int D, bool DEAL = false>
@@ -243,16 +249,16 @@ __global__ __launch_bounds__(256) void sdpa_combine_kernel(SdpaParams p)
 {
     constexpr int TPR = D / 4;
     constexpr int NG_MAX = 256 / TPR;
+    typedef float f2 __attribute__((ext_vector_type(2)));
     typedef float f4 __attribute__((ext_vector_type(4)));
     __shared__ float s_max[4];
     __shared__ f4 s_acc[NG_MAX][TPR];
     __shared__ float s_l[NG_MAX];
-    const int64_t row = blockIdx.x;                    // (b * Hq + hq) * Sq + i
+    constexpr int AHEAD = 4;
     const int tid = threadIdx.x;
     const int ng = blockDim.x / TPR;
-    const int i = (int)(row % p.Sq);
-    const int64_t bh = row / p.Sq;
-    const int hq = (int)(bh % p.Hq), b = (int)(bh / p.Hq);
+    const int i = blockIdx.x, hq = blockIdx.y, b = blockIdx.z;
+    const int64_t row = ((int64_t)b * p.Hq + hq) * p.Sq + i;
     int n = p.num_splits, w0 = 0, rows_per_place = 1, place_row = 0;
     if constexpr (DEAL) {
         const DealColumn column = deal_column<deal_unit<T, D>()>(p);
@@ -270,8 +276,21 @@ __global__ __launch_bounds__(256) void sdpa_combine_kernel(SdpaParams p)
     const float* ml = DEAL ? p.ws_ml : p.ws_ml + row * p.num_splits * 2;
     const float* ac = DEAL ? p.ws_acc : p.ws_acc + row * p.num_splits * D;
     auto at = [&](int s) __attribute__((always_inline)) { return DEAL ? deal_slot(w0 + s, s < n - 1, rows_per_place, place_row) : (int64_t)s; };
+    const int grp = tid / TPR, c = tid % TPR;
+    f2 first_ml[AHEAD];
+    f4 first_a[AHEAD];
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+        if (u * ng < n) {      // (uniform; a group whose split is beyond the last one reads that again)
+            const int64_t slot = at(min(grp + u * ng, n - 1));
+            first_ml[u] = *(const f2*)(ml + slot * 2);
+            first_a[u] = *(const f4*)(ac + slot * D + 4 * c);
+        }
     float m = -INFINITY;
-    for (int s = tid; s < n; s += blockDim.x) m = fmaxf(m, ml[at(s) * 2]);
+    for (int s = AHEAD * ng + tid; s < n; s += blockDim.x) m = fmaxf(m, ml[at(s) * 2]);
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+        if (u * ng < n) m = fmaxf(m, first_ml[u][0]);
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
     if ((tid & 63) == 0) s_max[tid >> 6] = m;
@@ -279,16 +298,20 @@ __global__ __launch_bounds__(256) void sdpa_combine_kernel(SdpaParams p)
     float M = s_max[0];
     for (int w = 1; w < (int)(blockDim.x >> 6); ++w) M = fmaxf(M, s_max[w]);
     const float M_use = (M == -INFINITY) ? 0.0f : M;
-    const int grp = tid / TPR, c = tid % TPR;
     f4 A = {0.0f, 0.0f, 0.0f, 0.0f};
     float L = 0.0f;
-    for (int s = grp; s < n; s += ng) {
-        const int64_t slot = at(s);
-        const float w = Softexp<T>::ex(ml[slot * 2] - M_use);
-        L = fmaf(w, ml[slot * 2 + 1], L);
-        const f4 a = *(const f4*)(ac + slot * D + 4 * c);
+    auto add = [&](f2 part, f4 a) __attribute__((always_inline)) {
+        const float w = Softexp<T>::ex(part[0] - M_use);
+        L = fmaf(w, part[1], L);
 #pragma unroll
         for (int e = 0; e < 4; ++e) A[e] = fmaf(w, a[e], A[e]);
+    };
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+        if (grp + u * ng < n) add(first_ml[u], first_a[u]);
+    for (int s = grp + AHEAD * ng; s < n; s += ng) {
+        const int64_t slot = at(s);
+        add(*(const f2*)(ml + slot * 2), *(const f4*)(ac + slot * D + 4 * c));
     }
     s_acc[grp][c] = A;
     if (c == 0) s_l[grp] = L;
@@ -315,15 +338,16 @@ template <typename T, int D>
 static hipError_t launch_combine_t(const SdpaParams& p, hipStream_t stream)
 {
     constexpr int TPR = D / 4;
+    const dim3 rows(p.Sq, p.Hq, p.B);      // (heads and batch entries: at most 65535 of each)
     int ng = 64 / TPR;                                  // at least one wavefront
     if constexpr (sizeof(T) == 2) {
         if (p.deal) {
-            hipLaunchKernelGGL((sdpa_combine_kernel<T, D, true>), dim3((unsigned)((int64_t)p.B * p.Hq * p.Sq)), dim3(256), 0, stream, p);
+            hipLaunchKernelGGL((sdpa_combine_kernel<T, D, true>), rows, dim3(256), 0, stream, p);
             return hipGetLastError();
         }
     }
     while (ng < 256 / TPR && ng < p.num_splits) ng *= 2;
-    hipLaunchKernelGGL((sdpa_combine_kernel<T, D>), dim3((unsigned)((int64_t)p.B * p.Hq * p.Sq)), dim3(ng * TPR), 0, stream, p);
+    hipLaunchKernelGGL((sdpa_combine_kernel<T, D>), rows, dim3(ng * TPR), 0, stream, p);
     return hipGetLastError();
 }
 

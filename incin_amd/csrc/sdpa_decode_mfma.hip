@@ -87,11 +87,13 @@ __global__ __launch_bounds__(256) void sdpa_decode_mfma_kernel(SdpaParams p)
         lim_hi = max(lim_hi, lim[rb]);
         if (valid[rb]) lim_lo = min(lim_lo, l);
     }
+    if (p.causal) {
 #pragma unroll
-    for (int off = 16; off >= 1; off >>= 1) {
-        lim_hi = max(lim_hi, __shfl_xor(lim_hi, off, 64));
-        lim_lo = min(lim_lo, __shfl_xor(lim_lo, off, 64));
-    }
+        for (int off = 16; off >= 1; off >>= 1) {
+            lim_hi = max(lim_hi, __shfl_xor(lim_hi, off, 64));
+            lim_lo = min(lim_lo, __shfl_xor(lim_lo, off, 64));
+        }
+    }      // (else every row that exists has the same, the first lane's among them)
     const int k_end = __builtin_amdgcn_readfirstlane(lim_hi);          // rows at and beyond are never read
     const int mask_from = __builtin_amdgcn_readfirstlane(lim_lo);      // blocks that end at or before need no mask
     const int n_blocks = k_end > k_begin ? (k_end - k_begin + BLOCK - 1) / BLOCK : 0;
@@ -358,29 +360,28 @@ __global__ __launch_bounds__(256) void sdpa_decode_mfma_kernel(SdpaParams p)
     }
 
     // ---- the four wavefronts' results meet (the rings are done with) --------------------------------------------------
+    // As they are, 16 bytes at a time, rows that exist only: whoever reads them scales them.
+    typedef float f4 __attribute__((ext_vector_type(4)));
     float* s_m = (float*)smem;                               // [4][CHUNK] maxima
-    float* s_l = s_m + 4 * CHUNK;                            // [4][CHUNK] sums, rescaled
-    float* s_o = s_l + 4 * CHUNK;                            // [4 wavefronts][NRB][NDB][16][64] O^T registers, rescaled
+    float* s_l = s_m + 4 * CHUNK;                            // [4][CHUNK] sums
+    f4* s_o = (f4*)(s_l + 4 * CHUNK);                        // [4 wavefronts][NRB][NDB][4][64] O^T registers
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // (the empty copies started past the last block too)
     __syncthreads();
 #pragma unroll
-    for (int rb = 0; rb < NRB; ++rb)
-        if (g == 0) s_m[wave * CHUNK + 32 * rb + ql] = m_run[rb];
-    __syncthreads();
-    float M[NRB];
-#pragma unroll
     for (int rb = 0; rb < NRB; ++rb) {
-        M[rb] = s_m[32 * rb + ql];
-#pragma unroll
-        for (int w = 1; w < 4; ++w) M[rb] = fmaxf(M[rb], s_m[w * CHUNK + 32 * rb + ql]);
-        const float M_use = (M[rb] == -INFINITY) ? 0.0f : M[rb];
-        const float f = __builtin_amdgcn_exp2f(m_run[rb] - M_use);
-        const float l_w = xor32_sum(l_run[rb]) * f;
-        if (g == 0) s_l[wave * CHUNK + 32 * rb + ql] = l_w;
+        const float l_w = xor32_sum(l_run[rb]);
+        if (!valid[rb]) continue;
+        if (g == 0) {
+            s_m[wave * CHUNK + 32 * rb + ql] = m_run[rb];
+            s_l[wave * CHUNK + 32 * rb + ql] = l_w;
+        }
 #pragma unroll
         for (int db = 0; db < NDB; ++db)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) s_o[(((wave * NRB + rb) * NDB + db) * 16 + r) * 64 + lane] = o_acc[rb][db][r] * f;
+            for (int r4 = 0; r4 < 4; ++r4) {
+                const f4 x = {o_acc[rb][db][4 * r4], o_acc[rb][db][4 * r4 + 1], o_acc[rb][db][4 * r4 + 2], o_acc[rb][db][4 * r4 + 3]};
+                s_o[(((wave * NRB + rb) * NDB + db) * 4 + r4) * 64 + lane] = x;
+            }
     }
     __syncthreads();
     // ---- this wavefront's NDBW blocks of 32 columns of every row (D = 64: the first two wavefronts' one) --------------
@@ -388,9 +389,15 @@ __global__ __launch_bounds__(256) void sdpa_decode_mfma_kernel(SdpaParams p)
 #pragma unroll
     for (int rb = 0; rb < NRB; ++rb) {
         if (!valid[rb]) continue;
-        float l_tot = 0.0f;
+        float M = s_m[32 * rb + ql], f[4], l_tot = 0.0f;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) l_tot += s_l[w * CHUNK + 32 * rb + ql];
+        for (int w = 1; w < 4; ++w) M = fmaxf(M, s_m[w * CHUNK + 32 * rb + ql]);
+        const float M_use = (M == -INFINITY) ? 0.0f : M;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            f[w] = __builtin_amdgcn_exp2f(s_m[w * CHUNK + 32 * rb + ql] - M_use);
+            l_tot = fmaf(s_l[w * CHUNK + 32 * rb + ql], f[w], l_tot);
+        }
         const float inv = (l_tot == 0.0f) ? __builtin_nanf("") : 1.0f / l_tot;      // no visible key: NaN, as the reference
         const int64_t slot = (((int64_t)b * p.Hq + hq[rb]) * Sq + qi[rb]) * p.num_splits + split;
 #pragma unroll
@@ -402,7 +409,11 @@ __global__ __launch_bounds__(256) void sdpa_decode_mfma_kernel(SdpaParams p)
 #pragma unroll
             for (int w = 0; w < 4; ++w)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) o[r] += s_o[(((w * NRB + rb) * NDB + db) * 16 + r) * 64 + lane];
+                for (int r4 = 0; r4 < 4; ++r4) {
+                    const f4 x = s_o[(((w * NRB + rb) * NDB + db) * 4 + r4) * 64 + lane];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) o[4 * r4 + e] = fmaf(x[e], f[w], o[4 * r4 + e]);
+                }
             if (p.num_splits == 1) {
                 T* orow = (T*)p.o + (int64_t)b * p.o_sb + (int64_t)hq[rb] * p.o_sh + (int64_t)qi[rb] * p.o_ss + 32 * db + 4 * g;
 #pragma unroll
@@ -417,7 +428,6 @@ __global__ __launch_bounds__(256) void sdpa_decode_mfma_kernel(SdpaParams p)
                 float* arow = p.ws_acc + slot * D + 32 * db + 4 * g;
 #pragma unroll
                 for (int r4 = 0; r4 < 4; ++r4) {
-                    typedef float f4 __attribute__((ext_vector_type(4)));
                     f4 w = {o[r4 * 4], o[r4 * 4 + 1], o[r4 * 4 + 2], o[r4 * 4 + 3]};
                     *(f4*)(arow + r4 * 8) = w;
                 }
@@ -426,9 +436,9 @@ __global__ __launch_bounds__(256) void sdpa_decode_mfma_kernel(SdpaParams p)
         if (wave == 0 && g == 0) {
             if (p.num_splits == 1) {
                 if (p.lse)      // the row's softmax normaliser, natural log (M and the sum are in log2 units)
-                    p.lse[((int64_t)b * p.Hq + hq[rb]) * Sq + qi[rb]] = l_tot == 0.0f ? -INFINITY : (M[rb] + __builtin_log2f(l_tot)) * 0.6931471805599453f;
+                    p.lse[((int64_t)b * p.Hq + hq[rb]) * Sq + qi[rb]] = l_tot == 0.0f ? -INFINITY : (M + __builtin_log2f(l_tot)) * 0.6931471805599453f;
             } else {
-                p.ws_ml[slot * 2 + 0] = M[rb];      // log2 units, as the combine kernel takes them for 16-bit storage
+                p.ws_ml[slot * 2 + 0] = M;      // log2 units, as the combine kernel takes them for 16-bit storage
                 p.ws_ml[slot * 2 + 1] = l_tot;
             }
         }

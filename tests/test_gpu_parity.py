@@ -835,6 +835,24 @@ def test_decode_splitkv_matrix_cores_f32_scale_lse_auto(gpu):
     check(got, oracle_full(q[:, :4], k[:, :, :300], v[:, :, :300], G=1), TOL[dt], "AUTO f32 decode over a short cache")
 
 
+@pytest.mark.parametrize("dtype", [capi.F32, capi.BF16], ids=lambda x: dtypes.NAMES[x])
+@pytest.mark.parametrize("D,counts", [(64, (2, 15, 17, 63, 64, 65)), (128, (2, 7, 9, 31, 32, 33, 70)), (256, (2, 3, 5, 15, 16, 17))])
+def test_combine_around_the_splits_asked_for_ahead(gpu, dtype, D, counts):
+    """The pass over the partial results holds four of them per group of threads (16, 8 or 4 groups at D = 64, 128, 256) before the
+    maximum is known and walks the rest: counts of splits on both sides of the groups and of what they hold, last splits ragged or
+    empty, two positions of two heads in two sequences of which one is half as long."""
+    for n in counts:
+        Skv = 256 * n - 100
+        q, k, v = inputs(1900 + n + D, 2, 4, 2, 2, Skv, D, D, dtype)
+        lens = np.asarray([Skv - 3, Skv // 2 + 1], np.int32)
+        got, lse, info = host.sdpa(q, k, v, dtype, causal=True, kv_lens=lens, num_splits=n, impl=capi.IMPL_SPLITKV_MFMA, return_lse=True, return_info=True)
+        assert info["splits"] == n
+        whole, lse1 = host.sdpa(q, k, v, dtype, causal=True, kv_lens=lens, num_splits=1, impl=capi.IMPL_SPLITKV_MFMA, return_lse=True)
+        check(got, oracle_full(q, k, v, G=2, causal=True, kv_lens=lens), TOL[dtype], "D=%d in %d splits" % (D, n))
+        assert np.max(np.abs(lse - lse1)) < (4e-6 if dtype == capi.F32 else 2e-3)      # (sums over 2^8 more or fewer roundings of P to storage)
+        check(got, whole, 4e-6 if dtype == capi.F32 else TOL[dtype], "against one split")
+
+
 HEAD_DIMS_16 = [(96, 96), (80, 80), (40, 40), (8, 8), (112, 72), (128, 64), (64, 128), (32, 16), (120, 128)]
 HEAD_DIMS_F32 = [(96, 96), (20, 20), (4, 4), (100, 36), (128, 64), (60, 128)]
 
