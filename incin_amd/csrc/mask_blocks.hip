@@ -5,28 +5,24 @@
 // The reference's operator knows one mask form, an additive tensor (crates/incin-backends/src/cpu/ops/shape_ops.rs:
 // 1262-1266), and its callers build the causal mask as full(-inf).triu(1): with the flags, such a tensor costs about
 // what the causal flag costs - blocks above the diagonal are skipped, blocks below it run the unmasked path.
-// One workgroup per strip of 32 rows x 256 keys (8 blocks): a thread takes 8 consecutive keys of 4 rows - one 16-byte
-// load each for 16-bit masks with unit key stride and aligned rows, element-wise loads otherwise - and the votes of a
+// One workgroup per strip of 32 rows x 256 keys (8 blocks): a thread takes 8 consecutive keys of 4 rows - 16-byte
+// loads for masks with unit key stride, element-wise loads otherwise and at the end of a row - and the votes of a
 // block meet in LDS; rows beyond Sq and keys beyond Skv do not vote.
 #include "sdpa_mfma_common.h"
 
 namespace incin_rocm {
 
+// Eight consecutive values of a mask's row in one load, wherever the row starts: the type asks for no more than an element's alignment, and
+// the compiler takes 16-byte loads for it, which the memory path allows at any address.  (By elements where rows were not multiples of 32 bytes:
+// whole call, f32, a bias per head, 8 heads x 1001 x 1001 134 -> 123 us, bf16 12 x 801 x 801 98 -> 85, 32 x 900 x 900 64 -> 60.)
+template <typename T> struct Mask8 { typedef T type __attribute__((ext_vector_type(8), aligned(sizeof(T)))); };
+
+// (one workgroup of 256 threads: block row rb of (mask batch entry, mask head) bh, the strip's 8 blocks)
 template <typename T, bool VEC>
-__global__ __launch_bounds__(256) void mask_classify_kernel(const T* mask, int64_t m_sb, int64_t m_sh, int64_t m_si, int64_t m_sj,
-                                                           int Hm, int Sq, int Skv, int nkb, uint8_t* flags, const int32_t* lims, int rows_m)
+__device__ __forceinline__ void classify_strip(const T* mask, int64_t m_sb, int64_t m_sh, int64_t m_si, int64_t m_sj,
+                                               int Hm, int Sq, int Skv, int nkb, int nrb, uint8_t* flags, int strip, int rb, int bh)
 {
     __shared__ int votes[8][2];
-    const int strip = blockIdx.x, rb = blockIdx.y, bh = blockIdx.z;
-    if (lims != nullptr) {
-        // Row limits are known (mask_row_limits_kernel ran before): the attention launches read the flags only of blocks of 128
-        // or 256 rows in which some row has no limit.  If every row of the 256 around these 32 has one, nobody will ask.
-        const int blk0 = (rb * 32 / 256) * 256, blk1 = min(blk0 + 256, Sq);
-        const int32_t* l = lims + (int64_t)bh * rows_m;
-        bool ok = true;
-        for (int i = blk0 + (int)threadIdx.x; i < blk1; i += 256) ok = ok && l[rows_m > 1 ? i : 0] >= 0;
-        if (__syncthreads_and(ok)) return;
-    }
     const int b = bh / Hm, h = bh % Hm;
     const T* base = mask + (int64_t)b * m_sb + (int64_t)h * m_sh;
     const int c8 = threadIdx.x & 31, r0 = threadIdx.x >> 5;       // 8 keys starting at strip * 256 + c8 * 8; rows r0, r0 + 8, ..
@@ -41,7 +37,7 @@ __global__ __launch_bounds__(256) void mask_classify_kernel(const T* mask, int64
             if (i >= Sq) continue;
             const T* row = base + (int64_t)i * m_si;
             if (VEC && j0 + 7 < Skv) {
-                typedef T vec8 __attribute__((ext_vector_type(8)));
+                typedef typename Mask8<T>::type vec8;
                 const vec8 x = *(const vec8*)(row + j0);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
@@ -63,8 +59,25 @@ __global__ __launch_bounds__(256) void mask_classify_kernel(const T* mask, int64
     __syncthreads();
     if (threadIdx.x < 8) {
         const int kb = strip * 8 + threadIdx.x;
-        if (kb < nkb) flags[((int64_t)bh * gridDim.y + rb) * nkb + kb] = !votes[threadIdx.x][0] ? 1 : (!votes[threadIdx.x][1] ? 2 : 0);
+        if (kb < nkb) flags[((int64_t)bh * nrb + rb) * nkb + kb] = !votes[threadIdx.x][0] ? 1 : (!votes[threadIdx.x][1] ? 2 : 0);
     }
+}
+
+template <typename T, bool VEC>
+__global__ __launch_bounds__(256) void mask_classify_kernel(const T* mask, int64_t m_sb, int64_t m_sh, int64_t m_si, int64_t m_sj,
+                                                           int Hm, int Sq, int Skv, int nkb, uint8_t* flags, const int32_t* lims, int rows_m)
+{
+    const int strip = blockIdx.x, rb = blockIdx.y, bh = blockIdx.z;
+    if (lims != nullptr) {
+        // Row limits are known (mask_row_limits_kernel ran before): the attention launches read the flags only of blocks of 128
+        // or 256 rows in which some row has no limit.  If every row of the 256 around these 32 has one, nobody will ask.
+        const int blk0 = (rb * 32 / 256) * 256, blk1 = min(blk0 + 256, Sq);
+        const int32_t* l = lims + (int64_t)bh * rows_m;
+        bool ok = true;
+        for (int i = blk0 + (int)threadIdx.x; i < blk1; i += 256) ok = ok && l[rows_m > 1 ? i : 0] >= 0;
+        if (__syncthreads_and(ok)) return;
+    }
+    classify_strip<T, VEC>(mask, m_sb, m_sh, m_si, m_sj, Hm, Sq, Skv, nkb, gridDim.y, flags, strip, rb, bh);
 }
 
 // Row limits: for every row of the mask, n if the row reads n zeros and then -inf to its end (n = Skv: all zeros, n = 0:
@@ -72,18 +85,18 @@ __global__ __launch_bounds__(256) void mask_classify_kernel(const T* mask, int64
 // every row it handles compares key numbers with it instead of reading the mask.  One wavefront per row: the first
 // position that is not zero and the number of -inf values decide.
 template <typename T, bool VEC>
-__global__ __launch_bounds__(256) void mask_row_limits_kernel(const T* mask, int64_t m_sb, int64_t m_sh, int64_t m_si, int64_t m_sj,
-                                                             int Hm, int rows_m, int Skv, int64_t n_rows, int32_t* lims)
+__device__ __forceinline__ void limits_of_rows(const T* mask, int64_t m_sb, int64_t m_sh, int64_t m_si, int64_t m_sj,
+                                               int Hm, int rows_m, int Skv, int64_t n_rows, int32_t* lims, unsigned group)
 {
     const int lane = threadIdx.x & 63;
-    const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);       // (mask batch entry, mask head, row)
+    const int64_t r = (int64_t)group * 4 + (threadIdx.x >> 6);       // (mask batch entry, mask head, row)
     if (r >= n_rows) return;
     const int i = (int)(r % rows_m);
     const int64_t bh = r / rows_m;
     const T* row = mask + (bh / Hm) * m_sb + (bh % Hm) * m_sh + (int64_t)i * m_si;
     int first = Skv, ninf = 0;
     if (VEC) {
-        typedef T vec8 __attribute__((ext_vector_type(8)));
+        typedef typename Mask8<T>::type vec8;
         for (int j0 = lane * 8; j0 < Skv; j0 += 512) {
             if (j0 + 7 < Skv) {
                 const vec8 x = *(const vec8*)(row + j0);
@@ -114,6 +127,26 @@ __global__ __launch_bounds__(256) void mask_row_limits_kernel(const T* mask, int
         ninf += __shfl_xor(ninf, off, 64);
     }
     if (lane == 0) lims[r] = ninf == Skv - first ? first : -1;
+}
+template <typename T, bool VEC>
+__global__ __launch_bounds__(256) void mask_row_limits_kernel(const T* mask, int64_t m_sb, int64_t m_sh, int64_t m_si, int64_t m_sj,
+                                                             int Hm, int rows_m, int Skv, int64_t n_rows, int32_t* lims)
+{
+    limits_of_rows<T, VEC>(mask, m_sb, m_sh, m_si, m_sj, Hm, rows_m, Skv, n_rows, lims, blockIdx.x);
+}
+
+// Limits and flags side by side in one launch: workgroups 0 .. n_strips - 1 classify a strip each (all of them: no limits to go by),
+// the others take four rows each.
+template <typename T, bool VEC>
+__global__ __launch_bounds__(256) void mask_both_kernel(const T* mask, int64_t m_sb, int64_t m_sh, int64_t m_si, int64_t m_sj,
+                                                       int Hm, int Sq, int Skv, int nkb, int nrb, uint8_t* flags, int32_t* lims, int rows_m, int64_t n_rows, unsigned n_strips)
+{
+    if (blockIdx.x >= n_strips) {
+        limits_of_rows<T, VEC>(mask, m_sb, m_sh, m_si, m_sj, Hm, rows_m, Skv, n_rows, lims, blockIdx.x - n_strips);
+        return;
+    }
+    const int across = (nkb + 7) / 8, strip = blockIdx.x % across, row = blockIdx.x / across;
+    classify_strip<T, VEC>(mask, m_sb, m_sh, m_si, m_sj, Hm, Sq, Skv, nkb, nrb, flags, strip, row % nrb, row / nrb);
 }
 
 // Both in one pass over the mask: a workgroup of sixteen wavefronts takes 32 whole rows, two per wavefront, and has the limits of
@@ -148,7 +181,7 @@ __global__ __launch_bounds__(1024) void mask_scan_kernel(const T* mask, int64_t 
                     not_hidden |= !(f == -INFINITY);
                 };
                 if (VEC && j0 + 7 < Skv) {
-                    typedef T vec8 __attribute__((ext_vector_type(8)));
+                    typedef typename Mask8<T>::type vec8;
                     const vec8 x = *(const vec8*)(row + j0);
 #pragma unroll
                     for (int e = 0; e < 8; ++e) see(to_f32(x[e]), j0 + e);
@@ -187,15 +220,29 @@ hipError_t launch_mask_classify(const SdpaParams& p, int dtype, hipStream_t stre
     const dim3 grid((nkb + 7) / 8, nrb, Bm * Hm);
     uint8_t* flags = (uint8_t*)p.mask_flags;
     const int esz = dtype == 0 ? 4 : 2;
-    // 8 consecutive elements in one vector load: unit key stride, every row start a multiple of the vector
-    const bool vec = p.m_sj == 1 && ((uintptr_t)p.mask % (8 * esz)) == 0 && p.m_sb % 8 == 0 && p.m_sh % 8 == 0 && p.m_si % 8 == 0;
+    const bool vec = p.m_sj == 1;      // 8 consecutive elements in one load
     const int rows_m = p.m_si ? p.Sq : 1;
-    // Limits and flags in one pass where its workgroups - one per 32 rows of the mask - are as many as compute units, or rows are so
-    // short that a launch is all there is to save; else two kernels, whose second reads nothing where all rows have limits.  Whole
-    // call, us, two / one: f32, a bias per head, 8 heads x 1024 x 1024 134 / 130, x 4096 887 / 824, 4 x 2048 x 16384 2200 / 2116, bf16 likewise 42.1 /
-    // 38.4, 231 / 231, 452 / 416; 129 x 129 30.7 / 27.7, 25.4 / 22.5; one causal mask of 256 x 256 19.6 / 18.2, 18.5 / 16.2, of 1024 x 1024 60.0 / 61.0,
-    // 24.5 / 24.9, 4096 x 4096 314 / 316, 74.4 / 79.3, 128 rows x 8192 291 / 304, 128 / 141.
-    if (p.mask_lims && (p.Skv <= 512 || (int64_t)nrb * Bm * Hm >= device_cus())) {
+    const int64_t n_rows = (int64_t)Bm * Hm * rows_m, n_strips = (int64_t)((nkb + 7) / 8) * nrb * Bm * Hm;
+    // Limits and flags side by side, so the mask read twice, where it is less than 16 MB: a launch and its latency saved.  Whole call, us, by the
+    // launches below / so: one causal mask, f32 1024 x 1024 59.6 / 58.5, 256 x 256 18.4 / 17.0, 129 x 129 18.9 / 16.2, bf16 1024 x 1024 23.4 / 21.8, 2048 x 2048 33.1
+    // / 32.0, 701 x 701 20.0 / 20.3; a bias per head, f32 4 x 8 x 300 x 300 44.6 / 41.7, 8 x 512 x 512 66.9 / 66.4, 1001 x 1001 (two launches either way, rows
+    // at any address) 134 / 123, bf16 12 x 800 x 800 40.3 / 35.7, 8 x 1024 x 1024 (16 MB) 38.4 / 39.3.
+    if (p.mask_lims && (int64_t)Bm * Hm * p.Sq * p.Skv * esz < 16 << 20) {
+        const dim3 bgrid((unsigned)(n_strips + (n_rows + 3) / 4));
+#define BOTH(T, V) hipLaunchKernelGGL((mask_both_kernel<T, V>), bgrid, dim3(256), 0, stream, (const T*)p.mask, p.m_sb, p.m_sh, p.m_si, p.m_sj, Hm, p.Sq, p.Skv, nkb, nrb, flags, (int32_t*)p.mask_lims, rows_m, n_rows, (unsigned)n_strips)
+        switch (dtype) {
+            case 0: if (vec) BOTH(float, true); else BOTH(float, false); break;
+            case 1: if (vec) BOTH(f16_t, true); else BOTH(f16_t, false); break;
+            default: if (vec) BOTH(bf16_t, true); else BOTH(bf16_t, false); break;
+        }
+#undef BOTH
+        return hipGetLastError();
+    }
+    // From there on limits and flags in one pass where its workgroups - one per 32 rows of the mask - are as many as compute units; else two
+    // kernels, whose second reads nothing where all rows have limits.  Whole call, us, two / one: a bias per head, f32 8 heads x 1024 x 1024 134 / 130,
+    // x 4096 887 / 824, 4 x 2048 x 16384 2200 / 2116, bf16 likewise 42.1 / 38.4, 231 / 231, 452 / 416; one causal mask of 4096 x 4096 314 / 316, 74.4 /
+    // 79.3, 128 rows x 8192 291 / 304, 128 / 141.
+    if (p.mask_lims && (int64_t)nrb * Bm * Hm >= device_cus()) {
 #define SCAN(T, V) hipLaunchKernelGGL((mask_scan_kernel<T, V>), dim3(nrb, Bm * Hm), dim3(1024), 0, stream, (const T*)p.mask, p.m_sb, p.m_sh, p.m_si, p.m_sj, Hm, p.Sq, p.Skv, nkb, flags, (int32_t*)p.mask_lims, rows_m)
         switch (dtype) {
             case 0: if (vec) SCAN(float, true); else SCAN(float, false); break;
@@ -206,7 +253,6 @@ hipError_t launch_mask_classify(const SdpaParams& p, int dtype, hipStream_t stre
         return hipGetLastError();
     }
     if (p.mask_lims) {       // the limits first: the flags of blocks whose rows all have one are not needed
-        const int64_t n_rows = (int64_t)Bm * Hm * rows_m;
         const dim3 lgrid((unsigned)((n_rows + 3) / 4));
 #define LIMITS(T, V) hipLaunchKernelGGL((mask_row_limits_kernel<T, V>), lgrid, dim3(256), 0, stream, (const T*)p.mask, p.m_sb, p.m_sh, p.m_si, p.m_sj, Hm, rows_m, p.Skv, n_rows, (int32_t*)p.mask_lims)
         switch (dtype) {
@@ -234,8 +280,7 @@ hipError_t launch_mask_row_limits(const void* mask, int dtype, const int64_t sha
     if (n_rows <= 0) return hipSuccess;
     if ((n_rows + 3) / 4 > 0x7fffffffLL) return hipErrorInvalidValue;
     const dim3 grid((unsigned)((n_rows + 3) / 4));
-    const int esz = dtype == 0 ? 4 : 2;
-    const bool vec = strides[3] == 1 && ((uintptr_t)mask % (8 * esz)) == 0 && strides[0] % 8 == 0 && strides[1] % 8 == 0 && strides[2] % 8 == 0;
+    const bool vec = strides[3] == 1;
 #define LIMITS(T, V) hipLaunchKernelGGL((mask_row_limits_kernel<T, V>), grid, dim3(256), 0, stream, (const T*)mask, strides[0], strides[1], strides[2], strides[3], (int)shape[1], (int)shape[2], (int)shape[3], n_rows, lims)
     switch (dtype) {
         case 0: if (vec) LIMITS(float, true); else LIMITS(float, false); break;

@@ -438,6 +438,27 @@ def test_auto_splits_the_keys_of_a_wide_prefill_launch_that_fills_the_device(gpu
         assert np.abs(got.reshape(Hq, Sq, 256)[rows[:, 0], rows[:, 1]] - ref).max() <= TOL[capi.BF16]
 
 
+@pytest.mark.parametrize("dtype", [capi.F32, capi.F16, capi.BF16], ids=lambda x: dtypes.NAMES[x])
+@pytest.mark.parametrize("Sq,Skv", [(65, 7), (130, 9), (97, 33), (300, 255), (140, 513), (129, 701), (70, 1030), (257, 2047)])
+def test_mask_limits_and_flags_side_by_side(gpu, dtype, Sq, Skv):
+    """Small masks: the workgroups that classify blocks and those that take row limits are one launch, and rows start wherever the
+    key count puts them (every alignment an element allows): limits, a hole, values in the last keys, rows without a key, in four heads -
+    against the kernels that read the mask's values as they are."""
+    H, D = 4, 64
+    q, k, v = inputs(5600 + Skv, 2, H, H, Sq, Skv, D, D, dtype)
+    r = rng(5601)
+    mask = np.zeros((1, H, Sq, Skv), np.float32)
+    for i in range(Sq):
+        mask[0, 0, i, min(1 + i * 3, Skv):] = -np.inf
+    mask[0, 1, : Sq // 2, Skv // 3: Skv // 2] = -np.inf
+    mask[0, 2, :, Skv - 2:] = dtypes.round_to(r.standard_normal((Sq, 2), dtype=np.float32), dtype)
+    mask[0, 3, Sq // 3:, 1:] = -np.inf
+    mask[0, 3, 40, :] = -np.inf
+    got = host.sdpa(q, k, v, dtype, mask=mask)
+    ref = host.sdpa(q, k, v, dtype, mask=mask, impl=capi.IMPL_GENERIC)
+    check(got, ref, TOL[dtype], "mask %d x %d" % (Sq, Skv))
+
+
 @pytest.mark.parametrize("dtype", [capi.F32, capi.BF16], ids=lambda x: dtypes.NAMES[x])
 @pytest.mark.parametrize("Skv", [4200, 4097, 4096, 8200])
 def test_mask_limits_and_flags_in_one_pass(gpu, dtype, Skv):
