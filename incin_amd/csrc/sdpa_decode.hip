@@ -242,9 +242,16 @@ __global__ __launch_bounds__(256) void sdpa_decode_split_kernel(SdpaParams p)
 // 10.2, four of 300 - 1000 10.5 / 10.3, 16 on 2 heads x 5 positions x 4 x 3000 18.6 / 17.3, 4 x 1000 - 3000 at D = 256 19.0 / 18.1; f32 2 x 8 on
 // 4 x 1000 - 2000 at D = 64 10.6 / 10.3.
 //
+// LONE: one wavefront does the row alone where its groups can ask for all splits so, eight each (16 splits at D = 128): sums meet over lanes, no barrier.
+// Us a call by groups / lone: bf16, 32 on 8 heads, one sequence of 1500 keys 10.9 / 10.3, 8 of 1000 - 2000 15.9 / 15.3, 4 x 5 positions x 3000 16.1 /
+// 15.4, 4 of 3000 - 16000 32.5 / 31.95, f32 2 x 8 on 4 x 1000 - 2000 at D = 64 10.15 / 9.7; dealt, 32 x 1031 - 8192 99.4 / 98.8.
+// (More splits than that keep the groups: with the choice between the two in the kernel they took 1 - 2 % longer.)
+//
 // DEAL: the partial results of a row are those of the shares that its sequence's units went to (decode_deal.h); rows of
 // sequences that one share holds are finished already.
-template <typename T, int D, bool DEAL = false>
+enum { COMBINE_GROUPS, COMBINE_LONE, COMBINE_DEAL };
+constexpr int COMBINE_LONE_AHEAD = 8;
+template <typename T, int D, int FORM>
 __global__ __launch_bounds__(256) void sdpa_combine_kernel(SdpaParams p)
 {
     constexpr int TPR = D / 4;
@@ -254,9 +261,9 @@ __global__ __launch_bounds__(256) void sdpa_combine_kernel(SdpaParams p)
     __shared__ float s_max[4];
     __shared__ f4 s_acc[NG_MAX][TPR];
     __shared__ float s_l[NG_MAX];
-    constexpr int AHEAD = 4;
+    constexpr bool DEAL = FORM == COMBINE_DEAL;
+    constexpr int AHEAD = FORM == COMBINE_GROUPS ? 4 : COMBINE_LONE_AHEAD, NG_WAVE = 64 / TPR;
     const int tid = threadIdx.x;
-    const int ng = blockDim.x / TPR;
     const int i = blockIdx.x, hq = blockIdx.y, b = blockIdx.z;
     const int64_t row = ((int64_t)b * p.Hq + hq) * p.Sq + i;
     int n = p.num_splits, w0 = 0, rows_per_place = 1, place_row = 0;
@@ -276,6 +283,9 @@ __global__ __launch_bounds__(256) void sdpa_combine_kernel(SdpaParams p)
     const float* ml = DEAL ? p.ws_ml : p.ws_ml + row * p.num_splits * 2;
     const float* ac = DEAL ? p.ws_acc : p.ws_acc + row * p.num_splits * D;
     auto at = [&](int s) __attribute__((always_inline)) { return DEAL ? deal_slot(w0 + s, s < n - 1, rows_per_place, place_row) : (int64_t)s; };
+    const bool lone = FORM == COMBINE_LONE || (DEAL && n <= AHEAD * NG_WAVE);      // (uniform)
+    if (lone && tid >= 64) return;
+    const int ng = lone ? NG_WAVE : blockDim.x / TPR;
     const int grp = tid / TPR, c = tid % TPR;
     f2 first_ml[AHEAD];
     f4 first_a[AHEAD];
@@ -292,11 +302,16 @@ __global__ __launch_bounds__(256) void sdpa_combine_kernel(SdpaParams p)
     for (int u = 0; u < AHEAD; ++u)
         if (u * ng < n) m = fmaxf(m, first_ml[u][0]);
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-    if ((tid & 63) == 0) s_max[tid >> 6] = m;
-    __syncthreads();
-    float M = s_max[0];
-    for (int w = 1; w < (int)(blockDim.x >> 6); ++w) M = fmaxf(M, s_max[w]);
+    for (int off = 32; off >= TPR; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+    float M = m;
+    if (!lone) {
+#pragma unroll
+        for (int off = TPR < 64 ? TPR / 2 : 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+        if ((tid & 63) == 0) s_max[tid >> 6] = m;
+        __syncthreads();
+        M = s_max[0];
+        for (int w = 1; w < (int)(blockDim.x >> 6); ++w) M = fmaxf(M, s_max[w]);
+    }
     const float M_use = (M == -INFINITY) ? 0.0f : M;
     f4 A = {0.0f, 0.0f, 0.0f, 0.0f};
     float L = 0.0f;
@@ -313,16 +328,26 @@ __global__ __launch_bounds__(256) void sdpa_combine_kernel(SdpaParams p)
         const int64_t slot = at(s);
         add(*(const f2*)(ml + slot * 2), *(const f4*)(ac + slot * D + 4 * c));
     }
-    s_acc[grp][c] = A;
-    if (c == 0) s_l[grp] = L;
-    __syncthreads();
-    if (tid < TPR) {
-        for (int g2 = 1; g2 < ng; ++g2) {
-            const f4 a = s_acc[g2][tid];
+    if (lone) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) A[e] += a[e];
-            L += s_l[g2];
+        for (int off = 32; off >= TPR; off >>= 1) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) A[e] += __shfl_xor(A[e], off, 64);
+            L += __shfl_xor(L, off, 64);
         }
+    } else {
+        s_acc[grp][c] = A;
+        if (c == 0) s_l[grp] = L;
+        __syncthreads();
+    }
+    if (tid < TPR) {
+        if (!lone)
+            for (int g2 = 1; g2 < ng; ++g2) {
+                const f4 a = s_acc[g2][tid];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) A[e] += a[e];
+                L += s_l[g2];
+            }
         typedef T vec4 __attribute__((ext_vector_type(4)));
         vec4 w;
 #pragma unroll
@@ -342,12 +367,16 @@ static hipError_t launch_combine_t(const SdpaParams& p, hipStream_t stream)
     int ng = 64 / TPR;                                  // at least one wavefront
     if constexpr (sizeof(T) == 2) {
         if (p.deal) {
-            hipLaunchKernelGGL((sdpa_combine_kernel<T, D, true>), rows, dim3(256), 0, stream, p);
+            hipLaunchKernelGGL((sdpa_combine_kernel<T, D, COMBINE_DEAL>), rows, dim3(256), 0, stream, p);
             return hipGetLastError();
         }
     }
+    if (p.num_splits <= COMBINE_LONE_AHEAD * ng) {
+        hipLaunchKernelGGL((sdpa_combine_kernel<T, D, COMBINE_LONE>), rows, dim3(64), 0, stream, p);
+        return hipGetLastError();
+    }
     while (ng < 256 / TPR && ng < p.num_splits) ng *= 2;
-    hipLaunchKernelGGL((sdpa_combine_kernel<T, D>), rows, dim3(ng * TPR), 0, stream, p);
+    hipLaunchKernelGGL((sdpa_combine_kernel<T, D, COMBINE_GROUPS>), rows, dim3(ng * TPR), 0, stream, p);
     return hipGetLastError();
 }
 

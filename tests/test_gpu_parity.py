@@ -857,11 +857,11 @@ def test_decode_splitkv_matrix_cores_f32_scale_lse_auto(gpu):
 
 
 @pytest.mark.parametrize("dtype", [capi.F32, capi.BF16], ids=lambda x: dtypes.NAMES[x])
-@pytest.mark.parametrize("D,counts", [(64, (2, 15, 17, 63, 64, 65)), (128, (2, 7, 9, 31, 32, 33, 70)), (256, (2, 3, 5, 15, 16, 17))])
+@pytest.mark.parametrize("D,counts", [(64, (2, 15, 17, 31, 32, 33, 63, 64, 65)), (128, (2, 7, 9, 15, 16, 17, 31, 32, 33, 70)), (256, (2, 3, 5, 7, 8, 9, 15, 16, 17))])
 def test_combine_around_the_splits_asked_for_ahead(gpu, dtype, D, counts):
     """The pass over the partial results holds four of them per group of threads (16, 8 or 4 groups at D = 64, 128, 256) before the
-    maximum is known and walks the rest: counts of splits on both sides of the groups and of what they hold, last splits ragged or
-    empty, two positions of two heads in two sequences of which one is half as long."""
+    maximum is known and walks the rest, or, up to eight per group of one wavefront, has that one do the row: counts of splits on both
+    sides of the groups, of what they hold and of the one wavefront's 32, 16 or 8, last splits ragged or empty, two positions of two heads in two sequences of which one is half as long."""
     for n in counts:
         Skv = 256 * n - 100
         q, k, v = inputs(1900 + n + D, 2, 4, 2, 2, Skv, D, D, dtype)
