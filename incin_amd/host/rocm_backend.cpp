@@ -62,14 +62,16 @@ struct PoolEvent {
 // once, which is what a thread that repeats an operator does.  Others may have it when an event recorded behind the release has
 // passed - and an event costs the stream 3 us, each further one without a launch between them 4.6 (a barrier and a write-back of
 // the caches: with two to eight per call the operator in f32 on 4 x 8 x 1024 x 64 with a mask took 69 us instead of 61, on 32 x 32 with gradients 59 instead of 37) - so a thread leaves
-// its last releases without one, up to ORDERED_BLOCKS blocks and ORDERED_BYTES bytes, and then stamps all of them with the same one.
+// its last releases without one, up to ORDERED_BLOCKS blocks and ORDERED_BYTES bytes, and stamps all of them with the same one when
+// there are more, or when it turns to another stream (so that a thread going back and forth has blocks of its own on either, and waits for nothing).
 struct IdleBlock {
     void* ptr;
     size_t bytes;
     void* stream;                          // the stream whose work may still be using the block
     bool ordered;                          // and no event says until when
     std::shared_ptr<PoolEvent> event;      // otherwise: until this has passed; none: nothing can be using it
-    std::weak_ptr<int> owner;              // (ordered) gone when the thread that released it is, or has turned to another stream
+    std::weak_ptr<int> owner;              // (ordered) gone when the thread that released it is
+    uint64_t waited = 0;                   // (ordered, nobody's) the device synchronisation that somebody has begun for it
 };
 constexpr int ORDERED_BLOCKS = 16;
 constexpr size_t ORDERED_BYTES = 64u << 20;
@@ -97,17 +99,42 @@ struct DevicePool {
     std::mutex mu;
     std::multimap<size_t, IdleBlock> idle;
     int64_t device_allocs = 0, reused = 0, idle_bytes = 0;
+    uint64_t waits = 0;      // device synchronisations begun for blocks of threads that are gone
 };
+// never evicted, like the reference's device cache (cuda/gpu.rs:99-152), and never destroyed: buffers released while the
+// process winds down still find their pool
+struct DevicePools {
+    std::mutex mu;
+    std::map<int32_t, DevicePool*> of;
+};
+DevicePools& device_pools()
+{
+    static DevicePools* pools = new DevicePools();
+    return *pools;
+}
 DevicePool& pool_of(int32_t device)
 {
-    // never evicted, like the reference's device cache (cuda/gpu.rs:99-152), and never destroyed: buffers released while the
-    // process winds down still find their pool
-    static std::mutex* mu = new std::mutex();
-    static std::map<int32_t, DevicePool*>* pools = new std::map<int32_t, DevicePool*>();
-    std::lock_guard<std::mutex> lock(*mu);
-    DevicePool*& p = (*pools)[device];
+    DevicePools& pools = device_pools();
+    std::lock_guard<std::mutex> lock(pools.mu);
+    DevicePool*& p = pools.of[device];
     if (!p) p = new DevicePool();
     return *p;
+}
+// One event on the calling thread's stream for everything of that stream's order in the pool, whoever released it: what they put on the
+// stream before is before the event.  False: there is no event to be had.
+bool stamp_ordered(int32_t device, DevicePool& pool)
+{
+    auto event = std::make_shared<PoolEvent>();
+    event->device = device;
+    if (incin_rocm_event_create(device, &event->event) != 0 || incin_rocm_event_record(device, event->event, t_stream) != 0) return false;
+    for (auto& kv : pool.idle) {
+        IdleBlock& b = kv.second;
+        if (!b.ordered || b.stream != t_stream) continue;
+        t_ordered.taken(b);
+        b.ordered = false;
+        b.event = event;
+    }
+    return true;
 }
 size_t pool_size_class(size_t bytes)
 {
@@ -122,7 +149,7 @@ int pool_alloc(int32_t device, size_t bytes, void** out, size_t* granted, bool* 
     const size_t want = pool_size_class(bytes);
     DevicePool& pool = pool_of(device);
     for (int attempt = 0; attempt < 2; ++attempt) {
-        std::lock_guard<std::mutex> lock(pool.mu);
+        std::unique_lock<std::mutex> lock(pool.mu);
         for (auto it = pool.idle.lower_bound(want); it != pool.idle.end() && it->first <= want + want / 4 + 4096; ++it) {
             IdleBlock& b = it->second;
             bool done = !b.ordered && !b.event;
@@ -138,13 +165,20 @@ int pool_alloc(int32_t device, size_t bytes, void** out, size_t* granted, bool* 
             return 0;
         }
         // Before the device is asked for more (which takes as long): blocks that were left in the order of a stream by a thread that is
-        // gone, or has gone to another stream, come back to everyone once the device has done all there is.
-        if (t_recording) break;
+        // gone come back to everyone once the device has done all there was.  Nobody else is kept waiting meanwhile; the blocks that this
+        // wait stands for are those marked before it, if they are still here.
+        if (t_recording || attempt) break;
         bool left = false;
         for (auto& kv : pool.idle) left = left || (kv.second.ordered && kv.second.bytes >= want && kv.second.bytes <= want + want / 4 + 4096 && kv.second.owner.expired());
-        if (!left || incin_rocm_sync(device) != 0) break;
+        if (!left) break;
+        const uint64_t wait = ++pool.waits;
         for (auto& kv : pool.idle)
-            if (kv.second.ordered && kv.second.owner.expired()) kv.second.ordered = false;
+            if (kv.second.ordered && kv.second.owner.expired()) kv.second.waited = wait;
+        lock.unlock();
+        if (incin_rocm_sync(device) != 0) break;
+        lock.lock();
+        for (auto& kv : pool.idle)
+            if (kv.second.ordered && kv.second.waited == wait) kv.second.ordered = false;
     }
     if (t_recording) {
         // (no message from the C ABI for this one: the refusal is the pool's)
@@ -179,19 +213,13 @@ void pool_release(int32_t device, void* ptr, size_t bytes)
     ++t_ordered.blocks;
     t_ordered.bytes += bytes;
     if (t_ordered.blocks <= ORDERED_BLOCKS && t_ordered.bytes <= ORDERED_BYTES) return;
-    auto event = std::make_shared<PoolEvent>();
-    event->device = device;
-    if (incin_rocm_event_create(device, &event->event) != 0 || incin_rocm_event_record(device, event->event, t_stream) != 0) {
-        // no event to be had: make sure nothing uses the blocks, then they need none
-        event.reset();
-        incin_rocm_sync(device);
-    }
-    for (auto& kv : pool.idle) {      // (whoever released them: what they put on the stream before that is before the event)
-        IdleBlock& b = kv.second;
-        if (!b.ordered || b.stream != t_stream) continue;
-        t_ordered.taken(b);
-        b.ordered = false;
-        b.event = event;
+    if (stamp_ordered(device, pool)) return;
+    // no event to be had: make sure nothing uses the blocks, then they need none
+    incin_rocm_sync(device);
+    for (auto& kv : pool.idle) {
+        if (!kv.second.ordered || kv.second.stream != t_stream) continue;
+        t_ordered.taken(kv.second);
+        kv.second.ordered = false;
     }
 }
 
@@ -279,7 +307,24 @@ RecordedGraph::~RecordedGraph()
 
 void RocmBackend::set_stream(void* stream)
 {
-    if (stream != t_stream && !t_winding_down) t_ordered.forget();      // (what this thread left in the old stream's order is nobody's now)
+    if (stream == t_stream) return;
+    if (!t_winding_down && t_ordered.blocks > 0) {
+        // What this thread left in the old stream's order gets its event now.  (Not while that stream may be recording - the event would become part
+        // of the graph and say nothing -, nor where there is none to be had: those blocks are as those of a thread that is gone.)
+        std::map<int32_t, DevicePool*> pools;
+        {
+            std::lock_guard<std::mutex> lock(device_pools().mu);
+            pools = device_pools().of;
+        }
+        for (auto& dp : pools) {
+            if (t_recording && t_recording->device == dp.first) continue;
+            std::lock_guard<std::mutex> lock(dp.second->mu);
+            bool own = false;
+            for (auto& kv : dp.second->idle) own = own || (kv.second.ordered && kv.second.owner.lock() == t_ordered.token);
+            if (own) stamp_ordered(dp.first, *dp.second);
+        }
+        t_ordered.forget();
+    }
     t_stream = stream;
 }
 void* RocmBackend::stream() { return t_stream; }

@@ -39,10 +39,13 @@ struct Error {
 };
 
 // One device allocation, released when the last storage that views it goes away.  Released, not freed: the buffer goes back
-// to a pool per device and is handed out again to the stream the releasing thread works on at once (its work is ordered behind
-// what still uses the buffer) or to another stream once an event on that one, recorded behind the release - at the latest when
-// the thread has left sixteen buffers or 64 MiB so -, has passed - the stream-ordered lifetime the reference's CUDA buffers have (cuda/storage.rs:171-177, 225-233).  So an
-// operator can drop temporaries and workspaces that its kernels are still using without waiting for the device.
+// to a pool per device.  The stream that the releasing thread works on may have it again at once (its work is ordered behind
+// what still uses the buffer); another stream when an event on that one, recorded behind the release, has passed - the
+// stream-ordered lifetime the reference's CUDA buffers have (cuda/storage.rs:171-177, 225-233).  The event is not recorded with each
+// release: a live thread leaves up to sixteen buffers or 64 MiB without one, until it releases more or turns to another stream
+// (set_stream, which for that expects the stream it leaves to exist still).  What a thread leaves when it ends is
+// given to other streams behind a device synchronisation, in the place of an allocation.  So an operator can drop temporaries and workspaces
+// that its kernels are still using without waiting for the device.
 class RocmBuffer {
   public:
     RocmBuffer(int32_t device, void* ptr, size_t bytes) : device_(device), ptr_(ptr), bytes_(bytes) {}

@@ -562,6 +562,51 @@ def test_blocks_left_in_stream_order_come_back(gpu):
         s.destroy()
 
 
+def test_a_thread_that_alternates_two_streams_has_blocks_on_either(gpu):
+    """One thread goes back and forth between two streams, the first of them busy for tens of milliseconds: the operator on the second
+    neither waits for that (an event behind the first one's work is still to come when its call has returned and its result is there) nor,
+    once either stream has blocks, asks the device for memory."""
+    import ctypes as C
+    from incin_amd import capi
+    q, k, v = (rnd(95 + i, (2, 4, 96, 64), RB.F32) for i in range(3))
+    ref = O.sdpa(q, k, v)
+    streams = [capi.Stream() for _ in range(2)]
+    sink = capi.DeviceBuffer(2048 * capi.device_info(0).compute_units)
+    src = capi.DeviceBuffer.from_numpy(np.zeros(65536, np.uint32))
+    behind = capi.Event()
+    S = [RB.RocmStorage.from_numpy(a) for a in (q, k, v)]
+    RB.scaled_dot_product_attention(*S).to_numpy()
+    RB.trim_pool()
+    allocs, busy = [], []
+    try:
+        for rep in range(5):
+            RB.set_stream(streams[0].ptr)
+            capi.matrix_rate(src, sink, 0, 1 << 19, stream=streams[0].ptr)      # some 50 ms
+            for _ in range(3):
+                RB.scaled_dot_product_attention(*S)
+            behind.record(streams[0].ptr)
+            RB.set_stream(streams[1].ptr)
+            for _ in range(3):
+                out = RB.scaled_dot_product_attention(*S)
+            streams[1].sync()
+            done = C.c_int32(1)
+            capi.check(capi.load().incin_rocm_event_query(0, behind.ptr, C.byref(done)))
+            busy.append(done.value == 0)
+            allocs.append(RB.pool_stats()[0])
+            close(out.to_numpy(), ref, TOL[RB.F32], "operator on the second stream")
+            del out
+            streams[0].sync()
+    finally:
+        RB.set_stream(None)
+    assert all(busy[1:]), "the second stream's operators waited for the first one's work: %r" % busy
+    assert allocs[1:] == [allocs[1]] * 4, "device allocations while alternating: %r" % allocs
+    RB.trim_pool()
+    for s in streams:
+        s.destroy()
+    sink.free()
+    src.free()
+
+
 def test_recorded_operator_with_a_transposed_k(gpu):
     """The operator with k handed over as a transposed view (gathered into a temporary first), recorded into a launch graph on
     a stream of the caller's and replayed: no step of it waits for the device or allocates while recording; every replay -
