@@ -564,7 +564,7 @@ def test_blocks_left_in_stream_order_come_back(gpu):
 
 def test_a_thread_that_alternates_two_streams_has_blocks_on_either(gpu):
     """One thread goes back and forth between two streams, the first of them busy for tens of milliseconds: the operator on the second
-    neither waits for that (an event behind the first one's work is still to come when its call has returned and its result is there) nor,
+    neither waits for that (an event behind the first one's work is still to come when its calls have returned) nor,
     once either stream has blocks, asks the device for memory."""
     import ctypes as C
     from incin_amd import capi
@@ -588,10 +588,10 @@ def test_a_thread_that_alternates_two_streams_has_blocks_on_either(gpu):
             RB.set_stream(streams[1].ptr)
             for _ in range(3):
                 out = RB.scaled_dot_product_attention(*S)
-            streams[1].sync()
             done = C.c_int32(1)
             capi.check(capi.load().incin_rocm_event_query(0, behind.ptr, C.byref(done)))
             busy.append(done.value == 0)
+            streams[1].sync()
             allocs.append(RB.pool_stats()[0])
             close(out.to_numpy(), ref, TOL[RB.F32], "operator on the second stream")
             del out
