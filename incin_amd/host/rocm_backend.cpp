@@ -64,59 +64,54 @@ struct PoolEvent {
 // the caches: with two to eight per call the operator in f32 on 4 x 8 x 1024 x 64 with a mask took 69 us instead of 61, on 32 x 32 with gradients 59 instead of 37) - so a thread leaves
 // its last releases without one, up to ORDERED_BLOCKS blocks and ORDERED_BYTES bytes, and stamps all of them with the same one when
 // there are more, or when it turns to another stream (so that a thread going back and forth has blocks of its own on either, and waits for nothing).
+
+// What a live thread has left so in one device's pool, all of it on the stream that it is on; counted under that pool's mutex, whoever
+// takes, stamps or frees a block.
+struct OrderedReleases {
+    int blocks = 0;
+    size_t bytes = 0;
+};
 struct IdleBlock {
     void* ptr;
     size_t bytes;
     void* stream;                          // the stream whose work may still be using the block
     bool ordered;                          // and no event says until when
     std::shared_ptr<PoolEvent> event;      // otherwise: until this has passed; none: nothing can be using it
-    std::weak_ptr<int> owner;              // (ordered) gone when the thread that released it is
+    std::weak_ptr<OrderedReleases> owner;  // (ordered) gone when the thread that released it is
     uint64_t waited = 0;                   // (ordered, nobody's) the device synchronisation that somebody has begun for it
+    // no longer left in the order of its stream: taken from the pool, stamped or freed
+    void counted_off()
+    {
+        if (auto o = owner.lock()) {
+            --o->blocks;
+            o->bytes -= bytes;
+        }
+        owner.reset();
+        ordered = false;
+    }
 };
 constexpr int ORDERED_BLOCKS = 16;
 constexpr size_t ORDERED_BYTES = 64u << 20;
 thread_local bool t_winding_down = false;      // (buffers may outlive the thread's other variables)
-struct OrderedReleases {      // the calling thread's, on its present stream
-    std::shared_ptr<int> token = std::make_shared<int>(0);
-    int blocks = 0;
-    size_t bytes = 0;
-    ~OrderedReleases() { t_winding_down = true; }
-    void forget()
-    {
-        token = std::make_shared<int>(0);
-        blocks = 0;
-        bytes = 0;
-    }
-    void taken(const IdleBlock& b)      // from the pool, or stamped
-    {
-        if (!b.ordered || b.owner.lock() != token) return;
-        --blocks;
-        bytes -= b.bytes;
-    }
+struct ThreadReleases {      // the calling thread's, by device
+    std::map<int32_t, std::shared_ptr<OrderedReleases>> of;
+    ~ThreadReleases() { t_winding_down = true; }
 };
-thread_local OrderedReleases t_ordered;
+thread_local ThreadReleases t_releases;
 struct DevicePool {
     std::mutex mu;
     std::multimap<size_t, IdleBlock> idle;
     int64_t device_allocs = 0, reused = 0, idle_bytes = 0;
     uint64_t waits = 0;      // device synchronisations begun for blocks of threads that are gone
 };
-// never evicted, like the reference's device cache (cuda/gpu.rs:99-152), and never destroyed: buffers released while the
-// process winds down still find their pool
-struct DevicePools {
-    std::mutex mu;
-    std::map<int32_t, DevicePool*> of;
-};
-DevicePools& device_pools()
-{
-    static DevicePools* pools = new DevicePools();
-    return *pools;
-}
 DevicePool& pool_of(int32_t device)
 {
-    DevicePools& pools = device_pools();
-    std::lock_guard<std::mutex> lock(pools.mu);
-    DevicePool*& p = pools.of[device];
+    // never evicted, like the reference's device cache (cuda/gpu.rs:99-152), and never destroyed: buffers released while the
+    // process winds down still find their pool
+    static std::mutex* mu = new std::mutex();
+    static std::map<int32_t, DevicePool*>* pools = new std::map<int32_t, DevicePool*>();
+    std::lock_guard<std::mutex> lock(*mu);
+    DevicePool*& p = (*pools)[device];
     if (!p) p = new DevicePool();
     return *p;
 }
@@ -130,8 +125,7 @@ bool stamp_ordered(int32_t device, DevicePool& pool)
     for (auto& kv : pool.idle) {
         IdleBlock& b = kv.second;
         if (!b.ordered || b.stream != t_stream) continue;
-        t_ordered.taken(b);
-        b.ordered = false;
+        b.counted_off();
         b.event = event;
     }
     return true;
@@ -155,7 +149,7 @@ int pool_alloc(int32_t device, size_t bytes, void** out, size_t* granted, bool* 
             bool done = !b.ordered && !b.event;
             if (!done && !b.ordered && !t_recording) done = b.event->query();      // (an event recorded into a graph cannot be asked; such blocks carry none)
             if (!done && b.stream != t_stream) continue;
-            if (!t_winding_down) t_ordered.taken(b);
+            b.counted_off();
             *out = b.ptr;
             *granted = b.bytes;
             *settled = done;
@@ -209,18 +203,17 @@ void pool_release(int32_t device, void* ptr, size_t bytes)
         pool.idle.emplace(bytes, IdleBlock{ptr, bytes, t_stream, true, nullptr, {}});
         return;
     }
-    pool.idle.emplace(bytes, IdleBlock{ptr, bytes, t_stream, true, nullptr, t_ordered.token});
-    ++t_ordered.blocks;
-    t_ordered.bytes += bytes;
-    if (t_ordered.blocks <= ORDERED_BLOCKS && t_ordered.bytes <= ORDERED_BYTES) return;
+    std::shared_ptr<OrderedReleases>& own = t_releases.of[device];
+    if (!own) own = std::make_shared<OrderedReleases>();
+    pool.idle.emplace(bytes, IdleBlock{ptr, bytes, t_stream, true, nullptr, own});
+    ++own->blocks;
+    own->bytes += bytes;
+    if (own->blocks <= ORDERED_BLOCKS && own->bytes <= ORDERED_BYTES) return;
     if (stamp_ordered(device, pool)) return;
     // no event to be had: make sure nothing uses the blocks, then they need none
     incin_rocm_sync(device);
-    for (auto& kv : pool.idle) {
-        if (!kv.second.ordered || kv.second.stream != t_stream) continue;
-        t_ordered.taken(kv.second);
-        kv.second.ordered = false;
-    }
+    for (auto& kv : pool.idle)
+        if (kv.second.ordered && kv.second.stream == t_stream) kv.second.counted_off();
 }
 
 std::vector<int64_t> contiguous_strides(const std::vector<int64_t>& shape)
@@ -308,22 +301,15 @@ RecordedGraph::~RecordedGraph()
 void RocmBackend::set_stream(void* stream)
 {
     if (stream == t_stream) return;
-    if (!t_winding_down && t_ordered.blocks > 0) {
+    if (!t_winding_down) {
         // What this thread left in the old stream's order gets its event now.  (Not while that stream may be recording - the event would become part
         // of the graph and say nothing -, nor where there is none to be had: those blocks are as those of a thread that is gone.)
-        std::map<int32_t, DevicePool*> pools;
-        {
-            std::lock_guard<std::mutex> lock(device_pools().mu);
-            pools = device_pools().of;
+        for (auto& own : t_releases.of) {
+            DevicePool& pool = pool_of(own.first);
+            std::lock_guard<std::mutex> lock(pool.mu);
+            if (own.second->blocks == 0) continue;
+            if ((t_recording && t_recording->device == own.first) || !stamp_ordered(own.first, pool)) own.second = std::make_shared<OrderedReleases>();
         }
-        for (auto& dp : pools) {
-            if (t_recording && t_recording->device == dp.first) continue;
-            std::lock_guard<std::mutex> lock(dp.second->mu);
-            bool own = false;
-            for (auto& kv : dp.second->idle) own = own || (kv.second.ordered && kv.second.owner.lock() == t_ordered.token);
-            if (own) stamp_ordered(dp.first, *dp.second);
-        }
-        t_ordered.forget();
     }
     t_stream = stream;
 }
@@ -368,7 +354,7 @@ Error RocmBackend::trim_pool(int32_t device)
     DevicePool& pool = pool_of(device);
     std::lock_guard<std::mutex> lock(pool.mu);
     for (auto& kv : pool.idle) {
-        if (!t_winding_down) t_ordered.taken(kv.second);
+        kv.second.counted_off();
         incin_rocm_free(device, kv.second.ptr);
     }
     pool.idle.clear();

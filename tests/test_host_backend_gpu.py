@@ -607,6 +607,49 @@ def test_a_thread_that_alternates_two_streams_has_blocks_on_either(gpu):
     src.free()
 
 
+@pytest.mark.parametrize("how", ["taken", "stamped", "freed"])
+def test_releases_that_others_see_to_are_not_counted_against_a_thread(gpu, how):
+    """A thread's last sixteen releases go without an event.  Those that another thread on the same stream has taken, has put an event
+    behind, or has freed are not among them any more: after sixteen such, one more release still goes without (and so is not there
+    for a third thread on another stream, which gets new memory)."""
+    from concurrent.futures import ThreadPoolExecutor
+    from incin_amd import capi
+    RB.trim_pool()
+    other = capi.Stream()
+    new = lambda n: RB.RocmStorage.from_numpy(np.zeros(n, np.float32))
+    with ThreadPoolExecutor(1) as first, ThreadPoolExecutor(1) as second, ThreadPoolExecutor(1) as third:
+        def drop(sizes):
+            kept = [new(n) for n in sizes]
+            del kept
+        sizes = [1 << 12] * 16
+        first.submit(drop, sizes).result()
+        if how == "taken":
+            taken = second.submit(lambda: [new(n) for n in sizes]).result()
+            second.submit(taken.clear).result()
+        elif how == "stamped":
+            second.submit(drop, [1 << 16] * 24).result()
+        else:
+            second.submit(RB.trim_pool).result()
+        if how != "freed":
+            second.submit(drop, [1 << 16] * 24).result()      # (what is there has its event: the pool is the third thread's as well)
+        capi.sync()
+        first.submit(drop, [1 << 20]).result()
+        capi.sync()
+
+        def elsewhere():
+            RB.set_stream(other.ptr)
+            before = RB.pool_stats()
+            s = new(1 << 20)
+            after = RB.pool_stats()
+            del s
+            RB.set_stream(None)
+            return after[0] - before[0]
+        assert third.submit(elsewhere).result() == 1, "the release had an event recorded behind it"
+    capi.sync()
+    RB.trim_pool()
+    other.destroy()
+
+
 def test_recorded_operator_with_a_transposed_k(gpu):
     """The operator with k handed over as a transposed view (gathered into a temporary first), recorded into a launch graph on
     a stream of the caller's and replayed: no step of it waits for the device or allocates while recording; every replay -
