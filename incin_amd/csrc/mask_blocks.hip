@@ -241,8 +241,10 @@ hipError_t launch_mask_classify(const SdpaParams& p, int dtype, hipStream_t stre
     // From there on limits and flags in one pass where its workgroups - one per 32 rows of the mask - are as many as compute units; else two
     // kernels, whose second reads nothing where all rows have limits.  Whole call, us, two / one: a bias per head, f32 8 heads x 1024 x 1024 134 / 130,
     // x 4096 887 / 824, 4 x 2048 x 16384 2200 / 2116, bf16 likewise 42.1 / 38.4, 231 / 231, 452 / 416; one causal mask of 4096 x 4096 314 / 316, 74.4 /
-    // 79.3, 128 rows x 8192 291 / 304, 128 / 141.
-    if (p.mask_lims && (int64_t)nrb * Bm * Hm >= device_cus()) {
+    // 79.3, 128 rows x 8192 291 / 304, 128 / 141.  Not where all query rows have the same mask row, as with key padding handed over as [B, 1, 1, Skv]: its limits
+    // are those of a few rows, the one pass would read each of them 32 times a workgroup (bf16, 16 x 16 x 4096 at D = 64 667 / 734, 8 x 16 x 2048 at D = 128 176 /
+    // 188, 32 x 12 x 512 42.5 / 46.3).
+    if (p.mask_lims && p.m_si != 0 && (int64_t)nrb * Bm * Hm >= device_cus()) {
 #define SCAN(T, V) hipLaunchKernelGGL((mask_scan_kernel<T, V>), dim3(nrb, Bm * Hm), dim3(1024), 0, stream, (const T*)p.mask, p.m_sb, p.m_sh, p.m_si, p.m_sj, Hm, p.Sq, p.Skv, nkb, flags, (int32_t*)p.mask_lims, rows_m)
         switch (dtype) {
             case 0: if (vec) SCAN(float, true); else SCAN(float, false); break;

@@ -486,6 +486,34 @@ def test_mask_limits_and_flags_in_one_pass(gpu, dtype, Skv):
     check(got, ref, TOL[dtype], "mask in one pass, %d keys" % Skv)
 
 
+def test_mask_row_that_all_queries_share(gpu):
+    """Key padding as a tensor [B, 1, 1, Skv], large: the one row of each sequence has a limit, so nothing is asked of the blocks of
+    its 1024 repetitions and their flags stay unwritten - but for the sequence whose row holds values, where they say so - and
+    the result is that of key counts."""
+    B, H, S, D = 8, 2, 1024, 64
+    q, k, v = inputs(5700, B, H, H, S, S, D, D, capi.BF16)
+    lens = np.array([1024, 1, 700, 64, 33, 1000, 512, 900], np.int32)
+    for values in (False, True):
+        mask = np.where(np.arange(S) < lens[:, None], 0.0, -np.inf).astype(np.float32).reshape(B, 1, 1, S)
+        if values:
+            mask[5, 0, 0, 100:200] = 0.5
+        tq, tk, tv = (host.DeviceTensor.from_f32(x, capi.BF16) for x in (q, k, v))
+        to, tm = host.DeviceTensor((B, H, S, D), capi.BF16), capi.DeviceBuffer.from_numpy(dtypes.encode(mask, capi.BF16))
+        d = host.make_desc(tq, tk, tv, to, mask=tm, mask_strides=host.mask_strides_for(mask.shape, B, H, S, S))
+        need, _, impl = capi.sdpa_workspace(d)
+        ws = capi.DeviceBuffer.from_numpy(np.full(need, 0x5A, np.uint8))
+        d.workspace, d.workspace_bytes = ws.ptr, need
+        capi.sdpa_fwd(d)
+        capi.sync()
+        assert impl == capi.IMPL_MFMA
+        flags = ws.to_numpy(np.uint8, (need,))[: B * 32 * 32].reshape(B, 32, 32)
+        written = [bool((flags[b] != 0x5A).any()) for b in range(B)]
+        assert written == [values and b == 5 for b in range(B)]
+        check(to.to_f32(), host.sdpa(q, k, v, capi.BF16, mask=mask, impl=capi.IMPL_GENERIC), TOL[capi.BF16], "one mask row per sequence")
+        if values:
+            assert set(np.unique(flags[5])) <= {0, 1, 2} and (flags[5][:, 3] == 0).all()
+
+
 @pytest.mark.parametrize("dtype", [capi.BF16, capi.F16], ids=lambda x: dtypes.NAMES[x])
 @pytest.mark.parametrize("rows", ["128", "256"])
 @pytest.mark.parametrize("D", [128, 64])
