@@ -16,6 +16,31 @@ namespace incin_rocm {
 // the compiler takes 16-byte loads for it, which the memory path allows at any address.  (By elements where rows were not multiples of 32 bytes:
 // whole call, f32, a bias per head, 8 heads x 1001 x 1001 134 -> 123 us, bf16 12 x 801 x 801 98 -> 85, 32 x 900 x 900 64 -> 60.)
 template <typename T> struct Mask8 { typedef T type __attribute__((ext_vector_type(8), aligned(sizeof(T)))); };
+// The values of keys j0 .. j0 + 7 that a row has, as elements from .. 7 of what is returned; key j0 exists.  VEC (unit key stride, eight keys
+// or more): at the end of the row the eight before it, so that nothing is read one element after the other there.
+template <typename T> struct RowPart {
+    T x[8];
+    int first_key, from;      // element e is key first_key + e; the first `from` belong to whoever has the eight keys before
+};
+template <typename T, bool VEC> __device__ __forceinline__ RowPart<T> row_part(const T* row, int64_t m_sj, int j0, int Skv)
+{
+    RowPart<T> r;
+    if constexpr (VEC) {
+        r.first_key = min(j0, Skv - 8);
+        r.from = j0 - r.first_key;
+        const typename Mask8<T>::type v = *(const typename Mask8<T>::type*)(row + r.first_key);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) r.x[e] = v[e];
+    } else {
+        // (key by key; the n that there are take the last n places, key j0 fills the others)
+        const int n = min(8, Skv - j0);
+        r.first_key = j0 + n - 8;
+        r.from = 8 - n;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) r.x[e] = row[(int64_t)max(r.first_key + e, j0) * m_sj];
+    }
+    return r;
+}
 
 // (one workgroup of 256 threads: block row rb of (mask batch entry, mask head) bh, the strip's 8 blocks)
 template <typename T, bool VEC>
@@ -29,30 +54,19 @@ __device__ __forceinline__ void classify_strip(const T* mask, int64_t m_sb, int6
     if (threadIdx.x < 16) votes[threadIdx.x >> 1][threadIdx.x & 1] = 0;
     __syncthreads();
     const int j0 = strip * 256 + c8 * 8;
-    int not_zero = 0, not_hidden = 0;
     if (j0 < Skv) {
+        RowPart<T> part[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int i = rb * 32 + r0 + 8 * u;
-            if (i >= Sq) continue;
-            const T* row = base + (int64_t)i * m_si;
-            if (VEC && j0 + 7 < Skv) {
-                typedef typename Mask8<T>::type vec8;
-                const vec8 x = *(const vec8*)(row + j0);
+        for (int u = 0; u < 4; ++u) part[u] = row_part<T, VEC>(base + (int64_t)min(rb * 32 + r0 + 8 * u, Sq - 1) * m_si, m_sj, j0, Skv);      // (for rows that do not exist the last one again)
+        int not_zero = 0, not_hidden = 0;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const float f = to_f32(x[e]);
-                    not_zero |= !(f == 0.0f);
-                    not_hidden |= !(f == -INFINITY);
-                }
-            } else {
-                for (int e = 0; e < 8 && j0 + e < Skv; ++e) {
-                    const float f = to_f32(row[(int64_t)(j0 + e) * m_sj]);
-                    not_zero |= !(f == 0.0f);
-                    not_hidden |= !(f == -INFINITY);
-                }
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float f = to_f32(part[u].x[e]);
+                not_zero |= e >= part[u].from && !(f == 0.0f);
+                not_hidden |= e >= part[u].from && !(f == -INFINITY);
             }
-        }
         if (not_zero) atomicOr(&votes[c8 >> 2][0], 1);
         if (not_hidden) atomicOr(&votes[c8 >> 2][1], 1);
     }
@@ -96,22 +110,13 @@ __device__ __forceinline__ void limits_of_rows(const T* mask, int64_t m_sb, int6
     const T* row = mask + (bh / Hm) * m_sb + (bh % Hm) * m_sh + (int64_t)i * m_si;
     int first = Skv, ninf = 0;
     if (VEC) {
-        typedef typename Mask8<T>::type vec8;
         for (int j0 = lane * 8; j0 < Skv; j0 += 512) {
-            if (j0 + 7 < Skv) {
-                const vec8 x = *(const vec8*)(row + j0);
+            const RowPart<T> part = row_part<T, true>(row, m_sj, j0, Skv);
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const float f = to_f32(x[e]);
-                    if (!(f == 0.0f)) first = min(first, j0 + e);
-                    ninf += f == -INFINITY;
-                }
-            } else {
-                for (int e = 0; j0 + e < Skv; ++e) {
-                    const float f = to_f32(row[j0 + e]);
-                    if (!(f == 0.0f)) first = min(first, j0 + e);
-                    ninf += f == -INFINITY;
-                }
+            for (int e = 0; e < 8; ++e) {
+                const float f = to_f32(part.x[e]);
+                if (!(f == 0.0f)) first = min(first, part.first_key + e);
+                ninf += f == -INFINITY && e >= part.from;
             }
         }
     } else {
@@ -220,7 +225,7 @@ hipError_t launch_mask_classify(const SdpaParams& p, int dtype, hipStream_t stre
     const dim3 grid((nkb + 7) / 8, nrb, Bm * Hm);
     uint8_t* flags = (uint8_t*)p.mask_flags;
     const int esz = dtype == 0 ? 4 : 2;
-    const bool vec = p.m_sj == 1;      // 8 consecutive elements in one load
+    const bool vec = p.m_sj == 1 && p.Skv >= 8;      // 8 consecutive elements in one load
     const int rows_m = p.m_si ? p.Sq : 1;
     const int64_t n_rows = (int64_t)Bm * Hm * rows_m, n_strips = (int64_t)((nkb + 7) / 8) * nrb * Bm * Hm;
     // Limits and flags side by side, so the mask read twice, where it is less than 16 MB: a launch and its latency saved.  Whole call, us, by the
@@ -282,7 +287,7 @@ hipError_t launch_mask_row_limits(const void* mask, int dtype, const int64_t sha
     if (n_rows <= 0) return hipSuccess;
     if ((n_rows + 3) / 4 > 0x7fffffffLL) return hipErrorInvalidValue;
     const dim3 grid((unsigned)((n_rows + 3) / 4));
-    const bool vec = strides[3] == 1;
+    const bool vec = strides[3] == 1 && shape[3] >= 8;
 #define LIMITS(T, V) hipLaunchKernelGGL((mask_row_limits_kernel<T, V>), grid, dim3(256), 0, stream, (const T*)mask, strides[0], strides[1], strides[2], strides[3], (int)shape[1], (int)shape[2], (int)shape[3], n_rows, lims)
     switch (dtype) {
         case 0: if (vec) LIMITS(float, true); else LIMITS(float, false); break;

@@ -486,6 +486,68 @@ def test_mask_limits_and_flags_in_one_pass(gpu, dtype, Skv):
     check(got, ref, TOL[dtype], "mask in one pass, %d keys" % Skv)
 
 
+def mask_with_blocks(r, H, Sq, Skv):
+    """Rows with limits, blocks of zeros and of -inf, single values next to the end of a row."""
+    m = np.zeros((1, H, Sq, Skv), np.float32)
+    for h in range(H):
+        kind = r.integers(0, 4, size=((Sq + 31) // 32, (Skv + 31) // 32))
+        big = np.kron(kind, np.ones((32, 32), np.int64))[:Sq, :Skv]
+        m[0, h][big == 1] = -np.inf
+        for i in np.flatnonzero(r.random(Sq) < 0.4):      # a limit
+            m[0, h, i] = 0.0
+            m[0, h, i, int(r.integers(0, Skv + 1)):] = -np.inf
+        for i in np.flatnonzero(r.random(Sq) < 0.1):      # something in the last nine keys, or anywhere
+            m[0, h, i, Skv - 1 - int(r.integers(0, min(Skv, 9)))] = r.choice([0.5, -np.inf, 0.0, np.nan])
+            m[0, h, i, int(r.integers(0, Skv))] = r.choice([0.5, -np.inf, 0.0])
+    return m
+
+
+def limits_and_flags(m):
+    """What the mask kernels state, element by element: n for a row of n zeros and then -inf, else -1; per 32 x 32 block 1 all zero, 2 all -inf, else 0."""
+    H, Sq, Skv = m.shape[1:]
+    zero, hidden = m[0] == 0, m[0] == -np.inf
+    n = np.where(zero.all(-1), Skv, np.argmin(zero, axis=-1))
+    lims = np.where(hidden.sum(-1) == Skv - n, n, -1).astype(np.int32)
+    pad = [(0, 0), (0, -Sq % 32), (0, -Skv % 32)]
+    block = lambda x: np.pad(x, pad, constant_values=True).reshape(H, -(-Sq // 32), 32, -(-Skv // 32), 32).all(axis=(2, 4))
+    return lims, np.where(block(zero), 1, np.where(block(hidden), 2, 0)).astype(np.uint8)
+
+
+@pytest.mark.parametrize("dtype", [capi.BF16, capi.F16], ids=lambda x: dtypes.NAMES[x])
+@pytest.mark.parametrize("shape", [(3, 65, 1), (3, 66, 7), (3, 70, 8), (3, 65, 9), (2, 97, 15), (2, 97, 16), (2, 100, 33), (2, 128, 197), (2, 300, 255), (2, 140, 257), (2, 90, 300), (1, 70, 1030)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_mask_limits_and_flags_element_by_element(gpu, dtype, shape):
+    """Limits of rows and flags of blocks as they stand in the workspace, and the limits by the call of their own: keys one to eight
+    behind a multiple of eight, rows of fewer than eight, keys that are not next to each other in memory, NaN."""
+    import ctypes as C
+    H, Sq, Skv = shape
+    m = mask_with_blocks(rng(5800 + Skv), H, Sq, Skv)
+    lims, flags = limits_and_flags(m)
+    q, k, v = inputs(5801, 1, H, H, Sq, Skv, 64, 64, dtype)
+    raw = dtypes.encode(m, dtype)
+    wide = np.zeros(raw.shape[:3] + (2 * Skv,), raw.dtype)
+    wide[..., ::2] = raw
+    for strides, stored in ((host.mask_strides_for(m.shape, 1, H, Sq, Skv), raw), ([0, 2 * Sq * Skv, 2 * Skv, 2], wide)):
+        tm = capi.DeviceBuffer.from_numpy(stored)
+        tq, tk, tv = (host.DeviceTensor.from_f32(x, dtype) for x in (q, k, v))
+        to = host.DeviceTensor((1, H, Sq, 64), dtype)
+        d = host.make_desc(tq, tk, tv, to, mask=tm, mask_strides=strides)
+        d.impl = capi.IMPL_MFMA
+        need = capi.sdpa_workspace(d)[0]
+        ws = capi.DeviceBuffer.from_numpy(np.full(need, 0x5A, np.uint8))
+        d.workspace, d.workspace_bytes = ws.ptr, need
+        capi.sdpa_fwd(d)
+        capi.sync()
+        got = ws.to_numpy(np.uint8, (need,))
+        assert np.array_equal(got[: flags.size].reshape(flags.shape), flags)
+        at = (flags.size + 255) // 256 * 256
+        assert np.array_equal(got[at: at + 4 * H * Sq].view(np.int32).reshape(H, Sq), lims)
+        out = capi.DeviceBuffer(4 * H * Sq)
+        capi.check(capi.load().incin_rocm_mask_row_limits(0, dtype, tm.ptr, (C.c_int64 * 4)(1, H, Sq, Skv), (C.c_int64 * 4)(*strides), out.ptr, None))
+        capi.sync()
+        assert np.array_equal(out.to_numpy(np.int32, (H, Sq)), lims)
+
+
 def test_mask_row_that_all_queries_share(gpu):
     """Key padding as a tensor [B, 1, 1, Skv], large: the one row of each sequence has a limit, so nothing is asked of the blocks of
     its 1024 repetitions and their flags stay unwritten - but for the sequence whose row holds values, where they say so - and
