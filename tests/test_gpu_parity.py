@@ -514,7 +514,8 @@ def limits_and_flags(m):
 
 
 @pytest.mark.parametrize("dtype", [capi.BF16, capi.F16], ids=lambda x: dtypes.NAMES[x])
-@pytest.mark.parametrize("shape", [(3, 65, 1), (3, 66, 7), (3, 70, 8), (3, 65, 9), (2, 97, 15), (2, 97, 16), (2, 100, 33), (2, 128, 197), (2, 300, 255), (2, 140, 257), (2, 90, 300), (1, 70, 1030)],
+@pytest.mark.parametrize("shape", [(3, 65, 1), (3, 66, 7), (3, 70, 8), (3, 65, 9), (2, 97, 15), (2, 97, 16), (2, 100, 33), (2, 128, 197), (2, 300, 255), (2, 140, 257), (2, 90, 300), (1, 70, 1030),
+                                   (128, 65, 1021), (128, 70, 1024), (64, 97, 4097)],      # (16 MB and strips for every compute unit: one pass over whole rows)
                          ids=lambda s: "x".join(map(str, s)))
 def test_mask_limits_and_flags_element_by_element(gpu, dtype, shape):
     """Limits of rows and flags of blocks as they stand in the workspace, and the limits by the call of their own: keys one to eight
