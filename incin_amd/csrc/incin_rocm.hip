@@ -164,23 +164,27 @@ bool mask_rows_stageable(const incin_rocm_sdpa_desc_t* d)
 }
 
 // 16-bit decode with key counts: into how many workgroups the keys of all sequences are dealt (sdpa_decode_deal.hip), 0 for a launch
-// by splits of the capacity.  The host does not know the counts, so what speaks for it is what does not depend on them: a cache
-// large enough (300 MB) for the pass over the partial results and the division of the shares - 4 us and 1 - not to show, five sequences or
-// more, shares that hold few pieces (at most two rounds of (sequence, KV head) pairs, each of some thousand keys).  Bf16, four
-// query heads on each of 8 KV heads, counts spread evenly, us by splits / dealt: 32 x 1031 - 8192 106 / 98, 12 x 2048 - 16384 97 / 78.5,
-// 12 x 1000 - 8192 49.7 / 43.6, 24 x 512 - 4096 49.3 / 43.1, 48 x 1031 - 8192 156 / 144, 64 x 2000 - 16384 405 / 367, 20 of 4096 at D = 256 82 /
-// 70, 20 of 8192 on 12 KV heads 109 / 94, 20 of 8192 at D = 64 45 / 39; equal counts 32 x 4608 94.8 / 93.5, 8 x 12000 64.0 / 64.7, 64 x 16000 622 / 631.
-// Outside: 4 x 16384 30.6 / 33.2, 4 x 32768 58.6 / 61.5, 8 x 8192 33.2 / 33.0, 7 x 20000 on 1 KV head 18.1 / 21.2, 64 x 2048 54.9 / 57.7, 32 x 32 x 8192 351 / 356.
-// Two workgroups per compute unit where their LDS allows (rows x head dimension up to 512: 32 x 8192 ragged level, 24 x 4096 44.9 one, 43.1 two).
+// by splits of the capacity.  The host does not know the counts, so what speaks for it is what does not depend on them: that the launch by
+// splits needs the pass over partial results as well, a cache large enough (300 MB) for the division of the shares - 1 us - not to
+// show, five sequences or more, shares that hold few pieces (at most two rounds of (sequence, KV head) pairs, each of some thousand keys).  Us by splits / dealt, counts from an eighth of
+// the longest to it, in brackets two thirds of it, the longest a 64th of the capacity, a 16th, a quarter, a half, all: bf16, 32 on 8 heads, 12 x 16384 14.1 / 10.0, 25 / 15.8 (25.8 / 16.8), 46.6 /
+// 27.1 (48.2 / 35.3), 50.8 / 43.0 (62.6 / 58.1), 91.6 / 75.4 (106.4 / 108.8); 8 x 32768 11.8 / 10.7, 27.3 / 16.4, 82.9 / 31.1 (84.8 / 42.3), 88.2 / 53.1 (92.7 / 73.3), 99.5 / 96.4 (132.8 / 137.9);
+// 16 on 8, 40 x 8192 at D = 256 33 / 20, 43 / 33, 84 / 69 (106 / 96), 135 / 124 (182 / 173), 241 / 230 (344 / 344).  Over 26 launches of all kinds it was ahead by
+// 5 - 60 % but for the two ends: near the capacity throughout (up to 8 % behind), and some dozens of keys (up to 1 us).
+// Where a split holds a whole sequence, its launch writes the results itself, and the second launch of the dealt form is 3 us whatever the counts: 32 on 8, 32 x 8192
+// 7.4 / 10.3, 12.4 / 17.5, 30.9 / 33.3 (38.2 / 42.9), 55.6 / 55.8 (70.9 / 75.0), 105 / 98 (137 / 140); 64 on 8, 48 x 4096 12.3 / 18.9, 14.9 / 25, 26.6 / 37, 43 / 52, 79 / 82.
+// Others outside: 4 x 16384 30.6 / 33.2, 4 x 32768 58.6 / 61.5, 8 x 8192 33.2 / 33.0, 7 x 20000 on 1 KV head 18.1 / 21.2, 64 x 2048 54.9 / 57.7, 32 x 32 x 8192 351 / 356.
+// Two workgroups per compute unit where their LDS allows (rows x head dimension up to 512).
 // INCIN_ROCM_DECODE_DEAL forces a count of workgroups (0: by splits), for tests.
-int decode_deal_workgroups(const incin_rocm_sdpa_desc_t* d, int64_t R, int64_t d_pad)
+int decode_deal_workgroups(const incin_rocm_sdpa_desc_t* d, int64_t R, int64_t d_pad, int64_t splits)
 {
     if (d->dtype == INCIN_ROCM_F32 || d->num_splits != 0 || d->add_mask || d->B > incin_rocm::DEAL_MAX_BATCH ||
         R * d_pad > incin_rocm::DEAL_MAX_VALUES || d->B * d->Hkv * (d->Skv / 128 + 2) > (1LL << 30)) return 0;
     const char* forced = getenv("INCIN_ROCM_DECODE_DEAL");
     if (forced) return std::min(std::max(atoi(forced), 0), 4096);
     const int64_t cus = compute_units_of(d->device), groups = d->B * d->Hkv, key_bytes = d->Skv * d_pad * 2;
-    if (d->impl != INCIN_ROCM_IMPL_AUTO || !d->kv_lens || d->B < 5 || groups > 2 * cus || 2 * groups * key_bytes < 300000000 || key_bytes < (groups > cus ? 1 << 20 : 3 << 18)) return 0;
+    if (splits < 2 || d->impl != INCIN_ROCM_IMPL_AUTO || !d->kv_lens || d->B < 5 || groups > 2 * cus || 2 * groups * key_bytes < 300000000 ||
+        key_bytes < (groups > cus ? 1 << 20 : 3 << 18)) return 0;
     return (int)(cus * (d_pad <= 128 && 2 * R * d_pad <= incin_rocm::DEAL_MAX_VALUES ? 2 : 1));
 }
 
@@ -404,7 +408,7 @@ int make_plan(const incin_rocm_sdpa_desc_t* d, Plan* plan)
         plan->splits = (int)splits;
         plan->split_len = (int)split_len;
         plan->ws_bytes = splits > 1 ? (size_t)(d->B * d->Hq * d->Sq * splits) * (size_t)(d_pad + 2) * sizeof(float) : 0;
-        plan->deal = decode_deal_workgroups(d, R, d_pad);
+        plan->deal = decode_deal_workgroups(d, R, d_pad, splits);
         if (plan->deal) plan->deal_bytes = incin_rocm::deal_workspace_bytes(plan->deal, (int)R, (int)d_pad);
     }
     if (impl == INCIN_ROCM_IMPL_MFMA && !d->add_mask && !d->q_lens && !(wide && d->dtype == INCIN_ROCM_F32)) {

@@ -244,7 +244,7 @@ __global__ __launch_bounds__(256) void sdpa_decode_split_kernel(SdpaParams p)
 //
 // LONE: one wavefront does the row alone where its groups can ask for all splits so, eight each (16 splits at D = 128): sums meet over lanes, no barrier.
 // Us a call by groups / lone: bf16, 32 on 8 heads, one sequence of 1500 keys 10.9 / 10.3, 8 of 1000 - 2000 15.9 / 15.3, 4 x 5 positions x 3000 16.1 /
-// 15.4, 4 of 3000 - 16000 32.5 / 31.95, f32 2 x 8 on 4 x 1000 - 2000 at D = 64 10.15 / 9.7; dealt, 32 x 1031 - 8192 99.4 / 98.8.
+// 15.4, 4 of 3000 - 16000 32.5 / 31.95, f32 2 x 8 on 4 x 1000 - 2000 at D = 64 10.15 / 9.7.
 // (More splits than that keep the groups: with the choice between the two in the kernel they took 1 - 2 % longer.)
 //
 // DEAL: the partial results of a row are those of the shares that its sequence's units went to (decode_deal.h); rows of

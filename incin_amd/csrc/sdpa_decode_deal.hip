@@ -3,13 +3,13 @@
 //
 // That kernel gives a workgroup one split of one sequence, and the host, which does not know the counts, makes splits of the
 // capacity: with counts spread evenly from an eighth of it to all of it the compute units are left with very different amounts,
-// and the memory system idles while the longest finish (32 sequences of 1031 - 8192 keys on 8 KV heads: 106 us where 604 MB take
-// 85; dealt 98 - 100).  Here the keys of all sequences are dealt to the workgroups of one round in equal shares (decode_deal.h).  A share is a run of
+// and the memory system idles while the longest finish (12 sequences of 2048 - 16384 keys on 8 KV heads: 91.6 us where 453 MB take
+// 64; dealt 75.4).  Here the keys of all sequences are dealt to the workgroups of one round in equal shares (decode_deal.h).  A share is a run of
 // one to a few sequences' keys, and the ring of copies runs through it without a break: when the blocks of one sequence are
 // all on their way, the next copies are the next sequence's, so that while the four wavefronts' results of the first meet
 // and its rows of Q give way to the next one's, the ring fills on.  For that the results have LDS of their own, behind the
 // rings: rows x columns of each wavefront, which is why this form is for few rows (rows x head dimension up to 1024).
-// (With a ring drained and refilled for each sequence the same launch took 103 us, equal counts of 4608 95.9 instead of 93.5.)
+// (With a ring drained and refilled for each sequence 32 x 1031 - 8192 keys took 103 us instead of 98, equal counts of 4608 95.9 instead of 93.5.)
 #include <atomic>
 
 #include "decode_deal.h"

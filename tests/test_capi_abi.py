@@ -54,6 +54,23 @@ def _plan(d):
     return capi.sdpa_workspace(d)
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,Skv,D,dealt", [
+    (32, 32, 8, 8192, 128, False), (64, 32, 8, 16384, 128, False), (32, 32, 8, 32768, 128, False), (48, 64, 8, 4096, 128, False),
+    (24, 32, 8, 4096, 128, False), (64, 32, 8, 32768, 64, False), (12, 32, 8, 16384, 128, True), (8, 32, 8, 32768, 128, True), (40, 16, 8, 8192, 256, True),
+], ids=str)
+def test_decode_by_whole_sequences_stays_one_launch(B, Hq, Hkv, Skv, D, dealt):
+    """Decode with key counts whose splits are whole sequences needs no partial results, and so no workspace, whatever the counts; the
+    keys are dealt (two places for partial results a workgroup) only where sequences are split in any case."""
+    d = _desc(B=B, Hq=Hq, Hkv=Hkv, Sq=1, Skv=Skv, D=D, Dv=D, kv_lens=0x10000)
+    for name, h, s in (("q_stride", Hq, 1), ("k_stride", Hkv, Skv), ("v_stride", Hkv, Skv), ("o_stride", Hq, 1)):
+        st = getattr(d, name)
+        st[0], st[1], st[2] = h * s * D, s * D, D
+    nbytes, splits, impl = _plan(d)
+    assert impl == capi.IMPL_SPLITKV_MFMA
+    by_splits = B * Hq * splits * (D + 2) * 4 if splits > 1 else 0
+    assert (splits > 1) == dealt and nbytes == (max(by_splits, (512 if D <= 128 and 2 * Hq // Hkv * D <= 1024 else 256) * 2 * (Hq // Hkv) * (D + 2) * 4) if dealt else 0)
+
+
 def test_dispatch_choices():
     assert _plan(_desc())[2] == capi.IMPL_MFMA
     # f32: the IEEE-f32 matrix-core prefill kernel where the launch gives it more than two 128-row workgroups per compute unit
