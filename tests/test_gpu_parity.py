@@ -825,7 +825,7 @@ def test_decode_splitkv_matrix_cores_d64(gpu, dtype, shape, slots, monkeypatch):
 def test_keys_dealt_in_equal_shares(gpu, dtype, case, monkeypatch):
     """Decode whose workgroups take equal shares of all sequences' keys (chosen for large ragged batches; forced here with counts of
     workgroups that cut sequences, hold several of them, and outnumber the units): against the oracle, row normalisers against
-    the launch by splits, twice the same bytes, and with less workspace than it asks for the launch by splits itself."""
+    the launch by splits, twice the same bytes."""
     Hq, Hkv, Sq, D, Dv, causal, Skv, counts = case
     B = 3 if counts is None else len(counts)
     lens = None if counts is None else np.array(counts, np.int32)
@@ -847,6 +847,65 @@ def test_keys_dealt_in_equal_shares(gpu, dtype, case, monkeypatch):
         assert np.array_equal(got, again, equal_nan=True)
 
 
+class TokenMajor:
+    """Logical [B, H, S, D] over what is stored [B, S, H, D]."""
+
+    def __init__(self, x, dtype):
+        B, H, S, D = x.shape
+        self.stored = host.DeviceTensor.from_f32(np.ascontiguousarray(x.transpose(0, 2, 1, 3)), dtype)
+        self.shape, self.dtype, self.dev, self.ptr = x.shape, dtype, 0, self.stored.ptr
+        self.strides = (S * H * D, D, H * D)
+
+    def to_f32(self):
+        return self.stored.to_f32().transpose(0, 2, 1, 3)
+
+
+@pytest.mark.parametrize("dtype", [capi.BF16, capi.F16], ids=lambda x: dtypes.NAMES[x])
+@pytest.mark.parametrize("Hq,Hkv,Sq,D,Dv,causal", [(8, 2, 1, 128, 128, False), (6, 3, 2, 64, 64, False), (4, 2, 1, 256, 200, False), (4, 2, 3, 80, 96, False), (8, 2, 2, 128, 128, True)], ids=str)
+def test_keys_dealt_out_of_views(gpu, dtype, Hq, Hkv, Sq, D, Dv, causal, monkeypatch):
+    """Queries, cache and output as token-major views whose rows at and beyond the key counts hold NaN and infinities; the workspace shows that
+    the keys were dealt (partial results where only that form has any), and, for a call with the workspace of the launch by splits and no more, that they
+    were not."""
+    B, Skv, counts = 5, 1500, [1500, 1, 897, 128, 1301]
+    lens = np.array(counts, np.int32)
+    q, k, v = inputs(5350 + D, B, Hq, Hkv, Sq, Skv, D, Dv, dtype)
+    ref = oracle_full(q, k, v, G=Hq // Hkv, causal=causal, kv_lens=lens)
+    for b in range(B):
+        k[b, :, lens[b]:], v[b, :, lens[b]:] = np.nan, np.inf
+        v[b, :, lens[b] + 1:] = -np.inf
+    tq, tk, tv = (TokenMajor(x, dtype) for x in (q, k, v))
+    tl = capi.DeviceBuffer.from_numpy(lens)
+    Dp, R = (64 if max(D, Dv) <= 64 else 128 if max(D, Dv) <= 128 else 256), Hq // Hkv * Sq
+    results = {}
+    for workgroups in (0, 7, 61):
+        monkeypatch.setenv("INCIN_ROCM_DECODE_DEAL", str(workgroups))
+        to = TokenMajor(np.zeros((B, Hq, Sq, Dv), np.float32), dtype)
+        d = host.make_desc(tq, tk, tv, to, causal=causal, kv_lens=tl, impl=capi.IMPL_SPLITKV_MFMA)
+        for name, t in (("q_stride", tq), ("k_stride", tk), ("v_stride", tv), ("o_stride", to)):
+            for a in range(3):
+                getattr(d, name)[a] = t.strides[a]
+        need, splits, _ = capi.sdpa_workspace(d)
+        by_splits = B * Hq * Sq * splits * (Dp + 2) * 4 if splits > 1 else 0
+        pairs_at = workgroups * 2 * R * Dp * 4      # where the dealt form keeps (maximum, sum)
+        for give in {need, by_splits}:
+            room = max(need, 256)
+            ws = capi.DeviceBuffer.from_numpy(np.full(room, 0x5A, np.uint8))
+            d.workspace, d.workspace_bytes = ws.ptr, give
+            capi.sdpa_fwd(d)
+            capi.sync()
+            got = to.to_f32()
+            written = ws.to_numpy(np.uint8, (room,)) != 0x5A
+            check(got, ref, TOL[dtype], "views, %d workgroups, %d bytes" % (workgroups, give))
+            if workgroups == 0:
+                results["by splits"] = got
+            elif give == need and pairs_at >= by_splits:
+                assert written[pairs_at:].any(), "the keys were not dealt"
+                results[workgroups] = got
+            elif give < need:
+                assert not written[by_splits:].any() and np.array_equal(got, results["by splits"])
+    assert 61 in results
+
+
 def test_keys_dealt_where_a_large_batch_is_ragged(gpu):
     """The library's own choice for a large ragged batch: key counts change between two launches of one descriptor, and a descriptor
     with no more workspace than the launch by splits needs is served as it was."""
@@ -864,14 +923,15 @@ def test_keys_dealt_where_a_large_batch_is_ragged(gpu):
         old = B * Hq * splits * (D + 2) * 4 if splits > 1 else 0
         assert impl == capi.IMPL_SPLITKV_MFMA and need >= 2 * 256 * 4 * (D + 2) * 4
         give = need if dealt else old
-        ws = capi.DeviceBuffer(give) if give else None
-        if ws is not None:
-            desc.workspace, desc.workspace_bytes = ws.ptr, give
+        ws = capi.DeviceBuffer.from_numpy(np.full(max(need, old), 0x5A, np.uint8))
+        desc.workspace, desc.workspace_bytes = ws.ptr, give
         for n in (lens, lens[::-1].copy()):
             capi.check(capi.load().incin_rocm_memcpy_h2d(0, tl.ptr, n.ctypes.data, n.nbytes))
             capi.sdpa_fwd(desc)
             capi.sync()
             outs.append(to.to_f32())
+        # (behind what the launch by splits takes: the dealt one's partial results, or nothing)
+        assert need > old and (ws.to_numpy(np.uint8, (need,))[old:] != 0x5A).any() == dealt
     for a, b in ((0, 2), (1, 3)):
         check(outs[a], outs[b], 8e-3, "dealt against splits")
     for o, n in ((outs[0], lens), (outs[1], lens[::-1])):
