@@ -1,11 +1,12 @@
 // Split-KV launches whose sequences differ in length (key counts on the device): the keys of all of them, dealt to the workgroups of
 // one round in equal shares.
 //
-// A launch has a column per KV head, and the same sequences one after the other in each, counted in units of the keys that the four wavefronts of a workgroup take in one turn (a sequence without keys counts one: somebody has to write its
-// rows).  Workgroup w of W walks units [w T / W, (w + 1) T / W) of the T there are, sequence by sequence.  A sequence that lies inside one
-// share is finished by that workgroup; of the others, a share holds at most one that ends in it and one that goes on behind it:
-// two places for partial results per workgroup, which the combine kernel (sdpa_decode.hip) adds up in order.  Nothing here is known to the host but
-// W: key counts may change between the replays of a recorded launch.
+// A launch has a column per KV head, and the same sequences one after the other in each, counted in units of the keys that the four
+// wavefronts of a workgroup take in one turn (a sequence without keys counts one: somebody has to write its rows).  Of W workgroups
+// and T units in all, the first min(W, T) have a share, T / W units in a row each and the first T mod W of them one more, sequence by
+// sequence.  A sequence that lies inside one share is finished by that workgroup; of the others, a share holds at most one that ends in it and
+// one that goes on behind it: two places for partial results per workgroup, which the combine kernel (sdpa_decode.hip) adds up in order.  Nothing here is
+// known to the host but W: key counts may change between the replays of a recorded launch.
 #pragma once
 #include "sdpa_params.h"
 
@@ -76,7 +77,7 @@ __device__ __forceinline__ void deal_place(const DealColumn& c, int b, int* firs
     *first = f;
     *units = u;
 }
-// The shares: of `total` units in all, workgroup w's start at share_begin(w); owner(u) holds unit u.
+// The shares: of `total` units in all, workgroup w's is [begin(w), begin(w + 1)); owner(u) holds unit u.
 struct DealShares {
     int count, each, more;      // workgroups with a share; units of each, the first `more` one more
     __device__ __forceinline__ DealShares(int total, int workgroups)

@@ -33,8 +33,8 @@ struct SdpaParams {
     int32_t split_turn;        // largest shift of work_split (a power of two minus one; 0: none)
     int32_t split_even;        // splits are equal shares of a batch entry's keys, not of the capacity (split_keys)
     int32_t deal;              // workgroups that the blocks of all sequences are dealt to in equal shares (decode_deal.h; 0: by splits as above)
-    float* ws_acc;             // [B, Hq, Sq, num_splits, Dp] f32 partial numerators (Dp == Dv for the vector-ALU kernel)
-    float* ws_ml;              // [B, Hq, Sq, num_splits, 2]  running max (natural-log domain) and denominator
+    float* ws_acc;             // [B, Hq, Sq, num_splits, Dp] f32 partial numerators (Dp == Dv for the vector-ALU kernel); dealt: [deal, 2, G * Sq, Dp]
+    float* ws_ml;              // [B, Hq, Sq, num_splits, 2]  running max (f32 natural-log domain, 16-bit log2) and denominator; dealt: [deal, 2, G * Sq, 2]
     // matrix-core prefill kernels with a dense mask: one byte per block of 32 query rows x 32 keys (0 mixed, 1 all zero,
     // 2 all -inf), written by mask_classify_kernel ahead of the attention kernel, in the caller's workspace;
     // [mask batch entries][mask heads][ceil(Sq / 32)][ceil(Skv / 32)], an extent of 1 where the mask is broadcast

@@ -211,9 +211,14 @@ typedef struct {
                                       (launches that split the key axis: their combine pass) */
 } incin_rocm_sdpa_desc_t;
 
-/* Validates the descriptor and reports the scratch bytes and the split count the
- * launch will use (0 bytes and 1 split when the chosen kernel needs none).
- * `impl_out` (nullable) receives the INCIN_ROCM_IMPL_* the library will run. */
+/* Validates the descriptor and reports the scratch bytes that the launch has use for and its split count
+ * (0 bytes and 1 split when the chosen kernel needs none).
+ * `impl_out` (nullable) receives the INCIN_ROCM_IMPL_* the library will run.
+ * 16-bit decode over a large batch with kv_lens is a launch of two forms: the keys of all sequences dealt to the
+ * workgroups in equal shares, or so many splits of the capacity for each sequence.  The bytes reported are enough for
+ * either, the split count is that of the second.  The first is what runs with the bytes reported; with less, but
+ * enough for the second's partial results, incin_rocm_sdpa_fwd runs that one.  The results of the two differ as those of different
+ * split counts do, in the last bits. */
 int incin_rocm_sdpa_workspace(const incin_rocm_sdpa_desc_t* desc, size_t* bytes, int32_t* splits, int32_t* impl_out);
 
 /* Enqueues the kernels on `stream` (NULL = the device's default stream) and
@@ -236,8 +241,9 @@ int incin_rocm_sdpa_fwd(const incin_rocm_sdpa_desc_t* desc, void* stream);
  * harnesses that forbid it).  No counterpart in the reference.  `workspace` and `workspace_bytes` of the
  * descriptor are ignored: the scratch memory is a buffer of INCIN_ROCM_STATIC_SCRATCH_BYTES that is part of the
  * library's code object (one copy per device, held until the process ends), and the call makes no device or
- * host allocation.  A request whose scratch need (incin_rocm_sdpa_workspace) exceeds the buffer is refused with
- * INCIN_ROCM_EWORKSPACE.  Every call on a device shares that device's buffer: calls that may overlap in time on
+ * host allocation.  A request whose scratch need (incin_rocm_sdpa_workspace; where a launch has two forms, that of its
+ * splits) exceeds the buffer is refused with INCIN_ROCM_EWORKSPACE - but for prefill launches whose keys the library
+ * itself chose to split, which then run unsplit.  Every call on a device shares that device's buffer: calls that may overlap in time on
  * one device race, so keep them on one stream or order them with events. */
 #define INCIN_ROCM_STATIC_SCRATCH_BYTES (8u << 20)
 int incin_rocm_sdpa_fwd_static(const incin_rocm_sdpa_desc_t* desc, void* stream);
