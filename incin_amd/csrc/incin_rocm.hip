@@ -1083,10 +1083,11 @@ static int bwd16_parts(const incin_rocm_sdpa_desc_t* d, int64_t blocks, int64_t 
 }
 // Head dimensions above 128 (kind 3): one launch holds the blocks of all three gradients (sdpa_bwd_wide.hip), a dK or dV block
 // walks every head of its group, and the launch ends with its longest item at the earliest: a walk is dealt to more workgroups
-// when it alone would take more than twice what a compute unit's share of the whole launch is.  Measured (bf16, D = 256, causal,
-// backward call, in 1 / 2 / 4 / 8 parts): 8 query heads on 1 KV head x 2048 positions 847 / 424 / 229 / 137 us, x 4096 1678 / 854 /
-// 483 / 405, 64 on 8 x 700 299 / 172 / 142 / 162; where a walk is not the longest thing in the launch the planes (written, read
-// and summed in f32) only cost: 2 x 16 on 8 x 1024 126 / 142 / 167 / 239, 8 x 16 x 512 159 / 292.
+// when it alone would take more than twice what a compute unit's share of the whole launch is.  Measured, all walks of dK and dV divided alike
+// (bf16, D = 256, causal, backward call, in 1 / 2 / 4 / 8 parts): 8 query heads on 1 KV head x 2048 positions 847 / 424 / 229 / 137 us, x 4096 1678 / 854 /
+// 483 / 405, 64 on 8 x 700 299 / 172 / 142 / 162; where the longest is not twice the share the planes of all of them (written, read
+// and summed in f32) cost more than its division gains: 2 x 16 on 8 x 1024 - 1.45 times - 126 / 142 / 167 / 239, 8 x 16 x 512 159 / 292.
+// (What dividing the longest walks alone would give was not measured.)
 static int bwd_wide_parts(const incin_rocm_sdpa_desc_t* d)
 {
     const int64_t G = d->Hq / d->Hkv, nqb = (d->Sq + 127) / 128, nkb = (d->Skv + 127) / 128;

@@ -38,10 +38,11 @@
 // (2 x 16 on 8 x 1024 causal 128.5 -> 126 us, nothing masked 234 -> 229, 8 x 2048 123.5 -> 119.5, 4 x 3000 at D = 160 161 -> 158).
 //
 // Measured, backward call, bf16: 2 x 16 heads on 8 x 1024 positions, D = 256, causal 13.86 -> 0.14 ms (302 TFLOP/s of
-// useful work; the generic kernels 3.1), 8 on 1 x 4096 0.48 ms, 4 x 16 on 4 x 1024 0.25 ms.  The matrix pipes are busy 45 % of the
-// time a workgroup is on a compute unit; beside them the LDS is the bound - in the first products every matrix instruction takes
-// 1 KiB of it, 128 bytes a clock over the four SIMDs.  With parts left out (2 x 16 on 8 x 1024, nothing masked, 229 us): no copies
-// 210, no exponentials and splits 209, neither 191.
+// useful work; the generic kernels 3.1), 8 on 1 x 4096 0.48 ms, 4 x 16 on 4 x 1024 0.25 ms.  That causal launch is bound by its longest item: the
+// dK block of the first keys, 64 tiles of four products, is 1.45 times a compute unit's share of the whole.  Where items are equal (nothing
+// masked) the matrix pipes are busy 45 % of the time a workgroup is on a compute unit, and beside them the LDS is the bound - in the first products every
+// matrix instruction takes 1 KiB of it, 128 bytes a clock over the four SIMDs.  With parts left out (2 x 16 on 8 x 1024, nothing masked, 229 us): no
+// copies 210, no exponentials and splits 209, neither 191.
 #include <type_traits>
 
 // (three bodies in one kernel spill scalar registers, copy descriptors among them: their copies take the five wait states)
