@@ -419,14 +419,16 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(2, 2))
 // length by a causal flag and heads have eight of them or more: with one group the two longest meet on a compute unit and end the
 // launch.  16 x 4096 (512) 191 / 148, 8 x 8192 (512) 370 / 271, 2 x 16 x 1536 (384) 74 / 53, 4 x 16 x 1024 (512) 55.4 / 53.4; but 6 x 16 x 512 (384)
 // 31.8 / 34.3, 16 x 8 x 300 (384) 22 / 30, nothing masked 2 x 16 x 2048 (512) 124 / 137, 4 x 16 x 2048 (1024) 139 / 164.
-// Either way there have to be keys enough for the results' meeting to be earned back: six tiles up to half a round, 4 x 16 x 65 on 96 keys (64) 10.9 /
-// 11.6, on 160 13.7 / 13.5, on 192 15.2 / 14.2, 8 x 16 x 128 (128) on 160 14.8 / 14.9, on 192 16.0 / 15.3; beyond it the launch runs into the memory system's
-// pace and thirteen are needed, 12 x 16 x 128 (192) on 256 19.5 / 19.0, 16 x 16 x 128 (256) on 128 14.9 / 16.4, on 256 20.9 / 21.6, on 320 23.2 / 23.8, on
-// 384 26.0 / 26.0, on 416 and more ahead (512 31.3 / 30.5, 1024 52.8 / 48.7).
+// Either way there have to be keys enough for the results' meeting to be earned back: six tiles, 4 x 16 x 65 on 96 keys (64 workgroups) 10.9 / 11.6, on
+// 160 13.7 / 13.5, on 192 15.2 / 14.2; and more where workgroups, and heads of K and V above all, are many, for then the launch goes at the memory
+// system's pace and not at the wavefronts'.  Two over one, on 160 / 192 / 224 / 256 / 320 / 384 keys: 9 x 16 x 128 (144 workgroups, 144 heads) 1.02 / 0.96 / 0.97 / 0.93 / 0.92 / 0.90, 12 x 16
+// x 128 (192, 192) 1.05 / 1.03 / 1.03 / 0.97 / 0.96 / 0.93, 14 x 16 x 128 (224, 224) 1.09 / 1.06 / 1.06 / 1.00 / 0.98 / 0.95, 16 x 16 x 128 (256, 256) 1.13 / 1.07 / 1.09 / 1.05 / 1.02 / 0.99,
+// 16 on 8 heads (256, 128) 1.06 / 1.02 / 1.03 / 1.00 / 0.96 / 0.93, 16 on 4 (256, 64) 1.03 / 0.98 / 0.98 / 0.92 / 0.91 / 0.89, 8 x 16 x 256 (256, 128) 1.07 / 1.03 / 1.03 / 0.97 / 0.96 / 0.93,
+// 4 x 16 x 375 (192, 64) 1.02 / 0.96 / 0.96 / 0.92 / 0.89 / 0.86.
 static bool two_groups(const SdpaParams& p, int64_t total, int nqb)
 {
     const int64_t cus = device_cus();
-    if (p.Skv <= (2 * total <= cus ? 160 : 384)) return false;
+    if (p.Skv <= 160 || 4 * (int64_t)p.Skv <= 3 * (int64_t)p.B * p.Hkv + 2 * total) return false;
     return total <= cus || (total <= 2 * cus && (p.causal || p.mask) && nqb >= 8 && p.Skv - p.Sq <= p.Sq / 4);
 }
 

@@ -1141,15 +1141,17 @@ def test_two_groups_of_wavefronts_above_128(gpu, dtype, dims):
 @pytest.mark.parametrize("dtype", [capi.BF16, capi.F16], ids=lambda x: dtypes.NAMES[x])
 @pytest.mark.parametrize("full", [False, True], ids=["few_workgroups", "one_per_compute_unit"])
 def test_two_groups_of_wavefronts_take_keys_enough(gpu, dtype, full):
-    """Few keys are not dealt to two groups: up to 160 of them, or 384 where there is a workgroup for more than half the compute units, a
-    launch gives the very bytes that its heads give among so many others that there is one group.  Above, against the oracle."""
+    """Few keys are not dealt to two groups: up to 160 of them, or, with a workgroup and a head of K and V for every compute unit, up to five
+    quarters as many as there are of those, a launch gives the very bytes that its heads give among so many others that there is one
+    group.  Above, against the oracle."""
     cus = capi.device_info(0).compute_units
     H = cus if full else 4
+    most = 5 * cus // 4 if full else 160
     more = 2 * cus // H + 1
-    for Skv in ((33, 256, 384, 385) if full else (31, 65, 128, 160, 161, 193)):
+    for Skv in (31, 65, 128, 160, 161, 193, most, most + 1, most + 64):
         q, k, v = inputs(5150 + Skv, 1, H, H, 66, Skv, 256, 256, dtype)
         got = host.sdpa(q, k, v, dtype, impl=capi.IMPL_MFMA)
-        if Skv <= (384 if full else 160):
+        if Skv <= most:
             among = host.sdpa(*(np.concatenate([x] * more, axis=1) for x in (q, k, v)), dtype, impl=capi.IMPL_MFMA)
             assert np.array_equal(got, among[:, :H]), "%d keys" % Skv
         ref = oracle_full(q[:, :4], k[:, :4], v[:, :4])
