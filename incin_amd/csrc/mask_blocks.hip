@@ -233,10 +233,11 @@ hipError_t launch_mask_classify(const SdpaParams& p, int dtype, hipStream_t stre
     const bool vec = p.m_sj == 1 && p.Skv >= 8;      // 8 consecutive elements in one load
     const int rows_m = p.m_si ? p.Sq : 1;
     const int64_t n_rows = (int64_t)Bm * Hm * rows_m, n_strips = (int64_t)((nkb + 7) / 8) * nrb * Bm * Hm;
-    // Limits and flags side by side, so the mask read twice, where it is less than 16 MB: a launch and its latency saved.  Whole call, us, by the
-    // launches below / so: one causal mask, f32 1024 x 1024 59.6 / 58.5, 256 x 256 18.4 / 17.0, 129 x 129 18.9 / 16.2, bf16 1024 x 1024 23.4 / 21.8, 2048 x 2048 33.1
-    // / 32.0, 701 x 701 20.0 / 20.3; a bias per head, f32 4 x 8 x 300 x 300 44.6 / 41.7, 8 x 512 x 512 66.9 / 66.4, 1001 x 1001 (two launches either way, rows
-    // at any address) 134 / 123, bf16 12 x 800 x 800 40.3 / 35.7, 8 x 1024 x 1024 (16 MB) 38.4 / 39.3.
+    // Limits and flags side by side, so the mask read twice, where it is less than 16 MB: a launch and its latency saved.  Whole call at D = 64, us, by two
+    // launches / by one: bf16, a causal mask, 1 x 1 x 128 x 128 13.3 / 12.1, 2 x 8 x 300 15.6 / 14.3, 16 x 12 x 256 18.0 / 16.7, 64 x 12 x 197 37.1 / 36.4, 4 x 8 x 1024
+    // 23.8 / 22.7; key padding [B, 1, 1, Skv] 15.0 / 14.1, 16.8 / 15.7, 35.1 / 34.7, 23.3 / 22.6 for the last four; a bias per head 2 x 8 x 300 25.1 / 21.8, 4 x 16 x 700 47.0 / 43.6, 4 x 8 x
+    // 1024 40.0 / 38.2; f32, a causal mask 2 x 8 x 300 20.4 / 19.2, 4 x 8 x 1024 59.8 / 59.4, a bias per head 2 x 8 x 300 43.1 / 39.9.  Above, masks of limits are behind by it
+    // (f32 key padding 4 x 8 x 1024 88.7 / 92.7, bf16 1 x 8 x 4096 causal 57 / 61).
     if (p.mask_lims && (int64_t)Bm * Hm * p.Sq * p.Skv * esz < 16 << 20) {
         const dim3 bgrid((unsigned)(n_strips + (n_rows + 3) / 4));
 #define BOTH(T, V) hipLaunchKernelGGL((mask_both_kernel<T, V>), bgrid, dim3(256), 0, stream, (const T*)p.mask, p.m_sb, p.m_sh, p.m_si, p.m_sj, Hm, p.Sq, p.Skv, nkb, nrb, flags, (int32_t*)p.mask_lims, rows_m, n_rows, (unsigned)n_strips)
@@ -249,11 +250,11 @@ hipError_t launch_mask_classify(const SdpaParams& p, int dtype, hipStream_t stre
         return hipGetLastError();
     }
     // From there on limits and flags in one pass where its workgroups - one per 32 rows of the mask - are as many as compute units; else two
-    // kernels, whose second reads nothing where all rows have limits.  Whole call, us, two / one: a bias per head, f32 8 heads x 1024 x 1024 134 / 130,
-    // x 4096 887 / 824, 4 x 2048 x 16384 2200 / 2116, bf16 likewise 42.1 / 38.4, 231 / 231, 452 / 416; one causal mask of 4096 x 4096 314 / 316, 74.4 /
-    // 79.3, 128 rows x 8192 291 / 304, 128 / 141.  Not where all query rows have the same mask row, as with key padding handed over as [B, 1, 1, Skv]: its limits
-    // are those of a few rows, the one pass would read each of them 32 times a workgroup (bf16, 16 x 16 x 4096 at D = 64 667 / 734, 8 x 16 x 2048 at D = 128 176 /
-    // 188, 32 x 12 x 512 42.5 / 46.3).
+    // kernels, whose second reads nothing where all rows have limits.  Whole call, us, two / one: bf16, a bias per head, 8 x 8 x 1024 40.8 / 37.0, 1 x 8 x 4096 162 / 151, 8 x 16 x 2048 at D = 128
+    // 233 / 217; a mask per head and sequence, 64 x 12 x 197 145 / 149, 32 x 12 x 512 158 / 127, 8 x 8 x 1024 87 / 66; causal and padding per sequence, 32 x 12 x 512 44.6 / 43.3, 8 x 16 x
+    // 2048 133 / 133; f32, 1 x 8 x 4096, a bias 660 / 599, a band 280 / 217.  Fewer workgroups: one causal mask, bf16, 1 x 8 x 4096 57 / 62, 8 x 16 x 2048 154 / 156.  Not where all query rows have
+    // the same mask row, as with key padding handed over as [B, 1, 1, Skv]: its limits are those of a few rows, the one pass would read each of them 32 times a workgroup (bf16, 16 x 16 x 4096
+    // at D = 64 667 / 734, 8 x 16 x 2048 at D = 128 176 / 182, 32 x 12 x 512 42.1 / 43.9).
     if (p.mask_lims && p.m_si != 0 && (int64_t)nrb * Bm * Hm >= device_cus()) {
 #define SCAN(T, V) hipLaunchKernelGGL((mask_scan_kernel<T, V>), dim3(nrb, Bm * Hm), dim3(1024), 0, stream, (const T*)p.mask, p.m_sb, p.m_sh, p.m_si, p.m_sj, Hm, p.Sq, p.Skv, nkb, flags, (int32_t*)p.mask_lims, rows_m)
         switch (dtype) {
