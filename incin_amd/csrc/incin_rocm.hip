@@ -28,8 +28,8 @@ hipError_t launch_matrix_rate(const void* src, void* sink, int mix, int iteratio
 hipError_t launch_sdpa_prefill_f32(const SdpaParams& p, hipStream_t stream);
 hipError_t launch_sdpa_prefill_wide(const SdpaParams& p, int dtype, hipStream_t stream);
 hipError_t launch_mask_classify(const SdpaParams& p, int dtype, hipStream_t stream);
-hipError_t launch_mask_row_limits(const void* mask, int dtype, const int64_t shape[4], const int64_t strides[4], int32_t* lims, hipStream_t stream);
 hipError_t launch_sdpa_decode_f32_limits(const SdpaParams& p, hipStream_t stream);
+hipError_t launch_mask_row_limits(const void* mask, int dtype, const int64_t shape[4], const int64_t strides[4], int32_t* lims, hipStream_t stream);
 hipError_t launch_sdpa_decode(const SdpaParams& p, int dtype, hipStream_t stream);
 hipError_t launch_sdpa_decode_mfma(const SdpaParams& p, int dtype, hipStream_t stream);
 hipError_t launch_sdpa_decode_deal(const SdpaParams& p, int dtype, hipStream_t stream);
@@ -120,6 +120,7 @@ struct Plan {
     size_t ws_bytes, deal_bytes;      // workspace of the launch by splits (it must have that), of the other (it is taken where there is that)
     size_t lims_offset;      // dense mask on the prefill kernels: where the mask's row limits start in the workspace (0: none)
     bool lims_splitkv;       // f32 with a dense mask: the blocks whose rows all have a limit go through the f32 split-KV kernel first
+    bool rows64;             // f32: an unsplit launch of the split-KV form goes 64 rows per workgroup (sdpa_prefill_f32.hip)
     bool empty;      // nothing to compute
 };
 
@@ -188,6 +189,29 @@ int decode_deal_workgroups(const incin_rocm_sdpa_desc_t* d, int64_t R, int64_t d
     return (int)(cus * (d_pad <= 128 && 2 * R * d_pad <= incin_rocm::DEAL_MAX_VALUES ? 2 : 1));
 }
 
+// Whether an f32 launch whose keys are not split is over sooner with 64 rows of a query head per workgroup (sdpa_prefill_f32.hip) than with 32 rows of a
+// KV head (sdpa_decode_f32.hip).  The former is the one for launches that fill the device, its matrix instructions being the faster ones; the latter's
+// workgroups are half as large and walk a quarter of the keys per wavefront, so a launch that leaves compute units idle ends sooner, and
+// they are the fuller ones where 64 divides the positions badly.  By
+// the 64-row workgroups of the launch against compute units (two on one up to head dimension 64, else one) - measured on 2 - 96 heads x 65 -
+// 2048 positions, us, split-KV / prefill: D = 64, causal, 256 workgroups 28.1 / 35.8 (16 heads x 1024), 18.4 / 21.2 (32 x 512), 384 43.9 / 36.6 (24 x
+// 1024), 35.4 / 28.7 (32 x 768), 29.5 / 21.5 (48 x 512), but over at most 256 positions from 144 workgroups on 13.5 / 11.7 (48 x 192), 13.6 /
+// 13.4 (48 x 256); nothing masked, 128 14.7 / 20.3 (8 x 512), 30.5 / 34.9 (8 x 1024), 144 19.6 / 17.1 (24 x 384), 192 24.0 / 21.0 (24 x 512), 256 41.5 / 36.5 (16 x 1024),
+// 512 76.9 / 54.6.  D = 80, causal, 256 38.3 / 49.3, 384 56.2 / 49.6, 512 70.3 / 58.0; nothing masked, 144 26.5 / 23.0, 256 59.1 / 50.5, but where a
+// second round of them is not nearly full 288 66.4 / 74.2, 384 85.9 / 94.9, 576 107.5 / 110.9.  D = 128, causal, 256 49.0 / 62.8, 384 71.9 / 62.9, 512
+// 89.6 / 73.8; nothing masked, 192 42.4 / 35.4, 288 85.2 / 95.0, 512 144.2 / 125.2, 768 207.7 / 186.4.
+// 48 positions over 300 keys, causal, 256 workgroups 20.2 / 16.7; 64 over 256, 1024 workgroups 65 / 41.
+bool f32_rows64_ahead(const incin_rocm_sdpa_desc_t* d, int64_t d_pad, bool uneven)
+{
+    const int64_t G = d->Hq / d->Hkv;
+    if (d_pad > 128 || 3 * G * ((d->Sq + 63) / 64 * 64) > 4 * ((G * d->Sq + 31) / 32 * 32)) return false;
+    const int64_t cus = compute_units_of(d->device), wgs = d->B * d->Hq * ((d->Sq + 63) / 64);
+    if (d_pad == 64) return uneven ? wgs > cus || (d->Sq <= 256 && 2 * wgs > cus) : 2 * wgs > cus;
+    if (uneven) return wgs > cus;
+    const int64_t rounds = (wgs + cus - 1) / cus;
+    return 2 * wgs > cus && (rounds == 1 || rounds > 4 || 5 * wgs >= 4 * cus * rounds);
+}
+
 int make_plan(const incin_rocm_sdpa_desc_t* d, Plan* plan)
 {
     if (!d) return fail(INCIN_ROCM_EINVAL, "scaled_dot_product_attention: null descriptor");
@@ -206,6 +230,7 @@ int make_plan(const incin_rocm_sdpa_desc_t* d, Plan* plan)
     plan->deal_bytes = 0;
     plan->lims_offset = 0;
     plan->lims_splitkv = false;
+    plan->rows64 = false;
     plan->empty = (d->B == 0 || d->Hq == 0 || d->Sq == 0 || d->Dv == 0);
     if (plan->empty) return 0;
     if (d->Hkv <= 0 || d->Hq % d->Hkv != 0)
@@ -237,7 +262,7 @@ int make_plan(const incin_rocm_sdpa_desc_t* d, Plan* plan)
     // the MFMA kernels address a K/V tile with 32-bit byte offsets from the tile's first row
     const int64_t stride_lim = d->dtype == INCIN_ROCM_F32 ? (1 << 22) : (1 << 24);
     const bool tile_off_ok = d->k_stride[2] >= 0 && d->v_stride[2] >= 0 && d->k_stride[2] < stride_lim && d->v_stride[2] < stride_lim;
-    // f32: the IEEE-f32 matrix-core kernel, any finite scale; f16 / bf16: the 16-bit kernels fold the scale into Q in
+    // f32: the f32 matrix-core kernel, any finite scale; f16 / bf16: the 16-bit kernels fold the scale into Q in
     // a way that needs it positive.  Both take a dense additive mask (any strides); the 64-row kernel does not.
     // (above 128: sdpa_prefill_wide.hip - 16-bit storage, any finite scale, a dense mask whose rows it can read 8 bytes at a time)
     const bool mfma_ok = wide ? layout_ok && d->dtype != INCIN_ROCM_F32 && tile_off_ok && std::isfinite(d->scale) && (!d->add_mask || mask_rows_vector_loadable(d))
@@ -307,15 +332,9 @@ int make_plan(const incin_rocm_sdpa_desc_t* d, Plan* plan)
         else if (d->dtype == INCIN_ROCM_F32 && split_mfma_ok && d->Sq <= 64 && len128 >= 256 &&
                  (R >= 2 || d->Skv >= (d_pad == 64 ? 1024 : 512)))
             impl = INCIN_ROCM_IMPL_SPLITKV_MFMA;
-        // f32 prefill launches that give the prefill kernel at most two 128-row workgroups per compute unit (one round of what a
-        // compute unit holds; since the 32-row form runs two workgroups per compute unit, longest chunks first: 2 x 16 heads x
-        // 2048 x 2048 at D = 128, 512 workgroups' worth, 0.384 -> 0.316 ms; 4 x 16 x 1024 x 1024 0.197 -> 0.180; level at 640
-        // workgroups' worth at D = 64; the prefill kernel 1.1 - 1.3 times ahead from 1024 on): the split-KV kernel
-        // takes them 32 rows per workgroup with the keys dealt to its four wavefronts - four times the workgroups, a quarter
-        // of the keys per wavefront - where the prefill kernel's wavefronts each walk all keys for their 32 rows behind
-        // 64-cycle matrix instructions (measured, causal: one head of 128 x 128 13.3 -> 8.6 us; 2 x 8 heads x 512 x 512 at
-        // D = 128 73 -> 28; 128 workgroups' worth of 1024 x 1024 80 -> 33; 256 - 4 x 8 heads x 1024 x 1024 at D = 64 - 80 -> 65; level at 512).
-        // Not the chunks of a long prompt, where the prefill kernel splits the keys itself (below) and runs at 80 % of the peak.
+        // f32 prefill launches of at most two 128-row blocks per compute unit: whichever of the two forms is over sooner
+        // (f32_rows64_ahead, below).  Larger ones go 64 rows per workgroup, 1.2 - 1.5 times ahead of 32.
+        // Not the chunks of a long prompt, where the prefill kernel splits the keys itself (below).
         else if (d->dtype == INCIN_ROCM_F32 && split_mfma_ok && d->Sq > 64 && !(d->Skv >= 4096 && d->Skv >= 4 * d->Sq) &&
                  d->B * d->Hq * ((d->Sq + 127) / 128) <= 2 * compute_units_of(d->device))
             impl = INCIN_ROCM_IMPL_SPLITKV_MFMA;
@@ -381,6 +400,8 @@ int make_plan(const incin_rocm_sdpa_desc_t* d, Plan* plan)
         const int64_t nchunks = (R + chunk - 1) / chunk;
         const int64_t groups = d->B * d->Hkv * nchunks;
         int64_t splits = d->num_splits;
+        plan->rows64 = d->dtype == INCIN_ROCM_F32 && splits <= 1 && f32_rows64_ahead(d, d_pad, d->causal != 0);
+        if (plan->rows64) splits = 1;
         if (splits == 0) {
             const int64_t cus = compute_units_of(d->device);
             // (from 65536 keys on a split keeps at least 1024: with one or two groups the filling alone would ask for 512 splits of
@@ -445,13 +466,14 @@ int make_plan(const incin_rocm_sdpa_desc_t* d, Plan* plan)
         if (nbh > 65535 || (d->Sq + 31) / 32 > 65535)
             return fail(INCIN_ROCM_ESHAPE, "scaled_dot_product_attention: mask too large for one launch of the matrix-core kernels");
         plan->ws_bytes = (size_t)(nbh * ((d->Sq + 31) / 32) * ((d->Skv + 31) / 32) + 255) / 256 * 256;
-        // f32: a small launch (what AUTO would hand the f32 split-KV kernel if there were no mask tensor: at most two 128-row
-        // blocks per compute unit) whose chunks of 32 rows do not straddle query heads gets the blocks whose mask rows all have
-        // a limit computed by that kernel, from the limits, ahead of the prefill kernel's dense-mask launch for the rest
-        // (benchmark config 2 with the causal mask as a tensor: 90 -> 66 us)
-        plan->lims_splitkv = d->dtype == INCIN_ROCM_F32 && !wide && d->impl == INCIN_ROCM_IMPL_AUTO && !d->q_lens && d->Sq > 64 &&
-                             (d->Hq == d->Hkv || d->Sq % 128 == 0) && d->B * d->Hq * ((d->Sq + 127) / 128) <= 2 * compute_units_of(d->device);
-        if (d->dtype != INCIN_ROCM_F32 || plan->lims_splitkv) {      // one int per mask row: its limit, if it is zeros up to one and -inf beyond
+        // one int per mask row: its limit, if it is zeros up to one and -inf beyond.  f32: launches that AUTO would hand to the split-KV form if there were no
+        // mask tensor (larger ones, and what names the kernel, have never asked for the room, so they read the values; so has a
+        // padded batch).  Those that this form takes 32 rows at a time get the blocks whose mask rows all have a limit computed by its kernel, from the
+        // limits, ahead of the prefill kernel's launch for the rest; in the others the prefill kernel takes the limits for the mask.
+        const bool small = d->dtype == INCIN_ROCM_F32 && !wide && d->impl == INCIN_ROCM_IMPL_AUTO && !d->q_lens && d->Sq > 64 &&
+                           (d->Hq == d->Hkv || d->Sq % 128 == 0) && d->B * d->Hq * ((d->Sq + 127) / 128) <= 2 * compute_units_of(d->device);
+        plan->lims_splitkv = small && !f32_rows64_ahead(d, d_pad, true);
+        if (d->dtype != INCIN_ROCM_F32 || small) {
             plan->lims_offset = plan->ws_bytes;
             plan->ws_bytes += (size_t)(nbh * (d->mask_stride[2] ? d->Sq : 1) * 4 + 255) / 256 * 256;
         }
@@ -864,6 +886,7 @@ static int launch_fwd(const incin_rocm_sdpa_desc_t* desc, const Plan& planned, v
                     pl.split_len = (int)((desc->Skv + 255) / 256 * 256);
                     e = incin_rocm::launch_sdpa_decode_f32_limits(pl, s);
                     if (e != hipSuccess) break;
+                    p.lims_rows = 128;      // (whose 128-row blocks with a limit in every row the next launch leaves alone)
                 }
             }
             e = p.Dp == 256                    ? incin_rocm::launch_sdpa_prefill_wide(p, desc->dtype, s)
@@ -871,7 +894,7 @@ static int launch_fwd(const incin_rocm_sdpa_desc_t* desc, const Plan& planned, v
                                                 : incin_rocm::launch_sdpa_prefill_mfma(p, desc->dtype, s);
             break;
         case INCIN_ROCM_IMPL_SPLITKV: e = incin_rocm::launch_sdpa_decode(p, desc->dtype, s); break;
-        case INCIN_ROCM_IMPL_SPLITKV_MFMA: e = p.deal ? incin_rocm::launch_sdpa_decode_deal(p, desc->dtype, s) : incin_rocm::launch_sdpa_decode_mfma(p, desc->dtype, s); break;
+        case INCIN_ROCM_IMPL_SPLITKV_MFMA: e = plan.rows64 ? incin_rocm::launch_sdpa_prefill_f32(p, s) : p.deal ? incin_rocm::launch_sdpa_decode_deal(p, desc->dtype, s) : incin_rocm::launch_sdpa_decode_mfma(p, desc->dtype, s); break;
         default: e = incin_rocm::launch_sdpa_generic(p, desc->dtype, s); break;
     }
     if (e != hipSuccess) return hip_fail(e, "attention kernel launch");

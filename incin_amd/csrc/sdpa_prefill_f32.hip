@@ -1,36 +1,36 @@
-// f32 attention forward on the gfx950 matrix cores with IEEE single-precision arithmetic
-// (v_mfma_f32_32x32x2_f32: f32 operands, f32 products and sums - no reduced-precision path), for head dimensions up to
-// 128 (instances for 64 and 128; a smaller D or Dv, in whole 16-byte vectors, is zero-padded on the way into LDS), optional causal mask, per-batch key lengths, a dense additive mask with arbitrary broadcast strides,
-// MHA and GQA.  f32 is the one dtype the reference's own operator runs end to end
+// f32 attention forward on the gfx950 matrix cores, for head dimensions up to 128 (instances for 64 and 128; a smaller D or Dv, in
+// whole 16-byte vectors, is zero-padded on the way into LDS), optional causal mask, per-batch key lengths, a dense additive mask with
+// arbitrary broadcast strides, MHA and GQA.  f32 is the one dtype the reference's own operator runs end to end
 // (crates/incin-backends/src/cpu/ops/shape_ops.rs:1245-1269 over cpu/ops/matmul.rs:234,254), with a 1e-5 bar.
 //
-// Shape of the computation - that of sdpa_prefill_mfma.hip (one workgroup = 4 wavefronts = 128 query rows, one
-// wavefront = 32 query rows), with the operand layouts of the k = 2 instruction:
+// Products go through the bf16 matrix instruction, every value as the sum of three bf16 ones (f32_split.h: six instructions, no
+// larger error than the IEEE-f32 instruction's and 2.7 times its rate; it also lets the vector work of the other wavefronts run beside it).
 //
-//   S^T = K_blk Q'^T   A = K: lane (key = lane % 32, g = lane / 32) supplies K[key][d]; B = Q'^T: the same lane
-//                      supplies Q'[query = lane % 32][d] (Q' = Q * scale * log2(e), kept in registers for the whole
-//                      kernel).  One instruction sums over two values of d: the one the g = 0 lanes hold and the one
-//                      the g = 1 lanes hold.  Which two is free as long as A and B agree, so a lane reads four
-//                      consecutive floats d = 8j + 4g .. 8j + 4g + 3 (one 16-byte LDS read) and they serve four
-//                      instructions.  In the 32 x 32 result a lane owns ONE query (column lane % 32) and 16 keys
-//                      (register r is key 8 (r / 4) + 4 g + r % 4): row maximum and row sum are in-lane reductions
-//                      plus one exchange with lane ^ 32.
-//   P^T                exp2 of that in registers; the accumulator layout of S^T is already the B-operand layout of
-//                      the next product: register r is the k-step of keys kappa(r, 0), kappa(r, 1).
-//   O^T += V^T P^T     A = V^T: lane (d = lane % 32, g) supplies V[kappa(r, g)][32 db + d]: a 4-byte LDS read of
-//                      32 consecutive floats of one row per half-wavefront; no transposition anywhere.
+// A workgroup (4 wavefronts) computes 64 query rows of one head; two wavefronts share 32 rows and take a block of 32 keys each of every
+// tile of 64, their results meet in LDS at the end.  Operand layouts as in the 16-bit prefill kernels:
+//   S^T = K Q'^T     A = K rows (16-byte LDS reads), B = Q'^T (Q' = Q * scale * log2 e, parts kept in registers): a lane owns one
+//                    query (column lane % 32) and 16 keys (register r is key 8 (r / 4) + 4 g + r % 4)
+//   O^T += V^T P^T   registers 8 h .. 8 h + 7 of P^T are the B operand of 16 keys; A = V^T by transposing LDS reads of the same keys
+// A tile's values go global -> registers -> three planes of bf16 rows in LDS, so each is split once per workgroup.  A matrix instruction
+// hides about six vector instructions of its own wavefront or another's, no more, so they are dealt out between them, and the loop is a step of two halves:
+//   S(t + 1) = K Q', between its products the exponentials and parts of P(t) | barrier
+//   O += V(t) P(t), between its products K(t + 2) and V(t + 1) into LDS, K(t + 3) and V(t + 2) asked for | barrier
+//
+// What bounds it: the 48 matrix instructions of a 32 x 32 block at D = 64 (1536 cycles) and the clock the device keeps under them (about 2.0 GHz with
+// N(0,1) data), then the 360 vector instructions beside them, half of which split K and V.  Without those (results wrong) 4 x 8 x 1024, nothing masked,
+// takes 42 us instead of 55; without any 39.  At D > 64 a workgroup has its compute unit to itself (422 registers, 144 KiB of LDS).
+// Measured, forward, us, IEEE-f32 products (the kernel of 128 rows, or that of 32 for launches it was ahead on) / so: 4 x 8 x 1024 x 64 causal 50.4 /
+// 37.6, nothing masked 77.4 / 55.3, 8 x 12 x 2048 x 64 822 / 585, 4 x 12 x 2000 x 64 causal 243 / 166, 8 on 2 x 256 over 8192 keys 85 / 40; 4 x 8 x
+// 1024 x 128 causal 90 / 74, 8 x 12 x 2048 x 128 causal 876 / 780, 4 x 8 x 1024 x 80 causal 70 / 57; the causal mask as a tensor, 4 x 8 x 1024 x 64, with the pass over
+// it 60.1 / 43.8.  Its error against 64 bits is 0.5 - 0.6 of what it was (2-norm, 4 x 8 x 1024 x 64 3.4e-7 -> 2.0e-7, 8 x 12 x 2048 x 64 8.4e-7 -> 2.6e-7, 4 x 8 x 1024 x
+// 128 causal 2.3e-7 -> 1.3e-7): sums are rounded at their own size once per product of leading parts, the smaller products meet apart.
 //
 // A dense additive mask comes with one flag per block of 32 rows x 32 keys (mask_blocks.hip): blocks the mask hides
-// completely are skipped, blocks where it is zero run without it, the rest add its values to the scores.
-//
-// The matrix pipe is the bound by a wide margin (an instruction occupies it for 64 cycles and needs one register of
-// each operand), so the loop is plain: per key tile one barrier, the global -> LDS copies of the next tile (K and V,
-// two buffers each, 16 KiB tiles: 64 keys at D = 64, 32 at D = 128), scores, exact online softmax, second product.
-// The other wavefront of the SIMD covers the vector work.  LDS rows are unpadded with their 16-byte chunks
-// XOR-swizzled by the row number so that both read patterns touch every bank once.
+// completely are skipped, blocks where it is zero run without it, the rest add its values to the scores.  Where the mask's row limits are there
+// too (small launches) and all rows of the workgroup have one, those are the mask.
 #include <type_traits>
 
-#include "sdpa_mfma_common.h"
+#include "f32_split.h"
 
 namespace incin_rocm {
 
@@ -39,36 +39,42 @@ namespace incin_rocm {
 // combine kernel finishes - for launches with too few (batch, head, row block) items to fill the device over a long key axis.
 //
 // DC: the columns that are multiplied, D or fewer: the head dimensions are at most DC, and the products with the zeros beyond are
-// left out (the LDS rows keep the layout of D).  The matrix instructions bound the kernel: 4 x 12 heads x 2048 at 80 770 -> 609 us.
-template <int D, bool DENSE, bool SPLIT = false, int DC = D>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void sdpa_prefill_f32_kernel(SdpaParams p)
+// left out (the LDS rows keep the layout of D).
+template <int D, int DC, bool DENSE, bool SPLIT>
+__global__ __launch_bounds__(256, D == 64 ? 2 : 1)
+void sdpa_prefill_f32_kernel(SdpaParams p, int pairs)
 {
 #if defined(__HIP_DEVICE_COMPILE__)   // the body uses device-only types (buffer descriptors); the host pass needs only the stub
-    typedef F32Layout<D> L;
-    typedef float float4v __attribute__((ext_vector_type(4)));
-    constexpr int NJ = DC / 8;             // groups of four k-steps of the S^T product
-    constexpr int NDB = DC / 32;           // 32-wide blocks of the head dimension
-    constexpr int LPW = L::LOADS_PER_WAVE;
-    constexpr int KT = L::KT, NB = L::NB;
-
-    __shared__ __attribute__((aligned(1024))) char smem[4 * L::TILE_BYTES];   // K buffers 0, 1, V buffers 0, 1
+    constexpr int KT = 64, RW = 2, KW = 4 / RW, OWN = 32 * KW;      // keys per tile, wavefronts that share rows, blocks of 32 rows side by side, rows of the workgroup
+    constexpr int NSTEP = DC / 16, NDB = DC / 32;
+    constexpr int MAX_FLAGS = 1024;
+    constexpr float LOG2E = 1.4426950408889634f;
+    typedef SplitTile<D, DC, KT, 256> Tile;
+    typedef typename Tile::L L;
+    __shared__ __attribute__((aligned(1024))) char smem[3 * Tile::BYTES];      // K, V of even tiles, V of odd ones
+    __shared__ int s_vote[8];
+    __shared__ uint8_t s_flags[DENSE ? MAX_FLAGS : 1];
+    char* const kbuf = smem;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int own = wave % KW, rs = wave / KW;
     const int ql = lane & 31, g = lane >> 5;
     const int Sq = p.Sq, Skv = p.Skv;
 
     // ---- which (batch, head, query block): the work order of the 16-bit kernels (longest blocks first, an XCD keeps
     // the heads that share K/V) -----------------------------------------------------------------------------------
-    const int nqb = (Sq + PF_BM - 1) / PF_BM;
+    const int nqb = (Sq + OWN - 1) / OWN;
     const int total = gridDim.x;
-    const WorkItem wi = (total & 7) == 0 ? work_item_of_share(blockIdx.x & 7, blockIdx.x >> 3, total >> 3, p.interleave, p.G, nqb, p.deal_groups)
+    int item = blockIdx.x >> 3;
+    // (one round, two workgroups to a compute unit, blocks of different lengths: the second 32 of an XCD go in reverse, a long one with a short one)
+    if (pairs && ((item >> 5) & 1)) item = 32 + ((total >> 3) - 1 - item);
+    const WorkItem wi = (total & 7) == 0 ? work_item_of_share(blockIdx.x & 7, item, total >> 3, p.interleave, p.G, nqb, p.deal_groups)
                                          : work_item(blockIdx.x, p.interleave, p.G, nqb);
-    const int gq = wi.gq, qb = wi.qblk, bhkv = wi.bhkv;
+    const int gq = wi.gq, bhkv = wi.bhkv;
     const int hkv = bhkv % p.Hkv, b = bhkv / p.Hkv;
     const int hq = hkv * p.G + gq;
-    const int q0 = qb * PF_BM;
+    const int q0 = wi.qblk * OWN;
 
     const float* qp = (const float*)p.q + (int64_t)b * p.q_sb + (int64_t)hq * p.q_sh;
     const float* kp = (const float*)p.k + (int64_t)b * p.k_sb + (int64_t)hkv * p.k_sh;
@@ -83,207 +89,384 @@ void sdpa_prefill_f32_kernel(SdpaParams p)
     const int rows_b = p.q_lens ? clampi(p.q_lens[b], 0, Sq) : Sq;      // query rows at and beyond are padding
     if (q0 >= rows_b) return;                                           // (uniform: before any barrier)
     const int coff = Skv - Sq;
-    int j_end = kv_len;
-    const int my_i = q0 + wave * 32 + ql;
-    int lim_lane = kv_len, lim_wave_min = kv_len, lim_wave_max = kv_len;
+    const int my_i = q0 + own * 32 + ql;
+    // keys the workgroup walks, this lane's row sees, all rows of the wavefront see
+    int j_end = kv_len, lim_lane = kv_len, lim_wave_min = kv_len;
     if (p.causal) {
-        const int last_row = min(q0 + PF_BM - 1, rows_b - 1);
-        j_end = clampi(last_row + coff + 1, 0, kv_len);
+        j_end = clampi(min(q0 + OWN - 1, rows_b - 1) + coff + 1, 0, kv_len);
         lim_lane = clampi(my_i + coff + 1, 0, kv_len);
-        lim_wave_min = clampi(q0 + wave * 32 + coff + 1, 0, kv_len);
-        lim_wave_max = clampi(min(q0 + wave * 32 + 31, rows_b - 1) + coff + 1, 0, kv_len);
+        lim_wave_min = clampi(q0 + own * 32 + coff + 1, 0, kv_len);
     }
-    if (q0 + wave * 32 >= rows_b) lim_wave_min = lim_wave_max = 0;      // a wavefront of padding rows only keeps the barriers company
-    if (DENSE && p.mask_lims != nullptr) {
+    bool values = DENSE;      // the mask's values are looked at
+    if (DENSE && p.mask_lims != nullptr && p.lims_rows) {
         // a launch of the f32 split-KV kernel went before this one and computed the 128-row blocks whose mask rows are all n
         // zeros and then -inf from their limits (sdpa_decode_f32.hip, LIMS): such a block is done
-        __shared__ int s_ok[4];
-        const bool no_limit = my_i < rows_b && mask_lims_of(p, b, hq)[p.m_si ? my_i : 0] < 0;
-        const bool wave_ok = __builtin_amdgcn_ballot_w64(no_limit) == 0;
-        if (lane == 0) s_ok[wave] = wave_ok ? 1 : 0;
+        const int32_t* lims = mask_lims_of(p, b, hq);
+        const int blk0 = q0 / 128 * 128, i = min(blk0 + (tid & 127), min(blk0 + 127, Sq - 1));
+        const bool wave_ok = __builtin_amdgcn_ballot_w64(lims[p.m_si ? i : 0] < 0) == 0;
+        if (lane == 0) s_vote[wave] = wave_ok ? 1 : 0;
         __syncthreads();
-        if ((s_ok[0] & s_ok[1] & s_ok[2] & s_ok[3]) != 0) return;      // (uniform)
+        if ((s_vote[0] & s_vote[1] & s_vote[2] & s_vote[3]) != 0) return;      // (uniform)
+        __syncthreads();
+    } else if (DENSE && p.mask_lims != nullptr) {
+        int lim = my_i < rows_b ? mask_lims_of(p, b, hq)[p.m_si ? my_i : 0] : 0;
+        const bool ok = __builtin_amdgcn_ballot_w64(lim < 0) == 0;
+        lim = min(lim, lim_lane);
+        int hi = lim, lo = my_i < rows_b ? lim : 0x7fffffff;
+#pragma unroll
+        for (int off = 16; off >= 1; off >>= 1) {
+            hi = max(hi, __shfl_xor(hi, off, 64));
+            lo = min(lo, __shfl_xor(lo, off, 64));
+        }
+        if (lane == 0) {
+            s_vote[wave] = ok ? 1 : 0;
+            s_vote[4 + wave] = hi;
+        }
+        __syncthreads();
+        if ((s_vote[0] & s_vote[1] & s_vote[2] & s_vote[3]) != 0) {      // (uniform)
+            values = false;
+            lim_lane = lim;
+            lim_wave_min = min(__builtin_amdgcn_readfirstlane(lo), kv_len);
+            j_end = __builtin_amdgcn_readfirstlane(max(max(s_vote[4], s_vote[5]), max(s_vote[6], s_vote[7])));
+        }
+        __syncthreads();
     }
-    const int n_tiles = (j_end + KT - 1) / KT;
+    int n_tiles = (j_end + KT - 1) / KT;
     const int t_first = SPLIT ? min(split * (p.split_len / KT), n_tiles) : 0;
-    const int n_act = lim_wave_max > 0 ? (lim_wave_max + KT - 1) / KT : 0;      // tiles this wavefront computes
-
-    // ---- global -> LDS copy plan: wavefront-wide load ii = wave * LPW + c fills LDS bytes [ii * 1024, +1024) of a tile
-    int k_voff[LPW], v_voff[LPW];
+    if (DENSE && values) {
+        // the flags of a tile's four blocks (0 mixed, 1 all zero, 2 all -inf), two bits each; tiles at the end that the mask hides are left out
+        const int nkb32 = (Skv + 31) >> 5, nrb32 = (Sq + 31) >> 5;
+        const uint8_t* fl = mask_flags_of(p, b, hq) + (int64_t)(q0 >> 5) * nkb32;
+        const int second = (q0 >> 5) + 1 < nrb32 ? nkb32 : 0;
+        int last = -1;
+        for (int t = tid; t < n_tiles; t += 256) {
+            const bool both = 2 * t + 1 < nkb32;
+            const unsigned f = fl[2 * t] | (both ? fl[2 * t + 1] : 2u) << 2 | (unsigned)fl[second + 2 * t] << 4 | (both ? fl[second + 2 * t + 1] : 2u) << 6;
+            if (t < MAX_FLAGS) s_flags[t] = (uint8_t)f;
+            if (f != 0xaau) last = t;
+        }
 #pragma unroll
-    for (int c = 0; c < LPW; ++c) {
-        const int pos = (wave * LPW + c) * 64 + lane;
-        const int row = pos / L::CPR, slot = pos % L::CPR;
-        k_voff[c] = dma_chunk_offset(row, (int)p.k_ss * 4, slot ^ L::f(row), p.D * 4);
-        v_voff[c] = dma_chunk_offset(row, (int)p.v_ss * 4, slot ^ L::f(row), p.Dv * 4);
+        for (int off = 32; off >= 1; off >>= 1) last = max(last, __shfl_xor(last, off, 64));
+        if (lane == 0) s_vote[wave] = last;
+        __syncthreads();
+        n_tiles = __builtin_amdgcn_readfirstlane(max(max(s_vote[0], s_vote[1]), max(s_vote[2], s_vote[3]))) + 1;
+        __syncthreads();
     }
-    const int64_t k_tile_bytes = (int64_t)KT * p.k_ss * 4, v_tile_bytes = (int64_t)KT * p.v_ss * 4;
-    auto issue = [&](const float* base, int64_t tile_bytes, int64_t row_stride, int row_floats, int t, int buf, const int (&voff)[LPW]) __attribute__((always_inline)) {
-        // bytes to the end of the last row this workgroup may see: loads past that return 0 (rows past a batch
-        // entry's key count are never read)
-        int64_t rem = (int64_t)(j_end - t * KT - 1) * row_stride * 4 + row_floats * 4;
-        if (rem > 0x7fffffffLL) rem = 0x7fffffffLL;
-        const uint4v r = dma_descriptor((const char*)base + t * tile_bytes, (int)rem);
-        const unsigned dst = lds_address(smem) + buf * L::TILE_BYTES + wave * LPW * 1024;
-#pragma unroll
-        for (int c = 0; c < LPW; ++c) dma_copy16(r, dst + c * 1024, voff[c]);
+    auto flags_of = [&](int t) __attribute__((always_inline)) {
+        return !DENSE || !values ? 0x55 : t < MAX_FLAGS ? __builtin_amdgcn_readfirstlane((int)s_flags[t]) : 0;
     };
-    auto issue_kv = [&](int t) __attribute__((always_inline)) {
-        issue(kp, k_tile_bytes, p.k_ss, p.D, t, t & 1, k_voff);
-        issue(vp, v_tile_bytes, p.v_ss, p.Dv, t, 2 + (t & 1), v_voff);
+    // the first tile at or behind t in which any row of the workgroup sees a key, n_tiles if there is none
+    auto visible_from = [&](int t) __attribute__((always_inline)) {
+        if (DENSE && values)
+            while (t < n_tiles && flags_of(t) == 0xaa) ++t;
+        return t;
     };
 
-    // ---- LDS read addresses (bytes inside a tile buffer), kept to a few registers: the rest is one vector
-    // instruction per read, which costs nothing beside a 64-cycle matrix instruction ---------------------------------
-    // K operand: lane (ql, g) reads row 32 kb + ql, logical chunk 2 j + g, stored at chunk (2 j + g) ^ f(ql).  With
-    // f = f_hi | f_0 (bit 0 apart): byte address = [ql * ROWB + ((g ^ f_0) << 4) + (f_hi << 4)] ^ (j << 5); the
-    // three terms in brackets share no bits, and neither does j << 5 with the first two.
-    const int k_base = ql * L::ROWB + (((g ^ L::f(ql)) & 1) << 4) + ((L::f(ql) & 0xe) << 4);
-    auto k_addr = [&](int j) __attribute__((always_inline)) { return k_base ^ (j << 5); };
-    // V operand of k-step r, block db: row 8 (r / 4) + 4 g + r % 4 of the 32-key block, float 32 db + ql, i.e. logical
-    // chunk 8 db + ql / 4 at chunk slot (8 db + ql / 4) ^ f(row), f(row) = r % 4 | 4 (r / 4 % 2) | 8 g: the low three
-    // bits of the slot are (ql / 4) ^ c with c = r % 4 | 4 (r / 4 % 2), the rest is db ^ g.
-    int v_low[8], v_high[NDB];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) v_low[c] = 4 * g * L::ROWB + (((ql >> 2) ^ c) << 4) + (ql & 3) * 4;
-#pragma unroll
-    for (int db = 0; db < NDB; ++db) v_high[db] = (db ^ g) << 7;
-
-    // ---- Q'^T operand, resident in registers ----------------------------------------------------------------------
-    // (fetched 16 bytes per lane, eight lanes to a 128-byte run of a row, and brought into the operand layout through this
-    // wavefront's 4 KiB of the K buffer the first copies do not fill: nothing is copied there before the loop's first barrier)
-    float4v qreg[NJ];
+    // operand addresses: K row ql of a block, chunk 2 s + g; V transposed, column block db, half h of 16 rows
+    const int k_base = rs * 32 * L::ROWB + ql * L::ROWB + ((g ^ (L::fk(ql) & 1)) << 4) + ((L::fk(ql) & ~1) << 4);      // chunk 2 s + g: ^ (s << 5)
+    int v_addr[NDB][2];
     {
-        uint4v qraw[NJ / 4][4];
-        fetch_q_rows(qraw, qp, q0 + wave * 32, Sq, p.q_ss, p.D, lane);
-        stage_q_rows(qreg, qraw, smem + ((t_first + 1) & 1) * L::TILE_BYTES + wave * 4096, lane);
-        const float c2 = p.scale * 1.4426950408889634f;      // scores in log2 units
+        const int n = lane & 15, dh = (lane >> 4) & 1;
 #pragma unroll
-        for (int j = 0; j < NJ; ++j)
+        for (int db = 0; db < NDB; ++db)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) qreg[j][e] *= c2;
+            for (int h = 0; h < 2; ++h) {
+                const int r = 8 * h + 4 * g + (n >> 2), c = 4 * db + 2 * dh + ((n & 3) >> 1);
+                v_addr[db][h] = (rs * 32 + r) * L::ROWB + ((c ^ L::fv(r)) << 4) + (n & 1) * 8;
+            }
     }
     const float* mrow = nullptr;          // this lane's row of the dense mask
-    const uint8_t* mflags = nullptr;      // block flags of this wavefront's 32 rows: 0 mixed, 1 all zero, 2 all -inf
-    if (DENSE) {
-        mrow = (const float*)p.mask + (int64_t)b * p.m_sb + (int64_t)hq * p.m_sh + (int64_t)min(my_i, Sq - 1) * p.m_si;
-        mflags = mask_flags_of(p, b, hq) + (int64_t)((q0 >> 5) + wave) * ((Skv + 31) / 32);
-    }
+    if (DENSE) mrow = (const float*)p.mask + (int64_t)b * p.m_sb + (int64_t)hq * p.m_sh + (int64_t)min(my_i, Sq - 1) * p.m_si;
+    const bool m_vec = DENSE && p.m_sj == 1 && ((p.m_sb | p.m_sh | p.m_si) & 3) == 0 && (reinterpret_cast<uintptr_t>(p.mask) & 15u) == 0;
+    const int flag_shift = own * 4 + rs * 2;
 
     floatx16 o_acc[NDB];
+    float m_run = 0.0f, l_run = 0.0f;      // the reference the row's probabilities are taken against (log2 units), this lane's share of their sum
+    auto walk = [&](auto exact_) __attribute__((always_inline)) {
+        constexpr bool EXACT = decltype(exact_)::value;
+        Tile xk, xv;                     // values on their way into LDS
+        Split8 qreg[NSTEP];              // Q', resident
+        int t = visible_from(t_first), t1 = visible_from(t + 1), t2 = visible_from(t1 + 1);
+        // ---- Q' into operands, through the place of the second V tile; the first K and V tiles ----
+        {
+            Tile xq;
+            xq.fetch_any(qp, p.q_ss, p.D, Sq, q0, tid);
+            xk.fetch(kp, p.k_ss, p.D, j_end, t * KT, tid);
+            xv.fetch(vp, p.v_ss, p.Dv, j_end, t * KT, tid);
 #pragma unroll
-    for (int db = 0; db < NDB; ++db)
+            for (int i = 0; i < Tile::N; ++i) xq.x[i] *= p.scale * LOG2E;
+            xq.template put<EXACT, true>(smem + 2 * Tile::BYTES, tid);
+            xk.template put<EXACT, true>(kbuf, tid);
+            xv.template put<EXACT, false>(smem + Tile::BYTES, tid);
+        }
+        xk.fetch(kp, p.k_ss, p.D, j_end, t1 * KT, tid);
+        xv.fetch(vp, p.v_ss, p.Dv, j_end, t1 * KT, tid);
+        lds_barrier();
 #pragma unroll
-        for (int r = 0; r < 16; ++r) o_acc[db][r] = 0.0f;
-    float m_run = -INFINITY;      // running maximum (log2 units) of this lane's query, the same in lanes l and l ^ 32
-    float l_run = 0.0f;           // this lane's share of the running denominator
+        for (int s = 0; s < NSTEP; ++s) qreg[s] = Tile::rows_operand(smem + 2 * Tile::BYTES + ((k_base + (own - rs) * 32 * L::ROWB) ^ (s << 5)));
 
-    if (n_tiles > t_first) issue_kv(t_first);
-    for (int t = t_first; t < n_tiles; ++t) {
-        // K(t), V(t) have arrived for everyone, everyone is done with tile t - 1: its buffers take tile t + 1
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        if (t + 1 < n_tiles) issue_kv(t + 1);
-        if (t >= n_act) continue;
-        const char* kb_ = smem + (t & 1) * L::TILE_BYTES;
-        const char* vb_ = smem + (2 + (t & 1)) * L::TILE_BYTES;
+        [[maybe_unused]] float mv[16];      // dense mask values of this lane's 16 keys
+        [[maybe_unused]] auto fetch_mask = [&](int t) __attribute__((always_inline)) {
+            typedef float float4v __attribute__((ext_vector_type(4)));
+            if (t >= n_tiles || ((flags_of(t) >> flag_shift) & 3) != 0) return;
+            const int j0 = t * KT + rs * 32;
+            if (m_vec && j0 + 32 <= Skv) {
 #pragma unroll
-        for (int kb = 0; kb < NB; ++kb) {
-            const int j0 = t * KT + kb * 32;
-            if (j0 >= lim_wave_max) break;                    // (uniform) nothing of this block is visible to the wavefront
-            int flag = 1;
-            if (DENSE) {
-                flag = __builtin_amdgcn_readfirstlane((int)mflags[j0 >> 5]);
-                if (flag == 2) continue;                      // the mask hides the whole block from these rows
-            }
-            // dense mask values of this lane's 16 keys, fetched ahead of the product that hides their latency
-            float mv[16];
-            if (DENSE && flag == 0) {
+                for (int r4 = 0; r4 < 4; ++r4) {
+                    const float4v w = *(const float4v*)(mrow + j0 + 8 * r4 + 4 * g);
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int j = min(j0 + 8 * (r / 4) + 4 * g + (r % 4), Skv - 1);
-                    mv[r] = mrow[(int64_t)j * p.m_sj];
+                    for (int e = 0; e < 4; ++e) mv[4 * r4 + e] = w[e];
                 }
+            } else {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) mv[r] = mrow[(int64_t)min(j0 + 8 * (r / 4) + 4 * g + (r % 4), Skv - 1) * p.m_sj];
             }
-            // ---- scores: two chains over the halves of the head dimension -------------------------------------
-            floatx16 s0, s1;
+        };
+        // S^T = K Q'^T of the tile in kbuf, `between(i)` behind each of its 6 NSTEP instructions
+        auto scores = [&](floatx16& s, auto between) __attribute__((always_inline)) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) { s0[r] = 0.0f; s1[r] = 0.0f; }
+            for (int r = 0; r < 16; ++r) s[r] = 0.0f;
+            // (the five smaller products of all steps, then the leading ones: the sum is rounded at its own size NSTEP times, not 6 NSTEP)
+            Split8 a = Tile::rows_operand(kbuf + k_base);
+            uint4p lead[NSTEP];
 #pragma unroll
-            for (int j = 0; j < NJ / 2; ++j) {
-                const float4v ka = *(const float4v*)(kb_ + kb * 32 * L::ROWB + k_addr(j));
-                const float4v kc = *(const float4v*)(kb_ + kb * 32 * L::ROWB + k_addr(j + NJ / 2));
+            for (int i = 0; i < NSTEP; ++i) {
+                Split8 n = a;
+                if (i + 1 < NSTEP) n = Tile::rows_operand(kbuf + (k_base ^ ((i + 1) << 5)));
+                __builtin_amdgcn_sched_barrier(0);
+                lead[i] = a.h;
+                if (EXACT) s = mma_split<true>(a, qreg[i], s);
+                mma_split_term<EXACT, 0>(a, qreg[i], s); between(5 * i);
+                mma_split_term<EXACT, 1>(a, qreg[i], s); between(5 * i + 1);
+                mma_split_term<EXACT, 2>(a, qreg[i], s); between(5 * i + 2);
+                mma_split_term<EXACT, 3>(a, qreg[i], s); between(5 * i + 3);
+                mma_split_term<EXACT, 4>(a, qreg[i], s); between(5 * i + 4);
+                a = n;
+            }
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    s0 = __builtin_amdgcn_mfma_f32_32x32x2f32(ka[e], qreg[j][e], s0, 0, 0, 0);
-                    s1 = __builtin_amdgcn_mfma_f32_32x32x2f32(kc[e], qreg[j + NJ / 2][e], s1, 0, 0, 0);
+            for (int i = 0; i < NSTEP; ++i) {
+                a.h = lead[i];
+                if (!EXACT) mma_split_term<EXACT, 5>(a, qreg[i], s);
+                between(5 * NSTEP + i);
+            }
+        };
+        floatx16 s;
+        scores(s, [](int) {});
+        if (DENSE && values) fetch_mask(t);
+        lds_barrier();
+        if (t1 < n_tiles) xk.template put<EXACT, true>(kbuf, tid);
+        xk.fetch(kp, p.k_ss, p.D, j_end, t2 * KT, tid);
+#pragma unroll
+        for (int db = 0; db < NDB; ++db)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o_acc[db][r] = 0.0f;
+        m_run = 0.0f;
+        l_run = 0.0f;
+        float rise = -INFINITY;      // the reference moves where a block's maximum passes it by more than this: at the first key seen, then by 2^8
+        lds_barrier();
+        for (int even = 0; t < n_tiles; even ^= 1) {
+            const int j0 = t * KT + rs * 32;
+            if (DENSE && values) {
+                const int flag = (flags_of(t) >> flag_shift) & 3;
+                if (flag == 0) {
+                    asm volatile("");
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) s[r] = __builtin_fmaf(mv[r], LOG2E, s[r]);
+                } else if (flag == 2) {
+                    asm volatile("");
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) s[r] = -INFINITY;
                 }
-            }
-            floatx16 s;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) s[r] = s0[r] + s1[r];
-            if (DENSE && flag == 0) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) s[r] = __builtin_fmaf(mv[r], 1.4426950408889634f, s[r]);
             }
             if (j0 + 32 > lim_wave_min) {                     // (uniform) the block crosses a limit of this wavefront
+                asm volatile("");      // (a branch, not sixteen selects in every block)
                 const int rel = lim_lane - (j0 + 4 * g);
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
                     if (8 * (r / 4) + (r % 4) >= rel) s[r] = -INFINITY;
             }
-            // ---- online softmax ------------------------------------------------------------------------------------
+            // ---- online softmax: probabilities are taken against a reference that moves rarely (they stay <= 2^8) ----
             float tmax = s[0];
 #pragma unroll
             for (int r = 1; r < 16; ++r) tmax = fmaxf(tmax, s[r]);
-            tmax = xor32_max(tmax);
-            const float m_new = fmaxf(m_run, tmax);
-            const float m_use = (m_new == -INFINITY) ? 0.0f : m_new;
-            const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);       // exp2(-inf) = 0: nothing accumulated yet
-            m_run = m_new;
-            float rsum = 0.0f;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                s[r] = __builtin_amdgcn_exp2f(s[r] - m_use);
-                rsum += s[r];
-            }
-            l_run = l_run * alpha + rsum;
-            if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
+            if (__builtin_amdgcn_ballot_w64(tmax - m_run > rise) != 0) {
+                tmax = xor32_max(tmax);
+                const bool need = tmax - m_run > rise;
+                const float to = need ? tmax : m_run, alpha = rise == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m_run - to);      // (first key: nothing summed yet)
+                if (need) rise = PF_RESCALE_THRESHOLD;
+                m_run = to;
+                l_run *= alpha;
 #pragma unroll
                 for (int db = 0; db < NDB; ++db)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) o_acc[db][r] *= alpha;
             }
-            // ---- O^T += V^T P^T: k-step r takes keys kappa(r, 0), kappa(r, 1) ------------------------------------
-            const char* vblk = vb_ + kb * 32 * L::ROWB;
+            // ---- P^T and its parts, between the next tile's first products ----
+            Split8 pr[2];
+            SplitPair pair;
+            float e0 = 0.0f, e1 = 0.0f, bsum = 0.0f;
+            auto soft = [&](int k) __attribute__((always_inline)) {      // piece k of 24: three per two values
+                const int q = k / 3, part = k % 3, h = q / 4;
+                if (part == 0) {
+                    e0 = __builtin_amdgcn_exp2f(s[2 * q] - m_run);
+                    e1 = __builtin_amdgcn_exp2f(s[2 * q + 1] - m_run);
+                    return;
+                }
+                unsigned x = pr[h].h[q % 4], y = pr[h].m[q % 4], z = pr[h].l[q % 4];
+                if (part == 1) {
+                    bsum += e0;
+                    bsum += e1;
+                    pair.template step<EXACT, 0>(e0, e1, x, y, z);
+                } else {
+                    pair.template step<EXACT, 1>(e0, e1, x, y, z);
+                    pair.template step<EXACT, 2>(e0, e1, x, y, z);
+                }
+                pr[h].h[q % 4] = x;
+                pr[h].m[q % 4] = y;
+                pr[h].l[q % 4] = z;
+            };
+            floatx16 s1;
+            if (t1 < n_tiles) {
+                scores(s1, [&](int i) __attribute__((always_inline)) {
+                    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                float vv[NDB];
+                    for (int k = 24 * i / (6 * NSTEP); k < 24 * (i + 1) / (6 * NSTEP); ++k) soft(k);
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+            } else {
 #pragma unroll
-                for (int db = 0; db < NDB; ++db)
-                    vv[db] = *(const float*)(vblk + ((r / 8) * 16 + 8 * ((r / 4) % 2) + r % 4) * L::ROWB + v_low[(r % 4) | (4 * ((r / 4) % 2))] + v_high[db]);
-#pragma unroll
-                for (int db = 0; db < NDB; ++db) o_acc[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv[db], s[r], o_acc[db], 0, 0, 0);
+                for (int k = 0; k < 24; ++k) soft(k);
             }
+            l_run += bsum;
+            lds_barrier();
+            // ---- O^T += V^T P^T, between them the next tiles' values into LDS ----
+            const int t3 = visible_from(t2 + 1);
+            if (DENSE && values) fetch_mask(t1);
+            const char* const vcur = smem + (1 + even) * Tile::BYTES;
+            char* const vnext = smem + (2 - even) * Tile::BYTES;
+            typename Tile::State st;
+            constexpr int NM = 12 * NDB, NS = Tile::STEPS;
+            auto put = [&](int i) __attribute__((always_inline)) {      // behind matrix instruction i
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int k = 2 * NS * i / NM; k < 2 * NS * (i + 1) / NM; ++k) {
+                    if (k < NS) xk.template put_step<EXACT, true>(k, st, kbuf, tid);
+                    else xv.template put_step<EXACT, false>(k - NS, st, vnext, tid);
+                    if (k == NS - 1) xk.fetch(kp, p.k_ss, p.D, j_end, t3 * KT, tid);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            // (the five smaller products of a block meet in registers of their own before the sums so far take them: O is rounded at its own
+            // size three times per 32 keys instead of twelve)
+            Split8 a = Tile::cols_operand(vcur, v_addr[0][0], v_addr[0][1]);
+            floatx16 small;
+#pragma unroll
+            for (int i = 0; i < 2 * NDB; ++i) {
+                const int db = i / 2, h = i % 2, dn = (i + 1) / 2, hn = (i + 1) % 2;
+                Split8 n = a;
+                if (i + 1 < 2 * NDB) n = Tile::cols_operand(vcur + hn * 16 * L::ROWB, v_addr[dn][0], v_addr[dn][1]);
+                __builtin_amdgcn_sched_barrier(0);
+                if (h == 0) {
+                    if (db > 0) {
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) o_acc[db > 0 ? db - 1 : 0][r] += small[r];
+                    }
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) small[r] = 0.0f;
+                }
+                mma_split_term<EXACT, 0>(a, pr[h], small); put(6 * i);
+                mma_split_term<EXACT, 1>(a, pr[h], small); put(6 * i + 1);
+                mma_split_term<EXACT, 2>(a, pr[h], small); put(6 * i + 2);
+                mma_split_term<EXACT, 3>(a, pr[h], small); put(6 * i + 3);
+                mma_split_term<EXACT, 4>(a, pr[h], small); put(6 * i + 4);
+                mma_split_term<EXACT, 5>(a, pr[h], o_acc[db]); put(6 * i + 5);
+                a = n;
+            }
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o_acc[NDB - 1][r] += small[r];
+            xv.fetch(vp, p.v_ss, p.Dv, j_end, t2 * KT, tid);
+            lds_barrier();
+            s = s1;
+            t = t1;
+            t1 = t2;
+            t2 = t3;
         }
+        // something that is not finite?
+        float chk = l_run * 0.0f;
+#pragma unroll
+        for (int db = 0; db < NDB; ++db)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) chk = __builtin_fmaf(o_acc[db][r], 0.0f, chk);
+        const bool bad = __builtin_amdgcn_ballot_w64(chk != 0.0f) != 0;
+        if (lane == 0) s_vote[wave] = bad ? 1 : 0;
+        lds_barrier();
+        return (s_vote[0] | s_vote[1] | s_vote[2] | s_vote[3]) != 0;      // (uniform)
+    };
+    if (n_tiles > t_first) {
+        if (walk(std::integral_constant<bool, false>{})) {
+            lds_barrier();
+            walk(std::integral_constant<bool, true>{});
+        }
+    } else {
+#pragma unroll
+        for (int db = 0; db < NDB; ++db)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o_acc[db][r] = 0.0f;
     }
 
+    // ---- the two wavefronts that share rows: each keeps the column blocks db with db % 2 == rs, and has the other's of them added ----
+    constexpr int NKEEP = (NDB + 1) / 2;
+    float l_tot = xor32_sum(l_run);
+    {
+        // (the tiles are done with) [wavefront][column block it gives away][16][64], behind them m and l of each wavefront's rows
+        float* const give = (float*)smem;
+        float* const ml = give + 4 * NKEEP * 16 * 64;
+#pragma unroll
+        for (int db = 0; db < NDB; ++db)
+            if (db % 2 != rs) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) give[((wave * NKEEP + db / 2) * 16 + r) * 64 + lane] = o_acc[db][r];
+            }
+        if (g == 0) {
+            ml[(wave * 32 + ql) * 2] = m_run;
+            ml[(wave * 32 + ql) * 2 + 1] = l_tot;
+        }
+        lds_barrier();
+        const int other = wave ^ KW;
+        const float m2 = ml[(other * 32 + ql) * 2], l2 = ml[(other * 32 + ql) * 2 + 1];
+        // (a wavefront that saw no key has l = 0, and its reference says nothing)
+        const float top = l_tot == 0.0f ? m2 : l2 == 0.0f ? m_run : fmaxf(m_run, m2);
+        const float f1 = l_tot == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(m_run - top), f2 = l2 == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(m2 - top);
+        m_run = top;
+        l_tot = l_tot * f1 + l2 * f2;
+#pragma unroll
+        for (int k = 0; k < NKEEP; ++k) {
+            if (2 * k + rs >= NDB) break;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float mine = 2 * k + 1 < NDB && rs == 1 ? o_acc[2 * k + 1 < NDB ? 2 * k + 1 : 0][r] : o_acc[2 * k][r];
+                o_acc[k][r] = mine * f1 + give[((other * NKEEP + k) * 16 + r) * 64 + lane] * f2;
+            }
+        }
+        lds_barrier();      // (what follows stages rows in the same place)
+    }
+    // o_acc[k]: column block 2 k + rs
     // ---- normalise and store --------------------------------------------------------------------------------------
-    const float l_tot = xor32_sum(l_run);
     if constexpr (SPLIT) {
         // partial result of this split: unnormalised O, and (maximum, sum) in the natural-log units the combine kernel takes
         // for f32 storage; a row that saw no key in this split has the maximum -inf
+        typedef float float4v __attribute__((ext_vector_type(4)));
         if (my_i < rows_b) {
             const int64_t slot = (((int64_t)b * p.Hq + hq) * Sq + my_i) * p.num_splits + split;
             float* arow = p.ws_acc + slot * D + g * 4;
 #pragma unroll
-            for (int db = 0; db < NDB; ++db)
+            for (int k = 0; k < NKEEP; ++k)
 #pragma unroll
                 for (int r4 = 0; r4 < 4; ++r4) {
-                    float4v w = {o_acc[db][r4 * 4], o_acc[db][r4 * 4 + 1], o_acc[db][r4 * 4 + 2], o_acc[db][r4 * 4 + 3]};
-                    *(float4v*)(arow + db * 32 + r4 * 8) = w;
+                    float4v w = {o_acc[k][r4 * 4], o_acc[k][r4 * 4 + 1], o_acc[k][r4 * 4 + 2], o_acc[k][r4 * 4 + 3]};
+                    if (2 * k + rs < NDB) *(float4v*)(arow + (2 * k + rs) * 32 + r4 * 8) = w;
                 }
-            if (g == 0) {
+            if (g == 0 && rs == 0) {
                 p.ws_ml[slot * 2 + 0] = l_tot == 0.0f ? -INFINITY : m_run * 0.6931471805599453f;
                 p.ws_ml[slot * 2 + 1] = l_tot;
             }
@@ -291,46 +474,56 @@ void sdpa_prefill_f32_kernel(SdpaParams p)
         return;
     }
     const float inv = (l_tot == 0.0f) ? __builtin_nanf("") : 1.0f / l_tot;   // no visible key: NaN, as the reference
-    if (p.lse && g == 0 && my_i < rows_b)
+    if (p.lse && g == 0 && rs == 0 && my_i < rows_b)
         p.lse[((int64_t)b * p.Hq + hq) * Sq + my_i] = l_tot == 0.0f ? -INFINITY : (m_run + __builtin_log2f(l_tot)) * 0.6931471805599453f;
-    // through this wavefront's 4 KiB of the K buffer the last tile did not use (every wavefront is past the barrier of that
-    // tile, i.e. done with the tile before it, and nothing has been copied since)
-    store_o_rows_f32(o_acc, inv, smem + (n_tiles & 1) * L::TILE_BYTES + wave * 4096, op, q0 + wave * 32, rows_b, p.o_ss, p.Dv, lane);
+#pragma unroll
+    for (int k = 0; k < NKEEP; ++k) {
+        const floatx16 one[1] = {o_acc[k]};
+        const int c0 = (2 * k + rs) * 32;
+        if (c0 >= DC) break;
+        store_o_rows_f32(one, inv, smem + wave * 4096, op + c0, q0 + own * 32, rows_b, p.o_ss, p.Dv - c0, lane);
+    }
 #endif
 }
 
 hipError_t launch_sdpa_combine(const SdpaParams& p, int dtype, hipStream_t stream);
 
-template <int D, bool DENSE, int DC = D>
+template <int D, int DC, bool DENSE>
 static hipError_t launch_prefill_f32_t(const SdpaParams& p0, hipStream_t stream)
 {
+    constexpr int OWN = 64;
     SdpaParams p = p0;
-    const int nqb = (p.Sq + PF_BM - 1) / PF_BM;
+    const int nqb = (p.Sq + OWN - 1) / OWN;
     const int64_t total = (int64_t)nqb * p.Hq * p.B;
     if (total <= 0) return hipSuccess;
     if (total > 0x7fffffffLL) return hipErrorInvalidValue;
-    p.interleave = work_interleave(p.causal != 0 || p.mask != nullptr, 2 * device_cus() / 8, p.G, nqb, (total & 7) == 0 ? total >> 3 : total);
-    p.deal_groups = (total & 7) == 0 ? work_deal(p.interleave, p.G, nqb, total >> 3, p.causal != 0 || p.mask != nullptr) : 0;
+    const bool uneven = p.causal != 0 || p.mask != nullptr;
+    p.interleave = work_interleave(uneven, (D == 64 ? 2 : 1) * device_cus() / 8, p.G, nqb, (total & 7) == 0 ? total >> 3 : total);
+    p.deal_groups = (total & 7) == 0 ? work_deal(p.interleave, p.G, nqb, total >> 3, uneven) : 0;
+    const int pairs = D == 64 && uneven && (total & 7) == 0 && total > 256 && total <= 512 ? 1 : 0;
     if constexpr (!DENSE) {
         if (p.num_splits > 1) {          // split launch: partial results, then the split-KV kernels' combine pass
-            hipLaunchKernelGGL((sdpa_prefill_f32_kernel<D, false, true, DC>), dim3((unsigned)total, (unsigned)p.num_splits), dim3(256), 0, stream, p);
+            hipLaunchKernelGGL((sdpa_prefill_f32_kernel<D, DC, false, true>), dim3((unsigned)total, (unsigned)p.num_splits), dim3(256), 0, stream, p, 0);
             hipError_t e = hipGetLastError();
             return e != hipSuccess ? e : launch_sdpa_combine(p, 0, stream);
         }
     }
-    hipLaunchKernelGGL((sdpa_prefill_f32_kernel<D, DENSE, false, DC>), dim3((unsigned)total), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((sdpa_prefill_f32_kernel<D, DC, DENSE, false>), dim3((unsigned)total), dim3(256), 0, stream, p, pairs);
     return hipGetLastError();
+}
+template <int D, int DC> static hipError_t launch_prefill_f32_m(const SdpaParams& p, hipStream_t stream)
+{
+    return p.mask ? launch_prefill_f32_t<D, DC, true>(p, stream) : launch_prefill_f32_t<D, DC, false>(p, stream);
 }
 
 // Host has validated: f32, D and Dv <= 128 in whole 16-byte vectors (p.Dp = the instance: 64 or 128), finite scale, rows 16-byte aligned with unit last-dim stride, row
-// strides below 2^24 elements (tile offsets fit the 32-bit buffer offset); the dense mask, if any, has any strides.
+// strides of K and V below 2^22 elements (tile offsets fit the 32-bit buffer offset); the dense mask, if any, has any strides.
 hipError_t launch_sdpa_prefill_f32(const SdpaParams& p, hipStream_t stream)
 {
-    // up to head dimension 96 in the 128 layout: three quarters of the products (they bound the kernel)
-    if (p.Dp == 128 && p.D <= 96 && p.Dv <= 96)
-        return p.mask ? launch_prefill_f32_t<128, true, 96>(p, stream) : launch_prefill_f32_t<128, false, 96>(p, stream);
-    if (p.mask) return p.Dp == 128 ? launch_prefill_f32_t<128, true>(p, stream) : launch_prefill_f32_t<64, true>(p, stream);
-    return p.Dp == 128 ? launch_prefill_f32_t<128, false>(p, stream) : launch_prefill_f32_t<64, false>(p, stream);
+    if (p.Dp == 64) return launch_prefill_f32_m<64, 64>(p, stream);
+    // up to head dimension 96 in the 128 layout: three quarters of the products
+    if (p.D <= 96 && p.Dv <= 96) return launch_prefill_f32_m<128, 96>(p, stream);
+    return launch_prefill_f32_m<128, 128>(p, stream);
 }
 
 }  // namespace incin_rocm
