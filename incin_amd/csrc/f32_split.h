@@ -167,25 +167,31 @@ template <int D, int DC, int ROWS, int THREADS> struct SplitTile {
             }
         }
     }
-    // Piece k of STEPS: what is fetched goes into LDS eight by eight.  (s: state between pieces)
+    // Piece k of STEPS of splitting what is fetched; eight values are in `s` after twelve of them, and put_step stores them then.
     struct State { SplitPair pair; Split8 o; };
-    template <bool EXACT, bool BY_K> __device__ __forceinline__ void put_step(int k, State& s, char* tile, int tid)
+    template <bool EXACT> __device__ __forceinline__ void split_step(int k, State& s, Split8& o)
     {
         const int i = k / 12, q = k / 3 % 4, part = k % 3;
-        unsigned h = s.o.h[q], m = s.o.m[q], l = s.o.l[q];
+        unsigned h = o.h[q], m = o.m[q], l = o.l[q];
         if (part == 0) s.pair.template step<EXACT, 0>(x[i][2 * q], x[i][2 * q + 1], h, m, l);
         else if (part == 1) s.pair.template step<EXACT, 1>(x[i][2 * q], x[i][2 * q + 1], h, m, l);
         else s.pair.template step<EXACT, 2>(x[i][2 * q], x[i][2 * q + 1], h, m, l);
-        s.o.h[q] = h;
-        s.o.m[q] = m;
-        s.o.l[q] = l;
-        if (k % 12 == 11) {
-            const int pos = i * THREADS + tid, row = pos / CPR, c = pos % CPR;
-            char* at = tile + row * ROWB + ((c ^ (BY_K ? L::fk(row) : L::fv(row))) << 4);
-            *(uint4p*)at = s.o.h;
-            *(uint4p*)(at + PLANE) = s.o.m;
-            *(uint4p*)(at + 2 * PLANE) = s.o.l;
-        }
+        o.h[q] = h;
+        o.m[q] = m;
+        o.l[q] = l;
+    }
+    template <bool BY_K> static __device__ __forceinline__ void store(char* tile, const Split8& o, int tid, int i = 0)      // (eight i of the thread's)
+    {
+        const int pos = i * THREADS + tid, row = pos / CPR, c = pos % CPR;
+        char* at = tile + row * ROWB + ((c ^ (BY_K ? L::fk(row) : L::fv(row))) << 4);
+        *(uint4p*)at = o.h;
+        *(uint4p*)(at + PLANE) = o.m;
+        *(uint4p*)(at + 2 * PLANE) = o.l;
+    }
+    template <bool EXACT, bool BY_K> __device__ __forceinline__ void put_step(int k, State& s, char* tile, int tid)
+    {
+        split_step<EXACT>(k, s, s.o);
+        if (k % 12 == 11) store<BY_K>(tile, s.o, tid, k / 12);
     }
     template <bool EXACT, bool BY_K> __device__ __forceinline__ void put(char* tile, int tid)
     {

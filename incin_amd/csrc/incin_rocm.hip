@@ -1180,6 +1180,25 @@ static int bwd_f32_parts(const incin_rocm_sdpa_desc_t* d, int which)
     if (parts == 1 && !uneven && tiles >= 16 && (rounds == 1 ? tiles >= 32 : rounds == 2 && 4 * (n_kv + n_q) <= 3 * rounds * slots)) parts = 2;
     return parts;
 }
+// Whether an f32 call with head dimensions up to 64 goes through the kernel whose values are three bf16 parts (sdpa_bwd_f32_split.hip): up to
+// 1.5 times ahead wherever the launch fills the device, but an item owns 128 rows and a compute unit, so few or half empty ones are better off
+// with the kernel above.  Backward call, us, that one / this: 32 heads x 1024 causal 144 / 102, nothing masked 243 / 162; 96 x 2048 causal 1487 / 963, 96 x 512 133 /
+// 96, 96 x 128 27 / 21; 64 on 16 x 2048 causal 966 / 637.
+//   The longest item may take 2.4 times a compute unit's share of the whole (dK / dV: four products a tile, dQ: three): 8 x 2048 causal (2.3) 153 / 139, 64 on 16 x
+//   1024 causal (2.3) 292 / 278, 32 on 8 x 1024 (2.3) 269 / 275; but 8 x 1536 causal (3.0) 97 / 106, 4 x 2048 causal (4.6) 114 / 136, 64 on 16 x 512 causal (4.6) 95 / 137.
+//   Walks of up to 16 tiles: from 48 blocks of keys on, 16 x 384 37 / 35, 8 x 768 62 / 58, 8 x 1024 76 / 74, 24 x 256 28 / 27, 48 x 128 19.4 / 19.7; below, 16 x 256 20 / 27.
+//   More than a round of items: only where three quarters of the owned rows exist, 300 x 96 46.0 / 45.6, 400 x 200 158 / 125, but 512 x 64 37 / 48, 1000 x 65 106 / 111.
+static bool bwd_f32_splits_values(const incin_rocm_sdpa_desc_t* d)
+{
+    if (d->D > 64 || d->Dv > 64 || getenv("INCIN_ROCM_BWD_PARTS")) return false;      // (forced parts: the kernel that takes parts)
+    const int64_t cus = compute_units_of(d->device), G = d->Hq / d->Hkv;
+    const int64_t nkb = (d->Skv + 127) / 128, nqb = (d->Sq + 127) / 128, blocks = nkb * d->Hkv * d->B, q_blocks = nqb * d->Hq * d->B;
+    const int64_t walk = (d->Sq + 63) / 64 * G, walk_q = (d->Skv + 63) / 64;
+    if (blocks + q_blocks > cus && (4 * d->Skv < 3 * 128 * nkb || 4 * d->Sq < 3 * 128 * nqb)) return false;
+    if (walk <= 16 && walk_q <= 16 && blocks >= 48) return true;
+    const int64_t all = (blocks * walk * 4 + q_blocks * walk_q * 3) / (d->causal || d->add_mask ? 2 : 1), longest = std::max(walk * 4, walk_q * 3);
+    return 5 * longest * cus <= 12 * all;
+}
 // Matrix-core kernels: into how many workgroups the key tiles of a dQ block (which = 0) or the query tiles of a dK/dV block (which =
 // 1) are dealt; the sums meet in planes of the workspace and a pass adds them (sdpa_bwd.h).
 static int bwd_parts(const incin_rocm_sdpa_desc_t* d, int kind, int which)
@@ -1301,6 +1320,7 @@ int incin_rocm_sdpa_bwd(const incin_rocm_sdpa_bwd_desc_t* bd, void* stream)
     bp.parts_q = parts_q;
     bp.parts_kv = parts_kv;
     bp.share = kind == 2 ? bwd_f32_share(&bd->fwd) : 0;
+    bp.split = kind == 2 && bwd_f32_splits_values(&bd->fwd);
     if (plane_bytes) {
         const incin_rocm_sdpa_desc_t* d = &bd->fwd;
         char* at = (char*)bd->workspace + bwd_rows_bytes(d) + flag_bytes;

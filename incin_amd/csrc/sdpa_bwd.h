@@ -25,6 +25,7 @@ struct SdpaBwdParams {
     // order.  f32: part 0 writes the gradient's rows itself and part k > 0 plane k - 1, which the pass adds to the rows; 16-bit
     // storage: every part writes a plane, and the pass rounds their sum into the rows.
     int32_t parts_q, parts_kv;
+    int32_t split;                 // f32: the kernel whose values are three bf16 parts (sdpa_bwd_f32_split.hip) takes the call
     int32_t share;                 // f32: wavefronts of a workgroup that share a block's walk (1, 2 or 4)
     float* part_dq;                // workspace, f32: [parts_q - 1][B, Hq, Sq, D]
     float* part_dk;                // workspace, f32: [parts_kv - 1][B, Hkv, Skv, D]; 16-bit storage: [parts_kv][...]
@@ -76,6 +77,7 @@ hipError_t launch_sdpa_bwd_wide(const SdpaBwdParams& bp, int dtype, hipStream_t 
 hipError_t launch_sdpa_bwd_delta(const SdpaBwdParams& bp, int dtype, hipStream_t stream);
 hipError_t launch_sdpa_bwd_sum_planes(const SdpaBwdParams& bp, int dtype, hipStream_t stream);
 hipError_t launch_sdpa_bwd_f32(const SdpaBwdParams& bp, hipStream_t stream);
+hipError_t launch_sdpa_bwd_f32_split(const SdpaBwdParams& bp, hipStream_t stream);
 hipError_t launch_sdpa_bwd_generic(const SdpaBwdParams& bp, int dtype, hipStream_t stream);
 
 }  // namespace incin_rocm

@@ -7,7 +7,7 @@
 //   dV_j = sum_i P_ij dO_i      dK_j = s sum_i dS_ij Q_i      dQ_i = s sum_j dS_ij K_j
 //
 // No atomics (results are the same on every run), P and dP recomputed for both kinds of gradient - the plan of sdpa_bwd_mfma.hip
-// with the operand layouts of sdpa_prefill_f32.hip:
+// with operands of one register: lane (m = lane % 32, g = lane / 32) supplies row (column) m of A (B) at one of the two summed places.
 //   bwd_f32_delta_kernel   per query row, into the workspace: -L_i log2(e) and -D_i, the values both kinds of block start
 //                          their S and dP accumulators from
 //   bwd_f32_kernel         one launch of both: dK / dV blocks first, dQ blocks behind them
@@ -23,7 +23,8 @@
 // layer).  At D = 128 the resident rows and the accumulators of a wavefront exceed 256 registers: those instances run one
 // wavefront per SIMD.  The call, causal, against two kernels on two streams with four blocks of 32 side by side in a workgroup: 32
 // heads x 1024, D = 64 214 -> 143 us (106 TFLOP/s of 153 that a large matrix product reaches), 64 x 2048 1129 -> 970, 12 x 501 at 80
-// 159 -> 66, 24 x 79 44 -> 14.
+// 159 -> 66, 24 x 79 44 -> 14.  (Head dimensions up to 64 in launches that fill the device go to sdpa_bwd_f32_split.hip: the second of these
+// calls 99, the third 632; the row statistics are computed here for both.)
 #include <type_traits>
 
 #include "sdpa_bwd.h"
@@ -33,7 +34,7 @@ namespace incin_rocm {
 
 typedef float float4v __attribute__((ext_vector_type(4)));
 
-// The LDS tile layout of sdpa_prefill_f32.hip: NB blocks of 32 unpadded rows, 16-byte chunks XOR-swizzled by f(row).
+// LDS tiles: NB blocks of 32 unpadded rows, 16-byte chunks XOR-swizzled by f(row) (reads down rows and across them touch every bank once).
 template <int D, int NB> struct F32Tile {
     static constexpr int ROWB = D * 4, CPR = D / 4, ROWS = 32 * NB, TILE_BYTES = ROWS * ROWB;
     static constexpr int LPW = TILE_BYTES / 1024 / 4;
@@ -748,10 +749,6 @@ static hipError_t launch_bwd_f32_t(const SdpaBwdParams& bp0, hipStream_t stream)
     const int64_t total = (int64_t)nqb * p.Hq * p.B, n_dkv = (int64_t)nkb * p.Hkv * p.B * bp.parts_kv, n_dq = total * bp.parts_q;
     if (n_dkv + n_dq > 0x7fffffffLL) return hipErrorInvalidValue;
     if (n_dkv + n_dq == 0) return hipSuccess;
-    if (rows > 0) {
-        if (p.Dv <= 64) hipLaunchKernelGGL(bwd_f32_delta_kernel<16>, dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, stream, bp);
-        else hipLaunchKernelGGL(bwd_f32_delta_kernel<32>, dim3((unsigned)((rows + 7) / 8)), dim3(256), 0, stream, bp);
-    }
     p.interleave = work_interleave(p.causal != 0 || p.mask != nullptr, (D == 128 || RW == 4 ? 1 : 2) * device_cus() / 8, p.G, nqb, (total & 7) == 0 ? total >> 3 : total);
     p.deal_groups = (total & 7) == 0 ? work_deal(p.interleave, p.G, nqb, total >> 3, p.causal != 0 || p.mask != nullptr) : 0;
     auto launch = [&](int64_t blocks, int64_t n) { hipLaunchKernelGGL((bwd_f32_kernel<D, DC, RW, DENSE>), dim3((unsigned)blocks), dim3(256), 0, stream, bp, (int)n); };
@@ -781,6 +778,12 @@ template <int D, int DC, int RW> static hipError_t launch_bwd_f32_d(const SdpaBw
 }
 hipError_t launch_sdpa_bwd_f32(const SdpaBwdParams& bp, hipStream_t stream)
 {
+    const int64_t rows = (int64_t)bp.f.B * bp.f.Hq * bp.f.Sq;
+    if (rows > 0) {
+        if (bp.f.Dv <= 64) hipLaunchKernelGGL(bwd_f32_delta_kernel<16>, dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, stream, bp);
+        else hipLaunchKernelGGL(bwd_f32_delta_kernel<32>, dim3((unsigned)((rows + 7) / 8)), dim3(256), 0, stream, bp);
+    }
+    if (bp.split) return launch_sdpa_bwd_f32_split(bp, stream);
     if (bp.f.Dp == 64)
         return bp.share == 4 ? launch_bwd_f32_d<64, 64, 4>(bp, stream) : bp.share == 2 ? launch_bwd_f32_d<64, 64, 2>(bp, stream) : launch_bwd_f32_d<64, 64, 1>(bp, stream);
     // (up to head dimension 96 in the 128 layout: three quarters of the products)

@@ -261,7 +261,7 @@ int incin_rocm_sdpa_fwd_static(const incin_rocm_sdpa_desc_t* desc, void* stream)
  * O, lse and d_o rows are never read, their d_q rows are written as zero and they add nothing to d_k and d_v).
  * fwd.impl picks the kernels: AUTO = matrix-core kernels where they apply - D and Dv up to 128 in whole 16-byte vectors (zero-padded
  * into instances for 64 and 128; f16 / bf16 without a dense mask: up to 256); f16 / bf16 with a positive scale (above 128: any finite
- * scale), f32 (IEEE single-precision matrix instructions) with any finite
+ * scale), f32 (IEEE single-precision matrix instructions, or every value as three bf16 parts) with any finite
  * scale; both with 16-byte aligned rows, and a dense mask of non-negative strides of which 64 rows fit 32-bit byte offsets
  * - and generic f32-arithmetic kernels otherwise; GENERIC and MFMA (up to 128) pin one or the other.  A query row with no visible key (NaN in the forward) gets a zero gradient and
  * contributes nothing to d_k and d_v, where the reference's tape would spread NaN over the whole head.

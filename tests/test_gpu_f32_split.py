@@ -72,3 +72,98 @@ def test_error_against_64_bits(gpu, S, D, causal):
     ref = (p / p.sum(-1, keepdims=True)) @ v64
     got = host.sdpa(q, k, v, capi.F32, causal=causal, impl=capi.IMPL_MFMA)
     assert np.linalg.norm(got - ref) / np.linalg.norm(ref) < 2.5e-7
+
+
+# ---- backward -----------------------------------------------------------------------------------------------------------
+
+BWD = [
+    # B, Hq, Hkv, Sq, Skv, D, Dv, causal, lens, mask: launches that the split kernel takes, with the edges of its tiles (64 rows) and blocks (128)
+    (3, 16, 16, 129, 127, 64, 64, False, None, None),
+    (4, 12, 12, 128, 193, 64, 32, True, None, None),
+    (2, 24, 24, 200, 256, 40, 64, True, None, None),
+    (4, 16, 16, 100, 100, 4, 4, True, (100, 65, 64, 1), None),
+    (4, 24, 12, 194, 194, 64, 64, True, (194, 1, 0, 129), None),
+    (50, 1, 1, 33, 31, 64, 64, False, None, None),
+    (2, 24, 24, 150, 150, 64, 64, False, None, "bias"),
+    (3, 16, 16, 129, 200, 64, 64, False, None, "window"),
+    (2, 32, 16, 160, 161, 64, 64, False, None, "rows"),
+]
+
+
+def bwd_case(shape, seed=3):
+    B, Hq, Hkv, Sq, Skv, D, Dv, causal, lens, mk = shape
+    r = np.random.Generator(np.random.PCG64(seed))
+    q, k, v, go = (r.standard_normal(s, dtype=np.float32) for s in ((B, Hq, Sq, D), (B, Hkv, Skv, D), (B, Hkv, Skv, Dv), (B, Hq, Sq, Dv)))
+    far = (np.arange(Sq)[:, None] + Skv - Sq - np.arange(Skv)[None]).astype(np.float32)
+    mask = None
+    if mk == "bias":
+        mask = np.where(far >= 0, -far[None] * 0.5 ** np.arange(1, Hq + 1, dtype=np.float32)[:, None, None], -np.inf)[None]
+    elif mk == "window":
+        mask = np.where(np.abs(far) < 40, 0.0, -np.inf)[None, None]
+    elif mk == "rows":
+        mask = r.standard_normal((1, 1, 1, Skv))
+    return q, k, v, go, None if mask is None else mask.astype(np.float32), None if lens is None else np.asarray(lens, np.int32)
+
+
+def f64_gradients(q, k, v, go, causal, mask, lens):
+    B, Hq, Sq, D = q.shape
+    Hkv, Skv = k.shape[1:3]
+    G = Hq // Hkv
+    q, k, v, go = (x.astype(np.float64) for x in (q, k, v, go))
+    k, v = (np.repeat(x, G, 1) for x in (k, v))
+    s = q @ k.transpose(0, 1, 3, 2) / np.sqrt(D)
+    if mask is not None:
+        s = s + mask
+    if causal:
+        s = np.where(np.arange(Skv)[None] > np.arange(Sq)[:, None] + Skv - Sq, -np.inf, s)
+    if lens is not None:
+        s = np.where(np.arange(Skv) >= lens[:, None, None, None], -np.inf, s)
+    m = s.max(-1, keepdims=True)
+    p = np.exp(s - np.where(np.isinf(m), 0, m))
+    p = p / np.maximum(p.sum(-1, keepdims=True), 1e-300)
+    o = p @ v
+    ds = p * (go @ v.transpose(0, 1, 3, 2) - (go * o).sum(-1, keepdims=True))
+    per = lambda x: x.reshape(B, Hkv, G, Skv, -1).sum(2)
+    return ds @ k / np.sqrt(D), per(ds.transpose(0, 1, 3, 2) @ q / np.sqrt(D)), per(p.transpose(0, 1, 3, 2) @ go)
+
+
+@pytest.mark.parametrize("shape", BWD, ids=lambda s: "x".join(map(str, s[:7])) + ("" if s[9] is None else s[9]))
+def test_backward_tile_edges(gpu, shape, monkeypatch):
+    """Gradients at the edges of tiles and blocks, key counts down to none, grouped queries, masks as tensors: against 64 bits at 1e-5 of the largest
+    gradient, and never further off (2-norm, all three together, 2 % for ties) than the kernel of IEEE-f32 products, which forced parts call."""
+    q, k, v, go, mask, lens = bwd_case(shape)
+    kw = dict(causal=shape[7], kv_lens=lens, mask=mask)
+    ref = f64_gradients(q, k, v, go, shape[7], mask, lens)
+    _, *got = host.sdpa_backward(q, k, v, go, capi.F32, **kw)
+    monkeypatch.setenv("INCIN_ROCM_BWD_PARTS", "1")
+    _, *ieee = host.sdpa_backward(q, k, v, go, capi.F32, **kw)
+    assert any(not np.array_equal(a, b) for a, b in zip(got, ieee)), "the same kernel"
+    off = [0.0, 0.0]
+    for name, a, b, r in zip(("dq", "dk", "dv"), got, ieee, ref):
+        assert np.max(np.abs(a - r)) <= 1e-5 * max(np.max(np.abs(r)), 1e-3), name
+        off[0] += np.sum((a - r) ** 2) / np.sum(r ** 2)
+        off[1] += np.sum((b - r) ** 2) / np.sum(r ** 2)
+    assert off[0] <= 1.04 * off[1]
+
+
+def test_backward_values_that_are_not_finite(gpu, monkeypatch):
+    """An infinite value of dO and a NaN in K reach what they reach in the kernel of IEEE-f32 products, and a dO whose first bf16 part would be
+    infinite stays finite."""
+    shape = (3, 16, 16, 129, 150, 64, 64, False, None, None)
+    q, k, v, go, _, _ = bwd_case(shape)
+    v[2, 0, :, 0] *= 0.01      # (so that dO V and dO O do not overflow where dO is the largest finite value)
+    for t, at, x in ((go, (0, 3, 128, 5), np.inf), (k, (1, 2, 149, 0), np.nan), (go, (2, 0, 0, 0), np.finfo(np.float32).max)):
+        was = t[at]
+        t[at] = x
+        with np.errstate(invalid="ignore", over="ignore"):
+            _, *got = host.sdpa_backward(q, k, v, go, capi.F32)
+            monkeypatch.setenv("INCIN_ROCM_BWD_PARTS", "1")
+            _, *ieee = host.sdpa_backward(q, k, v, go, capi.F32)
+            monkeypatch.delenv("INCIN_ROCM_BWD_PARTS")
+        t[at] = was
+        for name, a, b in zip(("dq", "dk", "dv"), got, ieee):
+            assert np.array_equal(np.isfinite(a), np.isfinite(b)) and np.array_equal(np.isnan(a), np.isnan(b)), (name, x)
+            for h in np.ndindex(a.shape[:2]):      # 1e-5 of a head's largest gradient, as above
+                fin = np.isfinite(b[h])
+                if fin.any():
+                    assert np.max(np.abs(a[h][fin] - b[h][fin])) <= 1e-5 * max(np.max(np.abs(b[h][fin])), 1), (name, x, h)
