@@ -16,6 +16,7 @@
 //   sdpa_bwd_dkv_kernel     the same with the roles swapped: a pair of wavefronts owns 32 keys (K and V rows resident),
 //                           Q / dO tiles of the group's query heads stream through LDS; S = Q K'^T and dP = dO V^T have a
 //                           lane-owns-a-key layout, the B-operand layout of dV^T += dO^T P and dK^T += Q^T dS
+#include <algorithm>
 #include <type_traits>
 
 #include "sdpa_bwd.h"
@@ -448,6 +449,41 @@ void sdpa_bwd_dq_kernel(SdpaBwdParams bp)
 
 // ---- dK, dV ---------------------------------------------------------------------------------------------------------------
 constexpr int BWD_KEYS = 128;      // keys per workgroup of the dK/dV kernel
+
+// Which key block of which (batch, KV head) pair a workgroup of the dK/dV kernels takes.  Workgroups reach the 8 XCDs round-robin by
+// id, and an XCD's reach its compute units in the same way.  All key blocks of a pair read the same Q and dO rows, so with a
+// multiple of 8 pairs a pair is given to one XCD (pair h to XCD h % 8).  The list runs over groups of F pairs (the last group takes what is
+// left), in a group over the key blocks, the one with the most visible queries (the first, under a causal mask) first, for each of them the group's pairs.
+struct KeyItem { int kblk, bhkv; };
+__device__ __forceinline__ KeyItem key_item(int id, int pairs, int nkb, int F)
+{
+    const bool by_xcd = (pairs & 7) == 0;
+    const int slot = by_xcd ? id >> 3 : id, per = by_xcd ? pairs >> 3 : pairs;
+    const int groups = max(per / F, 1), grp = min(slot / (F * nkb), groups - 1);
+    const int size = grp == groups - 1 ? per - grp * F : F, r = slot - grp * F * nkb;
+    const int pair = grp * F + r % size;
+    return {r / size, by_xcd ? pair * 8 + (id & 7) : pair};
+}
+// F for a launch (per_cu: workgroups on a compute unit).  Pair after pair (F = 1) starts every pair's longest walk while the pair
+// before ends on its shortest, ends the launch on a ragged round, and, where the key blocks of a pair divide the 32 compute units of an XCD, gives
+// one compute unit the first blocks of all pairs and another the last.  So F pairs that fill a round or two together; more lose a pair's
+// rows from the XCD's L2.  Without a multiple of 8 pairs F is one of 8, so that
+// what an XCD gets is not the same ranks of every pair.  Backward call, us, F = 1 / so: D = 128, causal, 8 x 16
+// heads x 4096 1886 / 1864 (all 16 pairs of an XCD 1932), x 2048 562 / 533, x 1024 197 / 176, x 512 82 / 72, 16 x 32 x 512 292 / 275, 4 x 32 on 8 x 2048 604 / 485, 1 x 20 x 4096
+// 475 / 353, 3 x 12 x 1500 149 / 118; D = 64, causal, 8 x 16 x 4096 970 / 926, x 1024 95 / 83, 8 x 32 x 512 68 / 62; D = 96, 12 x 16 x 900 186 / 168.
+// Key counts under no causal mask: the blocks behind a count are done at once, and the compute units that drew only those took no others - at D
+// = 64 three walks shared one of four compute units: 32 x 12 x 512, 128 keys each 75 / 58, 61 - 300 80 / 71, 61 - 512 89.8 / 88.3; D = 128, 61 - 512 232 / 213.
+// With key counts the walks differ between pairs as well, and the paired kernel's large ones are worse off with pairs that L2 does not hold: a round
+// of them (8 x 32 on 8 x 2048, 256 - 2048 keys 1079 / 1068, four pairs 1239; padded, causal, 8 x 16 x 4096 948 / 950, four 1053; x 1024 137 / 130).
+inline int64_t key_groups(int64_t pairs, int64_t nkb, int64_t cus, int64_t per_cu, bool narrow, bool uneven, bool counts)
+{
+    if (!uneven && !counts) return 1;
+    const int64_t slots = per_cu * (pairs % 8 ? cus : cus / 8);
+    auto rounds = [&](int64_t n) { return (n * slots + nkb - 1) / nkb; };      // pairs that fill n rounds
+    if (pairs % 8) return (rounds(uneven && (narrow || !counts) ? 2 : 1) + 7) / 8 * 8;
+    if (narrow) return uneven ? rounds(2) : 8;
+    return counts ? rounds(1) : std::max(rounds(1), (int64_t)4);
+}
 constexpr int BWD_RING = 4;        // matrix operands in flight from LDS (reads run this many matrix instructions ahead)
 
 // A wavefront that has a SIMD to itself pays for every instruction it issues on top of its matrix instructions (nothing
@@ -501,21 +537,8 @@ void sdpa_bwd_dkv_kernel(SdpaBwdParams bp)
     const int ql = lane & 31, g = lane >> 5;
     const int Sq = p.Sq, Skv = p.Skv;
     const int nkb = (Skv + BWD_KEYS - 1) / BWD_KEYS;
-    // Workgroups reach the 8 XCDs round-robin by id.  All key blocks of a (batch, KV head) pair read the same Q and dO
-    // rows, so a pair is given to one XCD (pair h to XCD h % 8) and its key blocks run there side by side, the
-    // block with the most visible queries (the first, under a causal mask) first.
-    int kblk, bhkv;
-    {
-        const int pairs = p.B * p.Hkv;
-        if ((pairs & 7) == 0) {
-            const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-            kblk = slot % nkb;
-            bhkv = (slot / nkb) * 8 + xcd;
-        } else {
-            kblk = blockIdx.x % nkb;
-            bhkv = blockIdx.x / nkb;
-        }
-    }
+    const KeyItem ki = key_item(blockIdx.x, p.B * p.Hkv, nkb, p.interleave);
+    const int kblk = ki.kblk, bhkv = ki.bhkv;
     const int hkv = bhkv % p.Hkv, b = bhkv / p.Hkv;
     const int j0 = kblk * BWD_KEYS;
     const int my_j = j0 + kb * 32 + ql;                // this lane's key
@@ -964,15 +987,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 3
     const int ql = lane & 31, g = lane >> 5;
     const int Sq = p.Sq, Skv = p.Skv;
     const int nkb = (Skv + BWD_KEYS - 1) / BWD_KEYS;
-    int kblk, bhkv;      // (a pair's key blocks on one XCD, the one with the most visible queries first: see sdpa_bwd_dkv_kernel)
-    if (((p.B * p.Hkv) & 7) == 0) {
-        const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-        kblk = slot % nkb;
-        bhkv = (slot / nkb) * 8 + xcd;
-    } else {
-        kblk = blockIdx.x % nkb;
-        bhkv = blockIdx.x / nkb;
-    }
+    const KeyItem ki = key_item(blockIdx.x, p.B * p.Hkv, nkb, p.interleave);
+    const int kblk = ki.kblk, bhkv = ki.bhkv;
     const int hkv = bhkv % p.Hkv, b = bhkv / p.Hkv;
     const int j0 = kblk * BWD_KEYS, wave_j0 = j0 + wave * 32, my_j = wave_j0 + ql;
 
@@ -1015,7 +1031,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 3
 
     // this lane's key: K row (scaled into log2 units) and V row as B operands, through 4 KiB per wavefront of the other stage
     vec8 kreg[NSTEP], vreg[NSTEP];
-    {
+    if (n_lo < n_hi) {      // (a block behind the key count has zeros to write and nothing to read)
         char* stage = smem + ((n_lo + 1) & 1) * STAGE + wave * 4096;
         static_assert(STAGE >= 4 * 4096, "a 4 KiB staging area per wavefront");
         uint4v kraw[NQH][4], vraw[NQH][4];
@@ -1241,10 +1257,12 @@ static hipError_t launch_bwd_t(const SdpaBwdParams& bp, hipStream_t stream)
     if (with_dkv) {
         const unsigned parts = bp.parts_kv > 1 ? (unsigned)bp.parts_kv : 1u;
         const dim3 grid((unsigned)((int64_t)nkb * p.Hkv * p.B), parts);
-        if (narrow && D == 64) hipLaunchKernelGGL((sdpa_bwd_dkv_narrow_kernel<T, 64, 64>), grid, dim3(256), 0, stream, bp);
-        else if (narrow) hipLaunchKernelGGL((sdpa_bwd_dkv_narrow_kernel<T, 128, 96>), grid, dim3(256), 0, stream, bp);
-        else if (DENSE && p.mask_chunks) hipLaunchKernelGGL((sdpa_bwd_dkv_kernel<T, D, DENSE ? 2 : 0>), grid, dim3(512), 0, stream, bp);
-        else hipLaunchKernelGGL((sdpa_bwd_dkv_kernel<T, D, DENSE ? 1 : 0>), grid, dim3(512), 0, stream, bp);
+        SdpaBwdParams bk = bp;
+        bk.f.interleave = (int)key_groups((int64_t)p.B * p.Hkv, nkb, cus, narrow ? (D == 64 ? 3 : 2) : 1, narrow, p.causal || DENSE, p.kv_lens != nullptr);
+        if (narrow && D == 64) hipLaunchKernelGGL((sdpa_bwd_dkv_narrow_kernel<T, 64, 64>), grid, dim3(256), 0, stream, bk);
+        else if (narrow) hipLaunchKernelGGL((sdpa_bwd_dkv_narrow_kernel<T, 128, 96>), grid, dim3(256), 0, stream, bk);
+        else if (DENSE && p.mask_chunks) hipLaunchKernelGGL((sdpa_bwd_dkv_kernel<T, D, DENSE ? 2 : 0>), grid, dim3(512), 0, stream, bk);
+        else hipLaunchKernelGGL((sdpa_bwd_dkv_kernel<T, D, DENSE ? 1 : 0>), grid, dim3(512), 0, stream, bk);
         if (parts > 1) sum_planes<T>(bp, stream);
     }
     if (forked) launch_dq(side.stream());
