@@ -502,6 +502,7 @@ void fill_params(const incin_rocm_sdpa_desc_t* d, const Plan& plan, SdpaParams* 
     p->scale = d->scale;
     p->causal = d->causal ? 1 : 0;
     p->interleave = 1;
+    p->groups = 1;
     p->deal_groups = 0;
     p->num_splits = plan.splits;
     p->split_len = plan.split_len;

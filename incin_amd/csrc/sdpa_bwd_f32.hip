@@ -174,8 +174,7 @@ __device__ __forceinline__ void bwd_f32_dq_body(const SdpaBwdParams& bp, char* s
     // (the parts of a block one behind the other, the blocks in the order of the work list)
     const bool eighths = (total & 7) == 0;
     const int part = eighths ? (id >> 3) % parts : id % parts;
-    const WorkItem wi = eighths ? work_item_of_share(id & 7, (id >> 3) / parts, total >> 3, p.interleave, p.G, nqb, p.deal_groups)
-                                : work_item(id / parts, p.interleave, p.G, nqb);
+    const WorkItem wi = work_item_of(p, eighths ? (id >> 3) / parts * 8 + (id & 7) : id / parts, total, nqb);
     const int hkv = wi.bhkv % p.Hkv, b = wi.bhkv / p.Hkv;
     const int hq = hkv * p.G + wi.gq;
     const int q0 = wi.qblk * OWN;
@@ -749,8 +748,7 @@ static hipError_t launch_bwd_f32_t(const SdpaBwdParams& bp0, hipStream_t stream)
     const int64_t total = (int64_t)nqb * p.Hq * p.B, n_dkv = (int64_t)nkb * p.Hkv * p.B * bp.parts_kv, n_dq = total * bp.parts_q;
     if (n_dkv + n_dq > 0x7fffffffLL) return hipErrorInvalidValue;
     if (n_dkv + n_dq == 0) return hipSuccess;
-    p.interleave = work_interleave(p.causal != 0 || p.mask != nullptr, (D == 128 || RW == 4 ? 1 : 2) * device_cus() / 8, p.G, nqb, (total & 7) == 0 ? total >> 3 : total);
-    p.deal_groups = (total & 7) == 0 ? work_deal(p.interleave, p.G, nqb, total >> 3, p.causal != 0 || p.mask != nullptr) : 0;
+    work_order(p, D == 128 || RW == 4 ? 1 : 2, nqb);
     auto launch = [&](int64_t blocks, int64_t n) { hipLaunchKernelGGL((bwd_f32_kernel<D, DC, RW, DENSE>), dim3((unsigned)blocks), dim3(256), 0, stream, bp, (int)n); };
     if (n_dkv + n_dq <= max_blocks(256)) launch(n_dkv + n_dq, n_dkv);
     else {

@@ -68,7 +68,7 @@ __device__ __forceinline__ void bwd_f32_split_body(const SdpaBwdParams& bp, char
         b = bhkv / p.Hkv;
     } else {
         const int nqb = (Sq + BS_OWN - 1) / BS_OWN, total = nqb * p.Hq * p.B;
-        const WorkItem wi = (total & 7) == 0 ? work_item_of_share(id & 7, id >> 3, total >> 3, p.interleave, p.G, nqb, p.deal_groups) : work_item(id, p.interleave, p.G, nqb);
+        const WorkItem wi = work_item_of(p, id, total, nqb);
         hkv = wi.bhkv % p.Hkv;
         b = wi.bhkv / p.Hkv;
         hq = hkv * p.G + wi.gq;
@@ -450,9 +450,7 @@ hipError_t launch_sdpa_bwd_f32_split(const SdpaBwdParams& bp0, hipStream_t strea
     SdpaParams& p = bp.f;
     const int nqb = (p.Sq + BS_OWN - 1) / BS_OWN, nkb = (p.Skv + BS_OWN - 1) / BS_OWN;
     const int64_t n_dq = (int64_t)nqb * p.Hq * p.B, n_dkv = (int64_t)nkb * p.Hkv * p.B;
-    const bool uneven = p.causal != 0 || p.mask != nullptr;
-    p.interleave = work_interleave(uneven, device_cus() / 8, p.G, nqb, (n_dq & 7) == 0 ? n_dq >> 3 : n_dq);
-    p.deal_groups = (n_dq & 7) == 0 ? work_deal(p.interleave, p.G, nqb, n_dq >> 3, uneven) : 0;
+    work_order(p, 1, nqb);
     auto launch = [&](int64_t blocks, int64_t n) {
         if (p.mask) hipLaunchKernelGGL(bwd_f32_split_kernel<true>, dim3((unsigned)blocks), dim3(BS_THREADS), 0, stream, bp, (int)n);
         else hipLaunchKernelGGL(bwd_f32_split_kernel<false>, dim3((unsigned)blocks), dim3(BS_THREADS), 0, stream, bp, (int)n);

@@ -155,10 +155,9 @@ void sdpa_bwd_dq_kernel(SdpaBwdParams bp)
     const int ql = lane & 31, g = lane >> 5;
     const int Sq = p.Sq, Skv = p.Skv;
     const int nqb = (Sq + PF_BM - 1) / PF_BM;
-    // the forward's work order: an eighth of the list per XCD, query blocks longest-first, heads interleaved
+    // the forward's work order: query blocks longest-first, heads interleaved
     const int total = gridDim.x;
-    const WorkItem wi = (total & 7) == 0 ? work_item_of_share(blockIdx.x & 7, blockIdx.x >> 3, total >> 3, p.interleave, p.G, nqb, p.deal_groups)
-                                         : work_item(blockIdx.x, p.interleave, p.G, nqb);
+    const WorkItem wi = work_item_of(p, blockIdx.x, total, nqb);
     const int gq = wi.gq, qb = wi.qblk, bhkv = wi.bhkv;
     const int hkv = bhkv % p.Hkv, b = bhkv / p.Hkv;
     const int hq = hkv * p.G + gq;
@@ -455,14 +454,20 @@ constexpr int BWD_KEYS = 128;      // keys per workgroup of the dK/dV kernel
 // multiple of 8 pairs a pair is given to one XCD (pair h to XCD h % 8).  The list runs over groups of F pairs (the last group takes what is
 // left), in a group over the key blocks, the one with the most visible queries (the first, under a causal mask) first, for each of them the group's pairs.
 struct KeyItem { int kblk, bhkv; };
-__device__ __forceinline__ KeyItem key_item(int id, int pairs, int nkb, int F)
+__device__ __forceinline__ KeyItem key_item(const SdpaParams& p, unsigned id, unsigned nkb)
 {
+    const unsigned F = p.interleave, last = p.groups - 1;
+    unsigned pairs = (unsigned)p.B * p.Hkv;
     const bool by_xcd = (pairs & 7) == 0;
-    const int slot = by_xcd ? id >> 3 : id, per = by_xcd ? pairs >> 3 : pairs;
-    const int groups = max(per / F, 1), grp = min(slot / (F * nkb), groups - 1);
-    const int size = grp == groups - 1 ? per - grp * F : F, r = slot - grp * F * nkb;
-    const int pair = grp * F + r % size;
-    return {r / size, by_xcd ? pair * 8 + (id & 7) : pair};
+    const unsigned xcd = id & 7;
+    if (by_xcd) {
+        id >>= 3;
+        pairs >>= 3;
+    }
+    unsigned grp = 0;
+    if (last > 0) grp = min(id / (F * nkb), last);
+    const unsigned size = grp == last ? pairs - grp * F : F, r = id - grp * F * nkb, kblk = r / size, pair = grp * F + r - kblk * size;
+    return {(int)kblk, (int)(by_xcd ? pair * 8 + xcd : pair)};
 }
 // F for a launch (per_cu: workgroups on a compute unit).  Pair after pair (F = 1) starts every pair's longest walk while the pair
 // before ends on its shortest, ends the launch on a ragged round, and, where the key blocks of a pair divide the 32 compute units of an XCD, gives
@@ -480,9 +485,8 @@ inline int64_t key_groups(int64_t pairs, int64_t nkb, int64_t cus, int64_t per_c
     if (!uneven && !counts) return 1;
     const int64_t slots = per_cu * (pairs % 8 ? cus : cus / 8);
     auto rounds = [&](int64_t n) { return (n * slots + nkb - 1) / nkb; };      // pairs that fill n rounds
-    if (pairs % 8) return (rounds(uneven && (narrow || !counts) ? 2 : 1) + 7) / 8 * 8;
-    if (narrow) return uneven ? rounds(2) : 8;
-    return counts ? rounds(1) : std::max(rounds(1), (int64_t)4);
+    if (pairs % 8) return std::min((rounds(uneven && (narrow || !counts) ? 2 : 1) + 7) / 8 * 8, pairs);
+    return std::min(narrow ? (uneven ? rounds(2) : 8) : counts ? rounds(1) : std::max(rounds(1), (int64_t)4), pairs / 8);
 }
 constexpr int BWD_RING = 4;        // matrix operands in flight from LDS (reads run this many matrix instructions ahead)
 
@@ -537,7 +541,7 @@ void sdpa_bwd_dkv_kernel(SdpaBwdParams bp)
     const int ql = lane & 31, g = lane >> 5;
     const int Sq = p.Sq, Skv = p.Skv;
     const int nkb = (Skv + BWD_KEYS - 1) / BWD_KEYS;
-    const KeyItem ki = key_item(blockIdx.x, p.B * p.Hkv, nkb, p.interleave);
+    const KeyItem ki = key_item(p, blockIdx.x, nkb);
     const int kblk = ki.kblk, bhkv = ki.bhkv;
     const int hkv = bhkv % p.Hkv, b = bhkv / p.Hkv;
     const int j0 = kblk * BWD_KEYS;
@@ -987,7 +991,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 3
     const int ql = lane & 31, g = lane >> 5;
     const int Sq = p.Sq, Skv = p.Skv;
     const int nkb = (Skv + BWD_KEYS - 1) / BWD_KEYS;
-    const KeyItem ki = key_item(blockIdx.x, p.B * p.Hkv, nkb, p.interleave);
+    const KeyItem ki = key_item(p, blockIdx.x, nkb);
     const int kblk = ki.kblk, bhkv = ki.bhkv;
     const int hkv = bhkv % p.Hkv, b = bhkv / p.Hkv;
     const int j0 = kblk * BWD_KEYS, wave_j0 = j0 + wave * 32, my_j = wave_j0 + ql;
@@ -1237,8 +1241,7 @@ static hipError_t launch_bwd_t(const SdpaBwdParams& bp, hipStream_t stream)
     const int nqb = (p.Sq + PF_BM - 1) / PF_BM;
     const int64_t total = dq_blocks;
     auto launch_dq = [&](hipStream_t s) {
-        bq.f.interleave = work_interleave(p.causal != 0 || p.mask != nullptr, 2 * device_cus() / 8, p.G, nqb, (total & 7) == 0 ? total >> 3 : total);
-        bq.f.deal_groups = (total & 7) == 0 ? work_deal(bq.f.interleave, p.G, nqb, total >> 3, p.causal != 0 || p.mask != nullptr) : 0;
+        work_order(bq.f, 2, nqb);
         if (D == 128 && !DENSE && p.D <= 96 && p.Dv <= 96) hipLaunchKernelGGL((sdpa_bwd_dq_kernel<T, D, 0, D == 128 ? 96 : D>), dim3((unsigned)total), dim3(256), 0, s, bq);
         else if (DENSE && p.mask_chunks) hipLaunchKernelGGL((sdpa_bwd_dq_kernel<T, D, DENSE ? 2 : 0>), dim3((unsigned)total), dim3(256), 0, s, bq);
         else hipLaunchKernelGGL((sdpa_bwd_dq_kernel<T, D, DENSE ? 1 : 0>), dim3((unsigned)total), dim3(256), 0, s, bq);
@@ -1258,7 +1261,9 @@ static hipError_t launch_bwd_t(const SdpaBwdParams& bp, hipStream_t stream)
         const unsigned parts = bp.parts_kv > 1 ? (unsigned)bp.parts_kv : 1u;
         const dim3 grid((unsigned)((int64_t)nkb * p.Hkv * p.B), parts);
         SdpaBwdParams bk = bp;
-        bk.f.interleave = (int)key_groups((int64_t)p.B * p.Hkv, nkb, cus, narrow ? (D == 64 ? 3 : 2) : 1, narrow, p.causal || DENSE, p.kv_lens != nullptr);
+        const int64_t pairs = (int64_t)p.B * p.Hkv;
+        bk.f.interleave = (int)key_groups(pairs, nkb, cus, narrow ? (D == 64 ? 3 : 2) : 1, narrow, p.causal || DENSE, p.kv_lens != nullptr);
+        bk.f.groups = (int)((pairs % 8 ? pairs : pairs / 8) / bk.f.interleave);
         if (narrow && D == 64) hipLaunchKernelGGL((sdpa_bwd_dkv_narrow_kernel<T, 64, 64>), grid, dim3(256), 0, stream, bk);
         else if (narrow) hipLaunchKernelGGL((sdpa_bwd_dkv_narrow_kernel<T, 128, 96>), grid, dim3(256), 0, stream, bk);
         else if (DENSE && p.mask_chunks) hipLaunchKernelGGL((sdpa_bwd_dkv_kernel<T, D, DENSE ? 2 : 0>), grid, dim3(512), 0, stream, bk);

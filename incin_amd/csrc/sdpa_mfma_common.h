@@ -2,6 +2,7 @@
 // instruction wrappers, the LDS tile layout (chunk-slot swizzle) and the
 // lane <-> lane^32 exchanges.
 #pragma once
+#include <algorithm>
 #include <atomic>
 
 #include "sdpa_params.h"
@@ -151,68 +152,64 @@ inline int device_cus()
 
 // ---- order of the work list ------------------------------------------------------------------------------------
 // A work item is (batch, KV head, query head of its group, block of query rows).  The list runs over groups of F
-// (batch, KV head) pairs; inside a group the query blocks go longest-first (under a causal mask the last block sees
-// the most keys), and for each block all F * G heads of the group follow one another.  With F * G * (blocks per head)
-// a multiple (twice, measured best) of the workgroups an XCD runs at a time, every round of workgroups gets items of
-// nearly equal length, which
-// list scheduling in plain head order does not give (it ends each head on its shortest blocks while the next head's
-// longest start, and the last round is left ragged: about 9 % at 4096 x 4096 causal).  F is kept small: F KV heads
-// are in an XCD's L2 at a time.
+// (batch, KV head) pairs (the last group takes what is left); inside a group the query blocks go longest-first (under a causal mask the last block sees
+// the most keys), and for each block all F * G heads of the group follow one another: plain head order ends each head on its shortest blocks
+// while the next head's longest start, and leaves the last round ragged (about 9 % at 4096 x 4096 causal).  F is kept small: F KV heads
+// are in an XCD's L2 at a time.  Workgroups reach the 8 XCDs round-robin by id.
+//   deal 1   pairs are dealt to the XCDs in turn - pair h to XCD h % 8 - and each XCD has a list of its own
+//   deal 0   an XCD has a contiguous eighth of the one list (of the list as it is, where it does not divide by 8)
+//   deal 2   the one list, dealt item by item, a group's pairs innermost: with F a multiple of 8 a pair stays on one XCD, or a few
+//   deal 3   likewise, a pair's query heads innermost: a pair is read by all XCDs
 struct WorkItem { int bhkv, gq, qblk; };
-__device__ __forceinline__ WorkItem work_item(int vid, int F, int G, int nqb)
+// (unsigned divisions by what the host could work out: every workgroup starts with them)
+__device__ __forceinline__ WorkItem work_item_of(const SdpaParams& p, unsigned id, unsigned total, unsigned nqb)
 {
-    const int per_group = F * G * nqb;
-    const int grp = vid / per_group, r = vid - grp * per_group;
-    const int rank = r / (F * G), m = r - rank * (F * G);
+    const unsigned G = p.G, F = p.interleave, last = p.groups - 1;
+    unsigned xcd = 0, pairs = (unsigned)p.B * p.Hkv;
+    if (p.deal_groups == 1) {
+        xcd = id & 7;
+        id >>= 3;
+        pairs >>= 3;
+    } else if (p.deal_groups == 0 && (total & 7) == 0) id = (id & 7) * (total >> 3) + (id >> 3);
+    unsigned grp = 0;
+    if (last > 0) grp = min(id / (F * G * nqb), last);
+    const unsigned size = grp == last ? pairs - grp * F : F, r = id - grp * F * G * nqb, rank = r / (size * G), m = r - rank * (size * G);
+    const bool inner = p.deal_groups == 2;
+    const unsigned den = inner ? size : G, quo = m / den, rem = m - quo * den, pair = grp * F + (inner ? rem : quo);
     WorkItem w;
-    w.bhkv = grp * F + m / G;
-    w.gq = m % G;
+    w.bhkv = p.deal_groups == 1 ? pair * 8 + xcd : pair;
+    w.gq = inner ? quo : rem;
     w.qblk = nqb - 1 - rank;
     return w;
 }
-// Item `item` of XCD `xcd`'s share of the work list (a share holds share_len items).  When a share holds whole
-// groups, (batch, KV head) pairs are dealt to the XCDs in turn - pair h goes to XCD h % 8, and an XCD groups the
-// pairs it holds F at a time - so the sequences of a ragged batch spread over all XCDs instead of one long sequence
-// filling the shares of two of them.  Otherwise a share is a contiguous eighth of the list - unless (deal = 2) a share is
-// less than one group and the group's blocks differ in length (a causal mask): a contiguous piece of a list that runs
-// longest-first would give one XCD the long blocks of every head and another the short ones (8 query heads on one KV head,
-// 64 blocks each: the first XCD would get 1.9 times the average), so the list is dealt item by item - item i of the list to
-// XCD i % 8, which is the order workgroups reach the XCDs in anyway.
-__device__ __forceinline__ WorkItem work_item_of_share(int xcd, int item, int share_len, int F, int G, int nqb, int deal)
+// The order of a launch with per_cu workgroups on a compute unit.
+//   A multiple of 8 pairs: 1.  Where blocks differ in length, F fills two rounds of workgroups (a slot that drew a long block first draws a short one next).
+//   Otherwise, where blocks differ in length, 2: eighths of the list, or the list as it is where that does not divide by 8, give one XCD the long
+// blocks of every head and another the short ones, or the long sequences of a batch and the short ones.  F fills two rounds, 8 to 64.  Us, so before / now, causal:
+// 1 x 12 heads x 8192 x 128 217 / 197, 1 x 16 on 4 x 8192 299 / 249, 5 x 12 x 4096 268 / 247, 1 x 20 x 2048 x 64 33.1 / 26.5, 3 x 12 x 1100 x 64 20.3 / 17.5, 5 x 16 on 4 x 1500 x
+// 256 140 / 111, 3 x 12 x 4000 of 600 - 4000 positions 148 / 84, f32 training step 3 x 12 x 700 x 64 118 / 96; 14 x 8 on 1 x 757 31.0 / 31.7, 1 x 32 on 2 x 3000 x 64 47.4 /
+// 48.2.  Key counts, nothing masked: training step of 33 x 12 x 512 x 64 137 / 133.
+//   Key or query counts, grouped queries and KV heads that 8 does not divide: 3, from more than a round of workgroups on - the KV heads of one sequence are on few
+// XCDs, and those of the longest then end the launch.  Padded batches of an eighth of the positions to all, causal: 5 x 32 on 4 x 8192 1920 / 950 (deal 2 1193), 8 x 8 on
+// 1 x 4096 203 / 136, 16 x 16 on 2 x 2048 151 / 138, 4 x 32 on 4 x 8192 880 / 780, 5 x 32 on 2 x 2048 x 256 299 / 162; 3 x 32 on 4 x 2000 with counts alone 158 / 133, 8 x 8 on 2 x
+// 2048 94.0 / 95.2.  (A round or less lasts as long as its longest block: 8 x 8 on 1 x 1024 23.4 / 24.3, so not there.)
+inline void work_order(SdpaParams& p, int per_cu, int nqb)
 {
-    if (deal == 2) return work_item(item * 8 + xcd, F, G, nqb);
-    if (!deal) return work_item(xcd * share_len + item, F, G, nqb);
-    const int per_group = F * G * nqb;
-    const int g_local = item / per_group, r = item - g_local * per_group;
-    const int rank = r / (F * G), m = r - rank * (F * G);
-    WorkItem w;
-    w.bhkv = (g_local * F + m / G) * 8 + xcd;
-    w.gq = m % G;
-    w.qblk = nqb - 1 - rank;
-    return w;
-}
-inline int work_deal(int F, int G, int nqb, long long share_items, bool uneven)
-{
-    const long long group = (long long)F * G * nqb;
-    // (item by item only where a share is less than a group - the few heads of such a launch fit the last-level cache whichever
-    //  XCD reads them.  With more heads than XCDs the contiguous shares keep a head's K and V in one L2, and dealing such lists
-    //  item by item loses more than the ragged shares cost: 12 heads x 8192 keys 932 -> 772 TFLOP/s, 5 x 12 heads x 4096 929 -> 734.)
-    return share_items % group == 0 ? 1 : (uneven && share_items < group ? 2 : 0);
-}
-
-// F for a launch: `slots` workgroups run on an XCD at a time, a range of the list (the whole list, or an eighth of it
-// when it divides by 8 and each XCD takes one) holds `range_items` items.
-// (`causal`: the blocks of a head differ in length - a causal flag, or a mask tensor, which more often than not is a causal
-// mask; with blocks of equal length the interleaved order costs nothing)
-inline int work_interleave(bool causal, int slots, int G, int nqb, long long range_items)
-{
-    if (!causal || slots <= 0) return 1;
-    int a = slots, b = (G * nqb) % slots;
-    while (b) { const int t = a % b; a = b; b = t; }          // a = gcd(slots, G * nqb)
-    int f = 2 * (slots / a);          // two rounds per group: a slot that drew a long block first draws a short one next
-    if (f > 8) f = 8;
-    while (f > 1 && range_items % ((long long)f * G * nqb)) --f;
-    return f;
+    const bool uneven = p.causal || p.mask, counts = p.kv_lens || p.q_lens;
+    const int64_t pairs = (int64_t)p.B * p.Hkv, list = (int64_t)p.G * nqb, slots = std::max((int64_t)per_cu * device_cus() / 8, (int64_t)1);
+    if (counts && p.G > 1 && p.Hkv % 8 && pairs * list > 8 * slots) p.deal_groups = 3;
+    else p.deal_groups = pairs % 8 == 0 ? 1 : uneven || counts ? 2 : 0;
+    int64_t F = 1;
+    if (p.deal_groups >= 2) F = std::min((2 * slots + list - 1) / std::max(list, (int64_t)1), (int64_t)8) * 8;
+    else if (uneven && list > 0) {
+        int64_t a = slots, b = list % slots;
+        while (b) { const int64_t t = a % b; a = b; b = t; }          // a = gcd(slots, list)
+        F = std::min(2 * (slots / a), (int64_t)8);
+        while (F > 1 && pairs / 8 % F) --F;
+    }
+    const int64_t per = std::max(p.deal_groups == 1 ? pairs / 8 : pairs, (int64_t)1);
+    p.interleave = (int)std::min(F, per);
+    p.groups = (int)(per / p.interleave);
 }
 
 // ---- Q rows in, O rows out: 16 bytes per lane, eight lanes to a 128-byte run of a row -------------------------------

@@ -25,8 +25,9 @@ struct SdpaParams {
     int32_t Dp;                // matrix-core kernels: the head dimension their instance is built for (64 or 128); D and Dv fit in it, zero-padded
     float scale;
     int32_t causal;
-    int32_t interleave;        // MFMA prefill kernels: (batch, KV head) pairs per group of the work list, set by their launchers
-    int32_t deal_groups;       // MFMA prefill kernels: (batch, KV head) pairs are dealt to the 8 XCDs in turn (else: contiguous eighths)
+    int32_t interleave;        // matrix-core prefill and backward kernels: (batch, KV head) pairs per group of the work list, set by their launchers
+    int32_t groups;            // the same: those groups per list
+    int32_t deal_groups;       // the same: how the list reaches the 8 XCDs (work_order)
     // split-KV only
     int32_t num_splits;
     int32_t split_len;         // keys per split (multiple of the kernel's key tile)

@@ -69,8 +69,7 @@ void sdpa_prefill_f32_kernel(SdpaParams p, int pairs)
     int item = blockIdx.x >> 3;
     // (one round, two workgroups to a compute unit, blocks of different lengths: the second 32 of an XCD go in reverse, a long one with a short one)
     if (pairs && ((item >> 5) & 1)) item = 32 + ((total >> 3) - 1 - item);
-    const WorkItem wi = (total & 7) == 0 ? work_item_of_share(blockIdx.x & 7, item, total >> 3, p.interleave, p.G, nqb, p.deal_groups)
-                                         : work_item(blockIdx.x, p.interleave, p.G, nqb);
+    const WorkItem wi = work_item_of(p, item * 8 + (blockIdx.x & 7), total, nqb);
     const int gq = wi.gq, bhkv = wi.bhkv;
     const int hkv = bhkv % p.Hkv, b = bhkv / p.Hkv;
     const int hq = hkv * p.G + gq;
@@ -498,8 +497,7 @@ static hipError_t launch_prefill_f32_t(const SdpaParams& p0, hipStream_t stream)
     if (total <= 0) return hipSuccess;
     if (total > 0x7fffffffLL) return hipErrorInvalidValue;
     const bool uneven = p.causal != 0 || p.mask != nullptr;
-    p.interleave = work_interleave(uneven, (D == 64 ? 2 : 1) * device_cus() / 8, p.G, nqb, (total & 7) == 0 ? total >> 3 : total);
-    p.deal_groups = (total & 7) == 0 ? work_deal(p.interleave, p.G, nqb, total >> 3, uneven) : 0;
+    work_order(p, D == 64 ? 2 : 1, nqb);
     const int pairs = D == 64 && uneven && (total & 7) == 0 && total > 256 && total <= 512 ? 1 : 0;
     if constexpr (!DENSE) {
         if (p.num_splits > 1) {          // split launch: partial results, then the split-KV kernels' combine pass

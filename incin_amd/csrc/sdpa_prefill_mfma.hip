@@ -135,8 +135,7 @@ void sdpa_prefill_mfma_kernel(SdpaParams p)
     // range of the work list so heads that share K/V stay in one L2.
     const int nqb = (Sq + BM - 1) / BM;
     const int total = gridDim.x;
-    const WorkItem wi = (total & 7) == 0 ? work_item_of_share(blockIdx.x & 7, blockIdx.x >> 3, total >> 3, p.interleave, p.G, nqb, p.deal_groups)
-                                         : work_item(blockIdx.x, p.interleave, p.G, nqb);
+    const WorkItem wi = work_item_of(p, blockIdx.x, total, nqb);
     const int gq = wi.gq, qb = wi.qblk, bhkv = wi.bhkv;
     const int hkv = bhkv % p.Hkv, b = bhkv / p.Hkv;
     const int hq = hkv * p.G + gq;
@@ -953,8 +952,7 @@ static hipError_t launch_prefill_nw(const SdpaParams& p0, hipStream_t stream)
     const int64_t total = (int64_t)nqb * p.Hq * p.B;
     // 256 registers per lane: eight wavefronts per compute unit, i.e. two workgroups of four or one of eight; an eighth
     // of the compute units per XCD
-    p.interleave = work_interleave(p.causal != 0 || p.mask != nullptr, (8 / NW) * device_cus() / 8, p.G, nqb, (total & 7) == 0 ? total >> 3 : total);
-    p.deal_groups = (total & 7) == 0 ? work_deal(p.interleave, p.G, nqb, total >> 3, p.causal != 0 || p.mask != nullptr) : 0;
+    work_order(p, 8 / NW, nqb);
     constexpr bool DENSE = MASK == 1 || MASK == 3;
     if constexpr (MASK == 0 && NW == 4) {
         if (p.num_splits > 1) {          // split launch: partial results, then the split-KV kernels' combine pass

@@ -66,8 +66,7 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(2, 2))
     // ---- which (batch, head, query block): the work order of the other prefill kernels ---------------------------------
     const int nqb = (Sq + PF_BM - 1) / PF_BM;
     const int total = gridDim.x;
-    const WorkItem wi = (total & 7) == 0 ? work_item_of_share(blockIdx.x & 7, blockIdx.x >> 3, total >> 3, p.interleave, p.G, nqb, p.deal_groups)
-                                         : work_item(blockIdx.x, p.interleave, p.G, nqb);
+    const WorkItem wi = work_item_of(p, blockIdx.x, total, nqb);
     const int hkv = wi.bhkv % p.Hkv, b = wi.bhkv / p.Hkv;
     const int hq = hkv * p.G + wi.gq;
     const int q0 = wi.qblk * PF_BM;
@@ -445,8 +444,7 @@ hipError_t launch_sdpa_prefill_wide(const SdpaParams& p0, int dtype, hipStream_t
     if (total <= 0) return hipSuccess;
     if (total > 0x7fffffffLL) return hipErrorInvalidValue;
     // two workgroups per compute unit, an eighth of the compute units per XCD
-    p.interleave = work_interleave(p.causal != 0 || p.mask != nullptr, 2 * device_cus() / 8, p.G, nqb, (total & 7) == 0 ? total >> 3 : total);
-    p.deal_groups = (total & 7) == 0 ? work_deal(p.interleave, p.G, nqb, total >> 3, p.causal != 0 || p.mask != nullptr) : 0;
+    work_order(p, 2, nqb);
     if (p.mask && p.mask_lims) {       // the blocks whose rows all have a limit; then, below, the others
         if (two_groups(p, total, nqb)) {      // (as the launch of the flag that such a mask stands for)
             if (dtype == 1) hipLaunchKernelGGL((sdpa_prefill_wide_kernel<f16_t, 2, false, 2>), dim3((unsigned)total), dim3(512), 0, stream, p);
