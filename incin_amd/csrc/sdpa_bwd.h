@@ -55,12 +55,15 @@ inline bool bwd16_narrow(int64_t D, int64_t Dv, bool mask, int64_t G, int64_t bl
 //   most two rounds too - of 16 tiles up to one and a half rounds, undivided: the second one leaves half of the compute units idle (40 x 1024 84 / 89,
 //   48 x 1024 88 / 92, 56 x 1024 113 / 105) - (8 x 8192 457 / 488, 2 x 32 / 8 x 2048 268 / 309, 16 / 4 x 2048 in 4 parts 145 / 126, 64 / 8 x 4096 975 / 891;
 //   without a mask 8 x 8192 942 / 823);
-//   the other: walks of 32 tiles under a causal mask or with grouped queries (8 x 8192, causal 278 / 305, 64 / 8 x 4096 466 / 518,
-//   4 x 32 / 8 x 4096 894 / 986; 32 x 12 x 512 118 / 103; without either 2 x 16 x 2048 135 / 121).
+//   the other: grouped queries with walks of 32 tiles and at most three key blocks per compute unit (training steps, D = 64: 64 on 8 x 4096 617 / 669, 2 x 64 on 8 x
+//   4096 1183 / 1263, 2 x 32 on 8 x 2048 208 / 229, 8 x 32 on 8 x 1024 208 / 213, but 8 x 32 on 8 x 2048 660 / 644); without, under a causal mask, two and a quarter
+//   with walks of 44, one and a half of 32 (8 x 8192 368 / 399, 12 x 4096 185 / 197, 2 x 12 x 3000 161 / 164, 2 x 8 x 2048 98 / 104, but 2 x 16 x 2048 119 / 114, 4 x 16 x 2048
+//   196 / 183, 2 x 16 x 4096 337 / 317, 8 x 16 x 4096 1218 / 1183; D = 96: 12 x 4096 223 / 263, 4 x 16 x 4096 921 / 882; neither: 32 x 12 x 512 118 / 103, 2 x 16 x 2048 135 / 121).
 inline bool bwd16_forks(bool narrow, bool causal, int64_t G, int64_t blocks, int64_t parts, int64_t walk, int64_t dq_blocks, int64_t cus)
 {
     const int64_t w = walk / parts;
-    if (narrow) return w >= 32 && (causal || G > 1);
+    if (narrow && G > 1) return w >= 32 && blocks <= 3 * cus;
+    if (narrow) return causal && ((w >= 44 && 4 * parts * blocks <= 9 * cus) || (w >= 32 && 2 * parts * blocks <= 3 * cus));
     if (2 * parts * blocks <= cus && w >= 12) return true;
     if (causal && parts == 1 && blocks > cus && 2 * blocks <= 3 * cus && dq_blocks <= 2 * cus && w >= 16) return true;
     return causal && parts * blocks <= 2 * cus && dq_blocks <= 4 * cus && w >= (parts > 1 ? 64 : 32);
