@@ -56,11 +56,11 @@ TRAFFIC_KIB = {   # leg/shape/variant: (FETCH_SIZE, WRITE_SIZE)
     "prefill_chunk/bf16_sq128_kv32768/auto": (66326.4 + 16680.5, 33392.9 + 1024), "prefill_chunk/bf16_sq128_kv32768/unsplit": (66199.5, 1024),
     "prefill_chunk/bf16_sq512_kv32768/auto": (67708 + 17448.5, 33677.2 + 4096), "prefill_chunk/bf16_sq512_kv32768/unsplit": (67735.5, 4096),
     "prefill_chunk/f32_sq128_kv32768/auto": (132204 + 16680, 33316.9 + 2048), "prefill_chunk/f32_sq128_kv32768/unsplit": (132192, 2048),
-    "f32/f32_c1": (187.2, 32), "f32/f32_c2": (12378.4, 8192), "f32/f32_large": (1523050, 262144),
-    "backward/bf16_d128": (432606 + 264544, 135168 + 262439),          # (dQ kernel with the row dots, dK/dV kernel)
-    "backward/bf16_d64": (133152 + 313584 + 269509, 8192 + 131072 + 270332),          # (row dots, dQ and dK/dV kernels)
-    "backward/f32_d64": (8350 + 26826, 256 + 24576),          # (row dots, one launch of all gradients)
-    "backward/f32_d128": (266271 + 3539515, 4096 + 786432),
+    "f32/f32_c1": (186, 32), "f32/f32_c2": (12401, 9216), "f32/f32_large": (756926, 262144),
+    "backward/bf16_d128": (432774 + 451685, 135168 + 262519),          # (dQ kernel with the row dots, dK/dV kernel)
+    "backward/bf16_d64": (371092 + 295714, 139264 + 262144),          # (dQ kernel with the row dots, dK/dV kernel)
+    "backward/f32_d64": (8350 + 25357, 256 + 24576),          # (row dots, one launch of all gradients)
+    "backward/f32_d128": (266270 + 3496110, 4096 + 786432),
 }
 TRAFFIC_PROFILE = "profiles/fetch_write_size_bench_legs.txt"
 
@@ -571,8 +571,8 @@ def matrix_rate():
 
 
 def f32_configs(steps, warmup, with_cpu, threads):
-    """BASELINE configs 1 and 2 - f32, the one dtype the reference's operator runs end to end - on the IEEE-f32
-    matrix-core kernel: absolute TFLOP/s against the fp32 matrix peak, config 2 also with the causal mask handed over
+    """BASELINE configs 1 and 2 - f32, the one dtype the reference's operator runs end to end - on the f32
+    matrix-core kernels: absolute TFLOP/s against the fp32 matrix peak, config 2 also with the causal mask handed over
     as the explicit [S, S] tensor of 0 / -inf a caller of the reference's operator passes, and the oracle's
     materialising restatement timed on all of config 2 beside it."""
     from oracle import oracle as O
@@ -586,8 +586,8 @@ def f32_configs(steps, warmup, with_cpu, threads):
         flops = causal_flops(B, H, S, S, D) if causal else 4.0 * D * B * H * S * S
         dur, dur_from = launch_duration(w, ev_mean)
         kernel = {capi.IMPL_MFMA: "sdpa_prefill_f32_kernel<%d>" % D, capi.IMPL_GENERIC: "sdpa_generic_kernel<float>",
-                  capi.IMPL_SPLITKV_MFMA: "sdpa_decode_f32_kernel<%d> (the f32 split-KV kernel, 32 rows per workgroup: AUTO's choice for launches "
-                                          "of at most one 128-row block per compute unit)" % D}.get(w.impl, str(w.impl))
+                  capi.IMPL_SPLITKV_MFMA: "sdpa_prefill_f32_kernel<%d>, or for launches that leave compute units idle sdpa_decode_f32_kernel<%d> "
+                                          "(32 rows per workgroup)" % (D, D)}.get(w.impl, str(w.impl))
         what = "BASELINE config %s" % key[-1] if key != "f32_large" else "not a BASELINE config (the shape of config 3 in f32: a launch that fills the machine)"
         rec = {"workload": "%s: f32 %s attention fwd B=%d H=%d S_q=S_kv=%d D=%d, %s" %
                            (what, "causal" if causal else "non-causal", B, H, S, D, scale_note),

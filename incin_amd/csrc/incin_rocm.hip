@@ -1001,7 +1001,7 @@ int incin_rocm_lds_fill(int32_t dev, uint32_t pattern, void* sink, void* stream)
 size_t incin_rocm_sizeof_sdpa_bwd_desc(void) { return sizeof(incin_rocm_sdpa_bwd_desc_t); }
 
 // Validates a backward request; *empty is set when there is nothing to compute, *kind says which kernels take it:
-// 0 the generic ones, 1 the 16-bit matrix-core ones, 2 the IEEE-f32 matrix-core ones, 3 the 16-bit ones above head dimension 128.
+// 0 the generic ones, 1 the 16-bit matrix-core ones, 2 the f32 matrix-core ones, 3 the 16-bit ones above head dimension 128.
 static int check_bwd(const incin_rocm_sdpa_bwd_desc_t* bd, bool* empty, int* kind)
 {
     static const char* OP = "scaled_dot_product_attention backward";
