@@ -55,7 +55,7 @@ TRAFFIC_KIB = {   # leg/shape/variant: (FETCH_SIZE, WRITE_SIZE)
     "head_dims/decode_d96": (393400, 192), "head_dims/decode_d256": (1048960, 512), "head_dims/prefill_d96_s4096": (206387, 123320),
     "prefill_chunk/bf16_sq128_kv32768/auto": (66326.4 + 16680.5, 33392.9 + 1024), "prefill_chunk/bf16_sq128_kv32768/unsplit": (66199.5, 1024),
     "prefill_chunk/bf16_sq512_kv32768/auto": (67708 + 17448.5, 33677.2 + 4096), "prefill_chunk/bf16_sq512_kv32768/unsplit": (67735.5, 4096),
-    "prefill_chunk/f32_sq128_kv32768/auto": (132204 + 16680, 33316.9 + 2048), "prefill_chunk/f32_sq128_kv32768/unsplit": (132192, 2048),
+    "prefill_chunk/f32_sq128_kv32768/auto": (135368 + 16678.9, 33280 + 2048), "prefill_chunk/f32_sq128_kv32768/unsplit": (132302, 2048),
     "f32/f32_c1": (186, 32), "f32/f32_c2": (12401, 9216), "f32/f32_large": (756926, 262144),
     "backward/bf16_d128": (432774 + 451685, 135168 + 262519),          # (dQ kernel with the row dots, dK/dV kernel)
     "backward/bf16_d64": (371092 + 295714, 139264 + 262144),          # (dQ kernel with the row dots, dK/dV kernel)
