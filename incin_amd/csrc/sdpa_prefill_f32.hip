@@ -284,7 +284,8 @@ void sdpa_prefill_f32_kernel(SdpaParams p, int pairs)
                 for (int r = 0; r < 16; ++r)
                     if (8 * (r / 4) + (r % 4) >= rel) s[r] = -INFINITY;
             }
-            // ---- online softmax: probabilities are taken against a reference that moves rarely (they stay <= 2^8) ----
+            // ---- online softmax: probabilities are taken against a reference that moves rarely (they stay <= 2^8; EXACT: <= 1, so that values
+            // of V up to the largest finite one do not overflow where the result does not) ----
             float tmax = s[0];
 #pragma unroll
             for (int r = 1; r < 16; ++r) tmax = fmaxf(tmax, s[r]);
@@ -292,7 +293,7 @@ void sdpa_prefill_f32_kernel(SdpaParams p, int pairs)
                 tmax = xor32_max(tmax);
                 const bool need = tmax - m_run > rise;
                 const float to = need ? tmax : m_run, alpha = rise == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m_run - to);      // (first key: nothing summed yet)
-                if (need) rise = PF_RESCALE_THRESHOLD;
+                if (need) rise = EXACT ? 0.0f : PF_RESCALE_THRESHOLD;
                 m_run = to;
                 l_run *= alpha;
 #pragma unroll

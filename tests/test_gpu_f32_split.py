@@ -59,6 +59,21 @@ def test_values_of_any_size(gpu, exponent):
         assert np.isfinite(got).all() and np.max(np.abs(got - gen) / np.maximum(np.abs(gen), 1)) <= 1e-5
 
 
+@pytest.mark.parametrize("D,splits", [(64, 0), (96, 0), (128, 0), (64, 2)])
+def test_large_values_under_a_late_maximum(gpu, D, splits):
+    """A key of a later tile 2^7 times as probable as the first ones, and V near the largest finite value there: 2^7 V overflows, the result does
+    not (weights of a row are at most one against its maximum).  Bound: the 24 bits of a weighted mean of V."""
+    q, k, v = inputs(7, 1, 2, 40, 640, D)
+    q[:], k[:] = 0.0, 0.0
+    q[..., 0], k[..., 600, 0] = 1.0, 7.0 * np.log(2.0) * np.sqrt(D)
+    v[..., :600, :] *= 1e-3
+    v[..., 600, :] = np.sign(v[..., 600, :]) * 2e38
+    got = host.sdpa(q, k, v, capi.F32, impl=capi.IMPL_MFMA, num_splits=splits)
+    w = np.exp(q.astype(np.float64) @ k.astype(np.float64).transpose(0, 1, 3, 2) / np.sqrt(D))
+    ref = (w / w.sum(-1, keepdims=True)) @ v.astype(np.float64)
+    assert np.isfinite(got).all() and np.max(np.abs(got / ref - 1)) <= 2e-6
+
+
 @pytest.mark.parametrize("S,D,causal", [(1024, 64, False), (512, 96, True), (700, 128, False)])
 def test_error_against_64_bits(gpu, S, D, causal):
     """No larger than that of IEEE-f32 products: those leave 2.2e-7 - 3.5e-7 of the 2-norm here, this kernel 1.2e-7 - 2.0e-7.  The bound is the
