@@ -284,6 +284,8 @@ void sdpa_prefill_f32_kernel(SdpaParams p, int pairs)
                 for (int r = 0; r < 16; ++r)
                     if (8 * (r / 4) + (r % 4) >= rel) s[r] = -INFINITY;
             }
+            // EXACT: a block that none of the wavefront's rows sees is left out of the product with V, whose rows may hold anything there
+            const bool unseen = EXACT && (((flags_of(t) >> flag_shift) & 3) == 2 || __builtin_amdgcn_ballot_w64(my_i < rows_b && j0 < lim_lane) == 0);
             // ---- online softmax: probabilities are taken against a reference that moves rarely (they stay <= 2^8; EXACT: <= 1, so that values
             // of V up to the largest finite one do not overflow where the result does not) ----
             float tmax = s[0];
@@ -379,7 +381,8 @@ void sdpa_prefill_f32_kernel(SdpaParams p, int pairs)
                 mma_split_term<EXACT, 2>(a, pr[h], small); put(6 * i + 2);
                 mma_split_term<EXACT, 3>(a, pr[h], small); put(6 * i + 3);
                 mma_split_term<EXACT, 4>(a, pr[h], small); put(6 * i + 4);
-                mma_split_term<EXACT, 5>(a, pr[h], o_acc[db]); put(6 * i + 5);
+                if (!unseen) mma_split_term<EXACT, 5>(a, pr[h], o_acc[db]);
+                put(6 * i + 5);
                 a = n;
             }
 #pragma unroll

@@ -45,6 +45,35 @@ def test_values_that_are_not_finite(gpu, D):
         assert fin.any() and not fin.all() and np.max(np.abs(got[fin] - ref[fin])) <= 1e-5, what
 
 
+@pytest.mark.parametrize("D", [64, 96])
+@pytest.mark.parametrize("how", ["causal", "limits", "window"])
+def test_hidden_blocks_may_hold_anything(gpu, D, how):
+    """A NaN in V reaches the rows whose block of 32 sees any of its block of 32 keys, and no other: under the causal flag, the same mask as a tensor
+    (through its row limits) and a mask of values with a hidden block inside a tile that is not hidden as a whole."""
+    H, S = 96, 192      # (enough workgroups that the planner hands the mask's limits to this kernel)
+    q, k, v = inputs(13, 1, H, S, S, D)
+    mask = np.zeros((S, S), np.float32)
+    if how == "window":
+        mask += np.random.Generator(np.random.PCG64(2)).standard_normal((S, S), dtype=np.float32)
+        mask[:32, 32:96] = mask[96:, 64:96] = -np.inf
+    else:
+        mask += np.triu(np.full((S, S), -np.inf, np.float32), 1)
+    ref = O.sdpa(q, k, v, mask=mask[None, None])
+    hit = [63, 70] + [191] * (how != "window")
+    v[0, :, hit, 5] = np.nan
+    if how == "causal":
+        got = host.sdpa(q, k, v, capi.F32, causal=True, impl=capi.IMPL_MFMA)
+    else:
+        got = host.sdpa(q, k, v, capi.F32, mask=mask[None, None], impl=capi.IMPL_AUTO if how == "limits" else capi.IMPL_MFMA)
+    seen = (mask > -np.inf).reshape(S // 32, 32, S // 32, 32).any(axis=(1, 3))
+    bad = np.repeat(seen[:, [x // 32 for x in hit]].any(axis=1), 32)
+    assert bad.any() and not bad.all()
+    want = ref.copy()
+    want[..., bad, 5] = np.nan
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.nanmax(np.abs(got - want)) <= 1e-5
+
+
 @pytest.mark.parametrize("exponent", [-60, -20, 20, 60, 120])
 def test_values_of_any_size(gpu, exponent):
     """Values far from 1 keep their 24 bits: Q large where K is small, V of any size; and values that round to infinity in bf16."""
