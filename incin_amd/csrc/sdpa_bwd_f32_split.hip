@@ -207,7 +207,13 @@ __device__ __forceinline__ void bwd_f32_split_body(const SdpaBwdParams& bp, char
                 if (k < 12) xa.template split_step<EXACT>(k, sa, na);
                 else xb.template split_step<EXACT>(k - 12, sb, nb);
             };
-            if (i0 < w_end && i0 + 32 > w_first && i0 < n_stream) {      // (uniform)
+            // (EXACT: a block that the mask hides is left out, like those that the causal flag hides: its rows may hold anything)
+            bool seen = i0 < w_end && i0 + 32 > w_first && i0 < n_stream;
+            if (EXACT && DENSE && p.mask_flags && seen) {
+                const int own32 = (o0 >> 5) + own, row32 = KEYS ? i0 >> 5 : own32, key32 = KEYS ? own32 : i0 >> 5;
+                seen = mask_flags_of(p, b, KEYS ? hkv * p.G + n / tiles : hq)[(int64_t)row32 * ((Skv + 31) >> 5) + key32] != 2;
+            }
+            if (seen) {      // (uniform)
                 [[maybe_unused]] float mv[16];
                 if (DENSE) {
                     if (KEYS) {

@@ -211,3 +211,19 @@ def test_backward_values_that_are_not_finite(gpu, monkeypatch):
                 fin = np.isfinite(b[h])
                 if fin.any():
                     assert np.max(np.abs(a[h][fin] - b[h][fin])) <= 1e-5 * max(np.max(np.abs(b[h][fin])), 1), (name, x, h)
+
+
+def test_backward_hidden_blocks_may_hold_anything(gpu):
+    """A NaN in a row of dO or K reaches the gradients of what sees it, by blocks of 32 x 32, and no other: the causal flag, and the same mask as a
+    tensor, whose hidden blocks lie inside the range that the walk trims to."""
+    shape = (2, 24, 24, 256, 256, 64, 64, True, None, None)
+    q, k, v, go, _, _ = bwd_case(shape)
+    tri = np.triu(np.full((256, 256), -np.inf, np.float32), 1)[None, None]
+    rdq, rdk, rdv = f64_gradients(q, k, v, go, True, None, None)
+    blocks = np.arange(256) // 32
+    go[1, :, 70, 3], k[0, :, 200, 2] = np.nan, np.nan
+    for kw in (dict(causal=True), dict(mask=tri)):
+        _, dq, dk, dv = host.sdpa_backward(q, k, v, go, capi.F32, **kw)
+        assert np.isnan(dv[1, :, blocks == 2, 3]).any() and np.isnan(dq[0, :, blocks == 7]).any()
+        for name, got, ref, clean in (("dk", dk[1], rdk[1], blocks > 2), ("dv", dv[1], rdv[1], blocks > 2), ("dq", dq[0], rdq[0], blocks < 6)):
+            assert np.max(np.abs(got[:, clean] - ref[:, clean])) <= 1e-5 * np.max(np.abs(ref)), (name, kw)
