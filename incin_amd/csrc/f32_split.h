@@ -8,9 +8,10 @@
 // wavefront of the SIMD run beside it (a loop of it with an equal time of v_fma, v_exp or v_add_u32 on the other wavefront takes the sum of both, 177
 // against 91 us; v_mfma_f32_32x32x16_bf16 with as much 224 against 186).  Six of the latter for eight of the former: 192 cycles instead of 512.
 //
-// Infinities and NaN: inf - inf is a NaN in the second part, so what such a value reaches is NaN.  Kernels look at their results and do
-// what is not finite over with EXACT, in the IEEE-f32 instruction on the same operands (the parts of a value that is not finite are then
-// itself and zeros), so such inputs give what they gave with that instruction; so do values whose first part rounds to infinity.
+// What the parts do not hold: an infinity (inf - inf is a NaN in the second part, so what it reaches is NaN), a value whose first part rounds to
+// infinity, and the last bits below 2^-110.  Kernels look at their results and at the sizes of their operands, and do a block
+// over with EXACT, in the IEEE-f32 instruction on the same operands (then kept whole, in two halves), where a result is not finite or where the bits
+// lost - at most 2^-134 of each operand - could be more than half of a rounding of the smallest result.
 #pragma once
 #include "sdpa_mfma_common.h"
 
@@ -34,21 +35,10 @@ template <bool EXACT> __device__ __forceinline__ void split_pair(float a, float 
         l = pack2<bf16_t>(ra - __uint_as_float(m << 16), rb - __uint_as_float(m & 0xffff0000u));
         return;
     }
-    // by truncation, which never rounds to infinity; a value that is not finite is its own first part
-    unsigned part[3][2];
-    const float x[2] = {a, b};
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const bool finite = __builtin_fabsf(x[i]) < INFINITY;
-        const float hi = x[i] != x[i] ? __builtin_nanf("") : __uint_as_float(__float_as_uint(x[i]) & 0xffff0000u);
-        const float r = finite ? x[i] - hi : 0.0f, mid = __uint_as_float(__float_as_uint(r) & 0xffff0000u);
-        part[0][i] = __float_as_uint(hi);
-        part[1][i] = __float_as_uint(mid);
-        part[2][i] = __float_as_uint(r - mid);
-    }
-    h = part[0][0] >> 16 | (part[0][1] & 0xffff0000u);
-    m = part[1][0] >> 16 | (part[1][1] & 0xffff0000u);
-    l = part[2][0] >> 16 | (part[2][1] & 0xffff0000u);
+    // the values as they are: their upper halves, their lower halves
+    h = __float_as_uint(a) >> 16 | (__float_as_uint(b) & 0xffff0000u);
+    m = (__float_as_uint(a) & 0xffffu) | __float_as_uint(b) << 16;
+    l = 0;
 }
 template <bool EXACT> __device__ __forceinline__ Split8 split8(const float8v& x)
 {
@@ -82,8 +72,7 @@ template <bool EXACT> __device__ __forceinline__ floatx16 mma_split(const Split8
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         auto whole = [&](const Split8& x) __attribute__((always_inline)) {
-            auto part = [&](unsigned w) __attribute__((always_inline)) { return __uint_as_float(e & 1 ? w & 0xffff0000u : w << 16); };
-            return part(x.h[e / 2]) + (part(x.m[e / 2]) + part(x.l[e / 2]));
+            return __uint_as_float(e & 1 ? (x.h[e / 2] & 0xffff0000u) | x.m[e / 2] >> 16 : x.h[e / 2] << 16 | (x.m[e / 2] & 0xffffu));
         };
         c = __builtin_amdgcn_mfma_f32_32x32x2f32(whole(a), whole(b), c, 0, 0, 0);
     }
@@ -123,6 +112,30 @@ struct SplitPair {
         }
     }
 };
+
+// ---- sizes: the largest of what is split (one instruction for two values), the smallest of what comes out --------------------------------
+// (the inputs of `largest` are values as loaded or multiplied, not results of matrix instructions: the compiler places no wait states for those here)
+__device__ __forceinline__ float largest(float top, float a, float b)
+{
+    asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(top) : "v"(a), "v"(b));
+    return top;
+}
+// Twice the bits of the smallest magnitude that is not zero, less one (zeros only: all ones).
+__device__ __forceinline__ unsigned smallest(unsigned low, float x) { return min(low, (__float_as_uint(x) << 1) - 1u); }
+__device__ __forceinline__ unsigned smallest_of(float x) { return (__float_as_uint(x) << 1) - 1u; }      // (x > 0)
+// A wavefront's maximum / minimum.
+template <bool MAX> __device__ __forceinline__ unsigned wave_extreme(unsigned x)
+{
+    auto take = [](unsigned a, unsigned b) __attribute__((always_inline)) { return MAX ? max(a, b) : min(a, b); };
+    x = take(x, (unsigned)__builtin_amdgcn_mov_dpp((int)x, 0xb1, 0xf, 0xf, true));       // lane ^ 1
+    x = take(x, (unsigned)__builtin_amdgcn_mov_dpp((int)x, 0x4e, 0xf, 0xf, true));       // lane ^ 2
+    x = take(x, (unsigned)__builtin_amdgcn_mov_dpp((int)x, 0x141, 0xf, 0xf, true));      // 7 - lane of the eight
+    x = take(x, (unsigned)__builtin_amdgcn_mov_dpp((int)x, 0x140, 0xf, 0xf, true));      // 15 - lane of the sixteen
+    auto at = [&](int lane) __attribute__((always_inline)) { return (unsigned)__builtin_amdgcn_readlane((int)x, lane); };
+    return take(take(at(0), at(16)), take(at(32), at(48)));
+}
+constexpr float SPLIT_TINY = 0x1p-100f;      // (parts hold values from 2^-110 on whole)
+constexpr float SPLIT_LOST = 0x1p-110f;      // 2^24 times the 2^-134 that a value below 2^-110 loses at most
 
 // Tiles of ROWS rows of a tensor as three planes of bf16 rows in LDS, 2 D bytes a row, 16-byte chunks swizzled as the 16-bit kernels'
 // K (BY_K) or V tiles: a workgroup's THREADS threads fetch the next tile's values into registers, eight to a thread at a time, and put
@@ -179,6 +192,25 @@ template <int D, int DC, int ROWS, int THREADS> struct SplitTile {
         o.h[q] = h;
         o.m[q] = m;
         o.l[q] = l;
+    }
+    // The largest magnitude of a thread's values, piece by piece of the splitting.
+    __device__ __forceinline__ float largest_step(int k, float top) const
+    {
+        return k % 3 ? top : largest(top, x[k / 12][2 * (k / 3 % 4)], x[k / 12][2 * (k / 3 % 4) + 1]);
+    }
+    __device__ __forceinline__ float largest_of(float top) const
+    {
+#pragma unroll
+        for (int k = 0; k < STEPS; k += 3) top = largest_step(k, top);
+        return top;
+    }
+    __device__ __forceinline__ unsigned smallest_in(unsigned low) const
+    {
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) low = smallest(low, x[i][e]);
+        return low;
     }
     template <bool BY_K> static __device__ __forceinline__ void store(char* tile, const Split8& o, int tid, int i = 0)      // (eight i of the thread's)
     {

@@ -52,7 +52,7 @@ void sdpa_prefill_f32_kernel(SdpaParams p, int pairs)
     typedef SplitTile<D, DC, KT, 256> Tile;
     typedef typename Tile::L L;
     __shared__ __attribute__((aligned(1024))) char smem[3 * Tile::BYTES];      // K, V of even tiles, V of odd ones
-    __shared__ int s_vote[8];
+    __shared__ int s_vote[12];
     __shared__ uint8_t s_flags[DENSE ? MAX_FLAGS : 1];
     char* const kbuf = smem;
 
@@ -185,6 +185,7 @@ void sdpa_prefill_f32_kernel(SdpaParams p, int pairs)
         constexpr bool EXACT = decltype(exact_)::value;
         Tile xk, xv;                     // values on their way into LDS
         Split8 qreg[NSTEP];              // Q', resident
+        [[maybe_unused]] float top = 0.0f;      // the largest magnitude of this thread's share of V; infinity: Q' wants EXACT
         int t = visible_from(t_first), t1 = visible_from(t + 1), t2 = visible_from(t1 + 1);
         // ---- Q' into operands, through the place of the second V tile; the first K and V tiles ----
         {
@@ -194,6 +195,9 @@ void sdpa_prefill_f32_kernel(SdpaParams p, int pairs)
             xv.fetch(vp, p.v_ss, p.Dv, j_end, t * KT, tid);
 #pragma unroll
             for (int i = 0; i < Tile::N; ++i) xq.x[i] *= p.scale * LOG2E;
+            // (a score's error by what K loses is negligible under a Q' up to 2^60, and Q' itself loses nothing from 2^-100 on)
+            if (!EXACT && (!(xq.largest_of(0.0f) <= 0x1p60f) || xq.smallest_in(~0u) < smallest_of(SPLIT_TINY))) top = INFINITY;
+            if (!EXACT) top = xv.largest_of(top);
             xq.template put<EXACT, true>(smem + 2 * Tile::BYTES, tid);
             xk.template put<EXACT, true>(kbuf, tid);
             xv.template put<EXACT, false>(smem + Tile::BYTES, tid);
@@ -353,7 +357,10 @@ void sdpa_prefill_f32_kernel(SdpaParams p, int pairs)
 #pragma unroll
                 for (int k = 2 * NS * i / NM; k < 2 * NS * (i + 1) / NM; ++k) {
                     if (k < NS) xk.template put_step<EXACT, true>(k, st, kbuf, tid);
-                    else xv.template put_step<EXACT, false>(k - NS, st, vnext, tid);
+                    else {
+                        if (!EXACT) top = xv.largest_step(k - NS, top);
+                        xv.template put_step<EXACT, false>(k - NS, st, vnext, tid);
+                    }
                     if (k == NS - 1) xk.fetch(kp, p.k_ss, p.D, j_end, t3 * KT, tid);
                 }
                 __builtin_amdgcn_sched_barrier(0);
@@ -394,16 +401,30 @@ void sdpa_prefill_f32_kernel(SdpaParams p, int pairs)
             t1 = t2;
             t2 = t3;
         }
-        // something that is not finite?
+        if constexpr (EXACT) return false;
+        // A result that is not finite, or one so small that what the parts lose (f32_split.h) could show: of V under the sum of the weights, of the
+        // weights under V.  (The sum is at most 2^8 a key.)
         float chk = l_run * 0.0f;
+        unsigned low = ~0u;
 #pragma unroll
         for (int db = 0; db < NDB; ++db)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) chk = __builtin_fmaf(o_acc[db][r], 0.0f, chk);
+            for (int r = 0; r < 16; ++r) {
+                chk = __builtin_fmaf(o_acc[db][r], 0.0f, chk);
+                low = smallest(low, o_acc[db][r]);
+            }
         const bool bad = __builtin_amdgcn_ballot_w64(chk != 0.0f) != 0;
-        if (lane == 0) s_vote[wave] = bad ? 1 : 0;
+        const unsigned w_top = wave_extreme<true>(__float_as_uint(top)), w_low = wave_extreme<false>(low);
+        if (lane == 0) {
+            s_vote[wave] = bad ? 1 : 0;
+            s_vote[4 + wave] = (int)w_top;
+            s_vote[8 + wave] = (int)w_low;
+        }
         lds_barrier();
-        return (s_vote[0] | s_vote[1] | s_vote[2] | s_vote[3]) != 0;      // (uniform)
+        const float v_top = __uint_as_float(max(max(s_vote[4], s_vote[5]), max(s_vote[6], s_vote[7])));
+        low = min(min((unsigned)s_vote[8], (unsigned)s_vote[9]), min((unsigned)s_vote[10], (unsigned)s_vote[11]));
+        const float bound = SPLIT_LOST * (float)((n_tiles - t_first) * KT) * (v_top + 256.0f);
+        return (s_vote[0] | s_vote[1] | s_vote[2] | s_vote[3]) != 0 || !(v_top < INFINITY) || low < smallest_of(bound) || (v_top > 0.0f && v_top < SPLIT_TINY);      // (uniform)
     };
     if (n_tiles > t_first) {
         if (walk(std::integral_constant<bool, false>{})) {

@@ -88,6 +88,44 @@ def test_values_of_any_size(gpu, exponent):
         assert np.isfinite(got).all() and np.max(np.abs(got - gen) / np.maximum(np.abs(gen), 1)) <= 1e-5
 
 
+def exact(q, k, v):
+    q, k, v = (x.astype(np.float64) for x in (q, k, v))
+    s = q @ k.transpose(0, 1, 3, 2) / np.sqrt(q.shape[-1])
+    p = np.exp(s - s.max(-1, keepdims=True))
+    return (p / p.sum(-1, keepdims=True)) @ v
+
+
+@pytest.mark.parametrize("D,splits", [(64, 0), (96, 0), (128, 0), (40, 0), (64, 2)])
+@pytest.mark.parametrize("what", ["v", "v column", "q", "k"])
+@pytest.mark.parametrize("exponent", [-104, -112, -118, -123])
+def test_values_whose_last_bits_no_part_holds(gpu, D, splits, what, exponent):
+    """Below 2^-110 the third bf16 part loses bits; f32 does not down to 2^-126.  V as small as that, or one of its columns beside ordinary ones, Q under
+    a K as large as Q is small, K under such a Q: each column within 1e-6 of 64 bits (the IEEE products: 3e-7; a column at 2^-125, whose values lie 2^-149 apart, 6e-8 more)."""
+    q, k, v = inputs(21, 1, 2, 70, 200, D)
+    small, large = np.float32(2.0 ** exponent), np.float32(2.0 ** -exponent)
+    if what == "v":
+        v *= small
+    elif what == "v column":
+        v[..., 3] *= small
+    else:
+        q, k = (q * small, k * large) if what == "q" else (q * large, k * small)
+    got, ref = host.sdpa(q, k, v, capi.F32, impl=capi.IMPL_MFMA, num_splits=splits), exact(q, k, v)
+    off = np.linalg.norm(got - ref, axis=2) / np.linalg.norm(ref, axis=2)
+    assert np.max(off) <= 1e-6
+
+
+def test_small_weights_of_large_values(gpu):
+    """A weight of 2^-121.5 whose value is 2^120 and makes up the result: what scores of that size leave (2^-23 of them, in the exponent)."""
+    q, k, v = inputs(22, 1, 2, 40, 200, 64)
+    q[:], k[:] = 0.0, 0.0
+    q[..., 0], k[..., 150, 0] = 1.0, -121.5 * np.log(2.0) * 8.0
+    big = np.sign(v[..., 150, :]) * 2.0 ** 120
+    v[:] = 0.0
+    v[..., 150, :] = big
+    got, ref = host.sdpa(q, k, v, capi.F32, impl=capi.IMPL_MFMA), exact(q, k, v)
+    assert np.max(np.abs(got / ref - 1)) <= 122 * np.log(2.0) * 3 * 2.0 ** -24
+
+
 @pytest.mark.parametrize("D,splits", [(64, 0), (96, 0), (128, 0), (64, 2)])
 def test_large_values_under_a_late_maximum(gpu, D, splits):
     """A key of a later tile 2^7 times as probable as the first ones, and V near the largest finite value there: 2^7 V overflows, the result does
@@ -98,9 +136,7 @@ def test_large_values_under_a_late_maximum(gpu, D, splits):
     v[..., :600, :] *= 1e-3
     v[..., 600, :] = np.sign(v[..., 600, :]) * 2e38
     got = host.sdpa(q, k, v, capi.F32, impl=capi.IMPL_MFMA, num_splits=splits)
-    w = np.exp(q.astype(np.float64) @ k.astype(np.float64).transpose(0, 1, 3, 2) / np.sqrt(D))
-    ref = (w / w.sum(-1, keepdims=True)) @ v.astype(np.float64)
-    assert np.isfinite(got).all() and np.max(np.abs(got / ref - 1)) <= 2e-6
+    assert np.isfinite(got).all() and np.max(np.abs(got / exact(q, k, v) - 1)) <= 2e-6
 
 
 @pytest.mark.parametrize("S,D,causal", [(1024, 64, False), (512, 96, True), (700, 128, False)])
