@@ -36,7 +36,7 @@ typedef SplitTile<64, 64, BS_OWN, BS_THREADS> BsOwn;
 constexpr int BS_LDS = 2 * BsOwn::BYTES + 2 * BsTile::BYTES;  // X, Y, A, B
 
 template <bool KEYS, bool DENSE>
-__device__ __forceinline__ void bwd_f32_split_body(const SdpaBwdParams& bp, char* smem, float (&s_stats)[2][BS_KT], int (&s_vote)[8], int id)
+__device__ __forceinline__ void bwd_f32_split_body(const SdpaBwdParams& bp, char* smem, float (&s_stats)[2][BS_KT], int (&s_vote)[6][8], int id)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
     constexpr float LOG2E = 1.4426950408889634f;
@@ -102,7 +102,7 @@ __device__ __forceinline__ void bwd_f32_split_body(const SdpaBwdParams& bp, char
     if (DENSE && p.mask_flags && t_end > t_begin) {
         // the tiles between the first and the last with a block that sees, or is seen by, any of the owned rows (keys: in any head of the group)
         const int nkb32 = (Skv + 31) >> 5, nrb32 = (Sq + 31) >> 5, lo32 = 2 * t_begin, n32 = min(2 * t_end, KEYS ? nrb32 : nkb32) - lo32;
-        if (tid == 0) { s_vote[0] = 0x7fffffff; s_vote[1] = -1; }
+        if (tid == 0) { s_vote[0][0] = 0x7fffffff; s_vote[0][1] = -1; }
         __syncthreads();
         int lo = 0x7fffffff, hi = -1;
         for (int x = tid; x < n32 * (KEYS ? p.G : 1); x += BS_THREADS) {
@@ -116,9 +116,9 @@ __device__ __forceinline__ void bwd_f32_split_body(const SdpaBwdParams& bp, char
             }
             if (seen) { lo = min(lo, s32); hi = max(hi, s32); }
         }
-        if (hi >= 0) { atomicMin(&s_vote[0], lo); atomicMax(&s_vote[1], hi); }
+        if (hi >= 0) { atomicMin(&s_vote[0][0], lo); atomicMax(&s_vote[0][1], hi); }
         __syncthreads();
-        const int a = __builtin_amdgcn_readfirstlane(s_vote[0]), z = __builtin_amdgcn_readfirstlane(s_vote[1]);
+        const int a = __builtin_amdgcn_readfirstlane(s_vote[0][0]), z = __builtin_amdgcn_readfirstlane(s_vote[0][1]);
         t_end = z < 0 ? t_begin : z / 2 + 1;
         t_begin = z < 0 ? t_begin : a / 2;
         __syncthreads();
@@ -176,6 +176,7 @@ __device__ __forceinline__ void bwd_f32_split_body(const SdpaBwdParams& bp, char
             if (KEYS && tid < 128) s_stats[tid >> 6][tid & 63] = stat;
         };
         fetch(0);
+        [[maybe_unused]] float top_a = 0.0f, top_b = 0.0f;      // the largest magnitudes of this thread's share of A and B; A infinity: X wants EXACT
         {
             BsOwn x;
             const int rows = max(n_own, 1);
@@ -183,10 +184,20 @@ __device__ __forceinline__ void bwd_f32_split_body(const SdpaBwdParams& bp, char
             else x.fetch_any(q_of(hq), p.q_ss, p.D, rows, o0, tid);
 #pragma unroll
             for (int i = 0; i < BsOwn::N; ++i) x.x[i] *= p.scale * LOG2E;
+            // (a score's error by what A loses is negligible under an X up to 2^60, and X itself loses nothing from 2^-100 on)
+            if (!EXACT && (!(x.largest_of(0.0f) <= 0x1p60f) || x.smallest_in(~0u) < smallest_of(SPLIT_TINY))) top_a = INFINITY;
             x.template put<EXACT, true>(own_x, tid);
             if (KEYS) x.fetch_any(vp, p.v_ss, p.Dv, rows, o0, tid);
             else x.fetch_any(g_of(hq), bp.do_ss, p.Dv, rows, o0, tid);
+            if (!EXACT) {
+                const unsigned top = wave_extreme<true>(__float_as_uint(x.largest_of(0.0f)));
+                if (lane == 0) s_vote[5][wave] = (int)top;
+            }
             x.template put<EXACT, true>(own_y, tid);
+        }
+        if (!EXACT) {
+            top_a = xa.largest_of(top_a);
+            top_b = xb.largest_of(top_b);
         }
         xa.template put<EXACT, true>(tile_a, tid);
         xb.template put<EXACT, true>(tile_b, tid);
@@ -204,8 +215,13 @@ __device__ __forceinline__ void bwd_f32_split_body(const SdpaBwdParams& bp, char
             BsTile::State sa, sb;
             // piece k of 24 of splitting them
             auto split_next = [&](int k) __attribute__((always_inline)) {
-                if (k < 12) xa.template split_step<EXACT>(k, sa, na);
-                else xb.template split_step<EXACT>(k - 12, sb, nb);
+                if (k < 12) {
+                    if (!EXACT) top_a = xa.largest_step(k, top_a);
+                    xa.template split_step<EXACT>(k, sa, na);
+                } else {
+                    if (!EXACT) top_b = xb.largest_step(k - 12, top_b);
+                    xb.template split_step<EXACT>(k - 12, sb, nb);
+                }
             };
             // (EXACT: a block that the mask hides is left out, like those that the causal flag hides: its rows may hold anything)
             bool seen = i0 < w_end && i0 + 32 > w_first && i0 < n_stream;
@@ -389,19 +405,45 @@ __device__ __forceinline__ void bwd_f32_split_body(const SdpaBwdParams& bp, char
             }
             lds_barrier();
         }
+        // A result that is not finite, or one so small that what the parts lose (f32_split.h) could show.  With a, b, y the largest
+        // magnitudes of A, B and Y: dp is at most 128 y b and off by 64 (y + b) units of 2^-134, P and dS by one each, A and B likewise.  Operands
+        // whose products are small throughout may leave zeros and are done over as well.
         float chk = 0.0f;
+        unsigned lx = ~0u, lv = ~0u;
 #pragma unroll
         for (int x = 0; x < NACC; ++x)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) chk = __builtin_fmaf(acc[x][r], 0.0f, chk);
+            for (int r = 0; r < 16; ++r) {
+                chk = __builtin_fmaf(acc[x][r], 0.0f, chk);
+                if (x < 2) lx = smallest(lx, acc[x][r]);
+                else lv = smallest(lv, acc[x][r]);
+            }
         const bool bad = __builtin_amdgcn_ballot_w64(chk != 0.0f) != 0;
-        if (lane == 0) s_vote[wave] = bad ? 1 : 0;
+        const unsigned w_a = wave_extreme<true>(__float_as_uint(top_a)), w_b = wave_extreme<true>(__float_as_uint(top_b));
+        const unsigned w_x = wave_extreme<false>(lx), w_v = wave_extreme<false>(lv);
+        if (lane == 0) {
+            s_vote[0][wave] = bad ? 1 : 0;
+            s_vote[1][wave] = (int)w_a;
+            s_vote[2][wave] = (int)w_b;
+            s_vote[3][wave] = (int)w_x;
+            s_vote[4][wave] = (int)w_v;
+        }
         lds_barrier();
-        int any = 0;
+        auto over_waves = [&](int i, auto take) __attribute__((always_inline)) {
+            unsigned v = (unsigned)s_vote[i][0];
 #pragma unroll
-        for (int w = 0; w < 8; ++w) any |= s_vote[w];
+            for (int w = 1; w < 8; ++w) v = take(v, (unsigned)s_vote[i][w]);
+            return (unsigned)__builtin_amdgcn_readfirstlane((int)v);
+        };
+        auto most = [](unsigned x, unsigned y) { return max(x, y); };
+        auto least = [](unsigned x, unsigned y) { return min(x, y); };
+        const unsigned any_bad = over_waves(0, most), low_x = over_waves(3, least), low_v = over_waves(4, least);
+        const float big_a = __uint_as_float(over_waves(1, most)), big_b = __uint_as_float(over_waves(2, most)), big_y = __uint_as_float(over_waves(5, most));
         lds_barrier();
-        return __builtin_amdgcn_readfirstlane(any) != 0;
+        const float lost = SPLIT_LOST * (float)n_tiles * BS_KT, yb = big_y * big_b;
+        const float bound_x = lost * (big_a * (128.0f * yb + 64.0f * (big_y + big_b) + 1.0f) + 128.0f * yb), bound_v = lost * (big_b + 1.0f);
+        const bool tiny = big_a > 0.0f && big_b > 0.0f && big_y > 0.0f && (big_b < SPLIT_TINY || yb < SPLIT_TINY || yb * big_a < SPLIT_TINY);
+        return any_bad != 0 || !(big_a < INFINITY) || !(big_b < INFINITY) || tiny || low_x < smallest_of(bound_x) || low_v < smallest_of(bound_v);      // (uniform)
     };
     if (n_tiles > 0) {
         if (walk(std::integral_constant<bool, false>{})) walk(std::integral_constant<bool, true>{});      // (f32_split.h)
@@ -442,7 +484,7 @@ template <bool DENSE> __global__ __launch_bounds__(BS_THREADS, 2) void bwd_f32_s
 #if defined(__HIP_DEVICE_COMPILE__)
     __shared__ __attribute__((aligned(1024))) char smem[BS_LDS];
     __shared__ __attribute__((aligned(16))) float s_stats[2][BS_KT];
-    __shared__ int s_vote[8];
+    __shared__ int s_vote[6][8];
     const int id = blockIdx.x;
     if (id < n_dkv) bwd_f32_split_body<true, DENSE>(bp, smem, s_stats, s_vote, id);
     else bwd_f32_split_body<false, DENSE>(bp, smem, s_stats, s_vote, id - n_dkv);

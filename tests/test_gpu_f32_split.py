@@ -249,6 +249,33 @@ def test_backward_values_that_are_not_finite(gpu, monkeypatch):
                     assert np.max(np.abs(a[h][fin] - b[h][fin])) <= 1e-5 * max(np.max(np.abs(b[h][fin])), 1), (name, x, h)
 
 
+@pytest.mark.parametrize("what", ["go", "go column", "q", "k", "v", "go and v", "go and q"])
+@pytest.mark.parametrize("exponent", [-104, -112, -118, -122])
+def test_backward_values_whose_last_bits_no_part_holds(gpu, what, exponent):
+    """As forward: dO below 2^-110, a column of it, Q or K as small under the other as large, V under such a dO, and two ordinary operands whose product is that
+    small.  Gradients, each column, within 3e-6 of 64 bits (the IEEE products: 1.3e-6) where they are not below f32's normal range."""
+    q, k, v, go, _, _ = bwd_case((3, 16, 16, 129, 127, 64, 64, False, None, None))
+    small, large, half = np.float32(2.0 ** exponent), np.float32(2.0 ** -exponent), np.float32(2.0 ** (exponent // 2))
+    if what == "go":
+        go *= small
+    elif what == "go column":
+        go[..., 3] *= small
+    elif what in "qk":
+        q, k = (q * small, k * large) if what == "q" else (q * large, k * small)
+    elif what == "v":
+        v, go = v * small, go * large
+    elif what == "go and v":
+        go, v = go * half, v * half
+    else:
+        go, q, k = go * half, q * half, k / half
+    _, *got = host.sdpa_backward(q, k, v, go, capi.F32)
+    for name, a, r in zip(("dq", "dk", "dv"), got, f64_gradients(q, k, v, go, False, None, None)):
+        norm = np.linalg.norm(r, axis=2)
+        normal = norm / np.sqrt(r.shape[2]) >= 2.0 ** -125
+        off = np.linalg.norm(a - r, axis=2) / norm
+        assert not normal.any() or np.max(off[normal]) <= 3e-6, name
+
+
 def test_backward_hidden_blocks_may_hold_anything(gpu):
     """A NaN in a row of dO or K reaches the gradients of what sees it, by blocks of 32 x 32, and no other: the causal flag, and the same mask as a
     tensor, whose hidden blocks lie inside the range that the walk trims to."""
