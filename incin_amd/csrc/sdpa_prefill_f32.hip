@@ -175,7 +175,7 @@ void sdpa_prefill_f32_kernel(SdpaParams p, int pairs)
             }
     }
     const float* mrow = nullptr;          // this lane's row of the dense mask
-    if (DENSE) mrow = (const float*)p.mask + (int64_t)b * p.m_sb + (int64_t)hq * p.m_sh + (int64_t)min(my_i, Sq - 1) * p.m_si;
+    if (DENSE) mrow = (const float*)p.mask + (int64_t)b * p.m_sb + (int64_t)hq * p.m_sh + (int64_t)min(my_i, rows_b - 1) * p.m_si;
     const bool m_vec = DENSE && p.m_sj == 1 && ((p.m_sb | p.m_sh | p.m_si) & 3) == 0 && (reinterpret_cast<uintptr_t>(p.mask) & 15u) == 0;
     const int flag_shift = own * 4 + rs * 2;
 
@@ -190,7 +190,7 @@ void sdpa_prefill_f32_kernel(SdpaParams p, int pairs)
         // ---- Q' into operands, through the place of the second V tile; the first K and V tiles ----
         {
             Tile xq;
-            xq.fetch_any(qp, p.q_ss, p.D, Sq, q0, tid);
+            xq.fetch_any(qp, p.q_ss, p.D, rows_b, q0, tid);      // (padding rows may hold anything, what starts EXACT among it: the last row in their place)
             xk.fetch(kp, p.k_ss, p.D, j_end, t * KT, tid);
             xv.fetch(vp, p.v_ss, p.Dv, j_end, t * KT, tid);
 #pragma unroll

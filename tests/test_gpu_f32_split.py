@@ -74,6 +74,25 @@ def test_hidden_blocks_may_hold_anything(gpu, D, how):
     assert np.nanmax(np.abs(got - want)) <= 1e-5
 
 
+@pytest.mark.parametrize("D", [64, 96])
+@pytest.mark.parametrize("bias", [False, True])
+def test_padding_rows_may_hold_anything(gpu, D, bias):
+    """NaN in the query rows behind a sequence's count, and in their mask rows, changes no bit of the rows before it: a block that is partly filled does not go
+    through its keys a second time for them (the second walk's products, and so its last bits, are others)."""
+    q, k, v = inputs(31, 3, 4, 200, 200, D)
+    lens = np.array([100, 137, 64], np.int32)
+    mask = np.random.Generator(np.random.PCG64(4)).standard_normal((3, 4, 200, 200), dtype=np.float32) if bias else None
+    run = lambda: host.sdpa(q, k, v, capi.F32, impl=capi.IMPL_MFMA, kv_lens=lens, q_lens=lens, mask=mask)
+    clean = run()
+    for b, n in enumerate(lens):
+        q[b, :, n:] = np.nan
+        if bias:
+            mask[b, :, n:] = np.nan
+    got = run()
+    for b, n in enumerate(lens):
+        assert np.isfinite(clean[b, :, :n]).all() and np.array_equal(got[b, :, :n], clean[b, :, :n])
+
+
 @pytest.mark.parametrize("exponent", [-60, -20, 20, 60, 120])
 def test_values_of_any_size(gpu, exponent):
     """Values far from 1 keep their 24 bits: Q large where K is small, V of any size; and values that round to infinity in bf16."""
