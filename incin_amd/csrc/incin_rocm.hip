@@ -121,6 +121,7 @@ struct Plan {
     size_t lims_offset;      // dense mask on the prefill kernels: where the mask's row limits start in the workspace (0: none)
     bool lims_splitkv;       // f32 with a dense mask: the blocks whose rows all have a limit go through the f32 split-KV kernel first
     bool rows64;             // f32: an unsplit launch of the split-KV form goes 64 rows per workgroup (sdpa_prefill_f32.hip)
+    bool rows64_unsplit;     // f32: the keys are split; without the workspace for that the launch goes unsplit, 64 rows per workgroup
     bool empty;      // nothing to compute
 };
 
@@ -192,24 +193,31 @@ int decode_deal_workgroups(const incin_rocm_sdpa_desc_t* d, int64_t R, int64_t d
 // Whether an f32 launch whose keys are not split is over sooner with 64 rows of a query head per workgroup (sdpa_prefill_f32.hip) than with 32 rows of a
 // KV head (sdpa_decode_f32.hip).  The former is the one for launches that fill the device, its matrix instructions being the faster ones; the latter's
 // workgroups are half as large and walk a quarter of the keys per wavefront, so a launch that leaves compute units idle ends sooner, and
-// they are the fuller ones where 64 divides the positions badly.  By
-// the 64-row workgroups of the launch against compute units (two on one up to head dimension 64, else one) - measured on 2 - 96 heads x 65 -
-// 2048 positions, us, split-KV / prefill: D = 64, causal, 256 workgroups 28.1 / 35.8 (16 heads x 1024), 18.4 / 21.2 (32 x 512), 384 43.9 / 36.6 (24 x
-// 1024), 35.4 / 28.7 (32 x 768), 29.5 / 21.5 (48 x 512), but over at most 256 positions from 144 workgroups on 13.5 / 11.7 (48 x 192), 13.6 /
+// they are the fuller ones where 64 divides the positions badly.  By the blocks of 64 rows and the chunks of 32 against compute units (of blocks two are on one up to
+// head dimension 64, else one; of chunks always two) - measured on 2 - 96 heads x 65 - 2048 positions, us, split-KV / prefill: D = 64, causal, 256 blocks 28.1 / 35.8 (16 heads x
+// 1024), 18.4 / 21.2 (32 x 512), 384 43.9 / 36.6 (24 x 1024), 35.4 / 28.7 (32 x 768), 29.5 / 21.5 (48 x 512), but over at most 256 positions from 144 blocks on 13.5 / 11.7 (48 x 192), 13.6 /
 // 13.4 (48 x 256); nothing masked, 128 14.7 / 20.3 (8 x 512), 30.5 / 34.9 (8 x 1024), 144 19.6 / 17.1 (24 x 384), 192 24.0 / 21.0 (24 x 512), 256 41.5 / 36.5 (16 x 1024),
 // 512 76.9 / 54.6.  D = 80, causal, 256 38.3 / 49.3, 384 56.2 / 49.6, 512 70.3 / 58.0; nothing masked, 144 26.5 / 23.0, 256 59.1 / 50.5, but where a
 // second round of them is not nearly full 288 66.4 / 74.2, 384 85.9 / 94.9, 576 107.5 / 110.9.  D = 128, causal, 256 49.0 / 62.8, 384 71.9 / 62.9, 512
 // 89.6 / 73.8; nothing masked, 192 42.4 / 35.4, 288 85.2 / 95.0, 512 144.2 / 125.2, 768 207.7 / 186.4.
-// 48 positions over 300 keys, causal, 256 workgroups 20.2 / 16.7; 64 over 256, 1024 workgroups 65 / 41.
+// 48 positions over 300 keys, causal, 256 blocks 20.2 / 16.7; 64 over 256, 1024 blocks 65 / 41.
+//   Chunks that have a compute unit each while nobody splits the keys: 48 x 143 over 402 15.5 / 18.9, 80 x 65 over 314 13.0 / 15.5, 48 x 152 over 301 x 80 15.1 / 21.3.
+//   Where 64 divides the positions badly (1.5 chunks a block), D up to 64: one round of chunks, but two of blocks on a compute unit, 272 blocks 42 / 51 (136 x 78 over
+// 1045), 288 61.9 / 76.4, causal 32.5 / 37.0, 63 / 72, 98 / 114; more of them are ahead, 576 43.6 / 42.6, 1344 94 / 87.  Above: all rounds, 288 causal 82.9 / 136, 384 121.7 / 158,
+// 658 191 / 223, 920 23.8 / 31.0, nothing masked 624 31 / 45, 1704 253 / 290.
+//   D above 64, causal: up to a third more blocks than compute units 280 29.6 / 33.1, 288 42 / 54, 320 66.5 / 74.3, 336 76.9 / 77.8, 340 53 / 51.5, 360 37.1 / 34.3; over a long key
+// axis blocks under a causal mask are as long as each other, 360 (310 positions over 891) 69 / 81, 348 (176 over 2765) 230 / 237, 384 149 / 166, 576 86.7 / 89.4, but 396 374 / 276, 432 167 / 146, 590 957 / 796, 960 137 / 126.
 bool f32_rows64_ahead(const incin_rocm_sdpa_desc_t* d, int64_t d_pad, bool uneven)
 {
-    const int64_t G = d->Hq / d->Hkv;
-    if (d_pad > 128 || 3 * G * ((d->Sq + 63) / 64 * 64) > 4 * ((G * d->Sq + 31) / 32 * 32)) return false;
-    const int64_t cus = compute_units_of(d->device), wgs = d->B * d->Hq * ((d->Sq + 63) / 64);
+    const int64_t cus = compute_units_of(d->device), wgs = d->B * d->Hq * ((d->Sq + 63) / 64), chunks = d->B * d->Hkv * ((d->Hq / d->Hkv * d->Sq + 31) / 32);
+    if (d_pad > 128 || 3 * wgs > 2 * chunks) return false;
+    if (chunks <= cus && (d->Skv < 512 || d->num_splits == 1 || d->add_mask)) return false;
+    if (wgs > cus && (d_pad == 64 ? chunks <= 2 * cus : 7 * wgs > 4 * chunks)) return false;
     if (d_pad == 64) return uneven ? wgs > cus || (d->Sq <= 256 && 2 * wgs > cus) : 2 * wgs > cus;
-    if (uneven) return wgs > cus;
+    if (uneven && 2 * d->Skv < 5 * d->Sq) return 3 * wgs > 4 * cus;
+    if (uneven && wgs <= cus) return false;
     const int64_t rounds = (wgs + cus - 1) / cus;
-    return 2 * wgs > cus && (rounds == 1 || rounds > 4 || 5 * wgs >= 4 * cus * rounds);
+    return 2 * wgs > cus && (rounds == 1 || rounds > 4 || (uneven ? 25 * wgs >= 19 * cus * rounds : 5 * wgs >= 4 * cus * rounds));
 }
 
 int make_plan(const incin_rocm_sdpa_desc_t* d, Plan* plan)
@@ -230,7 +238,7 @@ int make_plan(const incin_rocm_sdpa_desc_t* d, Plan* plan)
     plan->deal_bytes = 0;
     plan->lims_offset = 0;
     plan->lims_splitkv = false;
-    plan->rows64 = false;
+    plan->rows64 = plan->rows64_unsplit = false;
     plan->empty = (d->B == 0 || d->Hq == 0 || d->Sq == 0 || d->Dv == 0);
     if (plan->empty) return 0;
     if (d->Hkv <= 0 || d->Hq % d->Hkv != 0)
@@ -333,7 +341,7 @@ int make_plan(const incin_rocm_sdpa_desc_t* d, Plan* plan)
                  (R >= 2 || d->Skv >= (d_pad == 64 ? 1024 : 512)))
             impl = INCIN_ROCM_IMPL_SPLITKV_MFMA;
         // f32 prefill launches of at most two 128-row blocks per compute unit: whichever of the two forms is over sooner
-        // (f32_rows64_ahead, below).  Larger ones go 64 rows per workgroup, 1.2 - 1.5 times ahead of 32.
+        // (f32_rows64_ahead, above).  Larger ones go 64 rows per workgroup, 1.2 - 1.5 times ahead of 32.
         // Not the chunks of a long prompt, where the prefill kernel splits the keys itself (below).
         else if (d->dtype == INCIN_ROCM_F32 && split_mfma_ok && d->Sq > 64 && !(d->Skv >= 4096 && d->Skv >= 4 * d->Sq) &&
                  d->B * d->Hq * ((d->Sq + 127) / 128) <= 2 * compute_units_of(d->device))
@@ -401,7 +409,6 @@ int make_plan(const incin_rocm_sdpa_desc_t* d, Plan* plan)
         const int64_t groups = d->B * d->Hkv * nchunks;
         int64_t splits = d->num_splits;
         plan->rows64 = d->dtype == INCIN_ROCM_F32 && splits <= 1 && f32_rows64_ahead(d, d_pad, d->causal != 0);
-        if (plan->rows64) splits = 1;
         if (splits == 0) {
             const int64_t cus = compute_units_of(d->device);
             // (from 65536 keys on a split keeps at least 1024: with one or two groups the filling alone would ask for 512 splits of
@@ -410,9 +417,10 @@ int make_plan(const incin_rocm_sdpa_desc_t* d, Plan* plan)
             const int64_t min_len = d->Skv >= 65536 ? 1024 : 256;
             const int64_t max_by_len = d->Skv / min_len > 0 ? d->Skv / min_len : 1;
             const int64_t max_splits = std::min<int64_t>(max_by_len, std::max<int64_t>(1, 4 * cus / groups));
+            auto len_of = [&](int64_t s) { return ((d->Skv + s - 1) / s + 255) / 256 * 256; };
+            auto slots_of = [&](int64_t len) { return cus * incin_rocm::decode_mfma_workgroups_per_cu((int)chunk, len, d->dtype, (int)d_pad); };
             auto fill = [&](int64_t s) {           // (with the split length, and so the count, s really leads to)
-                const int64_t len = ((d->Skv + s - 1) / s + 255) / 256 * 256;
-                const int64_t at_a_time = cus * incin_rocm::decode_mfma_workgroups_per_cu((int)chunk, len, d->dtype, (int)d_pad);
+                const int64_t len = len_of(s), at_a_time = slots_of(len);
                 const int64_t wgs = groups * ((d->Skv + len - 1) / len), rounds = (wgs + at_a_time - 1) / at_a_time;
                 return (double)wgs / (double)(rounds * at_a_time);
             };
@@ -420,7 +428,21 @@ int make_plan(const incin_rocm_sdpa_desc_t* d, Plan* plan)
             for (int64_t s = 1; s <= max_splits; ++s) best = std::max(best, fill(s));
             splits = 1;
             while (splits < max_splits && fill(splits) < 0.98 * best) ++splits;
+            // 64 rows per workgroup do not split the keys.  Where this form would, they have one round of workgroups, each a compute unit to itself and
+            // all keys to walk, and the split ones their rounds of a split's length: level at 0.715 of the keys against those and a hundred for each round
+            // but the first.  Beyond 3072 keys the rounding of a split to 256 no longer costs this form anything, and it is ahead.
+            // Us, split-KV / 64 rows: 160 heads x 64 x 65536 1734 / 1888, 144 on 36 x 43 x 9600 x 80 246 / 397, 48 on 12 x 166 x 2732 (one round) 61 / 85, 88 x 80 x 3845 111 /
+            // 117, 36 x 211 x 918 (one) 29.5 / 33.1, 48 x 145 x 1125 (one) 36.9 / 39.2, 84 x 91 x 2424 causal (one) 61 / 75, 168 x 37 x 9045 x 80 350 / 378; but 8 x 1248 50.6 / 42.2,
+            // 5 x 1773 61.3 / 57.0, 48 x 189 x 1714 64.6 / 55.1, 24 x 407 x 2281 75.1 / 71.5, 80 x 103 x 1645 causal 64.8 / 53.4, 8 x 1034 x 128 77.7 / 65.1.
+            if (plan->rows64 && splits > 1) {
+                const int64_t len = len_of(splits), at_a_time = slots_of(len), wgs = groups * ((d->Skv + len - 1) / len), rounds = (wgs + at_a_time - 1) / at_a_time;
+                if (d->Skv > 3072 || 715 * d->Skv > 1000 * (rounds * (len + 100) - 100)) {
+                    plan->rows64 = false;
+                    plan->rows64_unsplit = true;
+                }
+            }
         }
+        if (plan->rows64) splits = 1;
         int64_t split_len = (d->Skv + splits - 1) / splits;
         split_len = (split_len + 255) / 256 * 256;      // whole rounds of the four wavefronts' blocks of 32 (D = 128) or 64 keys
         splits = (d->Skv + split_len - 1) / split_len;
@@ -861,6 +883,12 @@ static int launch_fwd(const incin_rocm_sdpa_desc_t* desc, const Plan& planned, v
     Plan plan = planned;
     // (a workspace that is enough for the launch by splits, or none where that needs none, is not refused)
     if (plan.deal && !(desc->workspace && desc->workspace_bytes >= plan.deal_bytes && aligned16(desc->workspace))) plan.deal = 0;
+    if (plan.rows64_unsplit && !(desc->workspace && desc->workspace_bytes >= plan.ws_bytes && aligned16(desc->workspace))) {
+        plan.rows64 = true;
+        plan.splits = 1;
+        plan.split_len = (int)desc->Skv;
+        plan.ws_bytes = 0;
+    }
     if (plan.ws_bytes > 0 && !plan.deal) {
         if (!desc->workspace || desc->workspace_bytes < plan.ws_bytes)
             return fail(INCIN_ROCM_EWORKSPACE,
@@ -947,7 +975,8 @@ int incin_rocm_sdpa_fwd_static(const incin_rocm_sdpa_desc_t* desc, void* stream)
         whole.num_splits = 1;
         if (int rc = make_plan(&whole, &plan)) return rc;
     }
-    if (plan.ws_bytes > (size_t)INCIN_ROCM_STATIC_SCRATCH_BYTES)
+    const bool unsplit = plan.rows64_unsplit && plan.ws_bytes > (size_t)INCIN_ROCM_STATIC_SCRATCH_BYTES;      // (launch_fwd has the form without a workspace)
+    if (plan.ws_bytes > (size_t)INCIN_ROCM_STATIC_SCRATCH_BYTES && !unsplit)
         return fail(INCIN_ROCM_EWORKSPACE,
                     "sdpa_fwd_static: this request needs %zu bytes of scratch memory, the static buffer holds %zu "
                     "(fewer splits, or incin_rocm_sdpa_fwd with a workspace of the caller's)",
@@ -957,7 +986,7 @@ int incin_rocm_sdpa_fwd_static(const incin_rocm_sdpa_desc_t* desc, void* stream)
     incin_rocm_sdpa_desc_t d = *desc;
     d.workspace = nullptr;
     d.workspace_bytes = 0;
-    if (plan.ws_bytes > 0) {
+    if (plan.ws_bytes > 0 && !unsplit) {
         if (int rc = use_device(desc->device)) return rc;
         void* scratch = nullptr;
         if (int rc = static_scratch_of(desc->device, &scratch)) return rc;

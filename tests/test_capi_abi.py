@@ -71,6 +71,22 @@ def test_decode_by_whole_sequences_stays_one_launch(B, Hq, Hkv, Skv, D, dealt):
     assert (splits > 1) == dealt and nbytes == (max(by_splits, (512 if D <= 128 and 2 * Hq // Hkv * D <= 1024 else 256) * 2 * (Hq // Hkv) * (D + 2) * 4) if dealt else 0)
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Skv,D,causal,splits", [
+    (1, 160, 160, 64, 65536, 64, 0, 3), (1, 160, 160, 64, 65536, 128, 0, 3), (36, 4, 1, 43, 9600, 80, 0, 2), (22, 4, 4, 80, 3845, 64, 0, 3), (3, 12, 12, 211, 918, 64, 0, 2),
+    (21, 4, 4, 91, 2424, 64, 1, 2), (4, 2, 2, 1248, 1248, 64, 0, 1), (4, 12, 12, 189, 1714, 64, 0, 1), (20, 4, 4, 103, 1645, 64, 1, 1), (2, 4, 4, 1034, 1034, 128, 0, 1),
+], ids=str)
+def test_f32_launches_that_leave_units_idle_split_a_long_key_axis(B, Hq, Hkv, Sq, Skv, D, causal, splits):
+    """f32 launches of at most one block of 64 rows per compute unit: 64 rows per workgroup only where walking all keys is over sooner than the split
+    form's rounds (256 compute units here: no device to ask)."""
+    d = _desc(dtype=capi.F32, B=B, Hq=Hq, Hkv=Hkv, Sq=Sq, Skv=Skv, D=D, Dv=D, causal=causal)
+    for name, h, s in (("q_stride", Hq, Sq), ("k_stride", Hkv, Skv), ("v_stride", Hkv, Skv), ("o_stride", Hq, Sq)):
+        st = getattr(d, name)
+        st[0], st[1], st[2] = h * s * D, s * D, D
+    nbytes, got, impl = _plan(d)
+    assert impl == capi.IMPL_SPLITKV_MFMA and got == splits
+    assert nbytes == (B * Hq * Sq * splits * ((64 if D <= 64 else 128) + 2) * 4 if splits > 1 else 0)
+
+
 def test_dispatch_choices():
     assert _plan(_desc())[2] == capi.IMPL_MFMA
     # f32: the IEEE-f32 matrix-core prefill kernel where the launch gives it more than two 128-row workgroups per compute unit

@@ -74,6 +74,44 @@ def test_hidden_blocks_may_hold_anything(gpu, D, how):
     assert np.nanmax(np.abs(got - want)) <= 1e-5
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Skv,D,causal,rows64", [
+    (48, 1, 1, 143, 402, 64, False, False), (80, 1, 1, 65, 314, 128, False, False), (24, 1, 1, 384, 384, 64, False, True), (48, 1, 1, 192, 192, 64, True, True),
+    (24, 4, 4, 152, 300, 64, True, False), (17, 8, 8, 78, 200, 64, False, False), (24, 8, 8, 92, 200, 64, False, True),
+    (8, 12, 12, 130, 260, 96, True, False), (25, 8, 8, 70, 300, 96, False, False), (8, 4, 4, 568, 568, 80, True, False), (6, 8, 8, 512, 512, 80, True, True),
+    (15, 8, 8, 173, 600, 128, True, False), (11, 6, 6, 350, 900, 128, True, True),
+], ids=str)
+def test_which_launches_take_64_rows_per_workgroup(gpu, B, Hq, Hkv, Sq, Skv, D, causal, rows64):
+    """Both sides of the rule's lines (they were measured on 256 compute units): what AUTO takes gives the bits of the prefill kernel, or others; both are right."""
+    if capi.device_info(0).compute_units != 256:
+        pytest.skip("the lines are by compute units")
+    r = np.random.Generator(np.random.PCG64(Sq + Skv))
+    q, k, v = (r.standard_normal(s, dtype=np.float32) for s in ((B, Hq, Sq, D), (B, Hkv, Skv, D), (B, Hkv, Skv, D)))
+    got, info = host.sdpa(q, k, v, capi.F32, causal=causal, return_info=True)
+    assert info["impl"] == capi.IMPL_SPLITKV_MFMA and info["splits"] == 1
+    ref = host.sdpa(q, k, v, capi.F32, causal=causal, impl=capi.IMPL_MFMA)
+    assert np.array_equal(got, ref) == rows64 and np.max(np.abs(got - ref)) <= 1e-5
+
+
+def test_split_launch_without_a_workspace(gpu):
+    """An f32 launch whose keys the planner splits runs without a workspace too, unsplit and 64 rows per workgroup - and so where its partial results exceed
+    the static buffer."""
+    for B, Hq, Hkv, Sq, Skv, D, fits in ((36, 4, 1, 43, 4096, 32, True), (18, 8, 8, 64, 5120, 128, True), (18, 8, 8, 64, 5120, 128, False)):
+        r = np.random.Generator(np.random.PCG64(17))
+        q, k, v = (r.standard_normal(s, dtype=np.float32) for s in ((B, Hq, Sq, D), (B, Hkv, Skv, D), (B, Hkv, Skv, D)))
+        tq, tk, tv = (host.DeviceTensor.from_f32(x, capi.F32) for x in (q, k, v))
+        to = host.DeviceTensor(q.shape, capi.F32)
+        d = host.make_desc(tq, tk, tv, to)
+        need, splits, _ = capi.sdpa_workspace(d)
+        assert need > 0 and splits > 1
+        if fits:
+            capi.sdpa_fwd(d)
+        else:
+            assert need > capi.STATIC_SCRATCH_BYTES
+            capi.sdpa_fwd_static(d)
+        capi.sync()
+        assert np.array_equal(to.to_f32(), host.sdpa(q, k, v, capi.F32, impl=capi.IMPL_MFMA, num_splits=1))
+
+
 @pytest.mark.parametrize("D", [64, 96])
 @pytest.mark.parametrize("bias", [False, True])
 def test_padding_rows_may_hold_anything(gpu, D, bias):
