@@ -69,11 +69,6 @@ inline bool bwd16_forks(bool narrow, bool causal, int64_t G, int64_t blocks, int
     return causal && parts * blocks <= 2 * cus && dq_blocks <= 4 * cus && w >= (parts > 1 ? 64 : 32);
 }
 
-// Blocks that one launch may have: its work-items along an axis stay below 2^32.  The kernels that hold the items of two or three
-// gradients in one launch pass that with very many small heads where a launch per gradient does not, and are then launched twice or
-// more (in multiples of 8: a block stays on the XCD it would have been on).
-constexpr int64_t max_blocks(int threads) { return (1ll << 32) / threads - 8; }
-
 hipError_t launch_sdpa_bwd_mfma(const SdpaBwdParams& bp, int dtype, hipStream_t stream);
 hipError_t launch_sdpa_bwd_wide(const SdpaBwdParams& bp, int dtype, hipStream_t stream);
 // (of sdpa_bwd_mfma.hip: the row dots, and the sum of the planes of a call with parts_kv > 1 into dK and dV)

@@ -478,14 +478,14 @@ __device__ __forceinline__ void bwd_f32_split_body(const SdpaBwdParams& bp, char
 #endif
 }
 
-// One launch: the dK/dV items, which are the longer ones, then the dQ items.
-template <bool DENSE> __global__ __launch_bounds__(BS_THREADS, 2) void bwd_f32_split_kernel(SdpaBwdParams bp, int n_dkv)
+// One list: the dK/dV items, which are the longer ones, then the dQ items; a launch takes those from `first` on.
+template <bool DENSE> __global__ __launch_bounds__(BS_THREADS, 2) void bwd_f32_split_kernel(SdpaBwdParams bp, int n_dkv, int first)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
     __shared__ __attribute__((aligned(1024))) char smem[BS_LDS];
     __shared__ __attribute__((aligned(16))) float s_stats[2][BS_KT];
     __shared__ int s_vote[6][8];
-    const int id = blockIdx.x;
+    const int id = first + blockIdx.x;
     if (id < n_dkv) bwd_f32_split_body<true, DENSE>(bp, smem, s_stats, s_vote, id);
     else bwd_f32_split_body<false, DENSE>(bp, smem, s_stats, s_vote, id - n_dkv);
 #endif
@@ -499,17 +499,15 @@ hipError_t launch_sdpa_bwd_f32_split(const SdpaBwdParams& bp0, hipStream_t strea
     const int nqb = (p.Sq + BS_OWN - 1) / BS_OWN, nkb = (p.Skv + BS_OWN - 1) / BS_OWN;
     const int64_t n_dq = (int64_t)nqb * p.Hq * p.B, n_dkv = (int64_t)nkb * p.Hkv * p.B;
     work_order(p, 1, nqb);
-    auto launch = [&](int64_t blocks, int64_t n) {
-        if (p.mask) hipLaunchKernelGGL(bwd_f32_split_kernel<true>, dim3((unsigned)blocks), dim3(BS_THREADS), 0, stream, bp, (int)n);
-        else hipLaunchKernelGGL(bwd_f32_split_kernel<false>, dim3((unsigned)blocks), dim3(BS_THREADS), 0, stream, bp, (int)n);
-    };
     if (n_dkv + n_dq > 0x7fffffffLL) return hipErrorInvalidValue;
-    if (n_dkv + n_dq <= max_blocks(BS_THREADS)) launch(n_dkv + n_dq, n_dkv);
-    else {
-        if (n_dkv > 0) launch(n_dkv, n_dkv);
-        if (n_dq > 0) launch(n_dq, 0);
+    hipError_t e = hipSuccess;
+    for (int64_t first = 0; first < n_dkv + n_dq && e == hipSuccess; first += max_blocks(BS_THREADS)) {
+        const dim3 grid((unsigned)min(n_dkv + n_dq - first, max_blocks(BS_THREADS)));
+        if (p.mask) hipLaunchKernelGGL(bwd_f32_split_kernel<true>, grid, dim3(BS_THREADS), 0, stream, bp, (int)n_dkv, (int)first);
+        else hipLaunchKernelGGL(bwd_f32_split_kernel<false>, grid, dim3(BS_THREADS), 0, stream, bp, (int)n_dkv, (int)first);
+        e = hipGetLastError();
     }
-    return hipGetLastError();
+    return e;
 }
 
 }  // namespace incin_rocm

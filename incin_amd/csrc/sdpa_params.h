@@ -61,6 +61,11 @@ __device__ __forceinline__ int causal_limit(int i, int Sq, int Skv) { return i +
 
 __device__ __forceinline__ int clampi(int x, int lo, int hi) { return x < lo ? lo : (x > hi ? hi : x); }
 
+// Blocks that one launch may have: its work-items along an axis stay below 2^32.  Kernels whose items are small, or that hold those of two or
+// three gradients in one launch, pass that with very many small heads, and are then launched twice or
+// more (in multiples of 8: a block stays on the XCD it would have been on).
+constexpr int64_t max_blocks(int threads) { return (1ll << 32) / threads - 8; }
+
 // Where the block flags of (batch b, query head hq) start, and the flags per row of blocks.
 __device__ __forceinline__ const uint8_t* mask_flags_of(const SdpaParams& p, int b, int hq)
 {

@@ -270,3 +270,72 @@ def test_very_many_small_heads(gpu, dt, shape):
         for name, g, r_ in zip(("dq", "dk", "dv"), (dq, dk, dv), BW.sdpa_backward(q[sl], k[sl], v[sl], go[sl], causal=causal)):
             err = float(np.abs(g[sl] - r_).max() / np.abs(r_).max())
             assert err <= TOL[dt], "%s of head (%d, %d): %.3e" % (name, b, h, err)
+
+
+def test_f32_forward_of_more_blocks_than_one_launch_takes(gpu):
+    """129 x 65535 heads of 65 positions, blocks of 64 rows: 16.9 million workgroups of 256, more than 2^32 work-items.  Q, K and V are the same for every
+    head (strides of 0); sampled heads - first, last, around the block at which the second launch starts - against the oracle."""
+    B, H, S, D = 129, 65535, 65, 4
+    say("f32 forward of %d x %d heads" % (B, H))
+    r = np.random.Generator(np.random.PCG64(91))
+    x = [r.standard_normal((1, 1, S, D), dtype=np.float32) for _ in range(3)]
+    ref = O.sdpa(*x)[0, 0]
+    ins = [host.DeviceTensor.from_f32(t, capi.F32) for t in x]
+    out = capi.DeviceBuffer(B * H * S * D * 4)
+    capi.check(capi.load().incin_rocm_memset(0, out.ptr, 0x7f, out.nbytes))
+    d = host.make_desc(*ins, ins[0])
+    d.B, d.Hq, d.Hkv, d.o = B, H, H, out.ptr
+    for name in ("q_stride", "k_stride", "v_stride"):
+        getattr(d, name)[0] = getattr(d, name)[1] = 0
+    d.o_stride[0], d.o_stride[1], d.o_stride[2] = H * S * D, S * D, D
+    need, _, impl = capi.sdpa_workspace(d)
+    assert impl == capi.IMPL_MFMA and need == 0
+    capi.sdpa_fwd(d)
+    capi.sync()
+    raw = np.empty((S, D), np.float32)
+    for h in [0, 1, B * H - 1, B * H // 2] + list(range(2 ** 23 - 12, 2 ** 23 + 4)) + [int(i) for i in r.integers(0, B * H, 200)]:
+        capi.check(capi.load().incin_rocm_memcpy_d2h(0, raw.ctypes.data, out.ptr + h * raw.nbytes, raw.nbytes))
+        assert np.abs(raw - ref).max() <= TOL[capi.F32], h
+    out.free()
+
+
+def test_f32_backward_of_more_key_blocks_than_one_launch_takes(gpu):
+    """33 x 63600 heads of 96 queries over 400 keys: 8.4 million blocks of 128 keys, one workgroup of 512 each, more than 2^32 work-items.  The inputs are
+    the same for every head (strides of 0); sampled heads against the oracle."""
+    from oracle import sdpa_backward as BW
+    B, H, Sq, Skv, D = 33, 63600, 96, 400, 4
+    assert B * H * 4 > 2 ** 23
+    say("f32 backward of %d x %d heads" % (B, H))
+    r = np.random.Generator(np.random.PCG64(92))
+    q, k, v, go = (r.standard_normal((1, 1, n, D), dtype=np.float32) for n in (Sq, Skv, Skv, Sq))
+    ref = [x[0, 0] for x in BW.sdpa_backward(q, k, v, go)]
+    s = (q.astype(np.float64) @ k.astype(np.float64).transpose(0, 1, 3, 2))[0, 0] * host.resolve_scale(None, D)
+    lse = np.log(np.exp(s).sum(-1))
+    tq, tk, tv, to, tg = (host.DeviceTensor.from_f32(x, capi.F32) for x in (q, k, v, O.sdpa(q, k, v), go))
+    tl = capi.DeviceBuffer.from_numpy(np.tile(lse.astype(np.float32), (B * H, 1)))
+    rows = (Sq, Skv, Skv)
+    grads = [capi.DeviceBuffer(B * H * n * D * 4) for n in rows]
+    for g in grads:
+        capi.check(capi.load().incin_rocm_memset(0, g.ptr, 0x7f, g.nbytes))
+    bd = capi.SdpaBwdDesc()
+    bd.fwd = host.make_desc(tq, tk, tv, to, lse=tl)
+    bd.fwd.B, bd.fwd.Hq, bd.fwd.Hkv = B, H, H
+    for name in ("q_stride", "k_stride", "v_stride", "o_stride"):
+        getattr(bd.fwd, name)[0] = getattr(bd.fwd, name)[1] = 0
+    bd.d_o, bd.d_q, bd.d_k, bd.d_v = tg.ptr, *(g.ptr for g in grads)
+    bd.d_o_stride[2] = D
+    for name, n in zip(("d_q", "d_k", "d_v"), rows):
+        st = getattr(bd, name + "_stride")
+        st[0], st[1], st[2] = H * n * D, n * D, D
+    ws = capi.DeviceBuffer(capi.sdpa_bwd_workspace(bd))
+    bd.workspace, bd.workspace_bytes = ws.ptr, ws.nbytes
+    capi.sdpa_bwd(bd)
+    capi.sync()
+    heads = [0, 1, B * H - 1, B * H // 2, B * H // 4] + list(range(2 ** 21 - 4, 2 ** 21 + 4)) + [int(i) for i in r.integers(0, B * H, 100)]
+    for h in heads:
+        for g, n, want, name in zip(grads, rows, ref, ("dq", "dk", "dv")):
+            raw = np.empty((n, D), np.float32)
+            capi.check(capi.load().incin_rocm_memcpy_d2h(0, raw.ctypes.data, g.ptr + h * raw.nbytes, raw.nbytes))
+            assert np.abs(raw - want).max() <= TOL[capi.F32] * np.abs(want).max(), (h, name)
+    for x in grads + [ws, tl]:
+        x.free()
