@@ -42,7 +42,7 @@ namespace incin_rocm {
 // left out (the LDS rows keep the layout of D).
 template <int D, int DC, bool DENSE, bool SPLIT>
 __global__ __launch_bounds__(256, D == 64 ? 2 : 1)
-void sdpa_prefill_f32_kernel(SdpaParams p, int pairs, int first, int total)
+void sdpa_prefill_f32_kernel(SdpaParams p, int paired, int first, int total)
 {
 #if defined(__HIP_DEVICE_COMPILE__)   // the body uses device-only types (buffer descriptors); the host pass needs only the stub
     constexpr int KT = 64, RW = 2, KW = 4 / RW, OWN = 32 * KW;      // keys per tile, wavefronts that share rows, blocks of 32 rows side by side, rows of the workgroup
@@ -67,8 +67,9 @@ void sdpa_prefill_f32_kernel(SdpaParams p, int pairs, int first, int total)
     const int nqb = (Sq + OWN - 1) / OWN;
     const int id = first + blockIdx.x;
     int item = id >> 3;
-    // (one round, two workgroups to a compute unit, blocks of different lengths: the second 32 of an XCD go in reverse, a long one with a short one)
-    if (pairs && ((item >> 5) & 1)) item = 32 + ((total >> 3) - 1 - item);
+    // (one round, two workgroups to a compute unit, blocks of different lengths: behind the first `paired` of an XCD, one for each of its compute units, the
+    // order is reversed, a long one with a short one)
+    if (paired && item >= paired) item = paired + ((total >> 3) - 1 - item);
     const WorkItem wi = work_item_of(p, item * 8 + (id & 7), total, nqb);
     const int gq = wi.gq, bhkv = wi.bhkv;
     const int hkv = bhkv % p.Hkv, b = bhkv / p.Hkv;
@@ -523,13 +524,14 @@ static hipError_t launch_prefill_f32_t(const SdpaParams& p0, hipStream_t stream)
     if (total > 0x7fffffffLL) return hipErrorInvalidValue;
     const bool uneven = p.causal != 0 || p.mask != nullptr;
     work_order(p, D == 64 ? 2 : 1, nqb);
-    const int pairs = D == 64 && uneven && (total & 7) == 0 && total > 256 && total <= 512 ? 1 : 0;
+    const int64_t cus = device_cus();
+    const int paired = D == 64 && uneven && (total & 7) == 0 && total > cus && total <= 2 * cus ? (int)(cus / 8) : 0;
     const bool split = !DENSE && p.num_splits > 1;      // partial results, then the split-KV kernels' combine pass
     hipError_t e = hipSuccess;
     for (int64_t first = 0; first < total && e == hipSuccess; first += max_blocks(256)) {
         const dim3 grid((unsigned)std::min(total - first, max_blocks(256)), split ? (unsigned)p.num_splits : 1u);
         if (split) hipLaunchKernelGGL((sdpa_prefill_f32_kernel<D, DC, false, !DENSE>), grid, dim3(256), 0, stream, p, 0, (int)first, (int)total);
-        else hipLaunchKernelGGL((sdpa_prefill_f32_kernel<D, DC, DENSE, false>), grid, dim3(256), 0, stream, p, pairs, (int)first, (int)total);
+        else hipLaunchKernelGGL((sdpa_prefill_f32_kernel<D, DC, DENSE, false>), grid, dim3(256), 0, stream, p, paired, (int)first, (int)total);
         e = hipGetLastError();
     }
     return split && e == hipSuccess ? launch_sdpa_combine(p, 0, stream) : e;

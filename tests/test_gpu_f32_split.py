@@ -74,6 +74,13 @@ def test_hidden_blocks_may_hold_anything(gpu, D, how):
     assert np.nanmax(np.abs(got - want)) <= 1e-5
 
 
+@pytest.mark.parametrize("B,H,S", [(3, 11, 512), (1, 152, 192), (9, 8, 250), (7, 9, 500), (2, 32, 450)])
+def test_one_round_of_uneven_blocks_is_paired(gpu, B, H, S):
+    """264, 456, 288, 504 and 512 blocks under a causal flag: the part of an XCD's list that goes in reverse is part of it, or all of the second half."""
+    q, k, v = inputs(S, B, H, S, S, 64)
+    assert np.max(np.abs(host.sdpa(q, k, v, capi.F32, causal=True, impl=capi.IMPL_MFMA) - O.sdpa(q, k, v, causal=True))) <= 1e-5
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,Sq,Skv,D,causal,rows64", [
     (48, 1, 1, 143, 402, 64, False, False), (80, 1, 1, 65, 314, 128, False, False), (24, 1, 1, 384, 384, 64, False, True), (48, 1, 1, 192, 192, 64, True, True),
     (24, 4, 4, 152, 300, 64, True, False), (17, 8, 8, 78, 200, 64, False, False), (24, 8, 8, 92, 200, 64, False, True),
