@@ -242,7 +242,8 @@ __device__ __forceinline__ void bwd_f32_split_body(const SdpaBwdParams& bp, char
 #pragma unroll
                         for (int r = 0; r < 16; ++r) mv[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, at, (8 * (r / 4) + (r % 4)) * row4, 0));
                     } else {
-                        const float* mrow = (const float*)p.mask + (int64_t)b * p.m_sb + (int64_t)hq * p.m_sh + (int64_t)min(mine, Sq - 1) * p.m_si;
+                        // (padding rows may hold anything, what starts EXACT among it: the last row in their place, as in Q' and dO)
+                        const float* mrow = (const float*)p.mask + (int64_t)b * p.m_sb + (int64_t)hq * p.m_sh + (int64_t)min(mine, rows_b - 1) * p.m_si;
                         const bool vec = p.m_sj == 1 && ((p.m_sb | p.m_sh | p.m_si) & 3) == 0 && (reinterpret_cast<uintptr_t>(p.mask) & 15u) == 0;
                         if (vec && i0 + 32 <= Skv) {
 #pragma unroll

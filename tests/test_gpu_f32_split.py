@@ -354,3 +354,18 @@ def test_backward_hidden_blocks_may_hold_anything(gpu):
         assert np.isnan(dv[1, :, blocks == 2, 3]).any() and np.isnan(dq[0, :, blocks == 7]).any()
         for name, got, ref, clean in (("dk", dk[1], rdk[1], blocks > 2), ("dv", dv[1], rdv[1], blocks > 2), ("dq", dq[0], rdq[0], blocks < 6)):
             assert np.max(np.abs(got[:, clean] - ref[:, clean])) <= 1e-5 * np.max(np.abs(ref)), (name, kw)
+
+
+def test_backward_padding_rows_may_hold_anything(gpu):
+    """NaN in the query rows behind a sequence's count - Q, dO, O, the row normalisers and the mask - changes no bit of any gradient: no block is done over for
+    them."""
+    B, H, S = 4, 16, 160
+    q, k, v, go, _, _ = bwd_case((B, H, H, S, S, 64, 64, False, None, None))
+    lens = np.array([100, 137, 64, 160], np.int32)
+    mask = np.random.Generator(np.random.PCG64(6)).standard_normal((B, H, S, S), dtype=np.float32)
+    run = lambda: host.sdpa_backward(q, k, v, go, capi.F32, q_lens=lens, mask=mask, poison_padding=True)[1:]
+    clean = run()
+    for b, n in enumerate(lens):
+        q[b, :, n:] = go[b, :, n:] = mask[b, :, n:] = np.nan
+    for name, a, c in zip(("dq", "dk", "dv"), run(), clean):
+        assert np.isfinite(c).all() and np.array_equal(a, c), name
