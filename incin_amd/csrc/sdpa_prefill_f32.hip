@@ -69,7 +69,7 @@ void sdpa_prefill_f32_kernel(SdpaParams p, int paired, int first, int total)
     int item = id >> 3;
     // (one round, two workgroups to a compute unit, blocks of different lengths: behind the first `paired` of an XCD, one for each of its compute units, the
     // order is reversed, a long one with a short one)
-    if (paired && item >= paired) item = paired + ((total >> 3) - 1 - item);
+    if (D == 64 && paired && item >= paired) item = paired + ((total >> 3) - 1 - item);
     const WorkItem wi = work_item_of(p, item * 8 + (id & 7), total, nqb);
     const int gq = wi.gq, bhkv = wi.bhkv;
     const int hkv = bhkv % p.Hkv, b = bhkv / p.Hkv;
