@@ -40,13 +40,22 @@ template <bool EXACT> __device__ __forceinline__ void split_pair(float a, float 
     m = (__float_as_uint(a) & 0xffffu) | __float_as_uint(b) << 16;
     l = 0;
 }
-template <bool EXACT> __device__ __forceinline__ Split8 split8(const float8v& x)
+// Eight values times c.  (The parts are those of the products before they are rounded: what the first leaves is one fused operation.)
+template <bool EXACT> __device__ __forceinline__ Split8 split8_scaled(const float8v& x, float c)
 {
     Split8 o;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
+        const float x0 = x[2 * i], x1 = x[2 * i + 1], a = x0 * c, b = x1 * c;
         unsigned h, m, l;
-        split_pair<EXACT>(x[2 * i], x[2 * i + 1], h, m, l);
+        if (EXACT) split_pair<true>(a, b, h, m, l);
+        else {
+            auto whole = [](unsigned w) __attribute__((always_inline)) { asm("" : "+v"(w)); return w; };
+            h = whole(pack2<bf16_t>(a, b));
+            const float ra = __builtin_fmaf(x0, c, -__uint_as_float(h << 16)), rb = __builtin_fmaf(x1, c, -__uint_as_float(h & 0xffff0000u));
+            m = whole(pack2<bf16_t>(ra, rb));
+            l = pack2<bf16_t>(ra - __uint_as_float(m << 16), rb - __uint_as_float(m & 0xffff0000u));
+        }
         o.h[i] = h;
         o.m[i] = m;
         o.l[i] = l;
@@ -230,6 +239,18 @@ template <int D, int DC, int ROWS, int THREADS> struct SplitTile {
         State s;
 #pragma unroll
         for (int k = 0; k < STEPS; ++k) put_step<EXACT, BY_K>(k, s, tile, tid);
+    }
+    // All of a thread's values times c.
+    template <bool EXACT, bool BY_K> __device__ __forceinline__ void put_scaled(char* tile, float c, int tid)
+    {
+#pragma unroll
+        for (int i = 0; i < N; ++i) store<BY_K>(tile, split8_scaled<EXACT>(x[i], c), tid, i);
+    }
+    // Whether one of them times c is outside of 2^-100 (zero apart) to 2^60.
+    __device__ __forceinline__ bool scaled_beyond(float c) const
+    {
+        const float low = __uint_as_float((smallest_in(~0u) + 1u) >> 1);      // (zeros only: zero)
+        return !(largest_of(0.0f) * __builtin_fabsf(c) <= 0x1p60f) || (low * __builtin_fabsf(c) < SPLIT_TINY && low * c != 0.0f);
     }
     static __device__ __forceinline__ Split8 rows_operand(const char* at)      // at: this lane's chunk in the first plane
     {

@@ -182,11 +182,9 @@ __device__ __forceinline__ void bwd_f32_split_body(const SdpaBwdParams& bp, char
             const int rows = max(n_own, 1);
             if (KEYS) x.fetch_any(kp, p.k_ss, p.D, rows, o0, tid);
             else x.fetch_any(q_of(hq), p.q_ss, p.D, rows, o0, tid);
-#pragma unroll
-            for (int i = 0; i < BsOwn::N; ++i) x.x[i] *= p.scale * LOG2E;
             // (a score's error by what A loses is negligible under an X up to 2^60, and X itself loses nothing from 2^-100 on)
-            if (!EXACT && (!(x.largest_of(0.0f) <= 0x1p60f) || x.smallest_in(~0u) < smallest_of(SPLIT_TINY))) top_a = INFINITY;
-            x.template put<EXACT, true>(own_x, tid);
+            if (!EXACT && x.scaled_beyond(p.scale * LOG2E)) top_a = INFINITY;
+            x.template put_scaled<EXACT, true>(own_x, p.scale * LOG2E, tid);
             if (KEYS) x.fetch_any(vp, p.v_ss, p.Dv, rows, o0, tid);
             else x.fetch_any(g_of(hq), bp.do_ss, p.Dv, rows, o0, tid);
             if (!EXACT) {

@@ -194,12 +194,10 @@ void sdpa_prefill_f32_kernel(SdpaParams p, int paired, int first, int total)
             xq.fetch_any(qp, p.q_ss, p.D, rows_b, q0, tid);      // (padding rows may hold anything, what starts EXACT among it: the last row in their place)
             xk.fetch(kp, p.k_ss, p.D, j_end, t * KT, tid);
             xv.fetch(vp, p.v_ss, p.Dv, j_end, t * KT, tid);
-#pragma unroll
-            for (int i = 0; i < Tile::N; ++i) xq.x[i] *= p.scale * LOG2E;
             // (a score's error by what K loses is negligible under a Q' up to 2^60, and Q' itself loses nothing from 2^-100 on)
-            if (!EXACT && (!(xq.largest_of(0.0f) <= 0x1p60f) || xq.smallest_in(~0u) < smallest_of(SPLIT_TINY))) top = INFINITY;
+            if (!EXACT && xq.scaled_beyond(p.scale * LOG2E)) top = INFINITY;
             if (!EXACT) top = xv.largest_of(top);
-            xq.template put<EXACT, true>(smem + 2 * Tile::BYTES, tid);
+            xq.template put_scaled<EXACT, true>(smem + 2 * Tile::BYTES, p.scale * LOG2E, tid);
             xk.template put<EXACT, true>(kbuf, tid);
             xv.template put<EXACT, false>(smem + Tile::BYTES, tid);
         }
