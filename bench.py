@@ -31,6 +31,7 @@ from incin_amd import capi, dtypes, host  # noqa: E402
 SEED0 = 20261125
 PEAK_BF16_TFLOPS = 2516.6   # 256 CUs x 2.4 GHz x 4096 dense bf16 FLOP/clk/CU (vendor: 2.5 PFLOP/s)
 PEAK_F32_TFLOPS = 157.3      # dense fp32 matrix peak, vendor figure (256 CUs x 2.4 GHz x 256 FLOP/clk/CU)
+PEAK_F32_SPLIT_TFLOPS = PEAK_BF16_TFLOPS / 6      # f32 values as three bf16 parts: six products of the bf16 instruction for one
 PEAK_HBM_GBS = 8000.0       # HBM3E, vendor figure
 # HBM bytes per launch, from rocprofv3 --pmc runs of this same script, one leg (and where a leg has several shapes on one
 # kernel, one shape) at a time: `rocprofv3 --pmc FETCH_SIZE -- python3 bench.py --only LEG [--shape NAME] --steps 10
@@ -55,12 +56,12 @@ TRAFFIC_KIB = {   # leg/shape/variant: (FETCH_SIZE, WRITE_SIZE)
     "head_dims/decode_d96": (393400, 192), "head_dims/decode_d256": (1048960, 512), "head_dims/prefill_d96_s4096": (206387, 123320),
     "prefill_chunk/bf16_sq128_kv32768/auto": (66326.4 + 16680.5, 33392.9 + 1024), "prefill_chunk/bf16_sq128_kv32768/unsplit": (66199.5, 1024),
     "prefill_chunk/bf16_sq512_kv32768/auto": (67708 + 17448.5, 33677.2 + 4096), "prefill_chunk/bf16_sq512_kv32768/unsplit": (67735.5, 4096),
-    "prefill_chunk/f32_sq128_kv32768/auto": (135368 + 16678.9, 33280 + 2048), "prefill_chunk/f32_sq128_kv32768/unsplit": (132302, 2048),
-    "f32/f32_c1": (186, 32), "f32/f32_c2": (12401, 9216), "f32/f32_large": (756926, 262144),
-    "backward/bf16_d128": (432774 + 451685, 135168 + 262519),          # (dQ kernel with the row dots, dK/dV kernel)
-    "backward/bf16_d64": (371092 + 295714, 139264 + 262144),          # (dQ kernel with the row dots, dK/dV kernel)
-    "backward/f32_d64": (8350 + 25357, 256 + 24576),          # (row dots, one launch of all gradients)
-    "backward/f32_d128": (266270 + 3496110, 4096 + 786432),
+    "prefill_chunk/f32_sq128_kv32768/auto": (135383 + 16679.3, 33281.5 + 2048), "prefill_chunk/f32_sq128_kv32768/unsplit": (132314, 2048),
+    "f32/f32_c1": (186, 32), "f32/f32_c2": (12416.5, 8192), "f32/f32_large": (760007, 262144),
+    "backward/bf16_d128": (435458 + 449479, 135168 + 264590),          # (dQ kernel with the row dots, dK/dV kernel)
+    "backward/bf16_d64": (377781 + 296636, 139264 + 262144),          # (dQ kernel with the row dots, dK/dV kernel)
+    "backward/f32_d64": (8350 + 25674.4, 256 + 24576),          # (row dots, one launch of all gradients)
+    "backward/f32_d128": (266270 + 3504400, 4096 + 786432),
 }
 TRAFFIC_PROFILE = "profiles/fetch_write_size_bench_legs.txt"
 
@@ -265,7 +266,7 @@ def prefill_chunk_leg(steps, warmup, only_shape=None):
         if only_shape is not None and only_shape != "%s_sq%d_kv%d" % (dtypes.NAMES[dt], Sq, Skv):
             continue
         flops = 4.0 * D * Hq * B * (Sq * Skv - Sq * (Sq - 1) / 2.0)
-        peak = PEAK_F32_TFLOPS if dt == capi.F32 else PEAK_BF16_TFLOPS
+        peak = PEAK_F32_SPLIT_TFLOPS if dt == capi.F32 else PEAK_BF16_TFLOPS
         kernel = "sdpa_prefill_f32_kernel<128>" if dt == capi.F32 else "sdpa_prefill_mfma_kernel<bf16,128>"
         entry = {"workload": "%s causal prefill chunk B=%d Hq=%d Hkv=%d S_q=%d over KV=%d D=128" % (dtypes.NAMES[dt], B, Hq, Hkv, Sq, Skv)}
         for name, ns in (("auto", 0), ("unsplit", 1)):
@@ -466,13 +467,14 @@ def backward_leg(steps, warmup, dtype=capi.BF16, B=8, H=16, S=4096, D=128, what=
     flops = 2.5 * causal_flops(B, H, S, S, D)
     for t in (tq.buf, tk.buf, tv.buf, tg.buf, to.buf, tdq.buf, tdk.buf, tdv.buf, lse, ws):
         t.free()
-    peak = PEAK_F32_TFLOPS if dtype == capi.F32 else PEAK_BF16_TFLOPS
+    # (f32: up to head dimension 64 the kernel of three bf16 parts, above the IEEE-f32 instruction's)
+    peak, peak_name = (PEAK_BF16_TFLOPS, "bf16_mfma") if dtype != capi.F32 else (PEAK_F32_SPLIT_TFLOPS, "f32_in_bf16_parts") if D <= 64 else (PEAK_F32_TFLOPS, "fp32_mfma")
     return {"workload": "backward of %s: %s causal B=%d H=%d S=%d D=%d, dQ dK dV from Q K V O dO and the "
                         "forward's row normalisers" % (what, name, B, H, S, D),
             "step": "one incin_rocm_sdpa_bwd call (%s)" % ("row dots, then dQ and dK/dV blocks in one launch" if dtype == capi.F32 else
                                                            "dQ and dK/dV kernels; row dots in the dQ kernel, or in one of their own where those two run side by side"), "dtype": name,
             "metric": "attn bwd TFLOP/s (2.5 x forward FLOPs)", "value": flops / (wall * 1e-3) / 1e12, "unit": "TFLOP/s",
-            "ms_per_step": wall, "steps": steps, "frac_of_%s_mfma_peak" % ("fp32" if dtype == capi.F32 else "bf16"): flops / (wall * 1e-3) / 1e12 / peak,
+            "ms_per_step": wall, "steps": steps, "frac_of_%s_peak" % peak_name: flops / (wall * 1e-3) / 1e12 / peak,
             "traffic": traffic_of("backward/%s_d%d" % (name, D))[0], "traffic_source": TRAFFIC_PROFILE,
             "parity_max_err_rel_to_max_abs_ref": err,
             "parity_sample": "dQ, dK, dV of slice (b=%d, h=%d) against the float64 oracle of the reference's tape gradients" % (b, h)}
@@ -572,7 +574,8 @@ def matrix_rate():
 
 def f32_configs(steps, warmup, with_cpu, threads):
     """BASELINE configs 1 and 2 - f32, the one dtype the reference's operator runs end to end - on the f32
-    matrix-core kernels: absolute TFLOP/s against the fp32 matrix peak, config 2 also with the causal mask handed over
+    matrix-core kernels: absolute TFLOP/s against the peak of the instruction that ran (IEEE-f32, or bf16 at six products
+    for one), config 2 also with the causal mask handed over
     as the explicit [S, S] tensor of 0 / -inf a caller of the reference's operator passes, and the oracle's
     materialising restatement timed on all of config 2 beside it."""
     from oracle import oracle as O
@@ -585,26 +588,30 @@ def f32_configs(steps, warmup, with_cpu, threads):
         wall, ev_mean, ev_med, ev_min = w.time(n, warmup)
         flops = causal_flops(B, H, S, S, D) if causal else 4.0 * D * B * H * S * S
         dur, dur_from = launch_duration(w, ev_mean)
-        kernel = {capi.IMPL_MFMA: "sdpa_prefill_f32_kernel<%d>" % D, capi.IMPL_GENERIC: "sdpa_generic_kernel<float>",
-                  capi.IMPL_SPLITKV_MFMA: "sdpa_prefill_f32_kernel<%d>, or for launches that leave compute units idle sdpa_decode_f32_kernel<%d> "
-                                          "(32 rows per workgroup)" % (D, D)}.get(w.impl, str(w.impl))
+        parity, pinned, prefill = w.parity(), None, w.impl == capi.IMPL_MFMA
+        if not prefill:        # the f32 prefill kernel on the same launch, pinned: the same bits where that is what ran
+            got = w.to.to_f32()
+            w.replan(impl=capi.IMPL_MFMA)
+            wall_p = w.time(n, warmup)[0]
+            prefill = bool(np.array_equal(got, w.to.to_f32()))
+            pinned = {"kernel": "sdpa_prefill_f32_kernel<%d>" % D, "ms_per_step": wall_p,
+                      "value": flops / (wall_p * 1e-3) / 1e12, "unit": "TFLOP/s", "parity_max_abs_err": w.parity()}
+            w.replan()
+        kernel = "sdpa_prefill_f32_kernel<%d>" % D if prefill else "sdpa_decode_f32_kernel<%d> (32 rows per workgroup)" % D
+        peak = PEAK_F32_SPLIT_TFLOPS if prefill else PEAK_F32_TFLOPS
         what = "BASELINE config %s" % key[-1] if key != "f32_large" else "not a BASELINE config (the shape of config 3 in f32: a launch that fills the machine)"
         rec = {"workload": "%s: f32 %s attention fwd B=%d H=%d S_q=S_kv=%d D=%d, %s" %
                            (what, "causal" if causal else "non-causal", B, H, S, D, scale_note),
                "metric": "attn fwd TFLOP/s", "value": flops / (wall * 1e-3) / 1e12, "unit": "TFLOP/s", "dtype": "f32",
                "ms_per_step": wall, "steps": n,
-               "roofline": {"bound": "mfma", "achieved": flops / (dur * 1e-3) / 1e12, "peak": PEAK_F32_TFLOPS, "unit": "TFLOP/s",
-                            "frac": flops / (dur * 1e-3) / 1e12 / PEAK_F32_TFLOPS,
+               "roofline": {"bound": "mfma", "achieved": flops / (dur * 1e-3) / 1e12, "peak": peak, "unit": "TFLOP/s",
+                            "frac": flops / (dur * 1e-3) / 1e12 / peak,
                             "traffic": traffic_of("f32/" + key)[0], "traffic_source": TRAFFIC_PROFILE, "kernel": kernel,
                             "algorithmic_flops_per_launch": flops, "launch_ms_mean": dur, "launch_ms_mean_from": dur_from,
                             "launch_ms_event_pair_mean": ev_mean, "launch_ms_median": ev_med, "launch_ms_min": ev_min},
-               "parity_max_abs_err": w.parity()}
-        if w.impl != capi.IMPL_MFMA:        # the f32 prefill kernel on the same launch, pinned
-            w.replan(impl=capi.IMPL_MFMA)
-            wall_p = w.time(n, warmup)[0]
-            rec["prefill_kernel_pinned"] = {"kernel": "sdpa_prefill_f32_kernel<%d>" % D, "ms_per_step": wall_p,
-                                            "value": flops / (wall_p * 1e-3) / 1e12, "unit": "TFLOP/s", "parity_max_abs_err": w.parity()}
-            w.replan()
+               "parity_max_abs_err": parity}
+        if pinned:
+            rec["prefill_kernel_pinned"] = pinned
         if key == "f32_c2":
             # the same problem with the mask as a tensor: the launch first classifies the tensor by blocks of 32 x 32 (hidden
             # blocks are skipped, zero blocks run unmasked), FLOPs counted as above

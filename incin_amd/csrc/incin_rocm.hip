@@ -463,6 +463,9 @@ int make_plan(const incin_rocm_sdpa_desc_t* d, Plan* plan)
         // (four times the rows or more): the partial results are rows x splits x D floats, and on a square causal launch
         // writing and combining them costs what the splits gain (one sequence, 8 heads, 4096 x 4096: 61 us whole, 64 in
         // two splits, 74 in four).  num_splits > 0 in the descriptor forces a count.
+        // The f32 kernel has 64 rows to a workgroup, and above head dimension 64 a compute unit holds one of them: what is counted here is half of its workgroups, and
+        // a full device comes to two of its rounds, or four.  At 64 that costs nothing (32 on 8 heads x 512 x 16384 in 2 / 4 / 8 splits 408 / 405 / 408 us, 16 heads
+        // 265 / 210 / 210), at 128 up to 8 % (32 on 8 917 / 931 / 966, 16 heads 480 / 489 / 495, 8 on 2 x 1024 x 8192 244 / 248 / 263, 2 x 16 x 128 x 8192 237 / 133 / 140).
         const int64_t cus = compute_units_of(d->device);
         const int64_t wgs = d->B * d->Hq * ((d->Sq + 127) / 128);
         int64_t splits = d->num_splits;

@@ -19,10 +19,10 @@
 // smaller products first, the row statistics added last: gradients are 0.3 - 0.45 of what the IEEE products left off 64 bits (2-norm, 24 heads x 600,
 // D = 64: 1.24e-6 -> 4.2e-7).
 //
-// What bounds it: the matrix instructions of a block (96 for keys, 72 for queries; pipes busy 46 % of the time) under the clock the device keeps with
-// them, and waits for LDS and barriers (38 % of wavefront time; both wavefronts of a SIMD belong to one workgroup).
-// Measured, backward call with the row statistics, us, IEEE products / so: 32 heads x 1024 causal 144 / 99, nothing masked 243 / 158, 96 x 2048 causal 1487 / 967, 96 x
-// 512 194 / 136, 96 x 128 27 / 21, 32 x 1000 with a bias per head under a causal mask as a tensor 230 / 128.
+// What bounds it: the matrix instructions of a block (96 for keys, 72 for queries; 32 heads x 1024 causal, pipes busy for 48 % of the time in which a compute unit has work) under
+// the clock the device keeps with them, and waits for LDS and barriers (36 % of wavefront time; both wavefronts of a SIMD belong to one workgroup).
+// Measured, backward call with the row statistics, us, IEEE products / so: 32 heads x 1024 causal 144 / 96, nothing masked 242 / 156, 96 x 2048 causal 1486 / 965, 96 x
+// 512 133 / 94, 96 x 128 26.5 / 19.9, 32 x 1000 with a bias per head under a causal mask, as a tensor, 163 / 114.
 #include <type_traits>
 
 #include "f32_split.h"

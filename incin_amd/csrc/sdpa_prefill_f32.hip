@@ -17,12 +17,15 @@
 //   O += V(t) P(t), between its products K(t + 2) and V(t + 1) into LDS, K(t + 3) and V(t + 2) asked for | barrier
 //
 // What bounds it: the 48 matrix instructions of a 32 x 32 block at D = 64 (1536 cycles) and the clock the device keeps under them (about 2.0 GHz with
-// N(0,1) data), then the 360 vector instructions beside them, half of which split K and V.  Without those (results wrong) 4 x 8 x 1024, nothing masked,
-// takes 42 us instead of 55; without any 39.  At D > 64 a workgroup has its compute unit to itself (422 registers, 144 KiB of LDS).
+// N(0,1) data), then the vector instructions beside them, ten to one of those, of which half split K and V: under a causal flag, 4 x 8 x 1024 x 64, the matrix pipes are busy for
+// 37 % of the time in which a compute unit has work, wavefronts wait for 19 % of theirs and for their turn to issue for 33 %.  At D > 64 a workgroup has its
+// compute unit to itself (434 registers, 144 KiB of LDS).  The instance for mask tensors at D = 64 keeps 11 registers in scratch (48 bytes a lane, 5.6 MB written
+// beside 8.4 MB of O in that launch); the others have none.
 // Measured, forward, us, IEEE-f32 products (the kernel of 128 rows, or that of 32 for launches it was ahead on) / so: 4 x 8 x 1024 x 64 causal 50.4 /
-// 37.6, nothing masked 77.4 / 55.3, 8 x 12 x 2048 x 64 822 / 585, 4 x 12 x 2000 x 64 causal 243 / 166, 8 on 2 x 256 over 8192 keys 85 / 40; 4 x 8 x
-// 1024 x 128 causal 90 / 74, 8 x 12 x 2048 x 128 causal 876 / 780, 4 x 8 x 1024 x 80 causal 70 / 57; the causal mask as a tensor, 4 x 8 x 1024 x 64, with the pass over
-// it 60.1 / 43.8.  Its error against 64 bits is 0.5 - 0.6 of what it was (2-norm, 4 x 8 x 1024 x 64 3.4e-7 -> 2.0e-7, 8 x 12 x 2048 x 64 8.4e-7 -> 2.6e-7, 4 x 8 x 1024 x
+// 37.1, nothing masked 77.5 / 54.8, 8 x 12 x 2048 x 64 822 / 586, 4 x 12 x 2000 x 64 causal 244 / 166, 8 on 2 x 256 over 8192 keys 85 / 41; 4 x 8 x
+// 1024 x 128 causal 90 / 76, 8 x 12 x 2048 x 128 causal 876 / 793, 4 x 8 x 1024 x 80 causal 70 / 60; the causal mask as a tensor, 4 x 8 x 1024 x 64, with the pass over
+// it 58.4 / 43.2.  The looks at sizes that decide about a second walk (f32_split.h) are 1 - 3 % of these.  Its error against 64 bits is 0.5 - 0.6 of what it was (2-norm, 4 x 8 x
+// 1024 x 64 3.4e-7 -> 2.0e-7, 8 x 12 x 2048 x 64 8.4e-7 -> 2.6e-7, 4 x 8 x 1024 x
 // 128 causal 2.3e-7 -> 1.3e-7): sums are rounded at their own size once per product of leading parts, the smaller products meet apart.
 //
 // A dense additive mask comes with one flag per block of 32 rows x 32 keys (mask_blocks.hip): blocks the mask hides

@@ -89,9 +89,9 @@ def test_f32_launches_that_leave_units_idle_split_a_long_key_axis(B, Hq, Hkv, Sq
 
 def test_dispatch_choices():
     assert _plan(_desc())[2] == capi.IMPL_MFMA
-    # f32: the IEEE-f32 matrix-core prefill kernel where the launch gives it more than two 128-row workgroups per compute unit
-    # (256 compute units here: no device to ask), the f32 split-KV kernel - 32 rows per workgroup, keys dealt to its wavefronts,
-    # two workgroups per compute unit - up to that
+    # f32: the matrix-core prefill kernel where the launch has more than two 128-row blocks per compute unit (256 compute units
+    # here: no device to ask); up to that the plan names the f32 split-KV form - 32 rows per workgroup, keys dealt to its
+    # wavefronts - and launches whose 64-row blocks fill the device run in the prefill kernel all the same
     assert _plan(_desc(dtype=capi.F32, B=8, Hq=16, Sq=4096, Skv=4096))[2] == capi.IMPL_MFMA
     assert _plan(_desc(dtype=capi.F32, B=4, Hq=8, Sq=1024, Skv=1024))[2] == capi.IMPL_SPLITKV_MFMA      # 4 x 8 heads x 1024 x 1024: 256 workgroups
     assert _plan(_desc(dtype=capi.F32, B=4, Hq=8, Sq=2048, Skv=2048))[2] == capi.IMPL_SPLITKV_MFMA      # 512
