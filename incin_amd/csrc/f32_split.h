@@ -247,10 +247,21 @@ template <int D, int DC, int ROWS, int THREADS> struct SplitTile {
         for (int i = 0; i < N; ++i) store<BY_K>(tile, split8_scaled<EXACT>(x[i], c), tid, i);
     }
     // Whether one of them times c is outside of 2^-100 (zero apart) to 2^60.
-    __device__ __forceinline__ bool scaled_beyond(float c) const
+    // (`width`: as fetched.  Where no value is zero, one instruction a value)
+    __device__ __forceinline__ bool scaled_beyond(float c, int width, int tid) const
     {
+        float least = INFINITY;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            float of = INFINITY;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) of = __builtin_fminf(of, __builtin_fabsf(x[i][e]));
+            if ((i * THREADS + tid) % CPR * 8 < width) least = __builtin_fminf(least, of);
+        }
+        const float most = largest_of(0.0f) * __builtin_fabsf(c);
+        if (most <= 0x1p60f && least * __builtin_fabsf(c) >= SPLIT_TINY) return false;
         const float low = __uint_as_float((smallest_in(~0u) + 1u) >> 1);      // (zeros only: zero)
-        return !(largest_of(0.0f) * __builtin_fabsf(c) <= 0x1p60f) || (low * __builtin_fabsf(c) < SPLIT_TINY && low * c != 0.0f);
+        return !(most <= 0x1p60f) || (low * __builtin_fabsf(c) < SPLIT_TINY && low * c != 0.0f);
     }
     static __device__ __forceinline__ Split8 rows_operand(const char* at)      // at: this lane's chunk in the first plane
     {

@@ -183,7 +183,7 @@ __device__ __forceinline__ void bwd_f32_split_body(const SdpaBwdParams& bp, char
             if (KEYS) x.fetch_any(kp, p.k_ss, p.D, rows, o0, tid);
             else x.fetch_any(q_of(hq), p.q_ss, p.D, rows, o0, tid);
             // (a score's error by what A loses is negligible under an X up to 2^60, and X itself loses nothing from 2^-100 on)
-            if (!EXACT && x.scaled_beyond(p.scale * LOG2E)) top_a = INFINITY;
+            if (!EXACT && x.scaled_beyond(p.scale * LOG2E, p.D, tid)) top_a = INFINITY;
             x.template put_scaled<EXACT, true>(own_x, p.scale * LOG2E, tid);
             if (KEYS) x.fetch_any(vp, p.v_ss, p.Dv, rows, o0, tid);
             else x.fetch_any(g_of(hq), bp.do_ss, p.Dv, rows, o0, tid);

@@ -198,7 +198,7 @@ void sdpa_prefill_f32_kernel(SdpaParams p, int paired, int first, int total)
             xk.fetch(kp, p.k_ss, p.D, j_end, t * KT, tid);
             xv.fetch(vp, p.v_ss, p.Dv, j_end, t * KT, tid);
             // (a score's error by what K loses is negligible under a Q' up to 2^60, and Q' itself loses nothing from 2^-100 on)
-            if (!EXACT && xq.scaled_beyond(p.scale * LOG2E)) top = INFINITY;
+            if (!EXACT && xq.scaled_beyond(p.scale * LOG2E, p.D, tid)) top = INFINITY;
             if (!EXACT) top = xv.largest_of(top);
             xq.template put_scaled<EXACT, true>(smem + 2 * Tile::BYTES, p.scale * LOG2E, tid);
             xk.template put<EXACT, true>(kbuf, tid);
@@ -405,7 +405,30 @@ void sdpa_prefill_f32_kernel(SdpaParams p, int paired, int first, int total)
         }
         if constexpr (EXACT) return false;
         // A result that is not finite, or one so small that what the parts lose (f32_split.h) could show: of V under the sum of the weights, of the
-        // weights under V.  (The sum is at most 2^8 a key.)
+        // weights under V.  (The sum is at most 2^8 a key.)  First whether all of a lane's are in a range where it could not, or zeros that no tiny V explains:
+        // two instructions for two values, where the precise look takes five, and a workgroup meets its instructions for the first time here.
+        {
+            float hi = 0.0f, lo = INFINITY;
+            auto take = [&](float x) __attribute__((always_inline)) {
+                hi = __builtin_elementwise_maximum(hi, __builtin_fabsf(x));      // (keeps a NaN)
+                lo = __builtin_fminf(lo, __builtin_fabsf(x));
+            };
+#pragma unroll
+            for (int db = 0; db < NDB; ++db)
+#pragma unroll
+                for (int r4 = 0; r4 < 4; ++r4) {
+                    if (DC < 128 && db * 32 + r4 * 8 >= p.Dv) continue;      // (uniform: columns of padding, zeros)
+                    if (DC < 128) asm volatile("");
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) take(o_acc[db][r4 * 4 + e]);
+                }
+            const bool fine = hi < INFINITY && l_run < INFINITY && (lo >= 0x1p-40f || hi == 0.0f) && top <= 0x1p50f && n_tiles - t_first <= (1 << 20) / KT;
+            const bool wave_fine = __builtin_amdgcn_ballot_w64(!fine) == 0 && __builtin_amdgcn_ballot_w64(top >= SPLIT_TINY) != 0;
+            if (lane == 0) s_vote[wave] = wave_fine ? 1 : 0;
+            lds_barrier();
+            if ((s_vote[0] & s_vote[1] & s_vote[2] & s_vote[3]) != 0) return false;      // (uniform)
+            lds_barrier();
+        }
         float chk = l_run * 0.0f;
         unsigned low = ~0u;
 #pragma unroll

@@ -178,6 +178,23 @@ def test_values_whose_last_bits_no_part_holds(gpu, D, splits, what, exponent):
     assert np.max(off) <= 1e-6
 
 
+@pytest.mark.parametrize("D,Dv", [(64, 64), (40, 36), (80, 68), (128, 100)])
+@pytest.mark.parametrize("what", ["small", "large", "zeros"])
+def test_results_at_the_ends_of_the_range_that_is_taken_at_once(gpu, D, Dv, what):
+    """Results of 2^-50 to 2^-30, V of 2^45 to 2^55, and a V of zeros but for one value too small for three parts; with and without columns of padding: each column
+    within 1e-6 of 64 bits, as above, and zeros where V is zero."""
+    q, k, v = inputs(23, 1, 2, 70, 100, D)
+    v = v[..., :Dv].copy()
+    if what == "zeros":
+        v[:] = 0.0
+        v[..., 7, 3] = np.float32(1.37 * 2.0 ** -118)
+    else:
+        v *= (2.0 ** (np.linspace(-50, -30, Dv) if what == "small" else np.linspace(45, 55, Dv))).astype(np.float32)
+    got, ref = host.sdpa(q, k, v, capi.F32, impl=capi.IMPL_MFMA), exact(q, k, v)
+    norm = np.linalg.norm(ref, axis=2)
+    assert np.max(np.linalg.norm(got - ref, axis=2)[norm > 0] / norm[norm > 0]) <= 1e-6 and np.all(got[ref == 0] == 0)
+
+
 def test_small_weights_of_large_values(gpu):
     """A weight of 2^-121.5 whose value is 2^120 and makes up the result: what scores of that size leave (2^-23 of them, in the exponent)."""
     q, k, v = inputs(22, 1, 2, 40, 200, 64)
