@@ -207,15 +207,19 @@ int decode_deal_workgroups(const incin_rocm_sdpa_desc_t* d, int64_t R, int64_t d
 // 658 191 / 223, 920 23.8 / 31.0, nothing masked 624 31 / 45, 1704 253 / 290.
 //   D above 64, causal: up to a third more blocks than compute units 280 29.6 / 33.1, 288 42 / 54, 320 66.5 / 74.3, 336 76.9 / 77.8, 340 53 / 51.5, 360 37.1 / 34.3; over a long key
 // axis blocks under a causal mask are as long as each other, 360 (310 positions over 891) 69 / 81, 348 (176 over 2765) 230 / 237, 384 149 / 166, 576 86.7 / 89.4, but 396 374 / 276, 432 167 / 146, 590 957 / 796, 960 137 / 126.
+//   A mask tensor costs the other form a launch more, whatever it holds, so none of these lines there: its row limits / values, 32 heads x 568 x 128 46.6 / 44.1, 56.0 / 52.1, 36 x 518 x
+// 80 38.9 / 35.6, 55.5 / 51.5, 96 x 150 17.4 / 16.2, 22.5 / 19.8, 72 x 90 14.2 / 13.7, 18.9 / 16.2; 24 x 695 x 128 47.5 / 50.8, 81 / 77.
 bool f32_rows64_ahead(const incin_rocm_sdpa_desc_t* d, int64_t d_pad, bool uneven)
 {
     const int64_t cus = compute_units_of(d->device), wgs = d->B * d->Hq * ((d->Sq + 63) / 64), chunks = d->B * d->Hkv * ((d->Hq / d->Hkv * d->Sq + 31) / 32);
     if (d_pad > 128 || 3 * wgs > 2 * chunks) return false;
-    if (chunks <= cus && (d->Skv < 512 || d->num_splits == 1 || d->add_mask)) return false;
-    if (wgs > cus && (d_pad == 64 ? chunks <= 2 * cus : 7 * wgs > 4 * chunks)) return false;
+    if (!d->add_mask) {
+        if (chunks <= cus && (d->Skv < 512 || d->num_splits == 1)) return false;
+        if (wgs > cus && (d_pad == 64 ? chunks <= 2 * cus : 7 * wgs > 4 * chunks)) return false;
+    }
     if (d_pad == 64) return uneven ? wgs > cus || (d->Sq <= 256 && 2 * wgs > cus) : 2 * wgs > cus;
+    if (uneven && (wgs <= cus || d->add_mask)) return wgs > cus;
     if (uneven && 2 * d->Skv < 5 * d->Sq) return 3 * wgs > 4 * cus;
-    if (uneven && wgs <= cus) return false;
     const int64_t rounds = (wgs + cus - 1) / cus;
     return 2 * wgs > cus && (rounds == 1 || rounds > 4 || (uneven ? 25 * wgs >= 19 * cus * rounds : 5 * wgs >= 4 * cus * rounds));
 }

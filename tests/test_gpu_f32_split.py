@@ -99,6 +99,18 @@ def test_which_launches_take_64_rows_per_workgroup(gpu, B, Hq, Hkv, Sq, Skv, D, 
     assert np.array_equal(got, ref) == rows64 and np.max(np.abs(got - ref)) <= 1e-5
 
 
+@pytest.mark.parametrize("B,H,S,D", [(8, 4, 568, 128), (12, 8, 144, 64), (6, 8, 150, 64), (1, 8, 300, 64)], ids=str)
+def test_mask_tensors_that_take_64_rows_per_workgroup(gpu, B, H, S, D):
+    """The causal mask as a tensor, on both sides of the lines of the flag (the last one fills no device and goes 32 rows per workgroup): the bits of the prefill kernel
+    under the flag where its blocks take the mask's limits, others elsewhere."""
+    if capi.device_info(0).compute_units != 256:
+        pytest.skip("the lines are by compute units")
+    q, k, v = inputs(S + D, B, H, S, S, D)
+    mask = np.triu(np.full((S, S), -np.inf, np.float32), 1)[None, None]
+    got, flag = host.sdpa(q, k, v, capi.F32, mask=mask), host.sdpa(q, k, v, capi.F32, causal=True, impl=capi.IMPL_MFMA)
+    assert np.array_equal(got, flag) == (B > 1) and np.max(np.abs(got - flag)) <= 1e-5
+
+
 def test_split_launch_without_a_workspace(gpu):
     """An f32 launch whose keys the planner splits runs without a workspace too, unsplit and 64 rows per workgroup - and so where its partial results exceed
     the static buffer."""
