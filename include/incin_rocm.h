@@ -219,7 +219,8 @@ typedef struct {
  * workgroups in equal shares, or so many splits of the capacity for each sequence.  The bytes reported are enough for
  * either, the split count is that of the second.  The first is what runs with the bytes reported; with less, but
  * enough for the second's partial results, incin_rocm_sdpa_fwd runs that one.  The results of the two differ as those of different
- * split counts do, in the last bits. */
+ * split counts do, in the last bits.  Some f32 launches whose keys the library splits (blocks of 64 rows for more than half of the compute
+ * units, at most one each) have a second form too: with less than the bytes reported, or none, they run unsplit. */
 int incin_rocm_sdpa_workspace(const incin_rocm_sdpa_desc_t* desc, size_t* bytes, int32_t* splits, int32_t* impl_out);
 
 /* Enqueues the kernels on `stream` (NULL = the device's default stream) and
