@@ -24,7 +24,7 @@
 // wavefront per SIMD.  The call, causal, against two kernels on two streams with four blocks of 32 side by side in a workgroup: 32
 // heads x 1024, D = 64 214 -> 143 us (106 TFLOP/s of 153 that a large matrix product reaches), 64 x 2048 1129 -> 970, 12 x 501 at 80
 // 159 -> 66, 24 x 79 44 -> 14.  (Head dimensions up to 64 in launches that fill the device go to sdpa_bwd_f32_split.hip: the second of these
-// calls 99, the third 632; the row statistics are computed here for both.)
+// calls 96, the third 632; the row statistics are computed here for both.)
 #include <type_traits>
 
 #include "sdpa_bwd.h"
