@@ -373,7 +373,7 @@ def test_matrix_core_backward_with_padded_head_dimensions(gpu, dtype, dims):
 ], ids=["tiny64", "tiny128_causal", "bench_head", "rect", "gqa_causal128", "gqa_rect_causal", "ragged_causal", "ragged128",
         "negative_scale", "dealt_pairs"])
 def test_matrix_core_backward_f32_against_the_oracle(gpu, shape):
-    """f32 through the IEEE-f32 matrix-core kernels (D = 64 and 128), picked by AUTO and pinned: 1e-5 of the largest
+    """f32 through the f32 matrix-core kernels (D = 64 and 128), picked by AUTO and pinned: 1e-5 of the largest
     gradient magnitude against the f64 oracle, and the generic f32 kernels within the same distance."""
     B, Hq, Hkv, Sq, Skv, D, causal, lens, scale = shape
     G = Hq // Hkv

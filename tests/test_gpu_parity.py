@@ -224,7 +224,7 @@ def test_mfma_prefill(gpu, dtype, shape, impl):
     (2, 3, 3, 1, 70, 128),
 ])
 def test_f32_matrix_core_prefill(gpu, shape):
-    """The IEEE-f32 matrix-core kernel on f32 operands - the reference's own dtype - against the oracle at 1e-5:
+    """The f32 matrix-core prefill kernel on f32 operands - the reference's own dtype - against the oracle at 1e-5:
     no mask, causal, ragged key counts with a causal mask, and dense additive masks of several broadcast shapes."""
     B, Hq, Hkv, Sq, Skv, D = shape
     G = Hq // Hkv
